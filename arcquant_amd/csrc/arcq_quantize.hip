@@ -621,6 +621,7 @@ __global__ __launch_bounds__(1024) void quantize_rows_unit_kernel(QuantParams p)
         ss = __builtin_fma(d0, d0, ss);  // exact squares, fp64 accumulation
         ss = __builtin_fma(d1, d1, ss);
       }
+      if (!active) ss = 0.0;  // a lane without channels (K % 1024 != 0) holds nothing that belongs to the row
       ss = wave_sum_to_lane63(ss);
       if ((tid & 63) == 63) red[tid >> 6] = ss;
       lds_barrier();  // partial sums visible; the previous row's gathers are over

@@ -78,6 +78,14 @@ def test_rmsnorm_quantize_x(agemm, oracle, fmt, M, K, S):
 
 
 @pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("M,K,S", [(2500, 3584, 128), (2100, 96, 32)])
+def test_rmsnorm_quantize_x_partial_last_wave(agemm, oracle, fmt, M, K, S):
+    """K not a multiple of 1024 and several rows per workgroup: the lanes of the last wave that own no channels stay
+    out of every row's sum of squares."""
+    test_rmsnorm_quantize_x(agemm, oracle, fmt, M, K, S)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
 def test_rmsnorm_quantize_x_benchmark_size(agemm, oracle, fmt):
     """The benchmark's launch (4096 x 4096, select_num 256) against the oracle, every row, and the same
     bits from every one of a series of back-to-back launches."""
