@@ -19,6 +19,15 @@ FORMATS = {"NVFP4": NVFP4, "MXFP4": MXFP4}
 _lib = None
 
 
+class GemmArgs(ctypes.Structure):
+    """arcq_gemm_args of include/arcq.h"""
+    _fields_ = [(n, ctypes.c_void_p) for n in ("a_codes", "a_scales", "b_codes", "b_scales")] + \
+               [(n, ctypes.c_int) for n in ("M", "N", "Kp", "fmt")] + [("alpha", ctypes.c_float), ("swiglu", ctypes.c_int)] + \
+               [(n, ctypes.c_void_p) for n in ("d_alpha_a", "d_alpha_b", "residual", "c", "seg_offsets")] + \
+               [("n_seg", ctypes.c_int), ("d_absmax", ctypes.c_void_p), ("workspace", ctypes.c_void_p),
+                ("workspace_bytes", ctypes.c_size_t)]
+
+
 class ArcqError(RuntimeError):
     def __init__(self, status: int, where: str):
         self.status = status
@@ -79,6 +88,10 @@ def lib() -> ctypes.CDLL:
     L.arcq_grouped_matmul_swiglu.argtypes = [vp, vp, vp, vp, vp, i, i, i, i, i, f, vp, vp, vp, vp, vp]
     L.arcq_matmul_swiglu.argtypes = [vp, vp, vp, vp, i, i, i, i, f, vp, vp, vp, vp, vp]
     L.arcq_scales_from_absmax.argtypes = [vp, i, f, vp]
+    L.arcq_gemm.argtypes = [ctypes.POINTER(GemmArgs), vp]
+    L.arcq_gemm.restype = i
+    L.arcq_gemm_workspace_bytes.argtypes = [i, i, i, i, i]
+    L.arcq_gemm_workspace_bytes.restype = sz
     for name in ("arcq_grouped_matmul_swiglu", "arcq_matmul_swiglu", "arcq_scales_from_absmax"):
         getattr(L, name).restype = i
     L.arcq_moe_combine.argtypes = [vp, vp, vp, i, i, i, i, vp, vp]

@@ -210,6 +210,20 @@ def _infer_fmt(A, SFA, fmt):
     raise RuntimeError(f"cannot tell the block format from SFA ({n} scale bytes for {M}x{2 * half} values)")
 
 
+def _gemm(A, SFA, B, SFB, M, N, Kp, f, c, *, alpha=1.0, da=None, db=None, residual=None, swiglu=0, seg=None, n_seg=0,
+          absmax=None):
+    """arcq_gemm with the scratch memory its fastest kernel for the problem takes, from torch's allocator"""
+    L = _lib.lib()
+    nbytes = L.arcq_gemm_workspace_bytes(M, N, Kp, f, n_seg)
+    work = torch.empty(nbytes, dtype=torch.uint8, device=A.device) if nbytes else None
+    args = _lib.GemmArgs(A.data_ptr(), SFA.data_ptr(), B.data_ptr(), SFB.data_ptr(), M, N, Kp, f, alpha, swiglu, da, db,
+                         None if residual is None else residual.data_ptr(), c.data_ptr(),
+                         None if seg is None else seg.data_ptr(), n_seg, None if absmax is None else absmax.data_ptr(),
+                         None if work is None else work.data_ptr(), nbytes)
+    with _on_device(A):
+        _lib.check(L.arcq_gemm(args, _stream(A)), "arcq_gemm")
+
+
 def matmul(A, B, SFA, SFB, scale, *, fmt=None, residual=None):
     """agemm.matmul (kernels/src/bindings.cpp:99-120): bf16 [M,N] = scale * dq(A) @ dq(B)^T.
 
@@ -242,14 +256,18 @@ def matmul(A, B, SFA, SFB, scale, *, fmt=None, residual=None):
         alpha, da, ka = _scalar(scale, A.device)
         db, kb = None, None
     C = torch.empty((M, N), dtype=torch.bfloat16, device=A.device)
+    if residual is not None:
+        _require(residual, "residual", torch.bfloat16, 2)
+        if tuple(residual.shape) != (M, N) or residual.device != A.device:
+            raise RuntimeError(f"residual must be bf16 [{M}, {N}] on A's device")
+    if M > 64:        # beyond the decode batches a kernel may want scratch memory
+        _gemm(A, SFA, B, SFB, M, N, Kp, f, C, alpha=alpha, da=da, db=db, residual=residual)
+        return C
     with _on_device(A):
         if residual is None:
             rc = L.arcq_matmul(A.data_ptr(), SFA.data_ptr(), B.data_ptr(), SFB.data_ptr(), M, N, Kp, f, alpha, da, db,
                                C.data_ptr(), _stream(A))
         else:
-            _require(residual, "residual", torch.bfloat16, 2)
-            if tuple(residual.shape) != (M, N) or residual.device != A.device:
-                raise RuntimeError(f"residual must be bf16 [{M}, {N}] on A's device")
             rc = L.arcq_matmul_add(A.data_ptr(), SFA.data_ptr(), B.data_ptr(), SFB.data_ptr(), M, N, Kp, f, alpha, da,
                                    db, residual.data_ptr(), C.data_ptr(), _stream(A))
     _lib.check(rc, "arcq_matmul")
@@ -380,11 +398,7 @@ def grouped_matmul(A, B, SFA, SFB, seg, scale_a=None, scale_b=None, *, fmt=None,
         if tuple(residual.shape) != (M, N) or residual.device != A.device:
             raise RuntimeError(f"residual must be bf16 [{M}, {N}] on A's device")
     C = torch.empty((M, N), dtype=torch.bfloat16, device=A.device)
-    with _on_device(A):
-        rc = _lib.lib().arcq_grouped_matmul(A.data_ptr(), SFA.data_ptr(), B.data_ptr(), SFB.data_ptr(), seg.data_ptr(), E,
-                                            M, N, Kp, f, 1.0, ptrs[0], ptrs[1],
-                                            None if residual is None else residual.data_ptr(), C.data_ptr(), _stream(A))
-    _lib.check(rc, "arcq_grouped_matmul")
+    _gemm(A, SFA, B, SFB, M, N, Kp, f, C, da=ptrs[0], db=ptrs[1], residual=residual, seg=seg, n_seg=E)
     return C
 
 
@@ -430,10 +444,7 @@ def matmul_swiglu(A, B, SFA, SFB, scale, *, fmt=None, tensor_scale=False):
         db, kb = None, None
     T = torch.empty((M, N // 2), dtype=torch.bfloat16, device=A.device)
     amax = torch.zeros(1, dtype=torch.float32, device=A.device) if tensor_scale else None
-    with _on_device(A):
-        rc = _lib.lib().arcq_matmul_swiglu(A.data_ptr(), SFA.data_ptr(), B.data_ptr(), SFB.data_ptr(), M, N, Kp, f, alpha,
-                                           da, db, T.data_ptr(), None if amax is None else amax.data_ptr(), _stream(A))
-    _lib.check(rc, "arcq_matmul_swiglu")
+    _gemm(A, SFA, B, SFB, M, N, Kp, f, T, alpha=alpha, da=da, db=db, swiglu=1, absmax=amax)
     del ka, kb
     if tensor_scale:
         return T, _absmax_to_scales(amax, 2688.0).reshape(())
@@ -468,11 +479,7 @@ def grouped_matmul_swiglu(A, B, SFA, SFB, seg, scale_a=None, scale_b=None, *, fm
         ptrs.append(t.data_ptr())
     T = torch.empty((M, N // 2), dtype=torch.bfloat16, device=A.device)
     amax = torch.zeros(E, dtype=torch.float32, device=A.device) if tensor_scale else None
-    with _on_device(A):
-        rc = _lib.lib().arcq_grouped_matmul_swiglu(A.data_ptr(), SFA.data_ptr(), B.data_ptr(), SFB.data_ptr(),
-                                                   seg.data_ptr(), E, M, N, Kp, f, 1.0, ptrs[0], ptrs[1], T.data_ptr(),
-                                                   None if amax is None else amax.data_ptr(), _stream(A))
-    _lib.check(rc, "arcq_grouped_matmul_swiglu")
+    _gemm(A, SFA, B, SFB, M, N, Kp, f, T, da=ptrs[0], db=ptrs[1], swiglu=1, seg=seg, n_seg=E, absmax=amax)
     if tensor_scale:
         return T, _absmax_to_scales(amax, 2688.0)
     return T

@@ -2,7 +2,6 @@
 
     python -m arcquant_amd.build            # build if stale
     python -m arcquant_amd.build --force    # rebuild even if up to date
-    python -m arcquant_amd.build --experiments   # with the measured-and-not-taken kernel variants (ARCQ_GEMM_KERNEL)
     python -m arcquant_amd.build --phases KERNEL # instruction counts between the ARCQ_PHASE markers of one kernel
 
 hipcc cross-compiles for gfx950 without a GPU present.  The built libraries live next to the
@@ -17,7 +16,7 @@ import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
-HIP_SOURCES = ["arcq_common.hip", "arcq_quantize.hip", "arcq_gemm.hip", "arcq_kvcache.hip", "arcq_moe.hip"]
+HIP_SOURCES = ["arcq_common.hip", "arcq_quantize.hip", "arcq_gemm.hip", "arcq_gemm_nv.hip", "arcq_kvcache.hip", "arcq_moe.hip"]
 HIP_LIB = os.path.join(CSRC, "libarcq_hip.so")
 # measurement only (plain copy kernels for bench.py and the counter calibration): its own library, so that the
 # product library holds operators only
@@ -47,14 +46,12 @@ def _stale(target: str, deps) -> bool:
     return any(os.path.getmtime(d) > t for d in deps)
 
 
-def build_hip(force: bool = False, verbose: bool = False, experiments: bool = False) -> str:
+def build_hip(force: bool = False, verbose: bool = False) -> str:
     srcs = [os.path.join(CSRC, s) for s in HIP_SOURCES]
-    deps = srcs + [os.path.join(CSRC, h) for h in ("arcq_math.h", "arcq_internal.h", "arcq_swiglu.h")] + [
+    deps = srcs + [os.path.join(CSRC, h) for h in ("arcq_math.h", "arcq_internal.h", "arcq_swiglu.h", "arcq_gemm_tile.h")] + [
         os.path.join(HERE, "..", "include", "arcq.h")]
     if force or _stale(HIP_LIB, deps):
-        # --experiments: also the kernel variants that were measured and not taken (reached only through
-        # ARCQ_GEMM_KERNEL; the counter summaries under profiles/ that name one were made with such a build)
-        cmd = [_hipcc(), *HIPCC_FLAGS, *(["-DARCQ_EXPERIMENTS"] if experiments else []), "-o", HIP_LIB, *srcs]
+        cmd = [_hipcc(), *HIPCC_FLAGS, "-o", HIP_LIB, *srcs]
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.check_call(cmd)
@@ -71,8 +68,8 @@ def build_probe(force: bool = False, verbose: bool = False) -> str:
     return PROBE_LIB
 
 
-def build_all(force: bool = False, verbose: bool = False, experiments: bool = False):
-    return (build_hip(force or experiments, verbose, experiments), build_probe(force, verbose))
+def build_all(force: bool = False, verbose: bool = False):
+    return (build_hip(force, verbose), build_probe(force, verbose))
 
 
 def phase_listing(kernel: str, source: str = "arcq_quantize.hip") -> str:
@@ -130,4 +127,4 @@ if __name__ == "__main__":
     if "--phases" in sys.argv:
         print(phase_listing(sys.argv[sys.argv.index("--phases") + 1]))
         sys.exit(0)
-    print(build_all(force="--force" in sys.argv, verbose=True, experiments="--experiments" in sys.argv))
+    print(build_all(force="--force" in sys.argv, verbose=True))

@@ -16,164 +16,10 @@
 #include <mutex>
 #include <type_traits>
 
-#include "arcq_internal.h"
-#include "arcq_math.h"
-#include "arcq_swiglu.h"
+#include "arcq_gemm_tile.h"
 
 namespace arcq {
 namespace {
-
-typedef int v8i __attribute__((ext_vector_type(8)));
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-
-struct GemmParams {
-  const uint8_t *a_codes, *a_scales;  // activations, M rows
-  const uint8_t *b_codes, *b_scales;  // weights, N rows
-  uint16_t *c;                        // bf16 [M,N]
-  const float *d_alpha_a, *d_alpha_b;
-  float alpha;
-  int M, N, Kp;
-  // split-K (tiled kernels): blockIdx.y selects one of k_slices ranges of K steps and the workgroup
-  // writes its fp32 partial tile to partial[slice][M][N] instead of C; splitk_reduce_kernel adds them
-  float *partial = nullptr;
-  int k_slices = 1;
-  // optional residual, bf16 [M,N]: C = bf16(bf16(alpha * acc) + residual), what a bf16 add of the
-  // rounded GEMM output and the residual gives
-  const uint16_t *residual = nullptr;
-  // grouped GEMM (tiled kernels): rows seg[e] .. seg[e+1]-1 of A and C belong to segment e, whose weights
-  // start seg_b_codes / seg_b_scales bytes after those of segment e-1; d_alpha_a / d_alpha_b are arrays
-  // indexed by segment.  A workgroup rewrites its copy of these parameters to its segment's sub-problem.
-  const int *seg = nullptr;
-  int n_seg = 0;
-  size_t seg_b_codes = 0, seg_b_scales = 0;
-  // fused SwiGLU epilogue (tiled kernels): the weight rows alternate gate, up, gate, up ..., so that output
-  // columns 2j and 2j+1 are gate_j and up_j of one token and sit in one lane; c then is bf16 [M, N/2] and
-  // receives act_fn(gate) * up formed from the bf16-rounded GEMM outputs, exactly what the unfused sequence
-  // (GEMM, then silu and multiply in bf16) gives.  absmax_bits: NULL, or one word per segment (one word when
-  // not grouped) that collects max |output| as the bits of a non-negative float (zeroed by the caller).
-  int swiglu = 0;
-  uint32_t *absmax_bits = nullptr;
-  int seg_index = 0;
-};
-
-// Grouped launches: maps the workgroup to (segment, tile) and turns p into that segment's problem (M = its
-// rows, operand pointers moved to its first row and its weights).  lin: tile number inside the segment, in
-// the order the ungrouped kernels use.  The launch holds an upper bound of the tile count; workgroups
-// beyond the real count return false.  G: elements per scale byte.
-template <int BM, int BN, int G>
-__device__ __forceinline__ bool enter_segment(GemmParams &p, int &lin) {
-  const int tiles_n = (p.N + BN - 1) / BN;
-  const int per_xcd = gridDim.x >> 3;  // the grid is a multiple of 8: contiguous runs of tiles per XCD
-  lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  const int rows = p.M;
-  int beg = min(max(p.seg[0], 0), rows);
-  for (int e = 0; e < p.n_seg; ++e) {
-    const int end = min(max(p.seg[e + 1], beg), rows);  // offsets that do not grow or leave the tensor: empty segments
-    const int cnt = end - beg;
-    const int t = ((cnt + BM - 1) / BM) * tiles_n;
-    if (lin < t) {
-      const size_t kbytes = p.Kp >> 1, ksc = p.Kp / G;
-      p.a_codes += (size_t)beg * kbytes;
-      p.a_scales += (size_t)beg * ksc;
-      p.c += (size_t)beg * (p.swiglu ? p.N >> 1 : p.N);
-      if (p.residual) p.residual += (size_t)beg * p.N;
-      p.b_codes += (size_t)e * p.seg_b_codes;
-      p.b_scales += (size_t)e * p.seg_b_scales;
-      if (p.d_alpha_a) p.d_alpha_a += e;
-      if (p.d_alpha_b) p.d_alpha_b += e;
-      p.M = cnt;
-      p.seg_index = e;
-      return true;
-    }
-    lin -= t;
-    beg = end;
-  }
-  return false;
-}
-
-// two bf16 pairs + two bf16 pairs, each sum rounded to bf16
-__device__ __forceinline__ uint32_t add_bf16_pair(uint32_t a, uint32_t b) {
-  return pack_bf16_rne(u2f(a << 16) + u2f(b << 16), u2f(a & 0xffff0000u) + u2f(b & 0xffff0000u));
-}
-__device__ __forceinline__ uint2 add_bf16_x4(uint2 a, uint2 b) {
-  return make_uint2(add_bf16_pair(a.x, b.x), add_bf16_pair(a.y, b.y));
-}
-
-__device__ __forceinline__ float effective_alpha(const GemmParams &p) {
-  float a = p.alpha;
-  if (p.d_alpha_a && p.d_alpha_b) {
-    a *= (*p.d_alpha_a) * (*p.d_alpha_b);
-  } else if (p.d_alpha_a) {
-    a *= *p.d_alpha_a;
-  } else if (p.d_alpha_b) {
-    a *= *p.d_alpha_b;
-  }
-  return a;
-}
-
-// One 32x32 accumulator tile -> C.  acc[v] is (n = n0 + 8*(v/4) + 4*(lane/32) + v%4, m = m0 + lane%32).
-__device__ __forceinline__ void store_tile(const GemmParams &p, const v16f &acc, int m0, int n0, int lane, float alpha) {
-  const int m = m0 + (lane & 31);
-  if (m0 + 32 <= p.M && n0 + 32 <= p.N && (p.N & 3) == 0) {  // tile fully inside: no per-element checks
-    uint16_t *crow = p.c + (size_t)m * p.N + n0 + 4 * (lane >> 5);
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      uint2 v = make_uint2(pack_bf16_rne(acc[4 * q] * alpha, acc[4 * q + 1] * alpha),
-                           pack_bf16_rne(acc[4 * q + 2] * alpha, acc[4 * q + 3] * alpha));
-      if (p.residual) v = add_bf16_x4(v, *reinterpret_cast<const uint2 *>(p.residual + (crow - p.c) + 8 * q));
-      *reinterpret_cast<uint2 *>(crow + 8 * q) = v;
-    }
-    return;
-  }
-  if (m >= p.M) return;
-  uint16_t *crow = p.c + (size_t)m * p.N;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int n = n0 + 8 * q + 4 * (lane >> 5);
-    uint32_t h[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) h[j] = f32_to_bf16_bits(acc[4 * q + j] * alpha);
-    if (p.residual) {
-      const uint16_t *rrow = p.residual + (size_t)m * p.N;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (n + j < p.N) h[j] = f32_to_bf16_bits(bf16_bits_to_f32(h[j]) + bf16_bits_to_f32(rrow[n + j]));
-    }
-    if (n + 3 < p.N && (p.N & 3) == 0) {
-      *reinterpret_cast<uint2 *>(crow + n) = make_uint2(h[0] | (h[1] << 16), h[2] | (h[3] << 16));
-    } else {
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (n + j < p.N) crow[n + j] = (uint16_t)h[j];
-    }
-  }
-}
-
-// One 32x32 accumulator tile that lies inside C, with 16-byte stores: lanes r and r + 32 hold the two halves of
-// eight consecutive columns of row r for every q; one half-wave swap (v_permlane32_swap) per register pair gives
-// the lower lane all eight columns of an even q and the upper lane those of the odd q behind it.
-// c: this lane's address for q = 0 (row m0 + lane % 32, column n0 + 8 * (lane / 32)); res: the same into the residual, or NULL.
-__device__ __forceinline__ void store_tile_rows16(const v16f &acc, uint16_t *c, const uint16_t *res, float alpha) {
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {  // q = 2h (lower lanes) and 2h + 1 (upper lanes)
-    const uint32_t e0 = pack_bf16_rne(acc[8 * h] * alpha, acc[8 * h + 1] * alpha);
-    const uint32_t e1 = pack_bf16_rne(acc[8 * h + 2] * alpha, acc[8 * h + 3] * alpha);
-    const uint32_t o0 = pack_bf16_rne(acc[8 * h + 4] * alpha, acc[8 * h + 5] * alpha);
-    const uint32_t o1 = pack_bf16_rne(acc[8 * h + 6] * alpha, acc[8 * h + 7] * alpha);
-    // swap(upper lanes of the first operand, lower lanes of the second): lower lanes end up with (own even q,
-    // partner's even q), upper lanes with (partner's odd q, own odd q)
-    const auto s0 = __builtin_amdgcn_permlane32_swap(e0, o0, false, false);
-    const auto s1 = __builtin_amdgcn_permlane32_swap(e1, o1, false, false);
-    uint4 v = make_uint4(s0[0], s1[0], s0[1], s1[1]);
-    if (res) {
-      const uint4 rv = *reinterpret_cast<const uint4 *>(res + 16 * h);
-      v = make_uint4(add_bf16_pair(v.x, rv.x), add_bf16_pair(v.y, rv.y), add_bf16_pair(v.z, rv.z), add_bf16_pair(v.w, rv.w));
-    }
-    *reinterpret_cast<uint4 *>(c + 16 * h) = v;
-  }
-}
 
 // ---------------------------------------------------------------------------------------------
 // Baseline kernels: operands straight from global memory into registers.  Correct for every
@@ -228,7 +74,10 @@ __global__ __launch_bounds__(256) void gemm_mxfp4_direct(GemmParams p) {
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) store_tile(p, acc[i][j], m_base + 32 * j, n_base + 32 * i, lane, alpha);
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        store_quad(p, Acc32<2, 2>{acc}.quad(4 * i + q, j), m_base + Acc32<2, 2>::m(j, lane), n_base + Acc32<2, 2>::n(4 * i + q, lane), alpha);
 }
 
 // 8 e2m1 codes (one dword, element 0 in the low nibble) times an NVFP4 block scale -> 8 bf16.
@@ -286,7 +135,10 @@ __global__ __launch_bounds__(256) void gemm_nvfp4_direct(GemmParams p) {
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j) store_tile(p, acc[i][j], m_base + 32 * j, n_base + 32 * i, lane, alpha);
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        store_quad(p, Acc32<2, 2>{acc}.quad(4 * i + q, j), m_base + Acc32<2, 2>::m(j, lane), n_base + Acc32<2, 2>::n(4 * i + q, lane), alpha);
 }
 
 
@@ -309,205 +161,6 @@ __global__ __launch_bounds__(256) void gemm_nvfp4_direct(GemmParams p) {
 // MFMAs, so its four E8M0 bytes are one dword of the row-major scale array and the byte is
 // picked by the instruction's op_sel.
 // ---------------------------------------------------------------------------------------------
-// These write M0.  The compiler reserves M0 and refuses it on a clobber list ("may lead to undefined
-// behaviour"), so the contract is kept by hand: the kernels that use these helpers contain nothing for
-// which the compiler would set or read M0 itself (no LDS-direct builtins, no indirect register
-// indexing, no s_sendmsg), and every helper sets M0 before its load.
-__device__ __forceinline__ void lds_dma16(const void *g, uint32_t lds_wave_base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               :
-               : "s"(lds_wave_base), "v"(g)
-               : "memory");
-}
-
-// The same with a wave-uniform base address and a 32-bit byte offset per lane.
-__device__ __forceinline__ void lds_dma16_at(const void *base, uint32_t lane_offset, uint32_t lds_wave_base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :
-               : "s"(lds_wave_base), "v"(lane_offset), "s"(base)
-               : "memory");
-}
-
-__device__ __forceinline__ void lds_dma4(const void *g, uint32_t lds_wave_base) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" : : "s"(lds_wave_base), "v"(g) : "memory");
-}
-
-__device__ __forceinline__ void wait_dma_and_sync() {
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-template <int WN, int WM, int NWM>
-__device__ __forceinline__ void store_workgroup_tile_swiglu_fwd(const GemmParams &p, v16f (&acc)[WN][WM], uint8_t *ldsA,
-                                                                uint8_t *ldsB, int m_base, int n_base, int wave, int lane);
-
-// Epilogue shared by the tiled kernels: acc[i][j] is the 32x32 tile (n-tile i, m-tile j) of the
-// wave tile.  The workgroup's waves form a 2 (along N) x NWM (along M) grid, wave = n + 2 * m.
-// ldsA / ldsB: two LDS areas of at least NWM*32*WM*64*WN bytes each, free for reuse.
-template <int WN, int WM, int NWM = 2>
-__device__ __forceinline__ void store_workgroup_tile(const GemmParams &p, v16f (&acc)[WN][WM], uint8_t *ldsA,
-                                                     uint8_t *ldsB, int m_base, int n_base, int wave, int lane) {
-  constexpr int BN = 64 * WN, BM = 32 * WM * NWM;
-  const int r = lane & 31, kh = lane >> 5;
-  const int wn0 = (wave & 1) * 32 * WN, wm0 = (wave >> 1) * 32 * WM;
-  if (p.swiglu) return store_workgroup_tile_swiglu_fwd<WN, WM, NWM>(p, acc, ldsA, ldsB, m_base, n_base, wave, lane);
-  if (p.partial) {  // split-K: the unscaled fp32 tile of this K range
-    float *part = p.partial + (size_t)blockIdx.y * p.M * p.N;
-#pragma unroll
-    for (int i = 0; i < WN; ++i)
-#pragma unroll
-      for (int j = 0; j < WM; ++j) {
-        const int m = m_base + wm0 + 32 * j + r;
-        if (m >= p.M) continue;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int n = n_base + wn0 + 32 * i + 8 * q + 4 * kh;
-          float *dst = part + (size_t)m * p.N + n;
-          if (n + 3 < p.N && (p.N & 3) == 0) {
-            *reinterpret_cast<float4 *>(dst) =
-                make_float4(acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]);
-          } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-              if (n + e < p.N) dst[e] = acc[i][j][4 * q + e];
-          }
-        }
-      }
-    return;
-  }
-  const float alpha = effective_alpha(p);
-  constexpr bool kPow2 = (WN & (WN - 1)) == 0;  // the swizzled transpose below needs 4*WN lanes per row to be a power of two
-  if (kPow2 && m_base + BM <= p.M && n_base + BN <= p.N && (p.N & 7) == 0) {
-    // Whole tile inside C: transpose each wave's tile through LDS (free now) so that every store
-    // instruction writes whole rows of the wave tile, 16 bytes per lane.
-    wait_dma_and_sync();  // every wave is done reading operands
-    constexpr int RB = 64 * WN;                       // bytes per row of the wave tile
-    constexpr int LPR = 4 * WN;                       // lanes per row when reading 16 bytes each
-    uint8_t *region = (wave < NWM ? ldsA : ldsB) + (wave % NWM) * (32 * WM * RB);
-#pragma unroll
-    for (int i = 0; i < WN; ++i)
-#pragma unroll
-      for (int j = 0; j < WM; ++j) {
-        const int m = 32 * j + r;
-        const int sw = (m & (LPR - 1)) << 1;          // even: keeps 8-byte chunk pairs adjacent
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const v16f &a = acc[i][j];                  // the hardware's round-to-nearest-even convert
-          const int c = 8 * i + 2 * q + kh;           // 8-byte chunk of the row
-          *reinterpret_cast<uint2 *>(region + m * RB + ((c ^ sw) << 3)) =
-              make_uint2(pack_bf16_rne(a[4 * q] * alpha, a[4 * q + 1] * alpha),
-                         pack_bf16_rne(a[4 * q + 2] * alpha, a[4 * q + 3] * alpha));
-        }
-      }
-    const int rr = lane / LPR, t = lane % LPR;
-    uint16_t *cbase = p.c + (size_t)(m_base + wm0) * p.N + n_base + wn0 + 8 * t;
-#pragma unroll
-    for (int it = 0; it < (32 * WM * LPR) / 64; ++it) {
-      const int m = it * (64 / LPR) + rr;
-      const int sw = (m & (LPR - 1)) << 1;
-      uint4 v = *reinterpret_cast<const uint4 *>(region + m * RB + (((2 * t) ^ sw) << 3));
-      if (p.residual) {
-        const uint4 rv = *reinterpret_cast<const uint4 *>(p.residual + (cbase - p.c) + (size_t)m * p.N);
-        v = make_uint4(add_bf16_pair(v.x, rv.x), add_bf16_pair(v.y, rv.y), add_bf16_pair(v.z, rv.z),
-                       add_bf16_pair(v.w, rv.w));
-      }
-      *reinterpret_cast<uint4 *>(cbase + (size_t)m * p.N) = v;
-    }
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < WN; ++i)
-#pragma unroll
-    for (int j = 0; j < WM; ++j)
-      store_tile(p, acc[i][j], m_base + wm0 + 32 * j, n_base + wn0 + 32 * i, lane, alpha);
-}
-
-// Fused SwiGLU epilogue of the tiled kernels (p.swiglu): a lane's four consecutive columns of one row are
-// (gate_j, up_j, gate_j+1, up_j+1); each is rounded to bf16 as the plain epilogue would store it, and the two
-// products act_fn(gate) * up leave as one dword.  Whole tiles go through LDS so that every store
-// instruction writes 16 bytes per lane along output rows; ragged tiles store dwords with bounds checks.
-template <int WN, int WM, int NWM>
-__device__ __forceinline__ void store_workgroup_tile_swiglu(const GemmParams &p, v16f (&acc)[WN][WM], uint8_t *ldsA,
-                                                            uint8_t *ldsB, int m_base, int n_base, int wave, int lane) {
-  constexpr int BN = 64 * WN, BM = 32 * WM * NWM;
-  const int r = lane & 31, kh = lane >> 5;
-  const int wn0 = (wave & 1) * 32 * WN, wm0 = (wave >> 1) * 32 * WM;
-  const float alpha = effective_alpha(p);
-  const int No = p.N >> 1;  // output columns
-  uint32_t amax = 0u;       // max |t| of this lane as bf16 bits without the sign
-  auto product = [&](const v16f &a, int q) {  // the hardware's RNE convert: the bits f32_to_bf16_bits gives
-    return swiglu_pair(pack_bf16_rne(a[4 * q] * alpha, a[4 * q + 2] * alpha),
-                       pack_bf16_rne(a[4 * q + 1] * alpha, a[4 * q + 3] * alpha));
-  };
-  auto track = [&](uint32_t t) {
-    const uint32_t lo = t & 0x7fffu, hi = (t >> 16) & 0x7fffu;
-    amax = lo > amax ? lo : amax;
-    amax = hi > amax ? hi : amax;
-  };
-  constexpr bool kPow2 = (WN & (WN - 1)) == 0;
-  if (kPow2 && m_base + BM <= p.M && n_base + BN <= p.N && (No & 7) == 0) {
-    wait_dma_and_sync();  // every wave is done reading operands
-    constexpr int RB = 32 * WN;   // bytes per row of the wave tile: 16 * WN products
-    constexpr int LPR = 2 * WN;   // lanes per row when reading 16 bytes each
-    uint8_t *region = (wave < NWM ? ldsA : ldsB) + (wave % NWM) * (32 * WM * RB);
-#pragma unroll
-    for (int i = 0; i < WN; ++i)
-#pragma unroll
-      for (int j = 0; j < WM; ++j) {
-        const int m = 32 * j + r;
-        const int sw = m & (LPR - 1);                 // swizzle of the row's 16-byte groups
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t t = product(acc[i][j], q);
-          track(t);
-          const int c = 8 * i + 2 * q + kh;           // dword of the row
-          *reinterpret_cast<uint32_t *>(region + m * RB + ((((c >> 2) ^ sw) << 2) | (c & 3)) * 4) = t;
-        }
-      }
-    const int rr = lane / LPR, tq = lane % LPR;
-    uint16_t *cbase = p.c + (size_t)(m_base + wm0) * No + ((n_base + wn0) >> 1) + 8 * tq;
-#pragma unroll
-    for (int it = 0; it < (32 * WM * LPR) / 64; ++it) {
-      const int m = it * (64 / LPR) + rr;
-      const int sw = m & (LPR - 1);
-      const uint4 v = *reinterpret_cast<const uint4 *>(region + m * RB + ((tq ^ sw) << 4));
-      *reinterpret_cast<uint4 *>(cbase + (size_t)m * No) = v;
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < WN; ++i)
-#pragma unroll
-      for (int j = 0; j < WM; ++j) {
-        const int m = m_base + wm0 + 32 * j + r;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const int n = n_base + wn0 + 32 * i + 8 * q + 4 * kh;
-          const uint32_t t = product(acc[i][j], q);   // every lane computes (the special-value test of the
-          if (m < p.M && n + 3 < p.N) {               // activation function is a vote of the whole wave)
-            track(t);
-            *reinterpret_cast<uint32_t *>(p.c + (size_t)m * No + (n >> 1)) = t;
-          }
-        }
-      }
-  }
-  if (p.absmax_bits) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const uint32_t v = (uint32_t)__shfl_xor((int)amax, o);
-      amax = v > amax ? v : amax;
-    }
-    if (lane == 0 && amax) atomicMax(p.absmax_bits + p.seg_index, amax << 16);  // bf16 bits -> fp32 bits
-  }
-}
-
-template <int WN, int WM, int NWM>
-__device__ __forceinline__ void store_workgroup_tile_swiglu_fwd(const GemmParams &p, v16f (&acc)[WN][WM], uint8_t *ldsA,
-                                                                uint8_t *ldsB, int m_base, int n_base, int wave, int lane) {
-  store_workgroup_tile_swiglu<WN, WM, NWM>(p, acc, ldsA, ldsB, m_base, n_base, wave, lane);
-}
-
 // An FP4 operand of the scaled MFMA is 4 registers; the builtin's type has 8, the upper 4 unused.
 __device__ __forceinline__ v8i fp4_operand(uint4 q) {
   const v4i v = {(int)q.x, (int)q.y, (int)q.z, (int)q.w};
@@ -887,38 +540,6 @@ __global__ __launch_bounds__(128 * NWM) void gemm_mxfp4_tiled(GemmParams p) {
 // packed fp16 multiplies by the block scale: 8 VALU instructions per 8 values.
 // Requires K' % 128 == 0.
 // ---------------------------------------------------------------------------------------------
-typedef _Float16 v8h __attribute__((ext_vector_type(8)));
-typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-
-// fp16 bits of two NVFP4 scale bytes sitting in bits 7:0 and 23:16: (1+m/8)*2^(e-9) = (b<<7) + 0x1800
-__device__ __forceinline__ uint32_t nv_scale_pair_f16(uint32_t two_bytes) { return (two_bytes << 7) + 0x18001800u; }
-
-// packed fp16 multiply of both halves of a by the LOW (HI=false) or HIGH half of s.  Plain vector
-// code, not inline asm: the compiler folds the broadcast into op_sel and, unlike with asm, keeps
-// the wait states the matrix pipe needs between a VALU write and an MFMA reading that register.
-typedef _Float16 v2h __attribute__((ext_vector_type(2)));
-template <bool HI>
-__device__ __forceinline__ uint32_t pk_mul_f16_bcast(uint32_t a, uint32_t s) {
-  const v2h av = __builtin_bit_cast(v2h, a), sv = __builtin_bit_cast(v2h, s);
-  const _Float16 k = HI ? sv[1] : sv[0];
-  const v2h kv = {k, k};
-  return __builtin_bit_cast(uint32_t, av * kv);
-}
-
-template <bool HI>
-__device__ __forceinline__ v8h decode8_nvfp4_f16(uint32_t codes, uint32_t scale_pair) {
-  // hardware FP4 -> fp16 conversion, two codes per instruction (low nibble first), then one packed
-  // multiply by the block scale: 8 VALU instructions per 8 values
-  v4u d;
-  d[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 1.0f, 0));
-  d[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 1.0f, 1));
-  d[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 1.0f, 2));
-  d[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 1.0f, 3));
-#pragma unroll
-  for (int k = 0; k < 4; ++k) d[k] = pk_mul_f16_bcast<HI>(d[k], scale_pair);
-  return __builtin_bit_cast(v8h, d);
-}
-
 template <int WN, int WM, int NWM = 2>
 __global__ __launch_bounds__(128 * NWM) void gemm_nvfp4_tiled(GemmParams p) {
   // waves: 2 along N x NWM along M (wave = n + 2 * m), each with WN x WM accumulator tiles of 32 x 32
@@ -1106,186 +727,6 @@ __global__ __launch_bounds__(128 * NWM) void gemm_nvfp4_tiled(GemmParams p) {
                                     n_base, wave, lane);
 }
 
-#ifdef ARCQ_EXPERIMENTS
-// ---------------------------------------------------------------------------------------------
-// EXPERIMENT (built only with -DARCQ_EXPERIMENTS, reached only through ARCQ_GEMM_KERNEL=86 / 46; measured slower than
-// the kernel above: 963 against 826 us on gate_up at M = 4096).
-// NVFP4 at large M: every operand value is decoded ONCE per workgroup.  In the kernel above each wave decodes
-// the operand rows it multiplies, so a weight row is decoded by every wave along M and an activation row by
-// every wave along N, and the decode instructions (six per MFMA) share the issue slots of the one wave per SIMD
-// with the MFMAs.  Here the workgroup's eight waves (2 along N x 4 along M, wave tile 128 x 64, two waves per
-// SIMD) first act as decoders: per K step of 64 elements a thread takes 32 codes of one weight row and 32 of
-// one activation row straight from global memory (16 bytes and two scale bytes each), decodes them exactly to
-// fp16 (code value x block scale has six significant bits) and writes them into an fp16 tile in LDS -- two
-// stages of 2 x 256 rows x 128 bytes -- and then as multipliers: v_mfma_f32_32x32x16_f16 on 16-byte operand
-// reads from that tile, two decode instructions per MFMA instead of six.  The decode of step t+1 is interleaved
-// with the MFMAs of step t, its codes were requested during step t-1; one barrier per step.
-// Requires K' % 128 == 0.
-// ---------------------------------------------------------------------------------------------
-template <int NWM>  // waves along M: 4 = eight waves of 128 x 64 (two per SIMD), 2 = four waves of 128 x 128
-__global__ __launch_bounds__(128 * NWM) void gemm_nvfp4_lds16(GemmParams p) {
-  constexpr int WN = 4, WM = 8 / NWM, BN = 256, BM = 256, NT = 128 * NWM, IPT = 512 / NT;  // IPT: decoder items per thread and operand
-  __shared__ uint4 sT[2 * (BN + BM) * 8];  // stage s: fp16 weights [BN rows x 8 chunks] at s*(BN+BM)*8, activations behind them
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int kbytes = p.Kp >> 1, ksc = p.Kp >> 4;
-
-  int lin;
-  if (p.seg) {
-    if (!enter_segment<BM, BN, 16>(p, lin)) return;
-  } else {
-    const int total = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
-    const int per_xcd = (total + 7) >> 3;
-    lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-    if (lin >= total) return;
-  }
-  const int tiles_m = (p.M + BM - 1) / BM;
-  const int n_base = (lin / tiles_m) * BN, m_base = (lin % tiles_m) * BM;
-  const int nk = p.Kp >> 6;  // K steps of 64 elements: 32 code bytes and 4 scale bytes per row
-
-  // ---- decoder role: item (row, half h of the step's 64 elements) of either tile; a thread takes items tid + it * NT
-  const int d_h = tid & 1;
-  int d_row[IPT], d_swz[IPT];
-  const uint8_t *wc[IPT], *xc[IPT], *wsc[IPT], *xsc[IPT];
-  // chunk c (16 bytes = 8 fp16) of row `row` sits at row * 8 + (c ^ ((row >> 1) & 7)): rows two apart use different
-  // chunk slots and neighbouring rows different halves of the banks, so neither the decoders' 16-byte writes nor the
-  // multipliers' 16-byte reads (32 consecutive rows, one chunk) collide
-#pragma unroll
-  for (int it = 0; it < IPT; ++it) {
-    d_row[it] = (tid + it * NT) >> 1;
-    d_swz[it] = (d_row[it] >> 1) & 7;
-    wc[it] = p.b_codes + (size_t)min(n_base + d_row[it], p.N - 1) * kbytes + 16 * d_h;
-    xc[it] = p.a_codes + (size_t)min(m_base + d_row[it], p.M - 1) * kbytes + 16 * d_h;
-    wsc[it] = p.b_scales + (size_t)min(n_base + d_row[it], p.N - 1) * ksc + 2 * d_h;
-    xsc[it] = p.a_scales + (size_t)min(m_base + d_row[it], p.M - 1) * ksc + 2 * d_h;
-  }
-  struct Codes { uint4 w[IPT], x[IPT]; uint32_t ws[IPT], xs[IPT]; };
-  auto request = [&](int kt, Codes &c) {
-#pragma unroll
-    for (int it = 0; it < IPT; ++it) {
-      c.w[it] = *reinterpret_cast<const uint4 *>(wc[it] + 32 * kt);
-      c.x[it] = *reinterpret_cast<const uint4 *>(xc[it] + 32 * kt);
-      c.ws[it] = *reinterpret_cast<const uint16_t *>(wsc[it] + 4 * kt);
-      c.xs[it] = *reinterpret_cast<const uint16_t *>(xsc[it] + 4 * kt);
-    }
-  };
-  // dword D (8 codes) of a thread's 32 codes + its block's scale byte -> chunk 4 * d_h + D of the row's fp16 tile
-  // (dwords 0, 1 belong to the first of the two blocks, 2, 3 to the second)
-  auto decode_dword = [&](const uint4 &q, uint32_t two_scales, uint4 *tile_row, int d_swz, auto dsel) {
-    constexpr int D = decltype(dsel)::value;
-    const uint32_t sp = nv_scale_pair_f16((two_scales & 0xffu) | ((two_scales & 0xff00u) << 8));  // (block 0, block 1) as fp16
-    const uint32_t c = D == 0 ? q.x : D == 1 ? q.y : D == 2 ? q.z : q.w;
-    const v8h v = D < 2 ? decode8_nvfp4_f16<false>(c, sp) : decode8_nvfp4_f16<true>(c, sp);
-    tile_row[(4 * d_h + D) ^ d_swz] = __builtin_bit_cast(uint4, v);
-  };
-  auto decode_part = [&](const Codes &c, int stage, auto dsel) {  // a quarter of a step: 16 * IPT VALU instructions, 2 * IPT LDS writes
-    uint4 *base = sT + stage * ((BN + BM) * 8);
-#pragma unroll
-    for (int it = 0; it < IPT; ++it) {
-      decode_dword(c.w[it], c.ws[it], base + d_row[it] * 8, d_swz[it], dsel);
-      decode_dword(c.x[it], c.xs[it], base + BN * 8 + d_row[it] * 8, d_swz[it], dsel);
-    }
-  };
-  auto decode_step = [&](const Codes &c, int stage) {
-    decode_part(c, stage, std::integral_constant<int, 0>{});
-    decode_part(c, stage, std::integral_constant<int, 1>{});
-    decode_part(c, stage, std::integral_constant<int, 2>{});
-    decode_part(c, stage, std::integral_constant<int, 3>{});
-  };
-
-  // ---- multiplier role
-  const int r = lane & 31, kh = lane >> 5;
-  const int swz = (r >> 1) & 7;
-  const int wn0 = (wave & 1) * 32 * WN, wm0 = (wave >> 1) * 32 * WM;
-  int w_rd[4], x_rd[4];  // chunk 2 * ks + kh of this lane's row in operand tile 0, per sub-step of 16 elements
-#pragma unroll
-  for (int ks = 0; ks < 4; ++ks) {
-    w_rd[ks] = (wn0 + r) * 8 + ((2 * ks + kh) ^ swz);
-    x_rd[ks] = BN * 8 + (wm0 + r) * 8 + ((2 * ks + kh) ^ swz);
-  }
-  v16f acc[WN][WM];
-#pragma unroll
-  for (int i = 0; i < WN; ++i)
-#pragma unroll
-    for (int j = 0; j < WM; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
-
-  auto lds_sync = [&]() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-  };
-
-  Codes ca, cb;  // the codes of the next step and of the one after it
-  request(0, ca);
-  if (nk > 1) request(1, cb);
-  decode_step(ca, 0);
-  lds_sync();
-  // One K step: the MFMAs of step kt and, if MORE, the decode of step kt + 1 (codes in cb, requested a step ago)
-  // into the other stage.  MORE is a compile-time flag so that a sub-step stays one basic block and the MFMAs,
-  // the decode instructions and the LDS traffic can be interleaved in it.
-  auto step = [&](int kt, auto more_t) {
-    constexpr bool MORE = decltype(more_t)::value;
-    const uint4 *t = sT + (kt & 1) * ((BN + BM) * 8);
-    uint4 wq[2][WN], xq[2][WM];
-    auto fetch = [&](int ks, int b) {
-#pragma unroll
-      for (int i = 0; i < (WN > WM ? WN : WM); ++i) {
-        if (i < WM) xq[b][i] = t[x_rd[ks] + i * 256];
-        if (i < WN) wq[b][i] = t[w_rd[ks] + i * 256];
-      }
-    };
-    fetch(0, 0);
-    // a quarter of the next step's decode (2 x (4 converts + 4 multiplies), two 16-byte LDS writes) rides behind the
-    // eight MFMAs of every sub-step: one MFMA, two decode instructions, and the operand reads of the next sub-step
-#define ARCQ_L16_SUBSTEP(KS)                                                                                     \
-  {                                                                                                              \
-    if (KS < 3) fetch(KS + 1, (KS + 1) & 1);                                                                     \
-    if (MORE) decode_part(cb, (kt + 1) & 1, std::integral_constant<int, KS>{});                                  \
-    _Pragma("unroll") for (int i = 0; i < WN; ++i) _Pragma("unroll") for (int j = 0; j < WM; ++j)                \
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, wq[KS & 1][i]),               \
-                                                          __builtin_bit_cast(v8h, xq[KS & 1][j]), acc[i][j], 0, 0, 0); \
-    _Pragma("unroll") for (int g = 0; g < WN * WM; ++g) {                                                        \
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                                                         \
-      if (MORE) __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);                                               \
-      if (KS < 3 && g < WN + WM) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);                              \
-      if (MORE && g >= WN * WM - 2 * IPT) __builtin_amdgcn_sched_group_barrier(0x200, 1, 0);                     \
-    }                                                                                                            \
-    __builtin_amdgcn_sched_barrier(0);                                                                           \
-  }
-    ARCQ_L16_SUBSTEP(0)
-    ARCQ_L16_SUBSTEP(1)
-    ARCQ_L16_SUBSTEP(2)
-    ARCQ_L16_SUBSTEP(3)
-#undef ARCQ_L16_SUBSTEP
-  };
-  for (int kt = 0; kt + 1 < nk; ++kt) {
-    if (kt + 2 < nk) request(kt + 2, ca);  // two steps ahead, into the register set decoded during the previous step
-    step(kt, std::true_type{});
-    {
-      const Codes tmp = ca;
-      ca = cb;
-      cb = tmp;
-    }
-    lds_sync();
-  }
-  step(nk - 1, std::false_type{});
-  lds_sync();
-  store_workgroup_tile<WN, WM, NWM>(p, acc, reinterpret_cast<uint8_t *>(sT), reinterpret_cast<uint8_t *>(sT + (BN + BM) * 8), m_base,
-                                    n_base, wave, lane);
-}
-
-template <int NWM>
-int launch_nvfp4_lds16(const GemmParams &p, hipStream_t st) {
-  const int total = ((p.M + 255) / 256 + (p.seg ? p.n_seg : 0)) * ((p.N + 255) / 256);
-  const int grid = ((total + 7) / 8) * 8;
-  hipLaunchKernelGGL(gemm_nvfp4_lds16<NWM>, dim3(grid), dim3(128 * NWM), 0, st, p);
-  ARCQ_HIP_TRY(hipGetLastError());
-  return ARCQ_OK;
-}
-#endif  // ARCQ_EXPERIMENTS
-
 // ---------------------------------------------------------------------------------------------
 // Skinny kernels for M <= 64 (decode batches): the GEMM is a stream of the weight matrix, read
 // exactly once, so nothing is staged through LDS.  A workgroup owns 16 weight rows; its NW waves
@@ -1296,8 +737,6 @@ int launch_nvfp4_lds16(const GemmParams &p, hipStream_t st) {
 // from L2 the same way, one 16-column tile at a time, each reusing the weight registers.
 // Requires K' % 128 == 0 and 16-byte aligned scale arrays.
 // ---------------------------------------------------------------------------------------------
-typedef float v4f __attribute__((ext_vector_type(4)));
-
 template <int MT, int AT, int NW>
 __device__ __forceinline__ void skinny_reduce_store(const GemmParams &p, v4f (&acc)[AT * MT], float (*red)[MT * AT][64][4],
                                                     int wave, int lane) {
@@ -1646,11 +1085,7 @@ GemmPlan plan_gemm(int M, int N, int Kp, int fmt, bool scales_aligned) {
     // against 74 us with 256x128 tiles), so the next smaller tile that still fills it
     const long t44 = (long)((M + 255) / 256) * ((N + 255) / 256), t42 = (long)((M + 127) / 128) * ((N + 255) / 256);
     const int pick = t44 >= 192 ? 44 : (M > 128 && !one_round_21 ? (t42 >= 192 ? 42 : 22) : 21);
-#ifdef ARCQ_EXPERIMENTS
-    const bool known = force == 44 || force == 84 || force == 86 || force == 46 || force == 42 || force == 22 || force == 21 || force == 11;
-#else
     const bool known = force == 44 || force == 42 || force == 22 || force == 21 || force == 11;
-#endif
     plan.kernel = known ? force : pick;  // a forced kernel that NVFP4 does not have is ignored
     return plan;
   }
@@ -1696,11 +1131,6 @@ int run_gemm(GemmParams p, const GemmPlan &plan, int fmt, float *scratch, hipStr
   } else {
     switch (plan.kernel) {
       case 44: return launch_nvfp4_tiled<4, 4>(p, st);
-#ifdef ARCQ_EXPERIMENTS
-      case 84: return launch_nvfp4_tiled<4, 2, 4>(p, st);  // 256x256 tile, eight waves of 128x64
-      case 86: return launch_nvfp4_lds16<4>(p, st);       // 256x256 tile, operands decoded once per workgroup: eight waves,
-      case 46: return launch_nvfp4_lds16<2>(p, st);       // four waves
-#endif
       case 42: return launch_nvfp4_tiled<4, 2>(p, st);
       case 22: return launch_nvfp4_tiled<2, 2>(p, st);
       case 21: return launch_nvfp4_tiled<2, 1>(p, st);
@@ -1743,15 +1173,32 @@ int check_gemm_args(const void *a_codes, const void *a_scales, const void *b_cod
   return ARCQ_OK;
 }
 
+// Whether this problem goes to the kernel that multiplies one operand decoded to fp16 ahead (arcq_gemm_nv.hip).
+// Its tile is 256x256, one workgroup per CU, and a round of tiles takes the same time however few there are (K' = 4352:
+// 80-95 us).  The kernels without a workspace are faster as long as their 256x128 tiles fit one round (2048 x 4096: 65
+// against 93 us), and slower beyond (2331 x 4096: 111 / 89; 1400 x 6144: 113 / 87; 4096 x 28672: 778 / 692 us).
+bool nvfp4_f16_wanted(int M, int N, int Kp, int fmt, int n_seg) {
+  const int force = tuning().gemm_kernel;
+  if (fmt != ARCQ_FMT_NVFP4 || Kp % 128 != 0 || Kp < 512 || (force >= 0 && force != 168)) return false;
+  // 32-bit byte offsets of rows in either operand
+  if ((size_t)M * Kp * 2 >= ((size_t)1 << 32) || (size_t)N * Kp / 2 >= ((size_t)1 << 32)) return false;
+  if (force == 168) return true;
+  if (n_seg > 0) return M / n_seg >= 768;
+  return (long)((M + 127) / 128) * ((N + 255) / 256) > 256;
+}
+
 int matmul_impl(const void *a_codes, const void *a_scales, const void *b_codes, const void *b_scales, int M, int N,
                 int Kp, int fmt, float alpha, const float *d_alpha_a, const float *d_alpha_b, const void *residual,
-                void *c, void *stream) {
+                void *c, void *workspace, size_t workspace_bytes, void *stream) {
   GemmParams p;
   const int rc = check_gemm_args(a_codes, a_scales, b_codes, b_scales, M, N, Kp, fmt, alpha, d_alpha_a, d_alpha_b,
                                  residual, c, &p);
   if (rc != ARCQ_OK || M == 0 || N == 0) return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const GemmPlan plan = plan_gemm(M, N, Kp, fmt, aligned16(a_scales) && aligned16(b_scales));
+  const bool scales_aligned = aligned16(a_scales) && aligned16(b_scales);
+  if (scales_aligned && workspace && nvfp4_f16_wanted(M, N, Kp, fmt, 0) && workspace_bytes >= nvfp4_f16_bytes(M, N, Kp, false))
+    return run_nvfp4_f16(p, workspace, st);
+  const GemmPlan plan = plan_gemm(M, N, Kp, fmt, scales_aligned);
   float *scratch = nullptr;
   if (plan.slices > 1) {
     int status = ARCQ_OK;
@@ -1844,7 +1291,7 @@ extern "C" int arcq_matmul(const void *a_codes, const void *a_scales, const void
                            int M, int N, int Kp, int fmt, float alpha, const float *d_alpha_a,
                            const float *d_alpha_b, void *c, void *stream) {
   return arcq::matmul_impl(a_codes, a_scales, b_codes, b_scales, M, N, Kp, fmt, alpha, d_alpha_a, d_alpha_b, nullptr, c,
-                           stream);
+                           nullptr, 0, stream);
 }
 
 extern "C" int arcq_matmul_add(const void *a_codes, const void *a_scales, const void *b_codes, const void *b_scales,
@@ -1853,7 +1300,7 @@ extern "C" int arcq_matmul_add(const void *a_codes, const void *a_scales, const 
   if (!residual) return ARCQ_ERR_NULL;
   if (!arcq::aligned16(residual)) return ARCQ_ERR_ALIGN;
   return arcq::matmul_impl(a_codes, a_scales, b_codes, b_scales, M, N, Kp, fmt, alpha, d_alpha_a, d_alpha_b, residual, c,
-                           stream);
+                           nullptr, 0, stream);
 }
 
 namespace arcq {
@@ -1862,7 +1309,7 @@ namespace {
 int grouped_matmul_impl(const void *a_codes, const void *a_scales, const void *b_codes, const void *b_scales,
                         const int *seg_offsets, int n_seg, int M, int N, int Kp, int fmt, float alpha,
                         const float *d_alpha_a, const float *d_alpha_b, const void *residual, void *c, bool swiglu,
-                        float *d_absmax, void *stream) {
+                        float *d_absmax, void *workspace, size_t workspace_bytes, void *stream) {
   GemmParams p;
   const int rc = check_gemm_args(a_codes, a_scales, b_codes, b_scales, M, N, Kp, fmt, alpha, d_alpha_a, d_alpha_b,
                                  residual, c, &p);
@@ -1885,6 +1332,8 @@ int grouped_matmul_impl(const void *a_codes, const void *a_scales, const void *b
   // 256x256 3.86-3.96; MXFP4 with the eight-wave 256x256 kernel against 128x128 tiles: 0.66 / 0.74 ms at 2048
   // rows, 1.00 / 1.03 at 4096, 1.18 / 1.32 at 6144, 1.52 / 1.65 at 8192.
   const int avg = M / n_seg;
+  if (workspace && nvfp4_f16_wanted(M, N, Kp, fmt, n_seg) && workspace_bytes >= nvfp4_f16_bytes(M, N, Kp, true))
+    return run_nvfp4_f16(p, workspace, static_cast<hipStream_t>(stream));
   GemmPlan plan;
   const int force = tuning().gemm_kernel;
   if (fmt == ARCQ_FMT_MXFP4)
@@ -1910,7 +1359,7 @@ extern "C" int arcq_grouped_matmul(const void *a_codes, const void *a_scales, co
                                    const float *d_alpha_a, const float *d_alpha_b, const void *residual, void *c,
                                    void *stream) {
   return arcq::grouped_matmul_impl(a_codes, a_scales, b_codes, b_scales, seg_offsets, n_seg, M, N, Kp, fmt, alpha,
-                                   d_alpha_a, d_alpha_b, residual, c, false, nullptr, stream);
+                                   d_alpha_a, d_alpha_b, residual, c, false, nullptr, nullptr, 0, stream);
 }
 
 extern "C" int arcq_grouped_matmul_swiglu(const void *a_codes, const void *a_scales, const void *b_codes,
@@ -1918,13 +1367,14 @@ extern "C" int arcq_grouped_matmul_swiglu(const void *a_codes, const void *a_sca
                                           int fmt, float alpha, const float *d_alpha_a, const float *d_alpha_b, void *t,
                                           float *d_absmax, void *stream) {
   return arcq::grouped_matmul_impl(a_codes, a_scales, b_codes, b_scales, seg_offsets, n_seg, M, N, Kp, fmt, alpha,
-                                   d_alpha_a, d_alpha_b, nullptr, t, true, d_absmax, stream);
+                                   d_alpha_a, d_alpha_b, nullptr, t, true, d_absmax, nullptr, 0, stream);
 }
 
-extern "C" int arcq_matmul_swiglu(const void *a_codes, const void *a_scales, const void *b_codes, const void *b_scales,
-                                  int M, int N, int Kp, int fmt, float alpha, const float *d_alpha_a,
-                                  const float *d_alpha_b, void *t, float *d_absmax, void *stream) {
-  using namespace arcq;
+namespace arcq {
+namespace {
+int matmul_swiglu_impl(const void *a_codes, const void *a_scales, const void *b_codes, const void *b_scales, int M, int N,
+                       int Kp, int fmt, float alpha, const float *d_alpha_a, const float *d_alpha_b, void *t, float *d_absmax,
+                       void *workspace, size_t workspace_bytes, void *stream) {
   GemmParams p;
   const int rc = check_gemm_args(a_codes, a_scales, b_codes, b_scales, M, N, Kp, fmt, alpha, d_alpha_a, d_alpha_b,
                                  nullptr, t, &p);
@@ -1933,6 +1383,8 @@ extern "C" int arcq_matmul_swiglu(const void *a_codes, const void *a_scales, con
   if (!aligned16(a_scales) || !aligned16(b_scales)) return ARCQ_ERR_ALIGN;
   p.swiglu = 1;
   p.absmax_bits = reinterpret_cast<uint32_t *>(d_absmax);
+  if (workspace && nvfp4_f16_wanted(M, N, Kp, fmt, 0) && workspace_bytes >= nvfp4_f16_bytes(M, N, Kp, false))
+    return run_nvfp4_f16(p, workspace, static_cast<hipStream_t>(stream));
   GemmPlan plan = plan_gemm(M, N, Kp, fmt, true);
   const int id = plan.kernel;  // (a kernel forced through the environment may not exist for this format)
   const bool tiled = plan.slices == 1 && (id == 84 || id == 44 || id == 42 || id == 22 || id == 21 ||
@@ -1942,6 +1394,36 @@ extern "C" int arcq_matmul_swiglu(const void *a_codes, const void *a_scales, con
     plan.kernel = M > 64 ? 22 : 21;
   }
   return run_gemm(p, plan, fmt, nullptr, static_cast<hipStream_t>(stream));
+}
+}  // namespace
+}  // namespace arcq
+
+extern "C" int arcq_matmul_swiglu(const void *a_codes, const void *a_scales, const void *b_codes, const void *b_scales,
+                                  int M, int N, int Kp, int fmt, float alpha, const float *d_alpha_a,
+                                  const float *d_alpha_b, void *t, float *d_absmax, void *stream) {
+  return arcq::matmul_swiglu_impl(a_codes, a_scales, b_codes, b_scales, M, N, Kp, fmt, alpha, d_alpha_a, d_alpha_b, t,
+                                  d_absmax, nullptr, 0, stream);
+}
+
+extern "C" int arcq_gemm(const arcq_gemm_args *a, void *stream) {
+  if (!a) return ARCQ_ERR_NULL;
+  if (a->workspace && !arcq::aligned16(a->workspace)) return ARCQ_ERR_ALIGN;
+  if (a->residual && !arcq::aligned16(a->residual)) return ARCQ_ERR_ALIGN;
+  if (a->n_seg < 0 || (a->swiglu && a->residual)) return ARCQ_ERR_SHAPE;
+  if (a->n_seg > 0)
+    return arcq::grouped_matmul_impl(a->a_codes, a->a_scales, a->b_codes, a->b_scales, a->seg_offsets, a->n_seg, a->M, a->N,
+                                     a->Kp, a->fmt, a->alpha, a->d_alpha_a, a->d_alpha_b, a->residual, a->c, a->swiglu != 0,
+                                     a->d_absmax, a->workspace, a->workspace_bytes, stream);
+  if (a->swiglu)
+    return arcq::matmul_swiglu_impl(a->a_codes, a->a_scales, a->b_codes, a->b_scales, a->M, a->N, a->Kp, a->fmt, a->alpha,
+                                    a->d_alpha_a, a->d_alpha_b, a->c, a->d_absmax, a->workspace, a->workspace_bytes, stream);
+  return arcq::matmul_impl(a->a_codes, a->a_scales, a->b_codes, a->b_scales, a->M, a->N, a->Kp, a->fmt, a->alpha,
+                           a->d_alpha_a, a->d_alpha_b, a->residual, a->c, a->workspace, a->workspace_bytes, stream);
+}
+
+extern "C" size_t arcq_gemm_workspace_bytes(int M, int N, int Kp, int fmt, int n_seg) {
+  if (M <= 0 || N <= 0 || Kp < 64 || n_seg < 0) return 0;
+  return arcq::nvfp4_f16_wanted(M, N, Kp, fmt, n_seg) ? arcq::nvfp4_f16_bytes(M, N, Kp, n_seg > 0) : 0;
 }
 
 extern "C" int arcq_scales_from_absmax(float *d_values, int n, float divisor, void *stream) {

@@ -1,0 +1,374 @@
+// arcq_gemm_tile.h -- what the GEMM kernels share: the problem, the mapping of workgroups to expert segments, LDS-direct
+// loads, NVFP4 decoding to fp16, and the epilogues.
+#ifndef ARCQ_GEMM_TILE_H_
+#define ARCQ_GEMM_TILE_H_
+
+#include <hip/hip_runtime.h>
+
+#include "arcq_internal.h"
+#include "arcq_math.h"
+#include "arcq_swiglu.h"
+
+namespace arcq {
+
+typedef int v8i __attribute__((ext_vector_type(8)));
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+
+struct GemmParams {
+  const uint8_t *a_codes, *a_scales;  // activations, M rows
+  const uint8_t *b_codes, *b_scales;  // weights, N rows
+  uint16_t *c;                        // bf16 [M,N]
+  const float *d_alpha_a, *d_alpha_b;
+  float alpha;
+  int M, N, Kp;
+  // split-K (tiled kernels): blockIdx.y selects one of k_slices ranges of K steps and the workgroup
+  // writes its fp32 partial tile to partial[slice][M][N] instead of C; splitk_reduce_kernel adds them
+  float *partial = nullptr;
+  int k_slices = 1;
+  // optional residual, bf16 [M,N]: C = bf16(bf16(alpha * acc) + residual), what a bf16 add of the
+  // rounded GEMM output and the residual gives
+  const uint16_t *residual = nullptr;
+  // grouped GEMM (tiled kernels): rows seg[e] .. seg[e+1]-1 of A and C belong to segment e, whose weights
+  // start seg_b_codes / seg_b_scales bytes after those of segment e-1; d_alpha_a / d_alpha_b are arrays
+  // indexed by segment.  A workgroup rewrites its copy of these parameters to its segment's sub-problem.
+  const int *seg = nullptr;
+  int n_seg = 0;
+  size_t seg_b_codes = 0, seg_b_scales = 0;
+  // fused SwiGLU epilogue (tiled kernels): the weight rows alternate gate, up, gate, up ..., so that output
+  // columns 2j and 2j+1 are gate_j and up_j of one token and sit in one lane; c then is bf16 [M, N/2] and
+  // receives act_fn(gate) * up formed from the bf16-rounded GEMM outputs, exactly what the unfused sequence
+  // (GEMM, then silu and multiply in bf16) gives.  absmax_bits: NULL, or one word per segment (one word when
+  // not grouped) that collects max |output| as the bits of a non-negative float (zeroed by the caller).
+  int swiglu = 0;
+  uint32_t *absmax_bits = nullptr;
+  int seg_index = 0;
+  // gemm_nvfp4_f16: one operand decoded to fp16 [rows, K'] ahead of the launch (the activations, or the weights
+  // where they have fewer rows)
+  const uint16_t *f16 = nullptr;
+};
+
+// arcq_gemm_nv.hip: bytes of the decoded operand, and the GEMM on it
+size_t nvfp4_f16_bytes(int M, int N, int Kp, bool grouped);
+int run_nvfp4_f16(GemmParams p, void *workspace, hipStream_t st);
+
+namespace {
+
+// Grouped launches: maps the workgroup to (segment, tile) and turns p into that segment's problem (M = its
+// rows, operand pointers moved to its first row and its weights).  lin: tile number inside the segment, in
+// the order the ungrouped kernels use.  The launch holds an upper bound of the tile count; workgroups
+// beyond the real count return false.  G: elements per scale byte.
+template <int BM, int BN, int G>
+__device__ __forceinline__ bool enter_segment(GemmParams &p, int &lin) {
+  const int tiles_n = (p.N + BN - 1) / BN;
+  const int per_xcd = gridDim.x >> 3;  // the grid is a multiple of 8: contiguous runs of tiles per XCD
+  lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  const int rows = p.M;
+  int beg = min(max(p.seg[0], 0), rows);
+  for (int e = 0; e < p.n_seg; ++e) {
+    const int end = min(max(p.seg[e + 1], beg), rows);  // offsets that do not grow or leave the tensor: empty segments
+    const int cnt = end - beg;
+    const int t = ((cnt + BM - 1) / BM) * tiles_n;
+    if (lin < t) {
+      const size_t kbytes = p.Kp >> 1, ksc = p.Kp / G;
+      p.a_codes += (size_t)beg * kbytes;
+      p.a_scales += (size_t)beg * ksc;
+      if (p.f16) p.f16 += (size_t)beg * p.Kp;
+      p.c += (size_t)beg * (p.swiglu ? p.N >> 1 : p.N);
+      if (p.residual) p.residual += (size_t)beg * p.N;
+      p.b_codes += (size_t)e * p.seg_b_codes;
+      p.b_scales += (size_t)e * p.seg_b_scales;
+      if (p.d_alpha_a) p.d_alpha_a += e;
+      if (p.d_alpha_b) p.d_alpha_b += e;
+      p.M = cnt;
+      p.seg_index = e;
+      return true;
+    }
+    lin -= t;
+    beg = end;
+  }
+  return false;
+}
+
+// two bf16 pairs + two bf16 pairs, each sum rounded to bf16
+__device__ __forceinline__ uint32_t add_bf16_pair(uint32_t a, uint32_t b) {
+  return pack_bf16_rne(u2f(a << 16) + u2f(b << 16), u2f(a & 0xffff0000u) + u2f(b & 0xffff0000u));
+}
+__device__ __forceinline__ uint2 add_bf16_x4(uint2 a, uint2 b) {
+  return make_uint2(add_bf16_pair(a.x, b.x), add_bf16_pair(a.y, b.y));
+}
+
+__device__ __forceinline__ float effective_alpha(const GemmParams &p) {
+  float a = p.alpha;
+  if (p.d_alpha_a && p.d_alpha_b) {
+    a *= (*p.d_alpha_a) * (*p.d_alpha_b);
+  } else if (p.d_alpha_a) {
+    a *= *p.d_alpha_a;
+  } else if (p.d_alpha_b) {
+    a *= *p.d_alpha_b;
+  }
+  return a;
+}
+
+// These write M0.  The compiler reserves M0 and refuses it on a clobber list ("may lead to undefined
+// behaviour"), so the contract is kept by hand: the kernels that use these helpers contain nothing for
+// which the compiler would set or read M0 itself (no LDS-direct builtins, no indirect register
+// indexing, no s_sendmsg), and every helper sets M0 before its load.
+__device__ __forceinline__ void lds_dma16(const void *g, uint32_t lds_wave_base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :
+               : "s"(lds_wave_base), "v"(g)
+               : "memory");
+}
+
+// The same with a wave-uniform base address and a 32-bit byte offset per lane.
+__device__ __forceinline__ void lds_dma16_at(const void *base, uint32_t lane_offset, uint32_t lds_wave_base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds_wave_base), "v"(lane_offset), "s"(base)
+               : "memory");
+}
+
+__device__ __forceinline__ void lds_dma4_at(const void *base, uint32_t lane_offset, uint32_t lds_wave_base) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+               :
+               : "s"(lds_wave_base), "v"(lane_offset), "s"(base)
+               : "memory");
+}
+
+__device__ __forceinline__ void wait_dma_and_sync() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The accumulator tiles of a wave, by matrix instruction.  In both a lane holds quads: four consecutive output columns n of
+// one row m (the weights sit in the instruction's A slot).
+//   quads / rows of tiles: kQuads along n, kTiles along m; columns and rows of the wave tile: kN, kM
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+template <int WN, int WM>
+struct Acc32 {  // v_mfma_*_32x32x*: element 4 q + e of a lane is n = 8 q + 4 (lane / 32) + e, m = lane % 32
+  static constexpr int kQuads = 4 * WN, kTiles = WM, kN = 32 * WN, kM = 32 * WM;
+  v16f (&a)[WN][WM];
+  static __device__ __forceinline__ int n(int q, int lane) { return 32 * (q >> 2) + 8 * (q & 3) + 4 * (lane >> 5); }
+  static __device__ __forceinline__ int m(int j, int lane) { return 32 * j + (lane & 31); }
+  __device__ __forceinline__ float4 quad(int q, int j) const {
+    const v16f &t = a[q >> 2][j];
+    const int e = 4 * (q & 3);
+    return make_float4(t[e], t[e + 1], t[e + 2], t[e + 3]);
+  }
+};
+
+template <int NT, int MT>
+struct Acc16 {  // v_mfma_*_16x16x*: element e of a lane is n = 4 (lane / 16) + e, m = lane % 16
+  static constexpr int kQuads = NT, kTiles = MT, kN = 16 * NT, kM = 16 * MT;
+  v4f (&a)[NT][MT];
+  static __device__ __forceinline__ int n(int q, int lane) { return 16 * q + 4 * (lane >> 4); }
+  static __device__ __forceinline__ int m(int j, int lane) { return 16 * j + (lane & 15); }
+  __device__ __forceinline__ float4 quad(int q, int j) const { return make_float4(a[q][j][0], a[q][j][1], a[q][j][2], a[q][j][3]); }
+};
+
+// Fused SwiGLU epilogue of the tiled kernels (p.swiglu): a lane's four consecutive columns of one row are
+// (gate_j, up_j, gate_j+1, up_j+1); each is rounded to bf16 as the plain epilogue would store it, and the two
+// products act_fn(gate) * up leave as one dword.  Whole tiles go through LDS so that every store
+// instruction writes 16 bytes per lane along output rows; ragged tiles store dwords with bounds checks.
+template <class Acc>
+__device__ __forceinline__ void store_wave_tile_swiglu(const GemmParams &p, const Acc &acc, uint8_t *region, int m0, int n0,
+                                                       bool whole, int lane) {
+  const float alpha = effective_alpha(p);
+  const int No = p.N >> 1;  // output columns
+  uint32_t amax = 0u;       // max |t| of this lane as bf16 bits without the sign
+  auto product = [&](int q, int j) {  // the hardware's RNE convert: the bits f32_to_bf16_bits gives
+    const float4 v = acc.quad(q, j);
+    return swiglu_pair(pack_bf16_rne(v.x * alpha, v.z * alpha), pack_bf16_rne(v.y * alpha, v.w * alpha));
+  };
+  auto track = [&](uint32_t t) {
+    const uint32_t lo = t & 0x7fffu, hi = (t >> 16) & 0x7fffu;
+    amax = lo > amax ? lo : amax;
+    amax = hi > amax ? hi : amax;
+  };
+  if (whole && (No & 7) == 0) {
+    wait_dma_and_sync();  // every wave is done reading operands
+    constexpr int RB = Acc::kN;        // bytes per row of the wave tile: kN / 2 products
+    constexpr int LPR = Acc::kN / 16;  // lanes per row when reading 16 bytes each
+    static_assert((LPR & (LPR - 1)) == 0, "the swizzle needs a power of two");
+#pragma unroll
+    for (int q = 0; q < Acc::kQuads; ++q)
+#pragma unroll
+      for (int j = 0; j < Acc::kTiles; ++j) {
+        const int m = Acc::m(j, lane), c = Acc::n(q, lane) >> 2;  // row and dword of the row
+        const int sw = m & (LPR - 1);                             // swizzle of the row's 16-byte groups
+        const uint32_t t = product(q, j);
+        track(t);
+        *reinterpret_cast<uint32_t *>(region + m * RB + ((((c >> 2) ^ sw) << 2) | (c & 3)) * 4) = t;
+      }
+    const int rr = lane / LPR, tq = lane % LPR;
+    uint16_t *cbase = p.c + (size_t)m0 * No + (n0 >> 1) + 8 * tq;
+#pragma unroll
+    for (int it = 0; it < (Acc::kM * LPR) / 64; ++it) {
+      const int m = it * (64 / LPR) + rr;
+      const int sw = m & (LPR - 1);
+      const uint4 v = *reinterpret_cast<const uint4 *>(region + m * RB + ((tq ^ sw) << 4));
+      *reinterpret_cast<uint4 *>(cbase + (size_t)m * No) = v;
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < Acc::kQuads; ++q)
+#pragma unroll
+      for (int j = 0; j < Acc::kTiles; ++j) {
+        const int m = m0 + Acc::m(j, lane), n = n0 + Acc::n(q, lane);
+        const uint32_t t = product(q, j);   // every lane computes (the special-value test of the
+        if (m < p.M && n + 3 < p.N) {       // activation function is a vote of the whole wave)
+          track(t);
+          *reinterpret_cast<uint32_t *>(p.c + (size_t)m * No + (n >> 1)) = t;
+        }
+      }
+  }
+  if (p.absmax_bits) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+      const uint32_t v = (uint32_t)__shfl_xor((int)amax, o);
+      amax = v > amax ? v : amax;
+    }
+    if (lane == 0 && amax) atomicMax(p.absmax_bits + p.seg_index, amax << 16);  // bf16 bits -> fp32 bits
+  }
+}
+
+// One quad with bounds checks: columns n .. n + 3 of row m.
+__device__ __forceinline__ void store_quad(const GemmParams &p, float4 v, int m, int n, float alpha) {
+  if (m >= p.M) return;
+  uint16_t *dst = p.c + (size_t)m * p.N + n;
+  const uint16_t *res = p.residual ? p.residual + (size_t)m * p.N + n : nullptr;
+  if (n + 3 < p.N && (p.N & 3) == 0) {
+    uint2 w = make_uint2(pack_bf16_rne(v.x * alpha, v.y * alpha), pack_bf16_rne(v.z * alpha, v.w * alpha));
+    if (res) w = add_bf16_x4(w, *reinterpret_cast<const uint2 *>(res));
+    *reinterpret_cast<uint2 *>(dst) = w;
+    return;
+  }
+  const float f[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+    if (n + e < p.N) {
+      uint32_t h = f32_to_bf16_bits(f[e] * alpha);
+      if (res) h = f32_to_bf16_bits(bf16_bits_to_f32(h) + bf16_bits_to_f32(res[e]));
+      dst[e] = (uint16_t)h;
+    }
+}
+
+// Epilogue shared by the tiled kernels, called by every wave of the workgroup.  m0 / n0: first row / column of C of this
+// wave's tile.  whole: the whole WORKGROUP tile lies inside C (the same for every wave: there is a barrier behind it).
+// region: 2 * kM * kN bytes of LDS of this wave's own, free for reuse once every wave is done reading operands.
+template <class Acc>
+__device__ __forceinline__ void store_wave_tile(const GemmParams &p, const Acc &acc, uint8_t *region, int m0, int n0,
+                                                bool whole, int lane) {
+  if (p.swiglu) return store_wave_tile_swiglu(p, acc, region, m0, n0, whole, lane);
+  if (p.partial) {  // split-K: the unscaled fp32 tile of this K range
+    float *part = p.partial + (size_t)blockIdx.y * p.M * p.N;
+#pragma unroll
+    for (int q = 0; q < Acc::kQuads; ++q)
+#pragma unroll
+      for (int j = 0; j < Acc::kTiles; ++j) {
+        const int m = m0 + Acc::m(j, lane), n = n0 + Acc::n(q, lane);
+        if (m >= p.M) continue;
+        const float4 v = acc.quad(q, j);
+        float *dst = part + (size_t)m * p.N + n;
+        if (n + 3 < p.N && (p.N & 3) == 0) {
+          *reinterpret_cast<float4 *>(dst) = v;
+        } else {
+          const float f[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < p.N) dst[e] = f[e];
+        }
+      }
+    return;
+  }
+  const float alpha = effective_alpha(p);
+  constexpr int RB = 2 * Acc::kN;   // bytes per row of the wave tile
+  constexpr int LPR = Acc::kN / 8;  // lanes per row when reading 16 bytes each
+  static_assert((LPR & (LPR - 1)) == 0, "the swizzle needs a power of two");
+  if (whole && (p.N & 7) == 0) {
+    // Whole tile inside C: transpose each wave's tile through LDS (free now) so that every store
+    // instruction writes whole rows of the wave tile, 16 bytes per lane.
+    wait_dma_and_sync();  // every wave is done reading operands
+#pragma unroll
+    for (int q = 0; q < Acc::kQuads; ++q)
+#pragma unroll
+      for (int j = 0; j < Acc::kTiles; ++j) {
+        const int m = Acc::m(j, lane), c = Acc::n(q, lane) >> 2;  // row and 8-byte chunk of the row
+        const int sw = (m & (LPR - 1)) << 1;                      // even: keeps 8-byte chunk pairs adjacent
+        const float4 v = acc.quad(q, j);                          // the hardware's round-to-nearest-even convert
+        *reinterpret_cast<uint2 *>(region + m * RB + ((c ^ sw) << 3)) =
+            make_uint2(pack_bf16_rne(v.x * alpha, v.y * alpha), pack_bf16_rne(v.z * alpha, v.w * alpha));
+      }
+    const int rr = lane / LPR, t = lane % LPR;
+    uint16_t *cbase = p.c + (size_t)m0 * p.N + n0 + 8 * t;
+#pragma unroll
+    for (int it = 0; it < (Acc::kM * LPR) / 64; ++it) {
+      const int m = it * (64 / LPR) + rr;
+      const int sw = (m & (LPR - 1)) << 1;
+      uint4 v = *reinterpret_cast<const uint4 *>(region + m * RB + (((2 * t) ^ sw) << 3));
+      if (p.residual) {
+        const uint4 rv = *reinterpret_cast<const uint4 *>(p.residual + (cbase - p.c) + (size_t)m * p.N);
+        v = make_uint4(add_bf16_pair(v.x, rv.x), add_bf16_pair(v.y, rv.y), add_bf16_pair(v.z, rv.z),
+                       add_bf16_pair(v.w, rv.w));
+      }
+      *reinterpret_cast<uint4 *>(cbase + (size_t)m * p.N) = v;
+    }
+    return;
+  }
+#pragma unroll
+  for (int q = 0; q < Acc::kQuads; ++q)
+#pragma unroll
+    for (int j = 0; j < Acc::kTiles; ++j) store_quad(p, acc.quad(q, j), m0 + Acc::m(j, lane), n0 + Acc::n(q, lane), alpha);
+}
+
+// The same for the kernels whose waves form a 2 (along N) x NWM (along M) grid, wave = n + 2 * m, of 32x32 tiles.
+// ldsA / ldsB: two LDS areas of at least NWM*32*WM*64*WN bytes each.
+template <int WN, int WM, int NWM = 2>
+__device__ __forceinline__ void store_workgroup_tile(const GemmParams &p, v16f (&acc)[WN][WM], uint8_t *ldsA,
+                                                     uint8_t *ldsB, int m_base, int n_base, int wave, int lane) {
+  constexpr int BN = 64 * WN, BM = 32 * WM * NWM;
+  const bool whole = m_base + BM <= p.M && n_base + BN <= p.N;
+  uint8_t *region = (wave < NWM ? ldsA : ldsB) + (wave % NWM) * (32 * WM * 64 * WN);
+  store_wave_tile(p, Acc32<WN, WM>{acc}, region, m_base + (wave >> 1) * 32 * WM, n_base + (wave & 1) * 32 * WN, whole, lane);
+}
+
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef uint32_t v4u __attribute__((ext_vector_type(4)));
+
+// fp16 bits of two NVFP4 scale bytes sitting in bits 7:0 and 23:16: (1+m/8)*2^(e-9) = (b<<7) + 0x1800
+__device__ __forceinline__ uint32_t nv_scale_pair_f16(uint32_t two_bytes) { return (two_bytes << 7) + 0x18001800u; }
+
+// packed fp16 multiply of both halves of a by the LOW (HI=false) or HIGH half of s.  Plain vector
+// code, not inline asm: the compiler folds the broadcast into op_sel and, unlike with asm, keeps
+// the wait states the matrix pipe needs between a VALU write and an MFMA reading that register.
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+template <bool HI>
+__device__ __forceinline__ uint32_t pk_mul_f16_bcast(uint32_t a, uint32_t s) {
+  const v2h av = __builtin_bit_cast(v2h, a), sv = __builtin_bit_cast(v2h, s);
+  const _Float16 k = HI ? sv[1] : sv[0];
+  const v2h kv = {k, k};
+  return __builtin_bit_cast(uint32_t, av * kv);
+}
+
+template <bool HI>
+__device__ __forceinline__ v8h decode8_nvfp4_f16(uint32_t codes, uint32_t scale_pair) {
+  // hardware FP4 -> fp16 conversion, two codes per instruction (low nibble first), then one packed
+  // multiply by the block scale: 8 VALU instructions per 8 values
+  v4u d;
+  d[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 1.0f, 0));
+  d[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 1.0f, 1));
+  d[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 1.0f, 2));
+  d[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(codes, 1.0f, 3));
+#pragma unroll
+  for (int k = 0; k < 4; ++k) d[k] = pk_mul_f16_bcast<HI>(d[k], scale_pair);
+  return __builtin_bit_cast(v8h, d);
+}
+
+}  // namespace
+}  // namespace arcq
+#endif  // ARCQ_GEMM_TILE_H_

@@ -197,6 +197,33 @@ int arcq_matmul_add(const void *a_codes, const void *a_scales, const void *b_cod
                     void *c, void *stream);
 
 /*
+ * Every form of the GEMM (plain, with a residual, grouped by expert, with the fused SwiGLU epilogue; the entry points
+ * above and below are these with the matching fields) as one call that may use device memory of the caller's:
+ *   workspace / workspace_bytes  16-byte aligned scratch memory, read and written by this call only, its contents need
+ *                                not be kept; arcq_gemm_workspace_bytes says how much the fastest kernel for the
+ *                                problem takes (0: none).  With less, or none, the call computes the same values by
+ *                                the kernel that needs none.
+ * NVFP4 problems of many rows use it: the operand with fewer rows is decoded to fp16 there once, instead of by every
+ * workgroup that multiplies it.  Fields that do not apply are 0 / NULL; n_seg > 0 makes it a grouped GEMM.
+ */
+typedef struct arcq_gemm_args {
+  const void *a_codes, *a_scales, *b_codes, *b_scales;
+  int M, N, Kp, fmt;
+  float alpha;
+  int swiglu;               /* 1: weight rows alternate gate, up; c is bf16 [M, N/2] (arcq_matmul_swiglu) */
+  const float *d_alpha_a, *d_alpha_b;
+  const void *residual;     /* bf16 [M, N] or NULL (arcq_matmul_add) */
+  void *c;
+  const int *seg_offsets;   /* device, [n_seg + 1] (arcq_grouped_matmul) */
+  int n_seg;
+  float *d_absmax;          /* with swiglu: fp32 [max(n_seg, 1)] or NULL */
+  void *workspace;
+  size_t workspace_bytes;
+} arcq_gemm_args;
+int arcq_gemm(const arcq_gemm_args *args, void *stream);
+size_t arcq_gemm_workspace_bytes(int M, int N, int Kp, int fmt, int n_seg);
+
+/*
  * arcq_matmul for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments, same kernel
  * choice and the same bits as arcq_matmul, but the split-K partial tiles live in a fixed 8 MiB array inside

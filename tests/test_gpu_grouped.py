@@ -384,3 +384,35 @@ def test_mixtral_block_with_non_finite_logits():
     # maximum; the clean tokens' outputs stay finite and close to the run without the bad logits
     assert bool(torch.isfinite(y[0][clean].float()).all())
     assert rel_fro(y[0][clean].float(), y2[0][clean].float()) < 5e-2
+
+
+@pytest.mark.parametrize("counts,N,K,S", [((2100, 0, 517), 528, 512, 128), ((1, 3000, 255, 257), 272, 1024, 128)])
+def test_grouped_matmul_nvfp4_decoded_ahead(agemm, counts, N, K, S):
+    """Enough rows per expert for the kernel that decodes the activations to fp16 ahead: every expert's rows against the
+    ungrouped GEMM of the same operands (the same exact products in fp32 sums: equal up to one bf16 rounding), the fused
+    SwiGLU form against the unfused sequence on the grouped output, bit for bit, with its per-expert maxima."""
+    T, E = sum(counts), len(counts)
+    x = recipes.activations(T, K, seed=8).cuda()
+    idx = torch.randperm(K, generator=torch.Generator().manual_seed(1)).to(torch.int16).cuda()
+    a, sfa = agemm.reorder_quantize_x(x, idx, S, global_scale=recipes.nvfp4_tensor_scale(x))
+    ws = [agemm.reorder_quantize_w(recipes.weights(N, K, seed=30 + e).cuda(), idx, S, global_scale=0.08 / 2688) for e in range(E)]
+    B, SFB = torch.stack([w[0] for w in ws]), torch.cat([w[1] for w in ws])
+    seg = segments(counts).cuda()
+    from arcquant_amd import _lib
+    assert _lib.lib().arcq_gemm_workspace_bytes(T, N, K + S, 0, E) == 2 * T * (K + S)
+    sa = torch.rand(E, generator=torch.Generator().manual_seed(3)).add(0.5).cuda() * 1e-3
+    y = agemm.grouped_matmul(a, B, sfa, SFB, seg, sa)
+    per = sfa.numel() // T
+    beg = 0
+    for e, n in enumerate(counts):
+        if n:
+            want = agemm.matmul(a[beg:beg + n], ws[e][0], sfa[beg * per:(beg + n) * per], ws[e][1], sa[e])
+            assert rel_fro(y[beg:beg + n].float(), want.float()) < 5e-4
+        beg += n
+    t, gs = agemm.grouped_matmul_swiglu(a, B, sfa, SFB, seg, sa, tensor_scale=True)
+    assert torch.equal(t, torch.nn.functional.silu(y[:, 0::2]) * y[:, 1::2])
+    beg = 0
+    for e, n in enumerate(counts):
+        m = t[beg:beg + n].float().abs().max() if n else torch.zeros((), device="cuda")
+        assert float(gs[e]) == float(torch.where(m == 0, torch.ones_like(m), m / torch.full_like(m, 2688.0)))
+        beg += n

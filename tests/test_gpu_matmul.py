@@ -242,3 +242,22 @@ def test_matmul_random_shapes(agemm, oracle, seed):
         err = float((y.float() - want).norm() / max(1e-20, float(want.norm())))
         assert err < 6e-3, (fmt, M, N, K, S, err)
         done += 1
+
+
+@pytest.mark.parametrize("M,N,K,S", [(300, 28672, 512, 128), (8300, 1030, 448, 64), (257, 33000, 1152, 256),
+                                     (6017, 2200, 1024, 128), (2048, 4352, 768, 0)])
+def test_nvfp4_one_operand_decoded_ahead(agemm, oracle, M, N, K, S):
+    """NVFP4 problems beyond one round of 256x128 tiles: the operand with fewer rows is decoded to fp16 ahead of the
+    GEMM (rows of either operand ending inside a 256-row tile, N not a multiple of 8, K' from two pairs of steps on,
+    with and without a residual).  Products are exact and sums fp32, so against fp32 matmul of the oracle's values only
+    the bf16 rounding (2^-9 per element, 1.7e-3 in norm) and the order of the sum remain."""
+    (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, K, S, "NVFP4", seed=17)
+    from arcquant_amd import _lib
+    assert _lib.lib().arcq_gemm_workspace_bytes(M, N, K + S, 0, 0) == 2 * min(M, N) * (K + S)
+    want = oracle_dq(oracle, a, sfa, "NVFP4") @ oracle_dq(oracle, b, sfb, "NVFP4").T * (gx * gw)
+    scale = (torch.tensor(gx, device="cuda"), torch.tensor(gw, device="cuda"))
+    y = agemm.matmul(a, b, sfa, sfb, scale)
+    assert rel_fro(y.float(), want) < 2.5e-3
+    assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
+    res = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
+    assert torch.equal(agemm.matmul(a, b, sfa, sfb, scale, residual=res), y + res)
