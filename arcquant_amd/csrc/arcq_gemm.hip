@@ -161,12 +161,6 @@ __global__ __launch_bounds__(256) void gemm_nvfp4_direct(GemmParams p) {
 // MFMAs, so its four E8M0 bytes are one dword of the row-major scale array and the byte is
 // picked by the instruction's op_sel.
 // ---------------------------------------------------------------------------------------------
-// An FP4 operand of the scaled MFMA is 4 registers; the builtin's type has 8, the upper 4 unused.
-__device__ __forceinline__ v8i fp4_operand(uint4 q) {
-  const v4i v = {(int)q.x, (int)q.y, (int)q.z, (int)q.w};
-  return __builtin_shufflevector(v, v, 0, 1, 2, 3, -1, -1, -1, -1);
-}
-
 // Scheduling pattern of one MXFP4 sub-step: NM MFMAs with NR LDS reads (the next sub-step's operands)
 // spread behind them, the first MFMAs taking the larger shares.
 template <int NM, int NR, int M = 0>
@@ -994,6 +988,11 @@ struct GemmPlan {
 // the largest scratch the plan ever asks for (the stream workspaces are this big)
 constexpr size_t kSplitMaxBytes = kWorkspaceBytes[kWsSplitK];
 
+// The 256x256 MXFP4 tile: with a long K the ping-pong kernel (88, arcq_gemm_mx.hip), whose main loop is faster (K' = 14592:
+// 16384 x 4096 485 -> 432 us, 4096 x 4096 119 -> 114; K' = 19072: 16384 x 3584 680 -> 543), else the one that requests the
+// next stage from one wave per SIMD (84), which gets in and out of a tile faster (K' = 4352, 4096 x 28672: 277 against 281).
+int large_mx_tile(int kernel, int Kp) { return kernel == 84 && Kp >= 8192 ? 88 : kernel; }
+
 GemmPlan plan_gemm(int M, int N, int Kp, int fmt, bool scales_aligned) {
   GemmPlan plan;
   const Tuning &tune = tuning();
@@ -1074,9 +1073,9 @@ GemmPlan plan_gemm(int M, int N, int Kp, int fmt, bool scales_aligned) {
                                               : (M <= 128 ? 21
                                                           : (M < 512 ? 22
                                                                      : (c44 < c42 && c44 < c22 ? 84 : (c42 <= c22 ? 82 : 22)))));
-    const bool known = force == 44 || force == 84 || force == 82 || force == 42 || force == 224 || force == 22 ||
+    const bool known = force == 88 || force == 44 || force == 84 || force == 82 || force == 42 || force == 224 || force == 22 ||
                        force == 214 || force == 21;
-    plan.kernel = known ? force : pick;
+    plan.kernel = known ? force : large_mx_tile(pick, Kp);
     return plan;
   }
   if (fmt == ARCQ_FMT_NVFP4 && force != 0 && tiled_ok) {
@@ -1116,7 +1115,8 @@ int run_gemm(GemmParams p, const GemmPlan &plan, int fmt, float *scratch, hipStr
     // (gate_up at M = 4096, seven tiles per CU: 333 -> 325 us; qkv, one and a half: 77.5 -> 74.9; one round: 1-3 % slower)
     const bool persist = !p.seg && !p.swiglu && tuning().gemm_persist != 0 && p.M % 256 == 0 && p.N % 256 == 0 &&
                          (long)(p.M / 256) * (p.N / 256) > 256;
-    switch (wide && plan.kernel == 84 ? 44 : (wide && plan.kernel == 82 ? 42 : plan.kernel)) {
+    if (plan.kernel == 88 && !wide) return run_mxfp4_pingpong(p, st);
+    switch (wide && (plan.kernel == 84 || plan.kernel == 88) ? 44 : (wide && plan.kernel == 82 ? 42 : plan.kernel)) {
       case 44: return launch_mxfp4_tiled<4, 4>(p, st);
       // 256x256 tile, eight waves of 128x64, and 256x128 tile, eight waves of 128x32
       case 84: return persist ? launch_mxfp4_persistent<4, 2>(p, st) : launch_mxfp4_tiled<4, 2, 2, 4>(p, st);
@@ -1337,10 +1337,10 @@ int grouped_matmul_impl(const void *a_codes, const void *a_scales, const void *b
   GemmPlan plan;
   const int force = tuning().gemm_kernel;
   if (fmt == ARCQ_FMT_MXFP4)
-    plan.kernel = avg >= 256 ? 84 : (avg >= 96 ? 22 : 21);
+    plan.kernel = avg >= 256 ? large_mx_tile(84, Kp) : (avg >= 96 ? 22 : 21);
   else
     plan.kernel = avg >= 2048 ? 44 : (avg >= 96 ? 22 : 21);
-  if (force == 84 || force == 44 || force == 42 || force == 22 || force == 21) plan.kernel = force;
+  if (force == 88 || force == 84 || force == 44 || force == 42 || force == 22 || force == 21) plan.kernel = force;
   return run_gemm(p, plan, fmt, nullptr, static_cast<hipStream_t>(stream));
 }
 
@@ -1387,7 +1387,7 @@ int matmul_swiglu_impl(const void *a_codes, const void *a_scales, const void *b_
     return run_nvfp4_f16(p, workspace, static_cast<hipStream_t>(stream));
   GemmPlan plan = plan_gemm(M, N, Kp, fmt, true);
   const int id = plan.kernel;  // (a kernel forced through the environment may not exist for this format)
-  const bool tiled = plan.slices == 1 && (id == 84 || id == 44 || id == 42 || id == 22 || id == 21 ||
+  const bool tiled = plan.slices == 1 && (id == 88 || id == 84 || id == 44 || id == 42 || id == 22 || id == 21 ||
                                           (fmt == ARCQ_FMT_MXFP4 && (id == 82 || id == 224 || id == 214)));
   if (!tiled) {  // the decode-batch kernels and split-K have no fused epilogue: a small tile instead
     plan = GemmPlan();

@@ -1,0 +1,215 @@
+// arcq_gemm_mx.hip -- MXFP4 GEMM for many rows: 256x256 tiles, ping-pong waves, 16x16x128 scaled MFMAs.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "arcq_gemm_tile.h"
+
+namespace arcq {
+namespace {
+
+// ---------------------------------------------------------------------------------------------
+// 256x256 tile, K in stages of 256.
+//
+// Eight waves, two per SIMD, in two groups of four: a wave owns 128 rows of the weights (wave >> 2) and 64 of the
+// activations (wave & 3).  It alternates between memory phases (operand reads from LDS, requests of later stages) and
+// compute phases (32 MFMAs, nothing else); the second group starts one phase late, so that one wave of every SIMD
+// multiplies while the other one reads, with a barrier between phases.
+//
+// The matrix instruction is 16x16x128: a register-only loop of it sustains 6.6-7.4 PFLOP/s on random codes against 5.1 for
+// 32x32x64 (which does not reach the peak rate on zeros either: 6.4 against 9.6), the upper figure when the tiles are
+// walked back and forth, so that neighbouring instructions share an operand.
+//
+// A stage has two phases: all activations with weight rows 0-63 of the wave, then with rows 64-127.  The activations and
+// the first half of the weights leave LDS in the first phase, so their buffers are requested again in the second one: two
+// stages of LDS (128 KB) hold requests for six phases ahead.  (Stages of 128 elements would do the same in four buffers,
+// but a row is then fetched in pieces of 64 bytes: twice the requests to L2, 54 instead of about 20 cycles per kilobyte.)
+//
+// LDS rows are 128 bytes of codes = 8 chunks, swizzled as the fp16 tile of the NVFP4 kernel (chunk ^ stage_swizzle(row)), and
+// windows of 16 scale bytes for two stages, the last of which ends with the row.  Lanes 16 g .. 16 g + 15 hold K blocks 2 g
+// and 2 g + 1 of the stage: their two scale bytes are one 16-bit read and picked by op_sel.
+// Requires K' % 128 == 0, K' >= 512.
+// ---------------------------------------------------------------------------------------------
+__global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
+  constexpr int BT = 256;
+  constexpr int kCodes = 2 * BT * 128, kScales = 2 * 2 * BT * 16;
+  constexpr int kRegion = 128 * 64 * 2;
+  static_assert(8 * kRegion <= 2 * kCodes, "the epilogue's transpose");
+  // weights, activations, scale bytes (512 rows per window; a lane without a block may read up to 10 bytes past its row)
+  __shared__ uint4 smem[(2 * kCodes + kScales) / 16 + 1];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int pos = wave & 3, group = wave >> 2;
+  const int kbytes = p.Kp >> 1, ksc = p.Kp >> 5;
+
+  int lin;
+  if (p.seg) {
+    if (!enter_segment<BT, BT, 32>(p, lin)) return;
+  } else {
+    const int total = ((p.M + BT - 1) / BT) * ((p.N + BT - 1) / BT);
+    lin = (blockIdx.x & 7) * ((total + 7) >> 3) + (blockIdx.x >> 3);
+    if (lin >= total) return;
+  }
+  const int tm = (p.M + BT - 1) / BT, tn = (p.N + BT - 1) / BT;
+  const int band = lin / (4 * tn), bw = min(4, tm - 4 * band), in_band = lin - band * 4 * tn;
+  const int n_base = (in_band / bw) * BT, m_base = (4 * band + in_band % bw) * BT;
+
+  const int ns = (p.Kp + 255) >> 8;                 // stages
+  const bool short_last = (p.Kp & 255) != 0;        // the last one then has blocks 0..3 only
+  const int nw = (ns + 1) >> 1, s_shift = 16 * nw - ksc;
+
+  // ---- global -> LDS
+  uint32_t wvo[4], xvo[4];
+  const int ld_row = 8 * wave + (lane >> 3);
+  const uint32_t ld_q = (lane & 7) ^ stage_swizzle(ld_row);   // (the swizzle has a period of 16 rows)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    wvo[i] = (uint32_t)min(n_base + 64 * i + ld_row, p.N - 1) * (uint32_t)kbytes + ld_q * 16;
+    xvo[i] = (uint32_t)min(m_base + 64 * i + ld_row, p.M - 1) * (uint32_t)kbytes + ld_q * 16;
+  }
+  const uint8_t *sbase = group ? p.a_scales : p.b_scales;
+  const uint32_t svo = (uint32_t)(group ? min(m_base + 64 * pos + lane, p.M - 1) : min(n_base + 64 * pos + lane, p.N - 1)) * (uint32_t)ksc;
+  const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(smem);
+  // requests behind the last stage fetch it again into buffers that nobody reads any more: the number of loads on their
+  // way is the same in every stage.  A short last stage has chunks 0..3: those twice.
+  auto request_codes = [&](const uint8_t *codes, const uint32_t *vo, int area, int s, int i) {
+    const int sf = min(s, ns - 1);
+    const uint32_t back = short_last && sf == ns - 1 && ld_q >= 4 ? 64u : 0u;
+    lds_dma16_at(codes + (size_t)sf * 128, vo[i] - back, lds0 + area + (s & 1) * (BT * 128) + i * 8192 + wave * 1024);
+  };
+  auto request_x = [&](int s, int i) { request_codes(p.a_codes, xvo, kCodes, s, i); };
+  auto request_w = [&](int s, int i) { request_codes(p.b_codes, wvo, 0, s, i); };  // i even: first phase's rows, odd: second's
+  auto request_scales = [&](int w) {
+    const int wf = min(w, nw - 1);
+    lds_dma16_at(sbase + wf * 16 - (wf == nw - 1 ? s_shift : 0), svo, lds0 + 2 * kCodes + (w & 1) * (2 * BT * 16) + wave * 1024);
+  };
+
+  // ---- LDS -> operands
+  const int r = lane & 15, g = lane >> 4;
+  const uint8_t *lds = reinterpret_cast<const uint8_t *>(smem);
+  const uint8_t *w_rd[2], *x_rd[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int c = ((2 * g + h) ^ stage_swizzle(r)) << 4;
+    w_rd[h] = lds + (128 * group + r) * 128 + c;
+    x_rd[h] = lds + kCodes + (64 * pos + r) * 128 + c;
+  }
+  const uint8_t *ws_rd = lds + 2 * kCodes + (128 * group + r) * 16 + 4 * (g >> 1);
+  const uint8_t *xs_rd = lds + 2 * kCodes + BT * 16 + (64 * pos + r) * 16 + 4 * (g >> 1);
+  const int s_half = 16 * (g & 1);
+
+  uint4 wq[4][2], xq[4][2];
+  int ws[4], xs[4];
+  v4f acc[8][4];
+#pragma unroll
+  for (auto &a : acc)
+#pragma unroll
+    for (auto &b : a) b = v4f{0.f, 0.f, 0.f, 0.f};
+
+  auto barrier = [&]() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+  };
+  auto scale_offset = [&](int s) { return ((s >> 1) & 1) * (2 * BT * 16) + 8 * (s & 1) + ((s >> 1) == nw - 1 ? s_shift : 0); };
+  auto read_w = [&](int s, int so, int t, int i) {
+    wq[i][0] = *reinterpret_cast<const uint4 *>(w_rd[0] + (s & 1) * (BT * 128) + t * 2048);
+    wq[i][1] = *reinterpret_cast<const uint4 *>(w_rd[1] + (s & 1) * (BT * 128) + t * 2048);
+    ws[i] = *reinterpret_cast<const int *>(ws_rd + so + t * 256);
+  };
+  auto multiply = [&](auto half_t) {
+    constexpr int W0 = decltype(half_t)::value * 4;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int i = j & 1 ? 3 - t : t;
+        acc[W0 + i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fp4_operand(wq[i][0]), fp4_operand(xq[j][0]), acc[W0 + i][j],
+                                                                         4, 4, 0, ws[i], 0, xs[j]);
+      }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int i = j & 1 ? 3 - t : t;
+        acc[W0 + i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fp4_operand(wq[i][1]), fp4_operand(xq[j][1]), acc[W0 + i][j],
+                                                                         4, 4, 1, ws[i], 1, xs[j]);
+      }
+  };
+
+  // in the order of the steady state, so that the same wait counts apply
+  request_scales(0);
+  request_w(0, 1);
+  request_w(0, 3);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) request_x(0, i);
+  request_w(0, 0);
+  request_w(0, 2);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) request_x(1, i);
+  request_w(1, 0);
+  request_w(1, 2);
+  asm volatile("s_waitcnt vmcnt(6)" ::: "memory");  // stage 0
+  barrier();
+  if (group) barrier();  // the second group runs one phase behind
+
+  for (int s = 0; s < ns; ++s) {
+    const int so = scale_offset(s);
+    // lanes without blocks (g >= 2 of a short last stage): both scales 2^-127, so that whatever codes they hold multiply to
+    // less than half the smallest number
+    const int present = short_last && s == ns - 1 && g >= 2 ? 0 : 16;
+    // first phase: activations and the first half of the weights
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      xq[i][0] = *reinterpret_cast<const uint4 *>(x_rd[0] + (s & 1) * (BT * 128) + i * 2048);
+      xq[i][1] = *reinterpret_cast<const uint4 *>(x_rd[1] + (s & 1) * (BT * 128) + i * 2048);
+      xs[i] = *reinterpret_cast<const int *>(xs_rd + so + i * 256);
+      read_w(s, so, i, i);
+      if (i == 0 && !(s & 1)) request_scales((s >> 1) + 1);
+      if (i == 1) request_w(s + 1, 1);
+      if (i == 2) request_w(s + 1, 3);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the second half of this stage's weights has to be there behind this barrier (the counts leave out the scale load of an
+    // even stage, which then may be waited for a little early)
+    asm volatile("s_waitcnt lgkmcnt(0) vmcnt(8)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 4; ++i) xs[i] = __builtin_amdgcn_ubfe(xs[i], s_half, present), ws[i] = __builtin_amdgcn_ubfe(ws[i], s_half, present);
+    barrier();
+    multiply(std::integral_constant<int, 0>{});
+    barrier();
+    // second phase: the second half of the weights
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      read_w(s, so, 4 + i, i);
+      request_x(s + 2, i);
+      if (i & 1) request_w(s + 2, i - 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the next stage's activations and first half of the weights
+    asm volatile("s_waitcnt lgkmcnt(0) vmcnt(8)" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ws[i] = __builtin_amdgcn_ubfe(ws[i], s_half, present);
+    barrier();
+    multiply(std::integral_constant<int, 1>{});
+    barrier();
+  }
+  if (!group) barrier();
+  const bool whole = m_base + BT <= p.M && n_base + BT <= p.N;
+  store_wave_tile(p, Acc16<8, 4>{acc}, reinterpret_cast<uint8_t *>(smem) + wave * kRegion, m_base + 64 * pos, n_base + 128 * group,
+                  whole, lane);
+}
+
+}  // namespace
+
+int run_mxfp4_pingpong(const GemmParams &p, hipStream_t st) {
+  const int total = ((p.M + 255) / 256 + (p.seg ? p.n_seg : 0)) * ((p.N + 255) / 256);
+  hipLaunchKernelGGL(gemm_mxfp4_pingpong, dim3(((total + 7) / 8) * 8), dim3(512), 0, st, p);
+  ARCQ_HIP_TRY(hipGetLastError());
+  return ARCQ_OK;
+}
+
+}  // namespace arcq

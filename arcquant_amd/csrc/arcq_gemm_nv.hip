@@ -29,15 +29,6 @@ __global__ __launch_bounds__(256) void nvfp4_decode_f16_kernel(const uint32_t *c
   }
 }
 
-// Swizzle of the fp16 tile's rows of eight 16-byte chunks.  A 16-byte LDS read is served in groups of 16 lanes that are not
-// consecutive: lanes 0-3 and 12-15 of one 16-lane quarter with lanes 4-11 of its neighbour, and the rest of the two.  Here
-// neighbouring quarters read chunks two apart, so rows 0-3, 12-15 get even numbers and rows 4-11 odd ones (chunk ^ row / 2,
-// which suits 32 rows on one chunk, costs a conflict cycle for every other group: 688 instead of 5xx cycles a phase).
-__device__ __forceinline__ int f16_swizzle(int row) {
-  const int q = (row >> 1) & 7;
-  return (((q >> 2) ^ (q >> 1)) & 1) | ((q & 1) << 1) | (q & 4);
-}
-
 // ---------------------------------------------------------------------------------------------
 // 256 rows of codes x 256 rows of fp16 per workgroup, K in steps of 64.
 //
@@ -53,7 +44,7 @@ __device__ __forceinline__ int f16_swizzle(int row) {
 //
 // LDS: three stages of the fp16 tile (64 elements of K: rows of 128 bytes), two of the codes (128 elements: rows of 64
 // bytes) and of the scale bytes (8 per row).  A stage is requested two steps ahead of its first read by LDS-direct
-// loads of all eight waves; chunks of 16 bytes are swizzled on the way (fp16: f16_swizzle, codes: chunk ^
+// loads of all eight waves; chunks of 16 bytes are swizzled on the way (fp16: stage_swizzle, codes: chunk ^
 // (row / 4 & 3)) so that the lanes of an operand read, 16 consecutive rows, spread over the banks.
 //
 // Which element of K a lane feeds to which MFMA is free as long as both operands agree: lanes 16 g .. 16 g + 15 take
@@ -100,7 +91,7 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
 #pragma unroll
   for (int i = 0; i < FI; ++i) {
     const int row = 64 * i + 8 * wave + (lane >> 3);
-    fvo[i] = (uint32_t)min(f_base + row, rows_f - 1) * (uint32_t)fbytes + (((lane & 7) ^ f16_swizzle(row)) << 4);
+    fvo[i] = (uint32_t)min(f_base + row, rows_f - 1) * (uint32_t)fbytes + (((lane & 7) ^ stage_swizzle(row)) << 4);
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
@@ -127,8 +118,8 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
   const int r = lane & 15, g = lane >> 4;
   const uint8_t *lds = reinterpret_cast<const uint8_t *>(smem);
   const int f_row = 16 * TF * group + r, c_row = 64 * cpos + r;
-  const uint8_t *f_rd[2] = {lds + f_row * 128 + (((2 * g) ^ f16_swizzle(r)) << 4),
-                            lds + f_row * 128 + (((2 * g + 1) ^ f16_swizzle(r)) << 4)};
+  const uint8_t *f_rd[2] = {lds + f_row * 128 + (((2 * g) ^ stage_swizzle(r)) << 4),
+                            lds + f_row * 128 + (((2 * g + 1) ^ stage_swizzle(r)) << 4)};
   const uint8_t *c_rd[2] = {lds + kF + c_row * 64 + (((g >> 1) ^ ((r >> 2) & 3)) << 4) + (g & 1) * 8,
                             lds + kF + c_row * 64 + ((((g >> 1) + 2) ^ ((r >> 2) & 3)) << 4) + (g & 1) * 8};
   const uint8_t *s_rd = lds + kF + kC + c_row * 4 + g;

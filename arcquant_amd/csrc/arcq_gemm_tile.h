@@ -53,6 +53,9 @@ struct GemmParams {
 size_t nvfp4_f16_bytes(int M, int N, int Kp, bool grouped);
 int run_nvfp4_f16(GemmParams p, void *workspace, hipStream_t st);
 
+// arcq_gemm_mx.hip
+int run_mxfp4_pingpong(const GemmParams &p, hipStream_t st);
+
 namespace {
 
 // Grouped launches: maps the workgroup to (segment, tile) and turns p into that segment's problem (M = its
@@ -344,6 +347,21 @@ __device__ __forceinline__ void store_workgroup_tile(const GemmParams &p, v16f (
   const bool whole = m_base + BM <= p.M && n_base + BN <= p.N;
   uint8_t *region = (wave < NWM ? ldsA : ldsB) + (wave % NWM) * (32 * WM * 64 * WN);
   store_wave_tile(p, Acc32<WN, WM>{acc}, region, m_base + (wave >> 1) * 32 * WM, n_base + (wave & 1) * 32 * WN, whole, lane);
+}
+
+// Swizzle of staged rows of eight 16-byte chunks for the 16x16 matrix instructions.  A 16-byte LDS read is served in groups of 16 lanes that are not
+// consecutive: lanes 0-3 and 12-15 of one 16-lane quarter with lanes 4-11 of its neighbour, and the rest of the two.  Here
+// neighbouring quarters read chunks two apart, so rows 0-3, 12-15 get even numbers and rows 4-11 odd ones (chunk ^ row / 2,
+// which suits 32 rows on one chunk, costs a conflict cycle for every other group: the NVFP4 kernel's phases took 688 instead of 654 cycles).
+__device__ __forceinline__ int stage_swizzle(int row) {
+  const int q = (row >> 1) & 7;
+  return (((q >> 2) ^ (q >> 1)) & 1) | ((q & 1) << 1) | (q & 4);
+}
+
+// An FP4 operand of the scaled MFMA is 4 registers; the builtin's type has 8, the upper 4 unused.
+__device__ __forceinline__ v8i fp4_operand(uint4 q) {
+  const v4i v = {(int)q.x, (int)q.y, (int)q.z, (int)q.w};
+  return __builtin_shufflevector(v, v, 0, 1, 2, 3, -1, -1, -1, -1);
 }
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));

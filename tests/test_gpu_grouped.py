@@ -416,3 +416,22 @@ def test_grouped_matmul_nvfp4_decoded_ahead(agemm, counts, N, K, S):
         m = t[beg:beg + n].float().abs().max() if n else torch.zeros((), device="cuda")
         assert float(gs[e]) == float(torch.where(m == 0, torch.ones_like(m), m / torch.full_like(m, 2688.0)))
         beg += n
+
+
+def test_grouped_matmul_mxfp4_long_rows(agemm):
+    """The grouped form of the MXFP4 kernel for long rows (an average of 256 rows per expert and more, K' >= 8192; here
+    half a stage at the end): every expert's rows against the ungrouped GEMM, equal up to one bf16 rounding."""
+    counts, N, K, S = (700, 0, 300, 257), 264, 8192, 128
+    T, E = sum(counts), len(counts)
+    x = recipes.activations(T, K, seed=9).cuda()
+    idx = torch.randperm(K, generator=torch.Generator().manual_seed(1)).to(torch.int16).cuda()
+    a, sfa = agemm.reorder_quantize_x(x, idx, S, fmt="MXFP4")
+    ws = [agemm.reorder_quantize_w(recipes.weights(N, K, seed=60 + e).cuda(), idx, S, fmt="MXFP4") for e in range(E)]
+    y = agemm.grouped_matmul(a, torch.stack([w[0] for w in ws]), sfa, torch.cat([w[1] for w in ws]), segments(counts).cuda())
+    per = sfa.numel() // T
+    beg = 0
+    for e, n in enumerate(counts):
+        if n:
+            want = agemm.matmul(a[beg:beg + n], ws[e][0], sfa[beg * per:(beg + n) * per], ws[e][1], 1.0, fmt="MXFP4")
+            assert rel_fro(y[beg:beg + n].float(), want.float()) < 5e-4
+        beg += n

@@ -261,3 +261,17 @@ def test_nvfp4_one_operand_decoded_ahead(agemm, oracle, M, N, K, S):
     assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
     res = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
     assert torch.equal(agemm.matmul(a, b, sfa, sfb, scale, residual=res), y + res)
+
+
+@pytest.mark.parametrize("M,N,K,S", [(3900, 4090, 8192, 128), (4096, 4096, 8192, 0), (3841, 4097, 8320, 64 + 64)])
+def test_mxfp4_long_rows(agemm, oracle, M, N, K, S):
+    """MXFP4 with K' of 8192 and more on problems that fill the chip with 256x256 tiles: the ping-pong kernel, with K' a
+    multiple of 256 and not (half a stage, half a window of scale bytes), rows of either operand ending inside a tile, N
+    not a multiple of 8.  Exact products, fp32 sums: the bf16 rounding (1.7e-3 in norm) and the sum's order remain."""
+    (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, K, S, "MXFP4", seed=23)
+    want = oracle_dq(oracle, a, sfa, "MXFP4") @ oracle_dq(oracle, b, sfb, "MXFP4").T * 0.5
+    y = agemm.matmul(a, b, sfa, sfb, 0.5, fmt="MXFP4")
+    assert rel_fro(y.float(), want) < 2.5e-3
+    assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
+    res = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
+    assert torch.equal(agemm.matmul(a, b, sfa, sfb, 0.5, fmt="MXFP4", residual=res), y + res)
