@@ -1395,6 +1395,8 @@ __global__ __launch_bounds__(kScaleThreads) void tensor_scale_kernel(const uint1
     }
 #pragma unroll
     for (int j = 0; j < U; ++j) {  // an absent chunk is zeros: act_fn(0) * 0 = 0 leaves the maximum alone
+      // (and one absent from the whole wave is not worth the activation's instructions)
+      if (SWIGLU && c0 - (threadIdx.x & 63) + j * stride >= total) break;
       uint32_t t[4] = {g[j].x, g[j].y, g[j].z, g[j].w};
       if (SWIGLU) {
         t[0] = swiglu_pair(g[j].x, u[j].x), t[1] = swiglu_pair(g[j].y, u[j].y);
@@ -1951,8 +1953,18 @@ int arcq_tensor_scale(const void *x, const void *up, int ld, int M, int K, float
   const size_t chunks = (size_t)M * (K >> 3);
   // at most one workgroup per CU; 512 threads x 8 chunks each while one trip of that covers the tensor (small
   // tensors: fewer waves to meet at the end), 1024 threads beyond
-  const int threads = chunks <= (size_t)256 * 512 * 8 ? 512 : arcq::kScaleThreads;
-  const size_t per_wg = (size_t)threads * 8;
+  int threads = chunks <= (size_t)256 * 512 * 8 ? 512 : arcq::kScaleThreads;
+  size_t per_wg = (size_t)threads * 8;
+  if (up) {
+    // The activation makes a chunk expensive (about thirty instructions per element), so small tensors are spread over
+    // more CUs: a chunk per thread; two where that keeps the launch within kScaleSingle workgroups, whose meeting is
+    // 2 us shorter.  Rows of 14336, two operands, us before -> now:
+    // 8 rows 10.1 -> 4.9, 16: 10.4 -> 5.7 (a chunk per thread, 56 workgroups: 8.3), 64: 10.5 -> 7.8, 128: 13.5 -> 8.8,
+    // 333: 14.0 -> 12.2, 1024: 20.9 -> 20.0; 16384: 180 -> 184, the price of the test for absent chunks.
+    if (chunks > (size_t)256 * 512) threads = arcq::kScaleThreads;
+    per_wg = threads;
+    if (chunks > (size_t)arcq::kScaleSingle * 512 && chunks <= (size_t)arcq::kScaleSingle * 1024) per_wg = 1024;
+  }
   int grid = (int)std::min<size_t>(256, (chunks + per_wg - 1) / per_wg);
   if (grid < 1) grid = 1;  // M == 0: one block writes the scale of an empty tensor, 1
   if (up)

@@ -428,3 +428,24 @@ def test_scale_and_quantize_when_the_workgroups_do_not_meet(agemm):
     out = subprocess.run([sys.executable, "-c", _ALONE, here], env=env, capture_output=True, text=True, timeout=300)
     print(out.stdout[-2000:], out.stderr[-2000:], flush=True)
     assert out.returncode == 0 and "ALONE-OK" in out.stdout
+
+
+@pytest.mark.parametrize("M,K", [(1, 32), (9, 14336), (10, 14336), (18, 14336), (19, 14336), (73, 14336), (74, 14336), (2331, 4128)])
+@pytest.mark.parametrize("special", [None, float("inf"), -float("inf"), float("nan")])
+def test_swiglu_tensor_scale_every_split(agemm, M, K, special):
+    """max |act_fn(gate) * up| / 2688 on both sides of every line of the launch rule (one or two chunks per thread, one or
+    two meeting points, waves without some of their chunks, several trips per wave): exactly torch's bf16 sequence, with the
+    maximum in the last chunk behind large negative gates, and with infinities and NaN."""
+    g = torch.Generator().manual_seed(M + K)
+    gu = torch.randn(M, 2 * K, generator=g)
+    gu[:, :K][torch.rand(M, K, generator=g) < 0.01] = -100.0  # |gate * up| is large there and the product next to nothing
+    gu[-1, K - 1], gu[-1, -1] = 9.0, -9.0
+    if special is not None:
+        gu[M // 2, K // 2 + 3] = special
+    gate, up = gu.to(torch.bfloat16).cuda()[:, :K], gu.to(torch.bfloat16).cuda()[:, K:]
+    # torch's own maximum, NaN propagated (-inf * sigmoid(-inf) is NaN as well)
+    want = (torch.nn.functional.silu(gate) * up).abs().float().max() / torch.full((), 2688.0, device="cuda")
+    idx = torch.arange(K, dtype=torch.int16, device="cuda")
+    for _ in range(2):
+        got = agemm.swiglu_quantize_x(gate, up, idx, 0, fmt="NVFP4", global_scale="absmax")[2]
+        assert torch.equal(got.reshape(()).isnan(), want.isnan()) and (want.isnan() or float(got) == float(want))
