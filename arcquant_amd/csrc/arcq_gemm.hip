@@ -723,7 +723,7 @@ __global__ __launch_bounds__(128 * NWM) void gemm_nvfp4_tiled(GemmParams p) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Skinny kernels for M <= 64 (decode batches): the GEMM is a stream of the weight matrix, read
+// Skinny kernels for M <= 64 (decode batches; NVFP4: a few rows on a narrow layer, see nvfp4_stream_wanted, and K' < 512): the GEMM is a stream of the weight matrix, read
 // exactly once, so nothing is staged through LDS.  A workgroup owns 16 weight rows; its NW waves
 // take the K steps of 128 round-robin in pairs (split-K: with four waves wave w does steps 2w, 2w+1, 2w+8, 2w+9, ...:
 // a pair of steps is one whole 128-byte line of every row, and the four waves walk neighbouring lines) and their partial sums meet in LDS.  A lane loads
@@ -1006,7 +1006,7 @@ int addressable_tile(int kernel, int M, int N, int Kp) {
 // The tiled kernels a format has: a kernel forced through the environment that is not among them is ignored.
 bool has_tile(int fmt, int kernel) {
   if (kernel == 44 || kernel == 42 || kernel == 22 || kernel == 21) return true;
-  return fmt == ARCQ_FMT_MXFP4 ? kernel == 88 || kernel == 84 || kernel == 82 || kernel == 224 || kernel == 214 : kernel == 11;
+  return fmt == ARCQ_FMT_MXFP4 ? kernel == 88 || kernel == 84 || kernel == 82 || kernel == 224 || kernel == 214 : false;
 }
 
 GemmPlan plan_gemm(int M, int N, int Kp, int fmt, bool scales_aligned) {
@@ -1024,12 +1024,8 @@ GemmPlan plan_gemm(int M, int N, int Kp, int fmt, bool scales_aligned) {
   // so it pays only where the single launch is far from the weight stream's time).
   int split = 0;
   bool one_round_21 = false;  // 128x64 tiles, no more of them than CUs, K not cut
-  // NVFP4 on a wide layer with up to 32 rows: decoding bounds the 128x64 tile (every weight row decoded by both
-  // of its M-waves, 64 activation rows multiplied of which at most 32 are real), so workgroups of two waves along
-  // N with a 64x32 tile -- each weight row decoded once -- and K in two slices to fill the CUs
-  // (gate_up 28672 x 4096: 30.7 -> 24.7 us at M = 16, 28.7 -> 26.7 at M = 32; slower on the narrow layers)
-  // (only while the two slices fit the 8 MiB array of the entry point that allocates nothing, which serves
-  // every decode batch: N up to 32768 at 32 rows)
+  // NVFP4 on a wide layer with up to 32 rows: plan 11, two slices of K (only while they fit the 8 MiB array of the entry point that
+  // allocates nothing).  The plan's name and scratch are what the callers' queries report; the launch is the weight stream's.
   const bool small_nv = fmt == ARCQ_FMT_NVFP4 && split_env == 0 && force < 0 && M >= 8 && M <= 32 && N >= 16384 && Kp < 8192 &&
                         (size_t)2 * M * N * sizeof(float) <= kNoAllocScratchBytes;
   if (split_env > 1) split = M <= 512 ? split_env : 0;
@@ -1055,7 +1051,7 @@ GemmPlan plan_gemm(int M, int N, int Kp, int fmt, bool scales_aligned) {
     const int slices = std::min(split, (Kp + 255) / 256 / 2);
     const size_t bytes = (size_t)slices * M * N * sizeof(float);
     if (slices > 1 && bytes <= kSplitMaxBytes) {
-      plan.kernel = fmt == ARCQ_FMT_MXFP4 ? 214 : ((small_nv || force == 11) ? 11 : 21);
+      plan.kernel = fmt == ARCQ_FMT_MXFP4 ? 214 : (small_nv ? 11 : 21);
       plan.slices = slices;
       plan.scratch = bytes;
       return plan;
@@ -1135,12 +1131,19 @@ GemmPlan plan_swiglu(int M, int N, int Kp, int fmt) {
   return plan;
 }
 
+// NVFP4 decode batches run as a stream of the weights, whichever tiles (and slices of K) the plan has for them, unless a kernel
+// or a number of slices is forced; plan 0 has operands that only the direct kernels take.
+bool takes_stream(const GemmPlan &plan, const GemmParams &p, int fmt) {
+  return fmt == ARCQ_FMT_NVFP4 && tuning().gemm_kernel < 0 && tuning().gemm_splitk == 0 && plan.kernel != 0 &&
+         nvfp4_stream_wanted(p.M, p.N, p.Kp, p.n_seg);
+}
+
 int run_gemm(GemmParams p, const GemmPlan &plan, int fmt, float *scratch, hipStream_t st) {
+  if (takes_stream(plan, p, fmt)) return run_nvfp4_stream(p, st);
   if (plan.slices > 1) {
     p.k_slices = plan.slices;
     p.partial = scratch;
-    const int rc = fmt == ARCQ_FMT_MXFP4 ? launch_mxfp4_tiled<2, 1, 4>(p, st)
-                   : (plan.kernel == 11 ? launch_nvfp4_tiled<1, 1, 1>(p, st) : launch_nvfp4_tiled<2, 1>(p, st));
+    const int rc = fmt == ARCQ_FMT_MXFP4 ? launch_mxfp4_tiled<2, 1, 4>(p, st) : launch_nvfp4_tiled<2, 1>(p, st);
     if (rc != ARCQ_OK) return rc;
     const size_t total4 = ((size_t)p.M * p.N) >> 2;
     hipLaunchKernelGGL(splitk_reduce_kernel, dim3((unsigned)std::min<size_t>((total4 + 255) / 256, 1024)), dim3(256), 0,
@@ -1175,7 +1178,6 @@ int run_gemm(GemmParams p, const GemmPlan &plan, int fmt, float *scratch, hipStr
       case 42: return launch_nvfp4_tiled<4, 2>(p, st);
       case 22: return launch_nvfp4_tiled<2, 2>(p, st);
       case 21: return launch_nvfp4_tiled<2, 1>(p, st);
-      case 11: return launch_nvfp4_tiled<1, 1, 1>(p, st);  // 64x32 tile, two waves along N
       default: break;
     }
   }
@@ -1251,7 +1253,7 @@ int matmul_impl(const void *a_codes, const void *a_scales, const void *b_codes, 
     return run_nvfp4_f16(p, workspace, st);
   const GemmPlan plan = plan_gemm(M, N, Kp, fmt, scales_aligned);
   float *scratch = nullptr;
-  if (plan.slices > 1) {
+  if (plan.slices > 1 && !takes_stream(plan, p, fmt)) {
     int status = ARCQ_OK;
     scratch = static_cast<float *>(stream_workspace(kWsSplitK, st, &status));
     if (!scratch) return status;
@@ -1321,7 +1323,7 @@ extern "C" int arcq_matmul_noalloc(const void *a_codes, const void *a_scales, co
   const GemmPlan plan = plan_gemm(M, N, Kp, fmt, aligned16(a_scales) && aligned16(b_scales));
   if (plan.scratch_bytes() > kNoAllocScratchBytes) return ARCQ_ERR_WORKSPACE;  // beyond the fixed array: nothing is launched
   float *ws = nullptr;
-  if (plan.slices > 1) {
+  if (plan.slices > 1 && !takes_stream(plan, p, fmt)) {
     int status = ARCQ_OK;
     ws = noalloc_scratch(&status);
     if (!ws) return status;

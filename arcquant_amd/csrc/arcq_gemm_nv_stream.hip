@@ -1,0 +1,355 @@
+// arcq_gemm_nv_stream.hip -- NVFP4 GEMM of decode batches (up to 64 rows, or experts of a few rows each): one pass over the
+// weights, all of whose bytes are on their way through many small workgroups.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+
+#include "arcq_gemm_tile.h"
+
+namespace arcq {
+namespace {
+
+// At most n of this wave's loads may still be on their way (more than the instruction's cases here: a stricter wait).
+__device__ __forceinline__ void wait_vmcnt(int n) {
+  switch (n) {
+    case 0: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
+    case 1: asm volatile("s_waitcnt vmcnt(1)" ::: "memory"); break;
+    case 2: asm volatile("s_waitcnt vmcnt(2)" ::: "memory"); break;
+    case 3: asm volatile("s_waitcnt vmcnt(3)" ::: "memory"); break;
+    case 4: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
+    case 5: asm volatile("s_waitcnt vmcnt(5)" ::: "memory"); break;
+    case 6: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
+    case 7: asm volatile("s_waitcnt vmcnt(7)" ::: "memory"); break;
+    case 8: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
+    case 9: asm volatile("s_waitcnt vmcnt(9)" ::: "memory"); break;
+    case 10: asm volatile("s_waitcnt vmcnt(10)" ::: "memory"); break;
+    default: asm volatile("s_waitcnt vmcnt(11)" ::: "memory"); break;
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
+// A workgroup multiplies 16 NT WN weight rows with 16 MT activation rows.  Its WN x WK waves share the K steps of 64 WK
+// elements: a wave takes 64 elements of every step and 16 NT rows, decodes both operands to fp16 in registers and feeds
+// v_mfma_f32_16x16x32_f16.  The WK partial sums of a tile meet in LDS at the end.
+//
+// What bounds such a problem is the stream of the weights, and in front of it everything that keeps a CU from asking for
+// more of them: waves that wait for one another, load instructions that touch a cache line for a few bytes, and the decoding,
+// which costs 8 VALU instructions (a wave's takes 2 ns on its SIMD once two or more waves offer them, 4 ns alone) per 512
+// codes and operand.  So:
+//  - NT is as large as the grid allows: the activations are decoded once per workgroup (WN = 1), whatever its rows.
+//  - Codes travel by LDS-direct loads in whole rows of 128 to 512 bytes, scale bytes in 64-byte windows (1024 elements): with
+//    16-byte windows, or straight to registers, the cache lines fetched for scale bytes outweigh the codes.
+//  - Two stages (one step on its way) and small workgroups, two to four per CU, that wait independently: 28672 x 4352 with 16
+//    rows 15.7 us (4.5 TB/s); three stages in the same shape 17.6, sixteen waves on 128 rows and four stages 20.3.
+// Before (64x32 and 128x64 tiles, the latter's K cut in slices and added up by a second launch, or a lane's operands straight
+// from global memory), us, weights from HBM, 16 / 32 / 64 rows: 28672 x 4352 23.2 / 25.7 / 28.2, now 15.7 / 18.5 / 24.7;
+// 14336 x 4352 17.8 / 26 / 26.4, now 10.9 / 14 / 16.9; 6144 x 4352 10.0 / 14.6 / 17.1, now 7.8 / 8.8 / 11.5; 4096 x 4352 6.6 / 9.0 /
+// 12.5, now 6.0 / 6.9 / 9.4; 4096 x 14592 16.9 / 20.8 / 22.2, now 12.1 / 15.3 / 21.3.
+// ---------------------------------------------------------------------------------------------
+template <int MT, int NT, int WN, int WK, int NS>
+struct StreamShape {
+  static constexpr int NW = WN * WK, BN = 16 * NT * WN, BM = 16 * MT;
+  static constexpr int RB = 32 * WK;             // code bytes of a row in one step (64 elements per wave)
+  static constexpr int SB = WK >= 16 ? 1 : 16 / WK;  // steps per scale window of 64 bytes
+  static constexpr int NB = (NS + SB - 2) / SB + 1;  // windows on their way or in use
+  static constexpr int kCodes = NS * (BN + BM) * RB, kScales = NB * (BN + BM) * 64;
+  static constexpr int kLds = kCodes + kScales;
+  // the waves' sums meet in LDS a few 16x16 tiles per wave at a time
+  static constexpr int kBatches = (NW * NT * MT * 1024 + kLds - 1) / kLds, kBatch = (NT * MT + kBatches - 1) / kBatches;
+  static_assert(NW * kBatch * 1024 <= kLds, "a batch of sums fits");
+};
+
+template <int MT, int NT, int WN, int WK, int NS>
+__device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, int m_base, uint8_t *smem) {
+  using S = StreamShape<MT, NT, WN, WK, NS>;
+  constexpr int NW = S::NW, BN = S::BN, BM = S::BM, RB = S::RB, SB = S::SB, NB = S::NB;
+  constexpr int CPR = RB / 16, RPI = 64 / CPR;      // 16-byte chunks per row, rows per load instruction
+  constexpr int WI = BN / RPI, NI = (BN + BM) / RPI;  // load instructions of the weights and of both operands per step
+  constexpr int PW = (NI + NW - 1) / NW;            // per wave, at most
+  constexpr int SI = (BN + BM) / 16;                // of a scale window: 16 rows of 64 bytes each
+  static_assert(BN % RPI == 0 && BM % RPI == 0, "whole instructions");
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const int kbytes = p.Kp >> 1, ksc = p.Kp >> 4;
+  const int nk = (kbytes + RB - 1) / RB;
+  const uint8_t *wc = p.b_codes + (size_t)n_base * kbytes, *ws = p.b_scales + (size_t)n_base * ksc;
+  const uint8_t *xc = p.a_codes + (size_t)m_base * kbytes, *xs = p.a_scales + (size_t)m_base * ksc;
+  const int rows_w = p.N - 1 - n_base, rows_x = p.M - 1 - m_base;  // last valid row of either tile
+  const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(smem);
+  // position of chunk c of a row: the 16 rows of an operand read spread over all banks
+  auto swizzle = [](int row) { return CPR == 8 ? (row >> 1) & 7 : row & 15; };
+
+  uint32_t ro[PW];
+  int co[PW];
+#pragma unroll
+  for (int i = 0; i < PW; ++i) {
+    const int k = wave + i * NW;
+    const bool x = k >= WI;
+    const int row = (x ? k - WI : k) * RPI + lane / CPR;
+    ro[i] = (uint32_t)min(row, x ? rows_x : rows_w) * (uint32_t)kbytes;
+    co[i] = ((lane % CPR) ^ swizzle(row)) * 16;
+  }
+  constexpr int PS = (SI + NW - 1) / NW;
+  uint32_t so[PS];
+  const int sp = ((lane & 3) ^ ((lane >> 4) & 3)) * 16;  // piece of the window; rows 4 apart take turns
+#pragma unroll
+  for (int i = 0; i < PS; ++i) {
+    const int k = wave + i * NW;
+    const bool x = k >= BN / 16;
+    const int row = (x ? k - BN / 16 : k) * 16 + (lane >> 2);
+    so[i] = (uint32_t)min(row, x ? rows_x : rows_w) * (uint32_t)ksc;
+  }
+
+  auto request = [&](int kt, int st, int win) {
+    if (kt % SB == 0) {
+#pragma unroll
+      for (int i = 0; i < PS; ++i) {
+        const int k = wave + i * NW;
+        if (k < SI)  // (pieces past the row's end: its last 16 bytes)
+          lds_dma16_at(k >= BN / 16 ? xs : ws, so[i] + (uint32_t)min((kt / SB) * 64 + sp, ksc - 16),
+                       lds0 + S::kCodes + win * ((BN + BM) * 64) + k * 1024);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+      const int k = wave + i * NW;
+      if (k < NI)
+        lds_dma16_at(k >= WI ? xc : wc, ro[i] + (uint32_t)min(kt * RB + co[i], kbytes - 16), lds0 + st * ((BN + BM) * RB) + k * 1024);
+    }
+  };
+  const int mine = (NI - wave + NW - 1) / NW;  // load instructions of this wave per step
+  const int mine_s = (SI - wave + NW - 1) / NW;
+  auto group = [&](int kt) { return mine + (kt % SB == 0 ? mine_s : 0); };
+
+  const int wn = wave % WN, wk = wave / WN;
+  v4f acc[NT][MT];
+#pragma unroll
+  for (auto &a : acc)
+#pragma unroll
+    for (auto &b : a) b = v4f{0.f, 0.f, 0.f, 0.f};
+  const int w_row = 16 * NT * wn + r, x_row = BN + r;
+  const int chunk = 2 * wk + (g >> 1);
+  const int w_rd = w_row * RB + ((chunk ^ swizzle(w_row)) << 4) + (g & 1) * 8;
+  const int x_rd = x_row * RB + ((chunk ^ swizzle(r)) << 4) + (g & 1) * 8;
+  const int swz_s = (r >> 2) & 3;
+
+  auto compute = [&](int kt, int st, int win) {
+    const int c64 = kt * WK + wk;  // this wave's 64 elements
+    if (c64 * 32 >= kbytes) return;
+    const int piece = c64 >> 2;
+    const int sb = (((piece & 3) ^ swz_s) << 4) + 4 * (c64 & 3) + g + ((ksc & 15) && piece == (ksc >> 4) ? 8 : 0);
+    const uint8_t *cs = smem + st * ((BN + BM) * RB), *ss = smem + S::kCodes + win * ((BN + BM) * 64) + sb;
+    uint2 wq[NT], xq[MT];
+    uint32_t wsc[NT], xsc[MT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      wq[i] = *reinterpret_cast<const uint2 *>(cs + w_rd + i * (16 * RB));
+      wsc[i] = ss[(w_row + 16 * i) * 64];
+    }
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      xq[j] = *reinterpret_cast<const uint2 *>(cs + x_rd + j * (16 * RB));
+      xsc[j] = ss[(x_row + 16 * j) * 64];
+    }
+#pragma unroll
+    for (int i = 0; i < NT; ++i) wsc[i] = (wsc[i] << 7) + 0x1800u;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) xsc[j] = (xsc[j] << 7) + 0x1800u;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      v8h b[MT];
+#pragma unroll
+      for (int j = 0; j < MT; ++j) b[j] = decode8_nvfp4_f16<false>(h ? xq[j].y : xq[j].x, xsc[j]);
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        const v8h a = decode8_nvfp4_f16<false>(h ? wq[i].y : wq[i].x, wsc[i]);
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b[j], acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  auto barrier = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+
+#pragma unroll
+  for (int a = 0; a < NS - 1; ++a)
+    if (a < nk) request(a, a, a / SB);
+  int st = 0, st_req = NS - 1, win = 0, win_req = ((NS - 1) / SB) % NB;  // stages and windows of step kt and of the step requested
+  for (int kt = 0; kt < nk; ++kt) {
+    int younger = 0;
+#pragma unroll
+    for (int a = 1; a < NS - 1; ++a)
+      if (kt + a < nk) younger += group(kt + a);
+    wait_vmcnt(younger);
+    barrier();  // step kt is there, and everyone is done with the stage of step kt - 1
+    if (kt + NS - 1 < nk) request(kt + NS - 1, st_req, win_req);
+    compute(kt, st, win);
+    st = st == NS - 1 ? 0 : st + 1;
+    st_req = st_req == NS - 1 ? 0 : st_req + 1;
+    if ((kt + 1) % SB == 0) win = win == NB - 1 ? 0 : win + 1;
+    if ((kt + NS) % SB == 0) win_req = win_req == NB - 1 ? 0 : win_req + 1;
+  }
+
+  // the sums of the waves that share a tile meet in LDS, added in the order of K
+  float4 *red = reinterpret_cast<float4 *>(smem);
+  const float alpha = effective_alpha(p);
+  uint32_t amax = 0u;
+  constexpr int Q = NT * MT, QB = S::kBatch;
+#pragma unroll
+  for (int b0 = 0; b0 < Q; b0 += QB) {
+    barrier();
+#pragma unroll
+    for (int q = 0; q < QB; ++q)
+      if (b0 + q < Q) {
+        const v4f a = acc[(b0 + q) / MT][(b0 + q) % MT];
+        red[(wave * QB + q) * 64 + lane] = make_float4(a[0], a[1], a[2], a[3]);
+      }
+    barrier();
+    for (int t = wave; t < WN * QB; t += NW) {
+      const int tn = t / QB, q = b0 + t % QB;  // tile q of the waves at position tn along N
+      if (q >= Q) continue;
+      float4 v = red[(tn * QB + t % QB) * 64 + lane];
+#pragma unroll
+      for (int w = 1; w < WK; ++w) {
+        const float4 u = red[((w * WN + tn) * QB + t % QB) * 64 + lane];
+        v.x += u.x, v.y += u.y, v.z += u.z, v.w += u.w;
+      }
+      const int m = m_base + 16 * (q % MT) + r, n = n_base + 16 * (NT * tn + q / MT) + 4 * g;
+      if (p.swiglu) {  // N is a multiple of 16: a quad is inside C or outside as a whole
+        const uint32_t o = swiglu_pair(pack_bf16_rne(v.x * alpha, v.z * alpha), pack_bf16_rne(v.y * alpha, v.w * alpha));
+        if (m < p.M && n < p.N) {
+          amax = max(amax, max(o & 0x7fffu, (o >> 16) & 0x7fffu));
+          *reinterpret_cast<uint32_t *>(p.c + (size_t)m * (p.N >> 1) + (n >> 1)) = o;
+        }
+        continue;
+      }
+      if (m >= p.M || n >= p.N) continue;
+      uint16_t *dst = p.c + (size_t)m * p.N + n;
+      if ((p.N & 3) == 0) {
+        uint2 o = make_uint2(pack_bf16_rne(v.x * alpha, v.y * alpha), pack_bf16_rne(v.z * alpha, v.w * alpha));
+        if (p.residual) o = add_bf16_x4(o, *reinterpret_cast<const uint2 *>(p.residual + (dst - p.c)));
+        *reinterpret_cast<uint2 *>(dst) = o;
+        continue;
+      }
+      const float f[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (n + e < p.N) {
+          uint32_t h = f32_to_bf16_bits(f[e] * alpha);
+          if (p.residual) h = f32_to_bf16_bits(bf16_bits_to_f32(h) + bf16_bits_to_f32(p.residual[(dst - p.c) + e]));
+          dst[e] = (uint16_t)h;
+        }
+    }
+  }
+  if (p.swiglu && p.absmax_bits) {
+    // All workgroups of an expert share one word, and atomics on one word are served one after the other (28672 x 4224, eight
+    // experts, one from every wave: 190 us, the GEMM alone 135): one per workgroup, and only if its maximum is above what the
+    // word, which never falls, was seen to hold.
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) amax = max(amax, (uint32_t)__shfl_xor((int)amax, o));
+    barrier();
+    uint32_t *top = reinterpret_cast<uint32_t *>(smem);
+    if (lane == 0) top[wave] = amax;
+    barrier();
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int w = 1; w < NW; ++w) amax = max(amax, top[w]);
+      uint32_t *word = p.absmax_bits + p.seg_index;
+      if ((amax << 16) > *const_cast<volatile uint32_t *>(word)) atomicMax(word, amax << 16);  // bf16 bits -> fp32 bits
+    }
+  }
+}
+
+template <int MT, int NT, int WN, int WK, int NS, bool GROUPED>
+__global__ __launch_bounds__(64 * WN * WK) void gemm_nvfp4_stream(GemmParams p) {
+  using S = StreamShape<MT, NT, WN, WK, NS>;
+  __shared__ uint4 smem[S::kLds / 16];
+  uint8_t *lds = reinterpret_cast<uint8_t *>(smem);
+  int lin;
+  if constexpr (GROUPED) {
+    if (!enter_segment<S::BM, S::BN, 16>(p, lin)) return;
+  } else {
+    const int total = ((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN);
+    lin = (blockIdx.x & 7) * ((total + 7) >> 3) + (blockIdx.x >> 3);
+    if (lin >= total) return;
+  }
+  const int tiles_m = (p.M + S::BM - 1) / S::BM;
+  const int n_base = (lin / tiles_m) * S::BN, m_base = (lin % tiles_m) * S::BM;
+  if constexpr (GROUPED && MT > 1) {  // experts of few rows: no matrix instructions for rows that are not there
+    const int rows = p.M - m_base;
+    if (rows <= 16) return nv_stream_tile<1, NT, WN, WK, NS>(p, n_base, m_base, lds);
+    if (MT > 2 && rows <= 32) return nv_stream_tile<2, NT, WN, WK, NS>(p, n_base, m_base, lds);
+    if (MT > 3 && rows <= 48) return nv_stream_tile<3, NT, WN, WK, NS>(p, n_base, m_base, lds);
+  }
+  nv_stream_tile<MT, NT, WN, WK, NS>(p, n_base, m_base, lds);
+}
+
+template <int MT, int NT, int WN, int WK, int NS, bool GROUPED = false>
+int launch(const GemmParams &p, hipStream_t st) {
+  using S = StreamShape<MT, NT, WN, WK, NS>;
+  const int total = ((p.M + S::BM - 1) / S::BM + (GROUPED ? p.n_seg : 0)) * ((p.N + S::BN - 1) / S::BN);
+  hipLaunchKernelGGL((gemm_nvfp4_stream<MT, NT, WN, WK, NS, GROUPED>), dim3(((total + 7) / 8) * 8), dim3(64 * S::NW), 0, st, p);
+  ARCQ_HIP_TRY(hipGetLastError());
+  return ARCQ_OK;
+}
+
+// Rows per workgroup.  Up to 12288 rows of weights make at most one workgroup per CU of 16, 32 or 48 rows, which then has
+// sixteen waves (us at 16 rows: 6144 x 4352 7.8, eight waves 8.9; 10240 x 8320 15.0 and 17.6).  Beyond, eight waves, and the
+// rows per workgroup by how many rounds of 256 workgroups they make: the rows and activation rows of a CU's workgroups
+// together, a quarter more where up to 32 rows have a single workgroup per CU to themselves (nothing else asks for weights
+// while it starts, waits and ends): 28672 rows take 64 per workgroup up to 32 rows and 112 above (64 rows: 24.7 us against
+// 25.4), 18944 rows 48 and 80.
+template <int MT>
+int launch_plain(const GemmParams &p, hipStream_t st) {
+  if (p.N <= 4096) return launch<MT, 1, 1, 16, (MT == 1 ? 3 : 2)>(p, st);
+  if (p.N <= 8192) return launch<MT, 2, 1, 16, 2>(p, st);
+  if (p.N <= 12288) return launch<MT, 3, 1, 16, 2>(p, st);
+  int best = 0;
+  double least = 0;
+  for (const int nt : {2, 3, 4, 5, 7}) {
+    const int groups = (p.N + 16 * nt - 1) / (16 * nt);
+    const double cost = (groups + 255) / 256 * (nt + 0.25 * MT) * (groups <= 256 && MT <= 2 ? 1.25 : 1.0);
+    if (!best || cost < least) best = nt, least = cost;
+  }
+  switch (best) {
+    case 2: return launch<MT, 2, 1, 8, 2>(p, st);
+    case 3: return launch<MT, 3, 1, 8, 2>(p, st);
+    case 4: return launch<MT, 4, 1, 8, 2>(p, st);
+    case 5: return launch<MT, 5, 1, 8, 2>(p, st);
+    default: return launch<MT, 7, 1, 8, 2>(p, st);
+  }
+}
+
+}  // namespace
+
+// Plain problems of up to 64 rows, but for a few rows on a narrow layer, where the kernel that reads its operands straight
+// into registers gets in and out faster (4 rows: 3584 x 3712 4.9 against 5.7 us; 1 row: 4096 x 14592 10.8 against 12.0, 8 rows
+// 12.8 against 12.0).  Experts: an average of fewer than 96 rows; from 40 rows on the 128x64 tiles
+// are as good where K is short (64 experts of 2048 x 1536, 64 rows each: 37 against 43 us).
+bool nvfp4_stream_wanted(int M, int N, int Kp, int n_seg) {
+  if (Kp % 128 != 0 || Kp < 512 || Kp > (1 << 24)) return false;
+  if (n_seg > 0) return M / n_seg < 96 && (M / n_seg <= 40 || Kp >= 2048);
+  return M <= 64 && !(N <= 8192 && M <= 4) && !(N <= 4096 && M <= 8 && Kp < 8192);
+}
+
+int run_nvfp4_stream(const GemmParams &p, hipStream_t st) {
+  if (p.seg) {
+    // Experts of very different sizes in one launch: a workgroup takes at most 48 rows of its expert (64 where the average is
+    // above 40) and leaves out the 16-row tiles that it has none for.  Eight experts of 28672 x 4224 with the SwiGLU epilogue and
+    // of 4096 x 14464, weights from HBM, us: 2 to 48 rows 139 and 70 (4.0 TB/s; 128x64 tiles: 186 and 101), 16 rows each 124 and
+    // 56, 32 rows each 134 and 60, 10 to 250 rows 270 and 150 (307 and 143).
+    if (p.M / p.n_seg > 40) return p.N > 8192 ? launch<4, 3, 2, 4, 2, true>(p, st) : launch<4, 4, 2, 4, 2, true>(p, st);
+    return p.N > 8192 ? launch<3, 4, 2, 4, 2, true>(p, st) : launch<3, 4, 1, 8, 2, true>(p, st);
+  }
+  switch ((p.M + 15) / 16) {
+    case 1: return launch_plain<1>(p, st);
+    case 2: return launch_plain<2>(p, st);
+    case 3: return launch_plain<3>(p, st);
+    default: return launch_plain<4>(p, st);
+  }
+}
+
+}  // namespace arcq

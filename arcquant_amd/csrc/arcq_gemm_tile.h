@@ -53,6 +53,10 @@ struct GemmParams {
 size_t nvfp4_f16_bytes(int M, int N, int Kp, bool grouped);
 int run_nvfp4_f16(GemmParams p, void *workspace, hipStream_t st);
 
+// arcq_gemm_nv_stream.hip: decode batches, plain (n_seg = 0, M <= 64) and grouped
+bool nvfp4_stream_wanted(int M, int N, int Kp, int n_seg);
+int run_nvfp4_stream(const GemmParams &p, hipStream_t st);
+
 // arcq_gemm_mx.hip
 int run_mxfp4_pingpong(const GemmParams &p, hipStream_t st);
 

@@ -49,7 +49,7 @@ constexpr size_t kNoAllocScratchBytes = 8u << 20;
 int noalloc_prepare();
 
 // Overrides for tuning runs, read from the environment once, when the library is first used:
-//   ARCQ_GEMM_KERNEL=<WN><WM>   force a GEMM tile (84 / 82 = 256x256 / 256x128 as eight waves, 44, 42, 22, 21, 11; 214 / 224 = four-stage
+//   ARCQ_GEMM_KERNEL=<WN><WM>   force a GEMM tile (84 / 82 = 256x256 / 256x128 as eight waves, 44, 42, 22, 21; 214 / 224 = four-stage
 //                               ring; 88 = MXFP4 256x256 ping-pong; 168 = NVFP4 with one operand decoded to fp16 ahead, where a workspace is
 //                               given; 1 = skinny, 0 = direct); a number the format has no kernel for is ignored
 //   ARCQ_GEMM_SPLITK=<slices>   force split-K for M <= 512 (1 = never split)

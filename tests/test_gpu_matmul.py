@@ -333,3 +333,23 @@ def test_gemm_workspace_too_small(agemm):
         assert L.arcq_gemm(args, stream) == 0
         out.append(c)
     assert torch.equal(*out) and bool((work == 77).all())
+
+
+@pytest.mark.parametrize("N", [24, 101, 4096, 4104, 8192, 12286, 14336, 18944, 20482, 28672, 33000])
+@pytest.mark.parametrize("M,K,S", [(5, 512, 0), (16, 640, 0), (17, 1024, 128), (32, 832, 64), (33, 1024, 256), (48, 2048, 128), (64, 576, 64)])
+def test_nvfp4_decode_batches(agemm, oracle, M, N, K, S):
+    """NVFP4 decode batches, one pass over the weights: every number of 16-row tiles of either operand, the last ones partly
+    empty, N not a multiple of 4, K' from one step on, ending inside a step and inside a 16-byte window of scale bytes.  Exact
+    products and fp32 sums: the bf16 rounding (2^-9 per element, 1.7e-3 in norm) and the sum's order remain."""
+    (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, K, S, "NVFP4", seed=41)
+    want = oracle_dq(oracle, a, sfa, "NVFP4") @ oracle_dq(oracle, b, sfb, "NVFP4").T * (gx * gw)
+    scale = (torch.tensor(gx, device="cuda"), torch.tensor(gw, device="cuda"))
+    y = agemm.matmul(a, b, sfa, sfb, scale)
+    assert rel_fro(y.float(), want) < 2.5e-3
+    assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
+    res = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
+    assert torch.equal(agemm.matmul(a, b, sfa, sfb, scale, residual=res), y + res)
+    if N % 16 == 0:
+        t, gs = agemm.matmul_swiglu(a, b, sfa, sfb, scale, tensor_scale=True)
+        h = torch.nn.functional.silu(y[:, 0::2]) * y[:, 1::2]
+        assert torch.equal(t, h) and float(gs) == float(h.abs().max().float().cpu() / torch.tensor(2688.0))
