@@ -115,6 +115,29 @@ def lib() -> ctypes.CDLL:
     return L
 
 
+HOST_LIB_PATH = os.path.join(_HERE, "csrc", "_arcq_host.so")
+
+
+class _Host:
+    """_arcq_host.so (csrc/arcq_host.cpp), loaded on the first call: the ordinary case of an operator in one native call
+    that returns None for arguments it does not take."""
+
+    def __getattr__(self, name):
+        lib()
+        if not os.path.exists(HOST_LIB_PATH):
+            raise RuntimeError(f"{HOST_LIB_PATH} is missing: build it with `python -m arcquant_amd.build`")
+        import importlib.util
+        import torch  # noqa: F401  (its libraries first: the module is linked against them)
+        spec = importlib.util.spec_from_file_location("_arcq_host", HOST_LIB_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        for f in ("quantize", "swiglu_quantize", "matmul", "decode_step"):
+            self.__dict__[f] = getattr(module, f)
+        return self.__dict__[name]
+
+
+host = _Host()
+
 PROBE_LIB_PATH = os.path.join(_HERE, "csrc", "libarcq_probe.so")
 _probe = None
 

@@ -45,6 +45,7 @@ def _fmt_id(fmt) -> int:
         raise RuntimeError(f"unknown quantization format {fmt!r} (expected 'NVFP4' or 'MXFP4')") from None
 
 
+_host = _lib.host      # the ordinary case of the operators below; None from it: the checks and the general route here
 _stream = _lib.stream_of
 _on_device = _lib.on_device_of
 
@@ -128,17 +129,20 @@ def reorder_quantize_x(X, reorder_index, KE, *, fmt="NVFP4", global_scale=None):
     global_scale="absmax" forms the NVFP4 tensor scale max|X| / 2688 on the device as part of the call (what the
     reference's callers compute with torch first, model/qLlamaLayer.py:73-77) and returns it as a third value:
     one launch and one pass over X while X fits the chip's LDS (up to 4096 rows of up to 4096 channels)."""
-    return _quantize("arcq_reorder_quantize_x", X, None, 0.0, reorder_index, KE, fmt, global_scale)
+    r = _host.quantize(0, X, None, 0.0, reorder_index, KE, fmt, global_scale)
+    return r if r is not None else _quantize("arcq_reorder_quantize_x", X, None, 0.0, reorder_index, KE, fmt, global_scale)
 
 
 def reorder_quantize_w(W, reorder_index, KE, *, fmt="NVFP4", global_scale=None):
     """agemm.reorder_quantize_w (kernels/src/bindings.cpp:170-210)."""
-    return _quantize("arcq_reorder_quantize_w", W, None, 0.0, reorder_index, KE, fmt, global_scale)
+    r = _host.quantize(1, W, None, 0.0, reorder_index, KE, fmt, global_scale)
+    return r if r is not None else _quantize("arcq_reorder_quantize_w", W, None, 0.0, reorder_index, KE, fmt, global_scale)
 
 
 def rmsnorm_quantize_x(X, W, eps, reorder_index, KE, *, fmt="NVFP4", global_scale=None):
     """agemm.rmsnorm_quantize_x (kernels/src/bindings.cpp:216-254); W is the RMSNorm weight bf16 [K]."""
-    return _quantize("arcq_rmsnorm_quantize_x", X, W, eps, reorder_index, KE, fmt, global_scale)
+    r = _host.quantize(2, X, W, eps, reorder_index, KE, fmt, global_scale)
+    return r if r is not None else _quantize("arcq_rmsnorm_quantize_x", X, W, eps, reorder_index, KE, fmt, global_scale)
 
 
 def tensor_scale(x, divisor=2688.0):
@@ -165,6 +169,9 @@ def swiglu_quantize_x(gate, up, reorder_index, KE, *, fmt="NVFP4", global_scale=
     halves of a fused gate_up output.  global_scale: None / float / 0-dim CUDA tensor;
     "absmax" computes the NVFP4 tensor scale max|t| / 2688 on the device first and returns it
     as a third value."""
+    r = _host.swiglu_quantize(gate, up, reorder_index, KE, fmt, global_scale)
+    if r is not None:
+        return r
     f = _fmt_id(fmt)
     L = _lib.lib()
     for t, name in ((gate, "gate"), (up, "up")):
@@ -249,6 +256,9 @@ def matmul(A, B, SFA, SFB, scale, *, fmt=None, residual=None):
     call (arcq_gemm_workspace_bytes); they sum in another order than arcq_matmul and arcq_matmul_noalloc, whose results
     may then differ by one bf16 rounding.
     """
+    C = _host.matmul(A, B, SFA, SFB, scale, fmt, residual)
+    if C is not None:
+        return C
     _require(A, "A", torch.uint8, 2)
     _require(B, "B", torch.uint8, 2)
     _require(SFA, "SFA", torch.uint8)

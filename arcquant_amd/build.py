@@ -21,6 +21,8 @@ HIP_LIB = os.path.join(CSRC, "libarcq_hip.so")
 # measurement only (plain copy kernels for bench.py and the counter calibration): its own library, so that the
 # product library holds operators only
 PROBE_LIB = os.path.join(CSRC, "libarcq_probe.so")
+# the Python operators' native host path over libarcq_hip.so
+HOST_LIB = os.path.join(CSRC, "_arcq_host.so")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
@@ -68,8 +70,29 @@ def build_probe(force: bool = False, verbose: bool = False) -> str:
     return PROBE_LIB
 
 
+def build_host(force: bool = False, verbose: bool = False) -> str:
+    """The operators' native host path: a CPython module against torch's headers, for torch's interpreter and library."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    src = os.path.join(CSRC, "arcq_host.cpp")
+    if force or _stale(HOST_LIB, [src, os.path.join(HERE, "..", "include", "arcq.h"), HIP_LIB]):
+        rocm = os.path.dirname(os.path.dirname(_hipcc()))
+        includes = [f"-isystem{d}" for d in (*cpp_extension.include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"])]
+        libs = [f"-L{d}" for d in cpp_extension.library_paths()]
+        cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+               f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *includes, "-o", HOST_LIB, src, *libs, "-lc10",
+               "-lc10_hip", "-ltorch_cpu", "-ltorch_python", f"-L{CSRC}", "-l:libarcq_hip.so", "-Wl,-rpath,$ORIGIN"]
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        subprocess.check_call(cmd)
+    return HOST_LIB
+
+
 def build_all(force: bool = False, verbose: bool = False):
-    return (build_hip(force, verbose), build_probe(force, verbose))
+    return (build_hip(force, verbose), build_probe(force, verbose), build_host(force, verbose))
 
 
 def phase_listing(kernel: str, source: str = "arcq_quantize.hip") -> str:

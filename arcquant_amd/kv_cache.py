@@ -326,6 +326,11 @@ class MultiLayerPagedKVCache4Bit:
         if self._rope is None:
             self._rope = rope_tables(self.pages.shape[0] // self.batch_size * self.page_size, self.head_dim,
                                      self.scales.dtype, self.device)
+        sp = self._specs
+        out = _lib.host.decode_step(qkv, num_qo_heads, self._rope[0], self._rope[1], self.positions, sp["kv_data"], sp["kv_param"],
+                                    sp["kv_indptr"], sp["kv_indices"], sp["last_page_offset"], layer_idx)
+        if out is not None:
+            return out
         q = rope_quantize_append(qkv, num_qo_heads, self._rope[0], self._rope[1], self.positions,
                                  layer_idx=layer_idx, **self._specs)
         out = torch.empty_like(q)

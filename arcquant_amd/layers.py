@@ -27,6 +27,7 @@ What differs from the reference, on purpose:
 """
 from __future__ import annotations
 
+import functools
 import math
 from typing import Optional
 
@@ -38,6 +39,18 @@ from . import agemm
 from . import kv_cache as _kvc
 
 NVFP4_RANGE = 448.0 * 6.0   # model/qLlamaLayer.py:74
+
+
+def _no_grad(forward):
+    """torch.no_grad() for a forward pass, entered only where gradients are on: a layer's modules call each other, and entering
+    it costs more than the rest of a module's Python"""
+    @functools.wraps(forward)
+    def run(*args, **kwargs):
+        if not torch.is_grad_enabled():
+            return forward(*args, **kwargs)
+        with torch.no_grad():
+            return forward(*args, **kwargs)
+    return run
 
 
 def _tensor_scale(t: torch.Tensor, signed: bool) -> torch.Tensor:
@@ -129,24 +142,26 @@ class QLinearLayer(nn.Module):
         else:
             self.bias = None
 
-    @torch.no_grad()
+    @_no_grad
     def forward(self, x, residual=None):
         """residual [..., out_features]: added to the output (in the GEMM's epilogue when the layer has
         no bias), same bits as `self(x) + residual`"""
         qx, scale_x, scale, bsz, q_len = x
-        alpha = (scale, self.scale) if isinstance(scale, torch.Tensor) else (float(scale), self.scale)
-        fused = residual is not None and self.bias is None
-        y = agemm.matmul(qx, self.W, scale_x, self.scale_w, alpha, fmt=self.quant_type,
+        own = self._buffers                # (each access through the module would search three dictionaries first)
+        alpha = (scale if isinstance(scale, torch.Tensor) else float(scale), own["scale"])
+        bias = self.bias if "bias" not in own else own["bias"]
+        fused = residual is not None and bias is None
+        y = agemm.matmul(qx, own["W"], scale_x, own["scale_w"], alpha, fmt=self.quant_type,
                          residual=residual.reshape(-1, self.out_features).contiguous() if fused else None)
-        if self.bias is not None:
-            y = y + self.bias
+        if bias is not None:
+            y = y + bias
         if residual is not None and not fused:
             y = y + residual.reshape(-1, self.out_features)
         if bsz is not None:
             return y.reshape(bsz, q_len, -1)
         return y.reshape(q_len, -1)
 
-    @torch.no_grad()
+    @_no_grad
     def forward_swiglu(self, x, tensor_scale):
         """for a gate/up projection whose weight rows alternate gate, up: act_fn(gate) * up [tokens, out/2]
         straight from the GEMM's epilogue (and its NVFP4 tensor scale when asked), same bits as
@@ -169,11 +184,12 @@ class RMSNormQuant(nn.Module):
         self.select_num = int(select_num)
         self.quant_type = quant_type
 
-    @torch.no_grad()
+    @_no_grad
     def forward(self, hidden_states):
         bsz, q_len, _ = hidden_states.shape
         flat = hidden_states.reshape(bsz * q_len, -1).contiguous()
-        A, SFA = agemm.rmsnorm_quantize_x(flat, self.weight, self.variance_epsilon, self.reorder_index,
+        own = self._buffers
+        A, SFA = agemm.rmsnorm_quantize_x(flat, own["weight"], self.variance_epsilon, own["reorder_index"],
                                           self.select_num, fmt=self.quant_type)
         return A, SFA, 1.0, bsz, q_len
 
@@ -236,7 +252,7 @@ class LlamaMLP(nn.Module):
         self.register_buffer("down_reorder_index", down_index.to(torch.int16))
         self.quant_type = quant_type
 
-    @torch.no_grad()
+    @_no_grad
     def forward(self, x, residual=None):
         """x: the tuple of the already quantized (normalised) hidden states; residual: added to the output"""
         sel = self.down_proj.select_num
@@ -270,7 +286,7 @@ class LlamaAttention(nn.Module):
         self.quant_type = quant_type
         self._rope = None                    # cos / sin tables of the fused rotary embedding, built on first use
 
-    @torch.no_grad()
+    @_no_grad
     def forward(self, x, kv_cache=None, past_len=0, layer_idx=0, residual=None):
         """x: quantized hidden states (tuple); residual: added to the output.  kv_cache: None, or (k, v) bf16 [bsz, kv_heads, L, d]
         holding past_len valid positions (the new keys/values are written behind them), or an
@@ -358,7 +374,7 @@ class LlamaDecoderLayer(nn.Module):
         self.mlp = LlamaMLP(self.linears["gate_up"], self.linears["down"], select_num, select_num_down, in_mlp,
                             down_idx, quant_type)
 
-    @torch.no_grad()
+    @_no_grad
     def forward(self, hidden_states, kv_cache=None, past_len=0, layer_idx=0):
         # both residual adds happen in the epilogues of the o and down projections
         h = self.self_attn(self.input_layernorm(hidden_states), kv_cache, past_len, layer_idx, residual=hidden_states)
@@ -376,7 +392,7 @@ class SplitQLinear(nn.Module):
         self.select_num = parts[0].select_num
         self.out_features = sum(p.out_features for p in parts)
 
-    @torch.no_grad()
+    @_no_grad
     def forward(self, x, residual=None):
         y = torch.cat([p(x) for p in self.parts], dim=-1)
         return y if residual is None else y + residual
@@ -392,7 +408,7 @@ class LlamaRMSNorm(nn.Module):
         self.register_buffer("weight", weight.to(torch.bfloat16).contiguous())
         self.variance_epsilon = float(eps)
 
-    @torch.no_grad()
+    @_no_grad
     def forward(self, hidden_states):
         dt = hidden_states.dtype
         h = hidden_states.to(torch.float32)
@@ -493,7 +509,7 @@ class QLlamaDecoderLayer(nn.Module):
             self.post_attention_layernorm = LlamaRMSNorm(norm_weights[1], eps)
         self.fuse_norm = bool(fuse_norm)
 
-    @torch.no_grad()
+    @_no_grad
     def forward(self, hidden_states, kv_cache=None, past_len=0, layer_idx=None):
         li = self.layer_idx if layer_idx is None else layer_idx
         a, m = self.self_attn, self.mlp
@@ -529,7 +545,7 @@ class MixtralExpertMLP(nn.Module):
         self.register_buffer("w2_reorder_index", w2_index.to(torch.int16))
         self.quant_type = quant_type
 
-    @torch.no_grad()
+    @_no_grad
     def forward(self, x):
         xq = quantize_tokens(x, self.w1_reorder_index, self.w13.select_num, self.quant_type)
         if self.interleaved:
@@ -619,7 +635,7 @@ class MixtralSparseMoeBlock(nn.Module):
                 gs2 = None
         return agemm.grouped_matmul(q2, self.w2_W, sf2, self.w2_scale_w, seg, gs2, self.w2_scale if nv else None, fmt=qt)
 
-    @torch.no_grad()
+    @_no_grad
     def forward(self, hidden_states, router_logits: Optional[torch.Tensor] = None):
         bsz, q_len, hid = hidden_states.shape
         x = hidden_states.reshape(-1, hid)
@@ -749,7 +765,7 @@ class QMixtralBlockSparseTop2MLP(nn.Module):
         self.register_buffer("w2_reorder_index", idx2)
         self.quant_type = quant_type
 
-    @torch.no_grad()
+    @_no_grad
     def forward(self, x):
         """x bf16 [tokens of this expert, hidden] (model/qMixtralLayer.py:523-543)"""
         xq = quantize_tokens(x, self.w1_reorder_index, self.w1.select_num, self.quant_type)
@@ -872,7 +888,7 @@ class GraphedDecodeStep:
     def _run(self):
         return self.layer(self.x, self.cache, self.cache.positions, self.layer_idx)
 
-    @torch.no_grad()
+    @_no_grad
     def __call__(self, hidden_states):
         if self.advance:
             self.cache.begin_step()
