@@ -28,6 +28,11 @@ class GemmArgs(ctypes.Structure):
                 ("workspace_bytes", ctypes.c_size_t)]
 
 
+class GemmParts(ctypes.Structure):
+    """arcq_gemm_parts_args of include/arcq.h"""
+    _fields_ = [("n", ctypes.c_int), ("end", ctypes.c_int * 4), ("d_alpha", ctypes.c_void_p * 4), ("bias", ctypes.c_void_p)]
+
+
 class ArcqError(RuntimeError):
     def __init__(self, status: int, where: str):
         self.status = status
@@ -90,6 +95,10 @@ def lib() -> ctypes.CDLL:
     L.arcq_scales_from_absmax.argtypes = [vp, i, f, vp]
     L.arcq_gemm.argtypes = [ctypes.POINTER(GemmArgs), vp]
     L.arcq_gemm.restype = i
+    L.arcq_gemm_parts.argtypes = [ctypes.POINTER(GemmArgs), ctypes.POINTER(GemmParts), vp]
+    L.arcq_gemm_parts.restype = i
+    L.arcq_rmsnorm.argtypes = [vp, vp, f, i, i, vp, f, vp, vp]
+    L.arcq_rmsnorm.restype = i
     L.arcq_gemm_workspace_bytes.argtypes = [i, i, i, i, i]
     L.arcq_gemm_workspace_bytes.restype = sz
     L.arcq_gemm_kernel.argtypes = [i, i, i, i, i, i]

@@ -35,7 +35,7 @@ __all__ = ["matmul", "reorder_quantize_x", "reorder_quantize_w", "rmsnorm_quanti
            "batch_decode_i4", "swiglu_quantize_x", "tensor_scale", "prepare_stream", "release_stream", "dequantize", "check_index",
            "unpack_codes", "scale_values", "grouped_tensor_scale", "grouped_reorder_quantize_x",
            "grouped_swiglu_quantize_x", "grouped_matmul", "moe_route", "moe_combine", "matmul_swiglu",
-           "grouped_matmul_swiglu", "interleave_gate_up"]
+           "grouped_matmul_swiglu", "interleave_gate_up", "matmul_parts", "rmsnorm"]
 
 
 def _fmt_id(fmt) -> int:
@@ -225,7 +225,7 @@ def _workspace_bytes(M, N, Kp, f, n_seg):
 
 
 def _gemm(A, SFA, B, SFB, M, N, Kp, f, c, *, alpha=1.0, da=None, db=None, residual=None, swiglu=0, seg=None, n_seg=0,
-          absmax=None):
+          absmax=None, parts=None):
     """arcq_gemm with the scratch memory its fastest kernel for the problem takes (up to 4 GiB, for the call), from torch's
     allocator; where there is none, by the kernel that takes none"""
     L = _lib.lib()
@@ -240,7 +240,10 @@ def _gemm(A, SFA, B, SFB, M, N, Kp, f, c, *, alpha=1.0, da=None, db=None, residu
                          None if seg is None else seg.data_ptr(), n_seg, None if absmax is None else absmax.data_ptr(),
                          None if work is None else work.data_ptr(), nbytes)
     with _on_device(A):
-        _lib.check(L.arcq_gemm(args, _stream(A)), "arcq_gemm")
+        if parts is None:
+            _lib.check(L.arcq_gemm(args, _stream(A)), "arcq_gemm")
+        else:
+            _lib.check(L.arcq_gemm_parts(args, parts, _stream(A)), "arcq_gemm_parts")
 
 
 def matmul(A, B, SFA, SFB, scale, *, fmt=None, residual=None):
@@ -299,6 +302,61 @@ def matmul(A, B, SFA, SFB, scale, *, fmt=None, residual=None):
     _lib.check(rc, "arcq_matmul")
     del ka, kb
     return C
+
+
+def matmul_parts(A, B, SFA, SFB, scale, part_rows, part_scales, *, fmt, bias=None):
+    """Several linears over one quantized input in one launch: B u8 [N, K'/2] and SFB hold the parts' quantized weights one behind
+    the other (q | k | v), part_rows[k] rows each, with the tensor scales part_scales[k] (0-dim fp32 CUDA tensors); scale: the
+    input's (float or 0-dim fp32 CUDA tensor).  bf16 [M, N], what torch.cat of the parts' ``matmul(..., (scale, part_scales[k]))`` is
+    (sums in another order: one bf16 rounding at most), plus ``bias`` bf16 [N] where given, added in bf16."""
+    _require(A, "A", torch.uint8, 2)
+    _require(B, "B", torch.uint8, 2)
+    _require(SFA, "SFA", torch.uint8)
+    _require(SFB, "SFB", torch.uint8)
+    f = _fmt_id(fmt)
+    M, N, Kp = A.shape[0], B.shape[0], 2 * A.shape[1]
+    G = _lib.GROUP_SIZE[f]
+    if B.shape[1] != A.shape[1] or SFA.numel() != M * (Kp // G) or SFB.numel() != N * (Kp // G):
+        raise RuntimeError("operands of matmul_parts do not match")
+    n = len(part_rows)
+    if not 1 <= n <= 4 or len(part_scales) != n or sum(part_rows) != N or any(r <= 0 or r % 32 for r in part_rows[:-1]) or \
+            part_rows[-1] <= 0 or Kp % 64:
+        raise RuntimeError(f"Value error in matmul_parts: parts of {list(part_rows)} rows, N={N}, K'={Kp}")
+    parts = _lib.GemmParts(n=n)
+    end = 0
+    for k in range(n):
+        t = _require(part_scales[k], "part scale", torch.float32)
+        if t.numel() != 1 or t.device != A.device:
+            raise RuntimeError("part scales must be fp32 scalars on the operands' device")
+        end += part_rows[k]
+        parts.end[k], parts.d_alpha[k] = end, t.data_ptr()
+    if bias is not None:
+        _require(bias, "bias", torch.bfloat16, 1)
+        if bias.numel() != N or bias.device != A.device:
+            raise RuntimeError(f"bias must be bf16 [{N}] on the operands' device")
+        parts.bias = bias.data_ptr()
+    alpha, da, keep = _scalar(scale, A.device)
+    C = torch.empty((M, N), dtype=torch.bfloat16, device=A.device)
+    _gemm(A, SFA, B, SFB, M, N, Kp, f, C, alpha=alpha, da=da, parts=parts)
+    del keep
+    return C
+
+
+def rmsnorm(X, W, eps, *, tensor_scale=False):
+    """RMSNorm as HF's LlamaRMSNorm has it (benchmarks/modeling_arc.py:237-242): bf16(W * bf16(X / sqrt(mean(X^2) + eps))) of bf16
+    X [M, K], W [K]; tensor_scale=True also returns the result's NVFP4 tensor scale max|Y| / 2688 (0-dim fp32 device tensor)."""
+    _require(X, "X", torch.bfloat16, 2)
+    _require(W, "W", torch.bfloat16, 1)
+    M, K = X.shape
+    if W.numel() != K or W.device != X.device:
+        raise RuntimeError(f"RMSNorm weight must have K={K} entries on X's device")
+    Y = torch.empty_like(X)
+    out = torch.empty((), dtype=torch.float32, device=X.device) if tensor_scale else None
+    with _on_device(X):
+        rc = _lib.lib().arcq_rmsnorm(X.data_ptr(), W.data_ptr(), float(eps), M, K, Y.data_ptr(), 2688.0,
+                                     None if out is None else out.data_ptr(), _stream(X))
+    _lib.check(rc, "arcq_rmsnorm")
+    return (Y, out) if tensor_scale else Y
 
 
 # ------------------------------------------------------------------------------------------

@@ -70,7 +70,7 @@ __global__ __launch_bounds__(256) void gemm_mxfp4_direct(GemmParams p) {
       for (int j = 0; j < 2; ++j)
         acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wf[i], xf[j], acc[i][j], 4, 4, 0, ws[i], 0, xs[j]);
   }
-  const float alpha = effective_alpha(p);
+  const Alpha alpha(p);
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(256) void gemm_nvfp4_direct(GemmParams p) {
       for (int j = 0; j < 2; ++j)
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[i], xf[j], acc[i][j], 0, 0, 0);
   }
-  const float alpha = effective_alpha(p);
+  const Alpha alpha(p);
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -432,7 +432,7 @@ __global__ __launch_bounds__(128 * NWM) void gemm_mxfp4_tiled(GemmParams p) {
                                       n_base, wave, lane);
   } else {
     // (the host sends only problems made of whole tiles here: M % BM == 0, N % BN == 0)
-    const float alpha = effective_alpha(p);
+    const Alpha by_column(p);
     for (;;) {
       const bool more = run_left > run_step;  // this workgroup has another tile
       const int cur_n = n_base, cur_m = m_base;
@@ -484,6 +484,7 @@ __global__ __launch_bounds__(128 * NWM) void gemm_mxfp4_tiled(GemmParams p) {
           const int sw = (r_e & (LPR - 1)) << 1;
 #pragma unroll
           for (int i = 0; i < WN; ++i) {
+            const float alpha = by_column.at(p, cur_n + wn0 + 32 * i);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
               const v16f &a = acc[i][j];
@@ -501,7 +502,7 @@ __global__ __launch_bounds__(128 * NWM) void gemm_mxfp4_tiled(GemmParams p) {
             const int swr = (m & (LPR - 1)) << 1;
             uint4 v = *reinterpret_cast<const uint4 *>(region + m * RB + (((2 * t) ^ swr) << 3));
             if (p.residual) {
-              const uint4 rv = *reinterpret_cast<const uint4 *>(p.residual + (cbase - p.c) + (size_t)m * p.N);
+              const uint4 rv = *reinterpret_cast<const uint4 *>(p.residual + (size_t)(cur_m + wm0 + 32 * j + m) * p.ld_residual + cur_n + wn0 + 8 * t);
               v = make_uint4(add_bf16_pair(v.x, rv.x), add_bf16_pair(v.y, rv.y), add_bf16_pair(v.z, rv.z), add_bf16_pair(v.w, rv.w));
             }
             *reinterpret_cast<uint4 *>(cbase + (size_t)m * p.N) = v;
@@ -741,9 +742,10 @@ __device__ __forceinline__ void skinny_reduce_store(const GemmParams &p, v4f (&a
   }
   __syncthreads();
   if (wave > 0) return;
-  const float alpha = effective_alpha(p);
+  const Alpha by_column(p);
 #pragma unroll
   for (int i = 0; i < AT; ++i) {
+    const float alpha = by_column.at(p, ((int)blockIdx.x * AT + i) * 16);
     const int n0 = ((int)blockIdx.x * AT + i) * 16 + 4 * (lane >> 4);
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
@@ -753,17 +755,18 @@ __device__ __forceinline__ void skinny_reduce_store(const GemmParams &p, v4f (&a
       const int m = 16 * j + (lane & 15);
       if (m >= p.M) continue;
       uint16_t *dst = p.c + (size_t)m * p.N + n0;
+      const uint16_t *res = p.residual ? p.residual + (size_t)m * p.ld_residual + n0 : nullptr;
       if (n0 + 3 < p.N && (p.N & 3) == 0) {
         const uint32_t lo = pack_bf16_rne(t[0] * alpha, t[1] * alpha), hi = pack_bf16_rne(t[2] * alpha, t[3] * alpha);
         uint2 v = make_uint2(lo, hi);
-        if (p.residual) v = add_bf16_x4(v, *reinterpret_cast<const uint2 *>(p.residual + (dst - p.c)));
+        if (res) v = add_bf16_x4(v, *reinterpret_cast<const uint2 *>(res));
         *reinterpret_cast<uint2 *>(dst) = v;
       } else {
 #pragma unroll
         for (int v = 0; v < 4; ++v)
           if (n0 + v < p.N) {
             uint32_t hb = f32_to_bf16_bits(t[v] * alpha);
-            if (p.residual) hb = f32_to_bf16_bits(bf16_bits_to_f32(hb) + bf16_bits_to_f32(p.residual[(dst - p.c) + v]));
+            if (res) hb = f32_to_bf16_bits(bf16_bits_to_f32(hb) + bf16_bits_to_f32(res[v]));
             dst[v] = (uint16_t)hb;
           }
       }
@@ -961,16 +964,19 @@ int launch_mxfp4_persistent(const GemmParams &p, hipStream_t st) {
 // reproducible.
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(GemmParams p) {
   const size_t total4 = ((size_t)p.M * p.N) >> 2, plane = (size_t)p.M * p.N;
-  const float alpha = effective_alpha(p);
+  const Alpha by_column(p);
+  const bool columns = p.parts || (p.residual && p.ld_residual == 0);  // something depends on the column
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total4; i += (size_t)gridDim.x * 256) {
     float4 t = reinterpret_cast<const float4 *>(p.partial)[i];
     for (int k = 1; k < p.k_slices; ++k) {
       const float4 u = reinterpret_cast<const float4 *>(p.partial + (size_t)k * plane)[i];
       t.x += u.x, t.y += u.y, t.z += u.z, t.w += u.w;
     }
+    const unsigned n = columns ? (unsigned)i % ((unsigned)p.N >> 2) * 4 : 0;  // (at most 512 rows: fewer than 2^32 quads)
+    const float alpha = by_column.at(p, n);
     const uint32_t lo = pack_bf16_rne(t.x * alpha, t.y * alpha), hi = pack_bf16_rne(t.z * alpha, t.w * alpha);
     uint2 v = make_uint2(lo, hi);
-    if (p.residual) v = add_bf16_x4(v, reinterpret_cast<const uint2 *>(p.residual)[i]);
+    if (p.residual) v = add_bf16_x4(v, p.ld_residual ? reinterpret_cast<const uint2 *>(p.residual)[i] : *reinterpret_cast<const uint2 *>(p.residual + n));
     reinterpret_cast<uint2 *>(p.c)[i] = v;
   }
 }
@@ -1213,6 +1219,7 @@ int check_gemm_args(const void *a_codes, const void *a_scales, const void *b_cod
   p->N = N;
   p->Kp = Kp;
   p->residual = static_cast<const uint16_t *>(residual);
+  p->ld_residual = N;
   return ARCQ_OK;
 }
 
@@ -1242,11 +1249,22 @@ bool nvfp4_f16_wanted(int M, int N, int Kp, int fmt, int n_seg) {
 
 int matmul_impl(const void *a_codes, const void *a_scales, const void *b_codes, const void *b_scales, int M, int N,
                 int Kp, int fmt, float alpha, const float *d_alpha_a, const float *d_alpha_b, const void *residual,
-                void *c, void *workspace, size_t workspace_bytes, void *stream) {
+                void *c, void *workspace, size_t workspace_bytes, void *stream, const arcq_gemm_parts_args *parts = nullptr) {
   GemmParams p;
   const int rc = check_gemm_args(a_codes, a_scales, b_codes, b_scales, M, N, Kp, fmt, alpha, d_alpha_a, d_alpha_b,
                                  residual, c, &p);
   if (rc != ARCQ_OK || M == 0 || N == 0) return rc;
+  if (parts) {
+    p.parts = parts->n;
+    for (int k = 0; k < parts->n; ++k) {
+      if (k + 1 < parts->n) p.part_end[k] = parts->end[k];
+      p.part_alpha[k] = parts->d_alpha[k];
+    }
+    if (parts->bias) {
+      p.residual = static_cast<const uint16_t *>(parts->bias);
+      p.ld_residual = 0;
+    }
+  }
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool scales_aligned = aligned16(a_scales) && aligned16(b_scales);
   if (scales_aligned && workspace && nvfp4_f16_wanted(M, N, Kp, fmt, 0) && workspace_bytes >= nvfp4_f16_bytes(M, N, Kp, false))
@@ -1450,6 +1468,21 @@ extern "C" int arcq_gemm(const arcq_gemm_args *a, void *stream) {
                                     a->d_alpha_a, a->d_alpha_b, a->c, a->d_absmax, a->workspace, a->workspace_bytes, stream);
   return arcq::matmul_impl(a->a_codes, a->a_scales, a->b_codes, a->b_scales, a->M, a->N, a->Kp, a->fmt, a->alpha,
                            a->d_alpha_a, a->d_alpha_b, a->residual, a->c, a->workspace, a->workspace_bytes, stream);
+}
+
+extern "C" int arcq_gemm_parts(const arcq_gemm_args *a, const arcq_gemm_parts_args *parts, void *stream) {
+  if (!a || !parts) return ARCQ_ERR_NULL;
+  if (a->workspace && !arcq::aligned16(a->workspace)) return ARCQ_ERR_ALIGN;
+  if (parts->bias && !arcq::aligned16(parts->bias)) return ARCQ_ERR_ALIGN;
+  if (a->n_seg != 0 || a->swiglu || a->residual || a->d_alpha_b) return ARCQ_ERR_SHAPE;
+  if (parts->n < 1 || parts->n > arcq::kMaxParts) return ARCQ_ERR_SHAPE;
+  for (int k = 0; k < parts->n; ++k) {
+    if (!parts->d_alpha[k]) return ARCQ_ERR_NULL;
+    const int beg = k ? parts->end[k - 1] : 0;
+    if (parts->end[k] <= beg || (k + 1 < parts->n ? parts->end[k] % 32 != 0 : parts->end[k] != a->N)) return ARCQ_ERR_SHAPE;
+  }
+  return arcq::matmul_impl(a->a_codes, a->a_scales, a->b_codes, a->b_scales, a->M, a->N, a->Kp, a->fmt, a->alpha, a->d_alpha_a,
+                           nullptr, nullptr, a->c, a->workspace, a->workspace_bytes, stream, parts);
 }
 
 extern "C" size_t arcq_gemm_workspace_bytes(int M, int N, int Kp, int fmt, int n_seg) {

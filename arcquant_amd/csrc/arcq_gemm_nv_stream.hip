@@ -195,7 +195,7 @@ __device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, 
 
   // the sums of the waves that share a tile meet in LDS, added in the order of K
   float4 *red = reinterpret_cast<float4 *>(smem);
-  const float alpha = effective_alpha(p);
+  const Alpha by_column(p);
   uint32_t amax = 0u;
   constexpr int Q = NT * MT, QB = S::kBatch;
 #pragma unroll
@@ -217,7 +217,8 @@ __device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, 
         const float4 u = red[((w * WN + tn) * QB + t % QB) * 64 + lane];
         v.x += u.x, v.y += u.y, v.z += u.z, v.w += u.w;
       }
-      const int m = m_base + 16 * (q % MT) + r, n = n_base + 16 * (NT * tn + q / MT) + 4 * g;
+      const int n_tile = n_base + 16 * (NT * tn + q / MT), m = m_base + 16 * (q % MT) + r, n = n_tile + 4 * g;
+      const float alpha = by_column.at(p, n_tile);
       if (p.swiglu) {  // N is a multiple of 16: a quad is inside C or outside as a whole
         const uint32_t o = swiglu_pair(pack_bf16_rne(v.x * alpha, v.z * alpha), pack_bf16_rne(v.y * alpha, v.w * alpha));
         if (m < p.M && n < p.N) {
@@ -228,9 +229,10 @@ __device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, 
       }
       if (m >= p.M || n >= p.N) continue;
       uint16_t *dst = p.c + (size_t)m * p.N + n;
+      const uint16_t *res = p.residual ? p.residual + (size_t)m * p.ld_residual + n : nullptr;
       if ((p.N & 3) == 0) {
         uint2 o = make_uint2(pack_bf16_rne(v.x * alpha, v.y * alpha), pack_bf16_rne(v.z * alpha, v.w * alpha));
-        if (p.residual) o = add_bf16_x4(o, *reinterpret_cast<const uint2 *>(p.residual + (dst - p.c)));
+        if (res) o = add_bf16_x4(o, *reinterpret_cast<const uint2 *>(res));
         *reinterpret_cast<uint2 *>(dst) = o;
         continue;
       }
@@ -239,7 +241,7 @@ __device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, 
       for (int e = 0; e < 4; ++e)
         if (n + e < p.N) {
           uint32_t h = f32_to_bf16_bits(f[e] * alpha);
-          if (p.residual) h = f32_to_bf16_bits(bf16_bits_to_f32(h) + bf16_bits_to_f32(p.residual[(dst - p.c) + e]));
+          if (res) h = f32_to_bf16_bits(bf16_bits_to_f32(h) + bf16_bits_to_f32(res[e]));
           dst[e] = (uint16_t)h;
         }
     }

@@ -16,6 +16,8 @@ typedef int v4i __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
+constexpr int kMaxParts = ARCQ_MAX_PARTS;
+
 struct GemmParams {
   const uint8_t *a_codes, *a_scales;  // activations, M rows
   const uint8_t *b_codes, *b_scales;  // weights, N rows
@@ -30,6 +32,7 @@ struct GemmParams {
   // optional residual, bf16 [M,N]: C = bf16(bf16(alpha * acc) + residual), what a bf16 add of the
   // rounded GEMM output and the residual gives
   const uint16_t *residual = nullptr;
+  int ld_residual = 0;  // elements from one of its rows to the next: N, or 0 for one row that is added to all (a bias)
   // grouped GEMM (tiled kernels): rows seg[e] .. seg[e+1]-1 of A and C belong to segment e, whose weights
   // start seg_b_codes / seg_b_scales bytes after those of segment e-1; d_alpha_a / d_alpha_b are arrays
   // indexed by segment.  A workgroup rewrites its copy of these parameters to its segment's sub-problem.
@@ -47,6 +50,11 @@ struct GemmParams {
   // gemm_nvfp4_f16: one operand decoded to fp16 [rows, K'] ahead of the launch (the activations, or the weights
   // where they have fewer rows)
   const uint16_t *f16 = nullptr;
+  // weights made of several parts with a tensor scale each (q | k | v): rows part_end[k - 1] .. part_end[k] - 1 have *part_alpha[k]
+  // in the place of *d_alpha_b.  Multiples of 32: a 16- or 32-column tile of accumulators lies in one part.
+  int parts = 0;
+  int part_end[kMaxParts - 1] = {};
+  const float *part_alpha[kMaxParts] = {};
 };
 
 // arcq_gemm_nv.hip: bytes of the decoded operand, and the GEMM on it
@@ -134,7 +142,7 @@ __device__ __forceinline__ bool enter_segment(GemmParams &p, int &lin) {
   p.a_scales += (size_t)row0 * ksc;
   if (p.f16) p.f16 += (size_t)row0 * p.Kp;
   p.c += (size_t)row0 * (p.swiglu ? p.N >> 1 : p.N);
-  if (p.residual) p.residual += (size_t)row0 * p.N;
+  if (p.residual) p.residual += (size_t)row0 * p.ld_residual;
   p.b_codes += (size_t)e * p.seg_b_codes;
   p.b_scales += (size_t)e * p.seg_b_scales;
   if (p.d_alpha_a) p.d_alpha_a += e;
@@ -163,6 +171,28 @@ __device__ __forceinline__ float effective_alpha(const GemmParams &p) {
   }
   return a;
 }
+
+// What a sum is multiplied by, by the tile of columns that it belongs to (n: the tile's first column, the same for the wave).
+struct Alpha {
+  float a[kMaxParts];
+  __device__ __forceinline__ explicit Alpha(const GemmParams &p) {
+    if (!p.parts) {
+      a[0] = effective_alpha(p);
+      return;
+    }
+#pragma unroll
+    for (int k = 0; k < kMaxParts; ++k)
+      if (k < p.parts) a[k] = p.alpha * (p.d_alpha_a ? *p.d_alpha_a * *p.part_alpha[k] : *p.part_alpha[k]);
+  }
+  __device__ __forceinline__ float at(const GemmParams &p, int n) const {
+    if (!p.parts) return a[0];
+    float v = a[0];
+#pragma unroll
+    for (int k = 1; k < kMaxParts; ++k)
+      if (k < p.parts && n >= p.part_end[k - 1]) v = a[k];
+    return v;
+  }
+};
 
 // These write M0.  The compiler reserves M0 and refuses it on a clobber list ("may lead to undefined
 // behaviour"), so the contract is kept by hand: the kernels that use these helpers contain nothing for
@@ -299,13 +329,14 @@ __device__ __forceinline__ void store_wave_tile_swiglu(const GemmParams &p, cons
 // where it ends inside C, and the address is formed once.  (Both per quad, here and in the store of split-K's partial
 // tiles: 64 x 6144 x 4352, four slices, 17.4 us against 16.3; MXFP4 64 x 4096 x 14592, eight slices, 16.0 against 15.0.)
 template <class Acc>
-__device__ __forceinline__ void store_tile(const GemmParams &p, const Acc &acc, int i, int j, int m0, int n0, int lane, float alpha) {
+__device__ __forceinline__ void store_tile(const GemmParams &p, const Acc &acc, int i, int j, int m0, int n0, int lane, const Alpha &by_column) {
   const int m = m0 + Acc::m(j, lane);
   if (m >= p.M) return;
   const int n_tile = n0 + Acc::kSide * i;
+  const float alpha = by_column.at(p, n_tile);
   const size_t at = (size_t)m * p.N + n_tile + Acc::lane_n(lane);
   uint16_t *dst = p.c + at;
-  const uint16_t *res = p.residual ? p.residual + at : nullptr;
+  const uint16_t *res = p.residual ? p.residual + (size_t)m * p.ld_residual + n_tile + Acc::lane_n(lane) : nullptr;
   const bool quads = (p.N & 3) == 0;  // a quad is 8-byte aligned, and inside C or outside as a whole
   auto store = [&](int q) {
     const float4 v = acc.quad(Acc::kTileQuads * i + q, j);
@@ -374,7 +405,7 @@ __device__ __forceinline__ void store_wave_tile(const GemmParams &p, const Acc &
     }
     return;
   }
-  const float alpha = effective_alpha(p);
+  const Alpha by_column(p);
   constexpr int RB = 2 * Acc::kN;   // bytes per row of the wave tile
   constexpr int LPR = Acc::kN / 8;  // lanes per row when reading 16 bytes each
   static_assert((LPR & (LPR - 1)) == 0, "the swizzle needs a power of two");
@@ -391,12 +422,13 @@ __device__ __forceinline__ void store_wave_tile(const GemmParams &p, const Acc &
     auto read_residual = [&](int first) {
 #pragma unroll
       for (int k = 0; k < RI; ++k)
-        res[k] = *reinterpret_cast<const uint4 *>(p.residual + (cbase - p.c) + (size_t)((first + k) * (64 / LPR) + rr) * p.N);
+        res[k] = *reinterpret_cast<const uint4 *>(p.residual + (size_t)(m0 + (first + k) * (64 / LPR) + rr) * p.ld_residual + n0 + 8 * t);
     };
     wait_dma_and_sync();  // every wave is done reading operands
     if (p.residual) read_residual(0);
 #pragma unroll
-    for (int q = 0; q < Acc::kQuads; ++q)
+    for (int q = 0; q < Acc::kQuads; ++q) {
+      const float alpha = by_column.at(p, n0 + Acc::kSide * (q / Acc::kTileQuads));
 #pragma unroll
       for (int j = 0; j < Acc::kTiles; ++j) {
         const int m = Acc::m(j, lane), c = Acc::n(q, lane) >> 2;  // row and 8-byte chunk of the row
@@ -405,6 +437,7 @@ __device__ __forceinline__ void store_wave_tile(const GemmParams &p, const Acc &
         *reinterpret_cast<uint2 *>(region + m * RB + ((c ^ sw) << 3)) =
             make_uint2(pack_bf16_rne(v.x * alpha, v.y * alpha), pack_bf16_rne(v.z * alpha, v.w * alpha));
       }
+    }
 #pragma unroll
     for (int it0 = 0; it0 < IT; it0 += RI) {
       if (p.residual && it0 > 0) read_residual(it0);
@@ -424,7 +457,7 @@ __device__ __forceinline__ void store_wave_tile(const GemmParams &p, const Acc &
 #pragma unroll
   for (int i = 0; i < Acc::kQuads / Acc::kTileQuads; ++i)
 #pragma unroll
-    for (int j = 0; j < Acc::kTiles; ++j) store_tile(p, acc, i, j, m0, n0, lane, alpha);
+    for (int j = 0; j < Acc::kTiles; ++j) store_tile(p, acc, i, j, m0, n0, lane, by_column);
 }
 
 // The same for the kernels whose waves form a 2 (along N) x NWM (along M) grid, wave = n + 2 * m, of 32x32 tiles.

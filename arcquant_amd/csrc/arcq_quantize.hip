@@ -1366,6 +1366,35 @@ constexpr unsigned kScaleGroups = 8;
 constexpr int kScaleLine = 32;  // words between the pairs: 128 bytes
 constexpr unsigned kScaleSingle = 32;  // launches of up to this many workgroups meet on one pair
 
+// A workgroup's maximum (bits of a non-negative float) on its way into *out; called by one thread of every workgroup.
+__device__ __forceinline__ void meet_for_scale(uint32_t m, float divisor, uint32_t *ws, float *out) {
+  // Every step below waits for the one before it to return (about half a microsecond each), so there are as few
+  // as the protocol allows: maximum, arrival; the last arrival of a group arrives at the top; the last arrival
+  // there reads the groups' maxima.  Up to kScaleSingle workgroups meet on the top pair alone.
+  uint32_t *top = ws;
+  if (gridDim.x > kScaleSingle) {
+    const int grp = (int)blockIdx.x % kScaleGroups;
+    const uint32_t members = ((uint32_t)gridDim.x - (uint32_t)grp + kScaleGroups - 1u) / kScaleGroups;
+    uint32_t *gw = ws + (1 + grp) * kScaleLine;  // this group's (maximum, counter)
+    const uint32_t old = atomicMax(gw, m);
+    if (atomicAdd(gw + 1, 1u + (old >> 31)) != members - 1u) return;  // old < 2^31: the add waits for the maximum
+    if (atomicAdd(top + 1, 1u) != kScaleGroups - 1u) return;
+    // every group's last arrival has been counted, each after all of its group's maxima: read them, zero them
+    for (int q = 0; q < kScaleGroups; ++q) {
+      const uint32_t v = atomicExch(ws + (1 + q) * kScaleLine, 0u);
+      m = q == 0 ? v : (v > m ? v : m);
+      __hip_atomic_store(ws + (1 + q) * kScaleLine + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  } else {
+    const uint32_t old = atomicMax(top, m);
+    if (atomicAdd(top + 1, 1u + (old >> 31)) != gridDim.x - 1u) return;
+    m = atomicExch(top, 0u);
+  }
+  __hip_atomic_store(top + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const float scale = u2f(m) / divisor;
+  *out = scale == 0.0f ? 1.0f : scale;
+}
+
 template <bool SWIGLU>
 __global__ __launch_bounds__(kScaleThreads) void tensor_scale_kernel(const uint16_t *x, const uint16_t *up, size_t ld, int rows,
                                                                       int K, float divisor, uint32_t *ws, float *out) {
@@ -1436,31 +1465,80 @@ __global__ __launch_bounds__(kScaleThreads) void tensor_scale_kernel(const uint1
   __syncthreads();
   if (threadIdx.x != 0) return;
   for (int w = 1; w < (int)(blockDim.x >> 6); ++w) m = wave_max[w] > m ? wave_max[w] : m;
-  // Every step below waits for the one before it to return (about half a microsecond each), so there are as few
-  // as the protocol allows: maximum, arrival; the last arrival of a group arrives at the top; the last arrival
-  // there reads the groups' maxima.  Up to kScaleSingle workgroups meet on the top pair alone.
-  uint32_t *top = ws;
-  if (gridDim.x > kScaleSingle) {
-    const int grp = (int)blockIdx.x % kScaleGroups;
-    const uint32_t members = ((uint32_t)gridDim.x - (uint32_t)grp + kScaleGroups - 1u) / kScaleGroups;
-    uint32_t *gw = ws + (1 + grp) * kScaleLine;  // this group's (maximum, counter)
-    const uint32_t old = atomicMax(gw, m);
-    if (atomicAdd(gw + 1, 1u + (old >> 31)) != members - 1u) return;  // old < 2^31: the add waits for the maximum
-    if (atomicAdd(top + 1, 1u) != kScaleGroups - 1u) return;
-    // every group's last arrival has been counted, each after all of its group's maxima: read them, zero them
-    for (int q = 0; q < kScaleGroups; ++q) {
-      const uint32_t v = atomicExch(ws + (1 + q) * kScaleLine, 0u);
-      m = q == 0 ? v : (v > m ? v : m);
-      __hip_atomic_store(ws + (1 + q) * kScaleLine + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  meet_for_scale(m, divisor, ws, out);
+}
+
+// RMSNorm of the reference's layers as the model has it in front of a quantizer (benchmarks/modeling_arc.py:237-242; the fused
+// form is the quantizers' MODE_NORM): y = bf16(gamma * bf16(x * rstd)), the mean of the squares in fp64, rstd correctly rounded.
+// With `out`, also the NVFP4 tensor scale of y, which its quantizer reads.  A read of x and a write of y, a wave per row whose
+// lanes keep their 16-byte chunks in registers (KEEP: rows of up to 4096 channels; longer ones are read again); beyond 256
+// workgroups of sixteen waves the rows take turns.  2331 rows of 3584: 8.4 us, 10.5 with the scale; eight launches of torch took
+// 81, the scale 10.
+template <bool KEEP>
+__global__ __launch_bounds__(1024) void rmsnorm_rows_kernel(const uint16_t *x, const uint16_t *gamma, float eps, int rows, int K,
+                                                            uint16_t *y, float divisor, uint32_t *ws, float *out) {
+  __shared__ uint32_t wave_max[16];
+  constexpr int CH = KEEP ? 8 : 1;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, chunks = K >> 3;
+  uint32_t top = 0u;
+  auto squares = [](double ss, const uint4 &q) {
+    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const double d0 = (double)u2f(w[j] << 16), d1 = (double)u2f(w[j] & 0xffff0000u);
+      ss = __builtin_fma(d0, d0, ss);
+      ss = __builtin_fma(d1, d1, ss);
     }
-  } else {
-    const uint32_t old = atomicMax(top, m);
-    if (atomicAdd(top + 1, 1u + (old >> 31)) != gridDim.x - 1u) return;
-    m = atomicExch(top, 0u);
+    return ss;
+  };
+  for (int r = blockIdx.x * 16 + wave; r < rows; r += gridDim.x * 16) {
+    const uint4 *src = reinterpret_cast<const uint4 *>(x + (size_t)r * K);
+    uint4 *dst = reinterpret_cast<uint4 *>(y + (size_t)r * K);
+    uint4 keep[CH];
+    double ss = 0.0;
+    if constexpr (KEEP) {
+#pragma unroll
+      for (int i = 0; i < CH; ++i) keep[i] = 64 * i + lane < chunks ? src[64 * i + lane] : make_uint4(0, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < CH; ++i) ss = squares(ss, keep[i]);
+    } else {
+#pragma unroll 4
+      for (int c = lane; c < chunks; c += 64) ss = squares(ss, src[c]);
+    }
+    ss = wave_sum_to_lane63(ss);
+    const uint64_t bits = __builtin_bit_cast(uint64_t, ss);
+    const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)bits, 63), hi = __builtin_amdgcn_readlane((int)(uint32_t)(bits >> 32), 63);
+    const double tot = __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+    const float rstd = 1.0f / sqrtf((float)(tot / (double)K) + eps);
+    auto finish = [&](const uint4 &q, int c) {
+      const uint4 g4 = reinterpret_cast<const uint4 *>(gamma)[c];
+      const uint32_t w[4] = {q.x, q.y, q.z, q.w}, g[4] = {g4.x, g4.y, g4.z, g4.w};
+      uint32_t t[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t h = pack_bf16_rne(u2f(w[j] << 16) * rstd, u2f(w[j] & 0xffff0000u) * rstd);
+        t[j] = pack_bf16_rne(u2f(h << 16) * u2f(g[j] << 16), u2f(h & 0xffff0000u) * u2f(g[j] & 0xffff0000u));
+        top = max(top, max((t[j] << 16) & 0x7fffffffu, t[j] & 0x7fff0000u));
+      }
+      dst[c] = make_uint4(t[0], t[1], t[2], t[3]);
+    };
+    if constexpr (KEEP) {
+#pragma unroll
+      for (int i = 0; i < CH; ++i)
+        if (64 * i + lane < chunks) finish(keep[i], 64 * i + lane);
+    } else {
+#pragma unroll 4
+      for (int c = lane; c < chunks; c += 64) finish(src[c], c);
+    }
   }
-  __hip_atomic_store(top + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const float scale = u2f(m) / divisor;
-  *out = scale == 0.0f ? 1.0f : scale;
+  if (!out) return;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, o));
+  if (lane == 0) wave_max[wave] = top;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < 16; ++w) top = max(top, wave_max[w]);
+  meet_for_scale(top, divisor, ws, out);
 }
 
 // Per-segment maxima for grouped launches (rows sorted by segment): max |x|, or max |act_fn(gate) * up|,
@@ -1991,6 +2069,26 @@ int arcq_tensor_scale(const void *x, const void *up, int ld, int M, int K, float
     hipLaunchKernelGGL(arcq::tensor_scale_kernel<false>, dim3(grid), dim3(threads), 0, st,
                        static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(nullptr), (size_t)ld, M, K, divisor, ws,
                        d_scale);
+  ARCQ_HIP_TRY(hipGetLastError());
+  return ARCQ_OK;
+}
+
+int arcq_rmsnorm(const void *x, const void *gamma, float eps, int M, int K, void *y, float divisor, float *d_scale, void *stream) {
+  if (M < 0 || K < 8 || K % 8 != 0 || K > 16384 || !(eps >= 0.0f) || (d_scale && !(divisor > 0.0f))) return ARCQ_ERR_SHAPE;
+  if (!gamma || (M > 0 && (!x || !y))) return ARCQ_ERR_NULL;
+  if (!arcq::aligned16(x) || !arcq::aligned16(gamma) || !arcq::aligned16(y)) return ARCQ_ERR_ALIGN;
+  if (M == 0 && !d_scale) return ARCQ_OK;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  uint32_t *ws = nullptr;
+  if (d_scale) {
+    int status = ARCQ_OK;
+    ws = static_cast<uint32_t *>(arcq::stream_workspace(arcq::kWsTensorScale, st, &status));
+    if (!ws) return status;
+  }
+  const dim3 grid((unsigned)std::min(256, std::max(1, (M + 15) / 16)));  // M == 0: the scale of an empty tensor, 1
+  const auto kernel = K <= 4096 ? arcq::rmsnorm_rows_kernel<true> : arcq::rmsnorm_rows_kernel<false>;
+  hipLaunchKernelGGL(kernel, grid, dim3(1024), 0, st, static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(gamma), eps, M, K,
+                     static_cast<uint16_t *>(y), divisor, ws, d_scale);
   ARCQ_HIP_TRY(hipGetLastError());
   return ARCQ_OK;
 }

@@ -381,20 +381,74 @@ class LlamaDecoderLayer(nn.Module):
         return self.mlp(self.post_attention_layernorm(h), residual=h)
 
 
+def _unhooked(module, cls):
+    """a call of the module is cls.forward and nothing else"""
+    return type(module) is cls and "forward" not in module.__dict__ and not (
+        module._forward_hooks or module._forward_pre_hooks or nn.modules.module._global_forward_hooks or
+        nn.modules.module._global_forward_pre_hooks)
+
+
 class SplitQLinear(nn.Module):
     """Several QLinearLayers over one quantized input, outputs concatenated along the features: q / k / v
     (or gate / up) kept as the reference keeps them, each with the tensor scale of its own weight
-    (model/qLinearLayer.py:25-28), where the fused layers above have one scale for the stacked weight."""
+    (model/qLinearLayer.py:25-28), where the fused layers above have one scale for the stacked weight.
+
+    The parts' quantized weights (and biases) are put one behind the other in one allocation, of which the parts hold
+    their pieces, and run as one GEMM that scales the columns by part, as long as they still lie so."""
 
     def __init__(self, parts):
         super().__init__()
         self.parts = nn.ModuleList(parts)
         self.select_num = parts[0].select_num
         self.out_features = sum(p.out_features for p in parts)
+        names = ["W", "scale_w"] + (["bias"] if all(p.bias is not None for p in parts) else [])
+        if len({p.W.shape[1] for p in parts}) == 1:
+            for name in names:
+                joint, at = torch.cat([getattr(p, name) for p in parts]), 0
+                for p in parts:
+                    n = getattr(p, name).shape[0]
+                    setattr(p, name, joint[at:at + n])
+                    at += n
+
+    def _joint(self, name):
+        """the parts' tensors as the one that they are pieces of; None if they are not"""
+        ts = [p._buffers.get(name) for p in self.parts]
+        if any(t is None or not t.is_contiguous() for t in ts):
+            return None
+        base = ts[0].untyped_storage().data_ptr()
+        at = ts[0].data_ptr()
+        for t in ts:
+            if t.data_ptr() != at or t.untyped_storage().data_ptr() != base or t.dtype != ts[0].dtype or t.shape[1:] != ts[0].shape[1:]:
+                return None
+            at += t.numel() * t.element_size()
+        return torch.as_strided(ts[0], (sum(t.shape[0] for t in ts), *ts[0].shape[1:]), ts[0].stride())
+
+    def _as_one(self, x):
+        """one GEMM over all parts, or None where they have to run one by one"""
+        qx, scale_x, scale, _, _ = x
+        ps = list(self.parts)
+        if not 2 <= len(ps) <= 4 or not all(_unhooked(p, QLinearLayer) and p.quant_type == ps[0].quant_type for p in ps) or \
+                any(p.out_features % 32 for p in ps) or not isinstance(scale, (float, int, torch.Tensor)):
+            return None
+        bias = None
+        if any(p.bias is not None for p in ps):
+            bias = self._joint("bias")
+            if bias is None or bias.dtype != torch.bfloat16:
+                return None
+        W, scale_w = self._joint("W"), self._joint("scale_w")
+        scales = [p._buffers["scale"] for p in ps]
+        if W is None or scale_w is None or any(s.dtype != torch.float32 or s.device != W.device for s in scales):
+            return None
+        return agemm.matmul_parts(qx, W, scale_x, scale_w, scale, [p.out_features for p in ps], scales, fmt=ps[0].quant_type,
+                                  bias=bias)
 
     @_no_grad
     def forward(self, x, residual=None):
-        y = torch.cat([p(x) for p in self.parts], dim=-1)
+        y = self._as_one(x)
+        if y is None:
+            y = torch.cat([p(x) for p in self.parts], dim=-1)
+        else:
+            y = y.reshape(x[3], x[4], -1) if x[3] is not None else y.reshape(x[4], -1)
         return y if residual is None else y + residual
 
 
@@ -408,8 +462,27 @@ class LlamaRMSNorm(nn.Module):
         self.register_buffer("weight", weight.to(torch.bfloat16).contiguous())
         self.variance_epsilon = float(eps)
 
+    def _in_one_launch(self, hidden_states):
+        """bf16 rows that arcq_rmsnorm takes, as [rows, K]; None for others"""
+        w, x = self._buffers["weight"], hidden_states
+        k = x.shape[-1] if x.dim() else 0
+        if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not x.is_cuda or x.device != w.device or x.dim() < 2 or \
+                w.shape != (k,) or k % 8 or not 8 <= k <= 16384 or not self.variance_epsilon >= 0:
+            return None
+        flat = x.reshape(-1, k).contiguous()
+        return flat if flat.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and w.is_contiguous() else None
+
+    @_no_grad
+    def forward_with_scale(self, hidden_states):
+        """the result [rows, K] and its NVFP4 tensor scale, or None where they do not come out of one launch"""
+        flat = self._in_one_launch(hidden_states)
+        return None if flat is None else agemm.rmsnorm(flat, self.weight, self.variance_epsilon, tensor_scale=True)
+
     @_no_grad
     def forward(self, hidden_states):
+        flat = self._in_one_launch(hidden_states)
+        if flat is not None:
+            return agemm.rmsnorm(flat, self.weight, self.variance_epsilon).view(hidden_states.shape)
         dt = hidden_states.dtype
         h = hidden_states.to(torch.float32)
         h = h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + self.variance_epsilon)
@@ -509,17 +582,24 @@ class QLlamaDecoderLayer(nn.Module):
             self.post_attention_layernorm = LlamaRMSNorm(norm_weights[1], eps)
         self.fuse_norm = bool(fuse_norm)
 
+    def _norm_and_quantize(self, norm, x, reorder_index, select_num):
+        """the norm, then the quantizer under the tensor scale of its result; the norm's launch forms that too"""
+        if self.fuse_norm:
+            return norm(x)
+        if self.quant_type == "NVFP4" and x.dim() == 3 and _unhooked(norm, LlamaRMSNorm):
+            r = norm.forward_with_scale(x)
+            if r is not None:
+                qx, sfx = agemm.reorder_quantize_x(r[0], reorder_index, select_num, fmt="NVFP4", global_scale=r[1])
+                return qx, sfx, r[1], x.shape[0], x.shape[1]
+        return quantize_tokens(norm(x), reorder_index, select_num, self.quant_type)
+
     @_no_grad
     def forward(self, hidden_states, kv_cache=None, past_len=0, layer_idx=None):
         li = self.layer_idx if layer_idx is None else layer_idx
         a, m = self.self_attn, self.mlp
-        t = self.input_layernorm(hidden_states)
-        if not self.fuse_norm:
-            t = quantize_tokens(t, a.q_reorder_index, a.q_proj.select_num, self.quant_type)
+        t = self._norm_and_quantize(self.input_layernorm, hidden_states, a.q_reorder_index, a.q_proj.select_num)
         h = a(t, kv_cache, past_len, li, residual=hidden_states)
-        t = self.post_attention_layernorm(h)
-        if not self.fuse_norm:
-            t = quantize_tokens(t, m.up_reorder_index, m.up_proj.select_num, self.quant_type)
+        t = self._norm_and_quantize(self.post_attention_layernorm, h, m.up_reorder_index, m.up_proj.select_num)
         return m(t, residual=h)
 
 

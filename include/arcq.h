@@ -157,6 +157,13 @@ int arcq_swiglu_absmax(const void *gate, const void *up, int ld, int M, int K, f
 int arcq_tensor_scale(const void *x, const void *up, int ld, int M, int K, float divisor, float *d_scale, void *stream);
 
 /*
+ * RMSNorm by itself: y = bf16(gamma * bf16(x / sqrt(mean(x^2) + eps))), bf16 [M, K] (benchmarks/modeling_arc.py:237-242), for layers
+ * that keep the model's norm in front of a quantizer (model/qLlamaLayer.py:180-197).  d_scale: NULL, or the NVFP4 tensor scale
+ * max |y| / divisor of the result as arcq_tensor_scale gives it.  K a multiple of 8, up to 16384.
+ */
+int arcq_rmsnorm(const void *x, const void *gamma, float eps, int M, int K, void *y, float divisor, float *d_scale, void *stream);
+
+/*
  * The tensor scale and the activation quantizer under it as one call: what the reference's callers write as
  * scale = x.abs().max() / (448 * 6) followed by reorder_quantize_x(x / scale, ...) (model/qLlamaLayer.py:73-77,
  * kernels/src/bindings.cpp:122-163).  d_scale receives max |x| / divisor (1 for an all-zero tensor); codes and
@@ -224,6 +231,22 @@ typedef struct arcq_gemm_args {
 } arcq_gemm_args;
 int arcq_gemm(const arcq_gemm_args *args, void *stream);
 size_t arcq_gemm_workspace_bytes(int M, int N, int Kp, int fmt, int n_seg);
+
+/*
+ * Several linears over one quantized input as one GEMM: their quantized weights lie behind one another in b_codes / b_scales
+ * (q | k | v, gate | up), rows end[k-1] .. end[k]-1 of part k carrying the tensor scale *d_alpha[k] (device).  What a GEMM per
+ * part with d_alpha_b = d_alpha[k] and a concatenation of the outputs gives (the order of the sums aside); with `bias`, bf16 [N], what
+ * adding it to the rounded output in bf16 gives (model/qLinearLayer.py:69-76).  args: n_seg = 0, swiglu = 0, no residual, no
+ * d_alpha_b.  end[n-1] = N, the others multiples of 32; at most ARCQ_MAX_PARTS parts.
+ */
+#define ARCQ_MAX_PARTS 4
+typedef struct {
+  int n;
+  int end[ARCQ_MAX_PARTS];
+  const float *d_alpha[ARCQ_MAX_PARTS];
+  const void *bias;
+} arcq_gemm_parts_args;
+int arcq_gemm_parts(const arcq_gemm_args *args, const arcq_gemm_parts_args *parts, void *stream);
 /* The kernel arcq_gemm takes for a problem when it has the workspace and aligned operands, by the numbers that the
  * ARCQ_GEMM_KERNEL environment variable forces (168 = one operand decoded ahead, 88 = MXFP4 ping-pong, ..., 1 = skinny,
  * 0 = direct); -1 for arguments arcq_gemm refuses.  NVFP4 problems of up to 64 rows, and experts of fewer than 96 on average, are

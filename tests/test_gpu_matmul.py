@@ -353,3 +353,28 @@ def test_nvfp4_decode_batches(agemm, oracle, M, N, K, S):
         t, gs = agemm.matmul_swiglu(a, b, sfa, sfb, scale, tensor_scale=True)
         h = torch.nn.functional.silu(y[:, 0::2]) * y[:, 1::2]
         assert torch.equal(t, h) and float(gs) == float(h.abs().max().float().cpu() / torch.tensor(2688.0))
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("M,rows", [(1, (512, 64, 32)), (17, (4096, 32, 520)), (64, (96, 100)), (64, (4096,)), (100, (3584, 512, 512)), (512, (1024, 2048, 512, 512)),
+                                    (300, (256, 260)), (700, (2048, 2048)), (2100, (6400, 1000))])
+def test_matmul_parts(agemm, M, rows, fmt):
+    """Several linears as one GEMM: the columns of each under its own scale (in every epilogue: decode batches, split-K, tiles
+    inside C and across its edge, parts that end inside a tile), against a GEMM per part; the bias exactly as a bf16 add.
+    Another tile sums in another order: one bf16 rounding at most, in fewer than one value in a hundred."""
+    N, K, S = sum(rows), 1024, 128
+    (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, K, S, fmt, seed=51)
+    dgx = torch.tensor(gx, device="cuda")
+    scales = [torch.tensor(0.5 + k, device="cuda") for k in range(len(rows))]
+    y = agemm.matmul_parts(a, b, sfa, sfb, dgx, rows, scales, fmt=fmt)
+    at, ones = 0, []
+    for n, s in zip(rows, scales):
+        ones.append(agemm.matmul(a, b[at:at + n], sfa, sfb.view(N, -1)[at:at + n].reshape(-1), (dgx, s), fmt=fmt))
+        at += n
+    one = torch.cat(ones, dim=1)
+    assert rel_fro(y.float(), one.float()) < 1e-3
+    assert torch.allclose(y.float(), one.float(), rtol=2 ** -7, atol=1e-4 * float(one.float().abs().max()))
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16).cuda()
+    assert torch.equal(agemm.matmul_parts(a, b, sfa, sfb, dgx, rows, scales, fmt=fmt, bias=bias), y + bias)
+    with pytest.raises(RuntimeError):
+        agemm.matmul_parts(a, b, sfa, sfb, dgx, (N - 16, 16), scales[:1] * 2, fmt=fmt)

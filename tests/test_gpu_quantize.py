@@ -451,3 +451,27 @@ def test_swiglu_tensor_scale_every_split(agemm, M, K, special):
     for _ in range(2):
         got = agemm.swiglu_quantize_x(gate, up, idx, 0, fmt="NVFP4", global_scale="absmax")[2]
         assert torch.equal(got.reshape(()).isnan(), want.isnan()) and (want.isnan() or float(got) == float(want))
+
+
+@pytest.mark.parametrize("M,K", [(1, 64), (5, 4096), (16, 4096), (17, 3584), (300, 520), (4099, 1024), (33, 4104), (9, 16384), (2, 8)])
+def test_rmsnorm(oracle, M, K):
+    """RMSNorm by itself against the oracle's normed rows, bit for bit, and the tensor scale of the result as arcq_tensor_scale
+    forms it; a row of zeros, and rows with an infinity and a NaN as torch has them."""
+    from arcquant_amd import agemm
+    x, gam = recipes.activations(M, K, seed=61), recipes.gamma(K, seed=62)
+    if M > 4:
+        x[3] = 0
+    y, gs = agemm.rmsnorm(x.cuda(), gam.cuda(), 1e-5, tensor_scale=True)
+    # torch's 1 / sqrt may be one fp32 step off: a bf16 step (2^-7) in h at a midpoint, and another in its product with gamma
+    h = (x.float() * (1.0 / torch.sqrt(x.double().pow(2).mean(-1, keepdim=True).float() + 1e-5))).to(torch.bfloat16)
+    assert torch.allclose(y.cpu().float(), (gam * h).float(), rtol=2 ** -6) and (y.cpu() != gam * h).float().mean() < 1e-3
+    if K % 32 == 0:
+        want = oracle.rmsnorm_quantize_x(x, gam, 1e-5, None, 0, "NVFP4", want_normed=True)["normed"]
+        assert torch.equal(y.cpu().view(torch.int16), torch.from_numpy(want.astype("int16")))
+    assert float(gs) == float(agemm.tensor_scale(y)) and torch.equal(agemm.rmsnorm(x.cuda(), gam.cuda(), 1e-5), y)
+    x[0, K // 2], x[M - 1, 0] = float("inf"), float("nan")
+    odd = agemm.rmsnorm(x.cuda(), gam.cuda(), 1e-5).float().cpu()
+    xf = x.float()
+    ref = (gam * (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + 1e-5)).to(torch.bfloat16)).float()
+    assert torch.equal(torch.isnan(odd), torch.isnan(ref))
+    assert agemm.rmsnorm(x[:0].cuda(), gam.cuda(), 1e-5, tensor_scale=True)[1].item() == 1.0
