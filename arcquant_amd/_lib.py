@@ -99,6 +99,8 @@ def lib() -> ctypes.CDLL:
     L.arcq_gemm_parts.restype = i
     L.arcq_rmsnorm.argtypes = [vp, vp, f, i, i, vp, f, vp, vp]
     L.arcq_rmsnorm.restype = i
+    L.arcq_attention_prefill.argtypes = [vp, i, vp, i, vp, i, i, i, i, i, i, f, vp, i, vp]
+    L.arcq_attention_prefill.restype = i
     L.arcq_gemm_workspace_bytes.argtypes = [i, i, i, i, i]
     L.arcq_gemm_workspace_bytes.restype = sz
     L.arcq_gemm_kernel.argtypes = [i, i, i, i, i, i]

@@ -16,7 +16,7 @@ import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
-HIP_SOURCES = ["arcq_common.hip", "arcq_quantize.hip", "arcq_gemm.hip", "arcq_gemm_nv.hip", "arcq_gemm_nv_stream.hip", "arcq_gemm_mx.hip", "arcq_kvcache.hip", "arcq_moe.hip"]
+HIP_SOURCES = ["arcq_common.hip", "arcq_quantize.hip", "arcq_gemm.hip", "arcq_gemm_nv.hip", "arcq_gemm_nv_stream.hip", "arcq_gemm_mx.hip", "arcq_kvcache.hip", "arcq_moe.hip", "arcq_attention.hip"]
 HIP_LIB = os.path.join(CSRC, "libarcq_hip.so")
 # measurement only (plain copy kernels for bench.py and the counter calibration): its own library, so that the
 # product library holds operators only

@@ -1472,8 +1472,8 @@ __global__ __launch_bounds__(kScaleThreads) void tensor_scale_kernel(const uint1
 // form is the quantizers' MODE_NORM): y = bf16(gamma * bf16(x * rstd)), the mean of the squares in fp64, rstd correctly rounded.
 // With `out`, also the NVFP4 tensor scale of y, which its quantizer reads.  A read of x and a write of y, a wave per row whose
 // lanes keep their 16-byte chunks in registers (KEEP: rows of up to 4096 channels; longer ones are read again); beyond 256
-// workgroups of sixteen waves the rows take turns.  2331 rows of 3584: 8.4 us, 10.5 with the scale; eight launches of torch took
-// 81, the scale 10.
+// workgroups of sixteen waves the rows take turns.  2331 rows of 3584, with the scale: 14.4 us; eight launches of torch took 81,
+// the scale 10.
 template <bool KEEP>
 __global__ __launch_bounds__(1024) void rmsnorm_rows_kernel(const uint16_t *x, const uint16_t *gamma, float eps, int rows, int K,
                                                             uint16_t *y, float divisor, uint32_t *ws, float *out) {

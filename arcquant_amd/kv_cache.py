@@ -112,6 +112,26 @@ def rope(qkv, q_len, pos0, num_qo_heads, num_kv_heads, cos_table, sin_table):
     return q, k
 
 
+def attention_prefill(q, k, v, q_len):
+    """Causal attention of whole prompts over their own keys (model/qLlamaLayer.py:340-370): q [tokens, heads, 128], k [tokens,
+    kv heads, 128] bf16 contiguous, v [tokens, kv heads * 128] bf16 with rows possibly strided (a slice of the fused projection's
+    output), q_len tokens per sequence.  Returns [tokens, heads * 128]; None for operands that arcq_attention_prefill does not take."""
+    tokens, heads, d = q.shape
+    kv_heads = k.shape[1]
+    ld = v.stride(0) if tokens > 1 else v.shape[1]
+    if d != 128 or any(t.dtype != torch.bfloat16 or not t.is_cuda or t.device != q.device or t.data_ptr() % 16 for t in (q, k, v)) or \
+            not (q.is_contiguous() and k.is_contiguous()) or v.stride(1) != 1 or ld % 8 or ld < v.shape[1] or q_len < 1 or tokens % q_len or \
+            tuple(k.shape) != (tokens, kv_heads, d) or tuple(v.shape) != (tokens, kv_heads * d) or heads % kv_heads or \
+            2 * q_len * max(ld, kv_heads * d) >= 1 << 32 or tokens * heads >= 1 << 30:
+        return None
+    o = torch.empty(tokens, heads * d, dtype=q.dtype, device=q.device)
+    with _lib.on_device_of(q):
+        rc = _lib.lib().arcq_attention_prefill(_ptr(q), heads * d, _ptr(k), kv_heads * d, _ptr(v), int(ld), tokens // q_len,
+                                               int(q_len), heads, kv_heads, d, 1.0 / math.sqrt(d), _ptr(o), heads * d, _stream(q))
+    _lib.check(rc, "arcq_attention_prefill")
+    return o
+
+
 def rope_quantize_append(qkv, num_qo_heads, cos_table, sin_table, positions, kv_data, kv_param, kv_indptr, kv_indices,
                          last_page_offset, layer_idx, q_out=None):
     """One decode step between the qkv projection and the attention (model/qLlamaLayer.py:316-327):

@@ -302,6 +302,7 @@ class LlamaAttention(nn.Module):
             return self.o_proj(quantize_tokens(out, self.o_reorder_index, self.o_proj.select_num, self.quant_type),
                                residual)
         v = qkv[..., (nh + nkv) * d:].view(bsz, q_len, nkv, d).transpose(1, 2)
+        rows = None
         if isinstance(past_len, int) and d == 128:
             # rotary embedding of q and k in one pass over the projection output (same values as
             # rotary_pos_emb below: every product and the sum rounded to bf16)
@@ -309,6 +310,7 @@ class LlamaAttention(nn.Module):
             if self._rope is None or self._rope[0].shape[0] < need:
                 self._rope = _kvc.rope_tables(max(need, 4096), d, qkv.dtype, qkv.device)
             q, k = _kvc.rope(qkv.view(bsz * q_len, -1), q_len, past_len, nh, nkv, *self._rope)
+            rows = (q, k, qkv.view(bsz * q_len, -1)[:, (nh + nkv) * d:(nh + 2 * nkv) * d])
             q = q.view(bsz, q_len, nh, d).transpose(1, 2)
             k = k.view(bsz, q_len, nkv, d).transpose(1, 2)
         else:
@@ -327,6 +329,11 @@ class LlamaAttention(nn.Module):
             kc[:, :, past_len:past_len + q_len] = k
             vc[:, :, past_len:past_len + q_len] = v
             k, v = kc[:, :, :past_len + q_len], vc[:, :, :past_len + q_len]
+        if rows is not None and kv_cache is None and past_len == 0:
+            out = _kvc.attention_prefill(*rows, q_len)          # a prompt's own keys, read where they are
+            if out is not None:
+                return self.o_proj(quantize_tokens(out.view(bsz, q_len, nh * d), self.o_reorder_index, self.o_proj.select_num,
+                                                   self.quant_type), residual)
         if q_len == 1:
             mask, causal = None, False
         elif isinstance(past_len, int) and past_len == 0:

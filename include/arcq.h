@@ -343,6 +343,16 @@ int arcq_matmul_swiglu(const void *a_codes, const void *a_scales, const void *b_
 int arcq_scales_from_absmax(float *d_values, int n, float divisor, void *stream);
 
 /*
+ * Causal attention of whole prompts (model/qLlamaLayer.py:340-370): o = softmax(q k^T * sm_scale) v over a sequence's own keys,
+ * query i of a sequence seeing keys 0 .. i.  bf16, head_dim 128; query heads a multiple of the KV heads.  Rows are tokens (sequence b's
+ * token t is row b * seq + t), a head's 128 values contiguous, ld* elements from row to row (multiples of 8; a fused projection's
+ * output is read in place); every operand 16-byte aligned and a sequence's keys below 4 GiB.  Scores, weights' sums and outputs
+ * accumulate in fp32, the weights enter the second product in bf16.
+ */
+int arcq_attention_prefill(const void *q, int ldq, const void *k, int ldk, const void *v, int ldv, int batch, int seq,
+                           int num_qo_heads, int num_kv_heads, int head_dim, float sm_scale, void *o, int ldo, void *stream);
+
+/*
  * Routing of a mixture-of-experts block (model/qMixtralLayer.py:441-452: softmax over the experts in fp32,
  * top-k, the k weights divided by their sum and cast to bf16; :456-471 then visits expert after expert and the
  * tokens routed to it).  Two launches, nothing read back: besides each token's choice the call writes what the

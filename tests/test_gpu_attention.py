@@ -1,0 +1,73 @@
+"""Causal attention of whole prompts (arcq_attention_prefill) against 64-bit softmax(q k^T / sqrt(d)) v on the CPU
+(model/qLlamaLayer.py:340-370)."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def operands(batch, seq, heads, kv_heads, gain=2.0, seed=1):
+    g = torch.Generator().manual_seed(seed + seq + heads)
+    t = batch * seq
+    q = (torch.randn(t, heads, 128, generator=g) * gain).to(torch.bfloat16)
+    k = torch.randn(t, kv_heads, 128, generator=g).to(torch.bfloat16)
+    qkv = torch.randn(t, (heads + 2 * kv_heads) * 128, generator=g).to(torch.bfloat16)
+    return q, k, qkv
+
+
+def reference(q, k, v, seq):
+    t, heads, d = q.shape
+    q, k, v = (x.double().view(t // seq, seq, -1, d).transpose(1, 2) for x in (q, k, v))
+    k, v = (x.repeat_interleave(heads // x.shape[1], 1) for x in (k, v))
+    s = (q @ k.transpose(-1, -2)) / math.sqrt(d)
+    s = s.masked_fill(torch.ones(seq, seq, dtype=torch.bool).triu(1), float("-inf"))
+    return (torch.softmax(s, -1) @ v).transpose(1, 2).reshape(t, heads * d)
+
+
+@pytest.mark.parametrize("batch,seq,heads,kv_heads", [(1, 1, 1, 1), (3, 2, 4, 4), (2, 31, 8, 2), (1, 32, 7, 1), (2, 33, 4, 2), (1, 63, 4, 1), (1, 64, 2, 2),
+                                                      (5, 65, 4, 2), (1, 127, 8, 8), (2, 128, 6, 2), (3, 129, 8, 1), (1, 257, 28, 4), (2, 500, 8, 2)])
+def test_attention_prefill(batch, seq, heads, kv_heads):
+    """Queries and keys ending inside a tile and at its edge, every kind of grouping, V as a strided slice.  What is left of the
+    rounding: the output's to bf16 (2^-9 at most, 1.66e-3 in norm) and the weights' (2^-9 each, partly cancelled by their sum)."""
+    from arcquant_amd import kv_cache
+    q, k, qkv = operands(batch, seq, heads, kv_heads)
+    v = qkv[:, (heads + kv_heads) * 128:]
+    got = kv_cache.attention_prefill(q.cuda(), k.cuda(), qkv.cuda()[:, (heads + kv_heads) * 128:], seq).cpu().double()
+    want = reference(q, k, v, seq)
+    assert float((got - want).norm() / want.norm()) < 2.3e-3
+    # a weight's error of 2^-9 of itself moves the result by 2^-9 of the weighted magnitudes, which abs() bounds; and the output's own
+    bound = reference(q, k, v.abs(), seq) * 2 ** -8 + want.abs() * 2 ** -8 + 1e-30
+    assert bool(((got - want).abs() <= bound).all())
+    first = got.view(batch, seq, heads, 128)[:, 0]                  # the first token sees itself alone: its V, unchanged
+    assert torch.equal(first, v.double().view(batch, seq, kv_heads, 128)[:, 0].repeat_interleave(heads // kv_heads, 1))
+
+
+def test_attention_prefill_large_scores_and_order():
+    """Scores of hundreds (one key takes all), equal scores (the mean), maxima that grow and fall along the keys"""
+    from arcquant_amd import kv_cache
+    seq, heads = 300, 2
+    q, k, qkv = operands(1, seq, heads, heads, gain=40.0)
+    for scale in (torch.zeros(seq, 1, 1), torch.linspace(0, 1, seq).view(-1, 1, 1), torch.linspace(1, 0, seq).view(-1, 1, 1)):
+        ks = (k.float() * scale).to(torch.bfloat16)
+        got = kv_cache.attention_prefill(q.cuda(), ks.cuda(), qkv.cuda()[:, 2 * heads * 128:], seq).cpu().double()
+        want = reference(q, ks, qkv[:, 2 * heads * 128:], seq)
+        assert float((got - want).norm() / want.norm()) < 2.3e-3
+
+
+def test_attention_prefill_refuses():
+    """what the kernel does not take is left to torch, and refused by the entry point"""
+    from arcquant_amd import _lib, kv_cache
+    q, k, qkv = operands(1, 8, 4, 2)
+    v = qkv[:, 6 * 128:]
+    q, k, v = q.cuda(), k.cuda(), v.cuda()
+    assert kv_cache.attention_prefill(q.half(), k, v, 8) is None
+    assert kv_cache.attention_prefill(q[:, :3].contiguous(), k, v, 8) is None       # 3 heads over 2
+    assert kv_cache.attention_prefill(q.transpose(0, 1).contiguous().transpose(0, 1), k, v, 8) is None
+    ok, f = 0x1000, _lib.lib().arcq_attention_prefill
+    good = dict(q=ok, ldq=512, k=ok, ldk=256, v=ok, ldv=256, b=0, s=8, h=4, g=2, d=128, c=0.1, o=ok, ldo=512)
+    call = lambda **kw: f(*{**good, **kw}.values(), None)
+    assert call() == 0 and call(b=1, s=0) == 0
+    assert call(d=64) == 2 and call(h=3) == 2 and call(ldq=511) == 2 and call(ldv=260) == 2 and call(ldk=128) == 2 and call(g=0) == 2
+    assert call(b=1, q=None) == 1 and call(b=1, v=0x1008) == 4 and call(b=1, s=1 << 23, ldk=512) == 2
