@@ -34,10 +34,11 @@ typedef v4s __attribute__((address_space(3))) lds_v4s;
 // CU, and the softmax of one runs beside the products of the other.  Rows of 256 bytes, 16-byte chunks swizzled: K by the key's
 // low four bits (sixteen keys on one chunk), V by its low two, in steps of 64 bytes (eight keys on 64 bytes).
 //
-// The weights' sum is taken over their bf16 values (v_dot2_f32_bf16, which is also one instruction for two), so that what is
-// left of their rounding is relative to one another; O is rescaled only when some query's maximum moves.  (Raising the maximum
-// only beyond 2^8 saves 4 % and costs accuracy: error against 64 bits 1.95e-3 in norm, so 1.82e-3, the bf16 output alone 1.66e-3;
-// torch's kernel 1.83e-3.)  us, torch's scaled_dot_product_attention before: 8 x 2048 tokens, 32 heads, 8 KV heads 744 -> 381
+// The running maximum is exact at every tile of 64 keys, and the weights' sum is taken before they are rounded to bf16: the
+// rounding of every weight is then that of torch's kernel (one output in 3000 to 10000 differs, by a bf16 step), behind which a quantizer
+// makes the same codes.  (Raising the maximum only beyond 2^8 saves 4 %, but a row's largest weight is then no longer exactly 1:
+// error against 64 bits 2.1e-3 in norm, so 1.8e-3 as torch's, the bf16 output alone 1.66e-3.)  O is rescaled only when some query's
+// maximum moves.  us, torch's scaled_dot_product_attention before: 8 x 2048 tokens, 32 heads, 8 KV heads 744 -> 381
 // (723 TFLOP/s), 4 x 1024 165 -> 62, 3 x 777, 28 heads, 4 KV heads 109 -> 39, 1 x 100 25 -> 7.
 //
 // XCDs get contiguous runs of (sequence, KV head) groups, whose K and V their L2 then holds, the longest query tiles first.
@@ -150,8 +151,8 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(AttentionPara
         for (int e = 0; e < 4; ++e) {
           const float a = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][8 * g + 2 * e], c, -mc));
           const float d = __builtin_amdgcn_exp2f(__builtin_fmaf(s[u][8 * g + 2 * e + 1], c, -mc));
+          l += a + d;
           w[e] = pack_bf16_rne(a, d);
-          l = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(v2bf, w[e]), __builtin_bit_cast(v2bf, 0x3f803f80u), l, false);
         }
         pf[2 * u + g] = __builtin_bit_cast(v8bf, make_uint4(w[0], w[1], w[2], w[3]));
       }
