@@ -103,6 +103,8 @@ def lib() -> ctypes.CDLL:
     L.arcq_attention_prefill.restype = i
     L.arcq_gemm_workspace_bytes.argtypes = [i, i, i, i, i]
     L.arcq_gemm_workspace_bytes.restype = sz
+    L.arcq_gemm_scratch_bytes.argtypes = [i, i, i, i, i]
+    L.arcq_gemm_scratch_bytes.restype = sz
     L.arcq_gemm_kernel.argtypes = [i, i, i, i, i, i]
     L.arcq_gemm_kernel.restype = i
     for name in ("arcq_grouped_matmul_swiglu", "arcq_matmul_swiglu", "arcq_scales_from_absmax"):

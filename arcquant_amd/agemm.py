@@ -220,8 +220,8 @@ def _infer_fmt(A, SFA, fmt):
 
 @functools.lru_cache(maxsize=4096)
 def _workspace_bytes(M, N, Kp, f, n_seg):
-    """arcq_gemm_workspace_bytes, a function of these numbers alone (0.9 us a call through ctypes)"""
-    return _lib.lib().arcq_gemm_workspace_bytes(M, N, Kp, f, n_seg)
+    """arcq_gemm_scratch_bytes, a function of these numbers alone (0.9 us a call through ctypes)"""
+    return _lib.lib().arcq_gemm_scratch_bytes(M, N, Kp, f, n_seg)
 
 
 def _gemm(A, SFA, B, SFB, M, N, Kp, f, c, *, alpha=1.0, da=None, db=None, residual=None, swiglu=0, seg=None, n_seg=0,
@@ -256,7 +256,7 @@ def matmul(A, B, SFA, SFB, scale, *, fmt=None, residual=None):
     in the epilogue, with the result of ``matmul(...) + residual`` bit for bit.
 
     Products are exact and sums fp32.  NVFP4 problems of many rows take scratch memory from torch's allocator for the
-    call (arcq_gemm_workspace_bytes); they sum in another order than arcq_matmul and arcq_matmul_noalloc, whose results
+    call (arcq_gemm_scratch_bytes); they sum in another order than arcq_matmul and arcq_matmul_noalloc, whose results
     may then differ by one bf16 rounding.
     """
     C = _host.matmul(A, B, SFA, SFB, scale, fmt, residual)

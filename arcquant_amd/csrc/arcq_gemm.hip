@@ -1247,6 +1247,23 @@ bool nvfp4_f16_wanted(int M, int N, int Kp, int fmt, int n_seg) {
   return (long)((M + 127) / 128) * tiles_n > 256;
 }
 
+// The same, and whether its last round of tiles is cut along K, which some problems take that are otherwise left to the kernels
+// without a workspace: bytes of scratch, 0 where it is not.
+size_t nvfp4_split_scratch(int M, int N, int Kp, int fmt, int n_seg) {
+  const int force = tuning().gemm_kernel;
+  if (fmt != ARCQ_FMT_NVFP4 || force >= 0 || (size_t)M * Kp * 2 >= ((size_t)1 << 32) || (size_t)N * Kp / 2 >= ((size_t)1 << 32)) return 0;
+  const size_t slots = nvfp4_split_bytes(M, N, Kp, n_seg);
+  return slots ? nvfp4_f16_bytes(M, N, Kp, n_seg > 0) + slots : 0;
+}
+
+// How a problem with this much workspace multiplies one operand decoded ahead: 0 not at all, 1 tile by tile, 2 with its last
+// round cut.
+int f16_way(int M, int N, int Kp, int fmt, int n_seg, size_t workspace_bytes) {
+  const size_t split = nvfp4_split_scratch(M, N, Kp, fmt, n_seg);
+  if (split && workspace_bytes >= split) return 2;
+  return nvfp4_f16_wanted(M, N, Kp, fmt, n_seg) && workspace_bytes >= nvfp4_f16_bytes(M, N, Kp, n_seg > 0) ? 1 : 0;
+}
+
 int matmul_impl(const void *a_codes, const void *a_scales, const void *b_codes, const void *b_scales, int M, int N,
                 int Kp, int fmt, float alpha, const float *d_alpha_a, const float *d_alpha_b, const void *residual,
                 void *c, void *workspace, size_t workspace_bytes, void *stream, const arcq_gemm_parts_args *parts = nullptr) {
@@ -1267,8 +1284,7 @@ int matmul_impl(const void *a_codes, const void *a_scales, const void *b_codes, 
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool scales_aligned = aligned16(a_scales) && aligned16(b_scales);
-  if (scales_aligned && workspace && nvfp4_f16_wanted(M, N, Kp, fmt, 0) && workspace_bytes >= nvfp4_f16_bytes(M, N, Kp, false))
-    return run_nvfp4_f16(p, workspace, st);
+  if (const int way = scales_aligned && workspace ? f16_way(M, N, Kp, fmt, 0, workspace_bytes) : 0) return run_nvfp4_f16(p, workspace, st, way == 2);
   const GemmPlan plan = plan_gemm(M, N, Kp, fmt, scales_aligned);
   float *scratch = nullptr;
   if (plan.slices > 1 && !takes_stream(plan, p, fmt)) {
@@ -1396,8 +1412,8 @@ int grouped_matmul_impl(const void *a_codes, const void *a_scales, const void *b
   p.seg_b_scales = (size_t)N * (Kp / G);
   p.swiglu = swiglu ? 1 : 0;
   p.absmax_bits = reinterpret_cast<uint32_t *>(d_absmax);
-  if (workspace && nvfp4_f16_wanted(M, N, Kp, fmt, n_seg) && workspace_bytes >= nvfp4_f16_bytes(M, N, Kp, true))
-    return run_nvfp4_f16(p, workspace, static_cast<hipStream_t>(stream));
+  if (const int way = workspace ? f16_way(M, N, Kp, fmt, n_seg, workspace_bytes) : 0)
+    return run_nvfp4_f16(p, workspace, static_cast<hipStream_t>(stream), way == 2);
   return run_gemm(p, plan_grouped(M, Kp, fmt, n_seg), fmt, nullptr, static_cast<hipStream_t>(stream));
 }
 
@@ -1440,8 +1456,8 @@ int matmul_swiglu_impl(const void *a_codes, const void *a_scales, const void *b_
   if (!aligned16(a_scales) || !aligned16(b_scales)) return ARCQ_ERR_ALIGN;
   p.swiglu = 1;
   p.absmax_bits = reinterpret_cast<uint32_t *>(d_absmax);
-  if (workspace && nvfp4_f16_wanted(M, N, Kp, fmt, 0) && workspace_bytes >= nvfp4_f16_bytes(M, N, Kp, false))
-    return run_nvfp4_f16(p, workspace, static_cast<hipStream_t>(stream));
+  if (const int way = workspace ? f16_way(M, N, Kp, fmt, 0, workspace_bytes) : 0)
+    return run_nvfp4_f16(p, workspace, static_cast<hipStream_t>(stream), way == 2);
   return run_gemm(p, plan_swiglu(M, N, Kp, fmt), fmt, nullptr, static_cast<hipStream_t>(stream));
 }
 }  // namespace
@@ -1488,6 +1504,11 @@ extern "C" int arcq_gemm_parts(const arcq_gemm_args *a, const arcq_gemm_parts_ar
 extern "C" size_t arcq_gemm_workspace_bytes(int M, int N, int Kp, int fmt, int n_seg) {
   if (M <= 0 || N <= 0 || Kp < 64 || n_seg < 0) return 0;
   return arcq::nvfp4_f16_wanted(M, N, Kp, fmt, n_seg) ? arcq::nvfp4_f16_bytes(M, N, Kp, n_seg > 0) : 0;
+}
+
+extern "C" size_t arcq_gemm_scratch_bytes(int M, int N, int Kp, int fmt, int n_seg) {
+  if (M <= 0 || N <= 0 || Kp < 64 || n_seg < 0) return 0;
+  return std::max(arcq::nvfp4_split_scratch(M, N, Kp, fmt, n_seg), arcq_gemm_workspace_bytes(M, N, Kp, fmt, n_seg));
 }
 
 extern "C" int arcq_gemm_kernel(int M, int N, int Kp, int fmt, int n_seg, int swiglu) {

@@ -9,6 +9,16 @@
 namespace arcq {
 namespace {
 
+// When the last round of tiles is cut along K: behind at least one whole round, and where the CUs without a tile times its steps are
+// worth more than the sums' way through memory and the second launch (30 to 35 us; what is left idle is not all lost, the
+// others run at a higher clock).  NVFP4, us, uncut and cut: 3000 x 6144 x 10240 (288 tiles) 391 and 292, 6000 x 4096 x 14592 (384) 560
+// and 512; 2331 x 4096 x 14592 (160, no whole round) 260 and 292, 2048 x 4096 x 8320 (128) 116 and 122.
+__host__ __device__ inline bool last_round_cut(long tiles, int pairs) {
+  const int rest = (int)(tiles & 255);
+  return tiles > 256 && rest > 0 && (256 - rest) * pairs > 6500;
+}
+constexpr int kSplitPairs = 12;   // pairs of steps that a workgroup has at least, about
+
 // codes + scale bytes -> fp16 values, row-major [rows, K'] (exact: at most six significant bits).  Codes, scale bytes and
 // values are dense, so that row boundaries play no part: dword i holds codes 8i .. 8i+7, all of block i / 2.
 __global__ __launch_bounds__(256) void nvfp4_decode_f16_kernel(const uint32_t *codes, const uint8_t *scales, uint4 *out,
@@ -56,37 +66,43 @@ __global__ __launch_bounds__(256) void nvfp4_decode_f16_kernel(const uint32_t *c
 // columns).  Requires K' % 128 == 0, K' >= 256.
 // ---------------------------------------------------------------------------------------------
 template <bool CODES_W>
-__global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
-  constexpr int TF = 8;  // 16-row tiles of the fp16 side per wave
-  constexpr int BC = 256, BF = 32 * TF;
-  constexpr int BM = CODES_W ? BF : BC, BN = CODES_W ? BC : BF;
-  constexpr int FI = BF / 64;                       // fp16 load instructions per wave and step
-  constexpr int kF = 3 * BF * 128, kC = 2 * BC * 64, kS = 2 * BC * 8;
-  constexpr int kRegion = 64 * 16 * TF * 2;         // bytes per wave of the epilogue's transpose
+struct F16Shape {
+  static constexpr int TF = 8;  // 16-row tiles of the fp16 side per wave
+  static constexpr int BC = 256, BF = 32 * TF;
+  static constexpr int BM = CODES_W ? BF : BC, BN = CODES_W ? BC : BF;
+  static constexpr int FI = BF / 64;                       // fp16 load instructions per wave and step
+  static constexpr int kF = 3 * BF * 128, kC = 2 * BC * 64, kS = 2 * BC * 8;
+  static constexpr int kRegion = 64 * 16 * TF * 2;         // bytes per wave of the epilogue's transpose
   static_assert(8 * kRegion <= kF + kC, "the epilogue's transpose");
-  __shared__ uint4 smem[(kF + kC + kS) / 16];
-  const int tid = threadIdx.x, lane = tid & 63;
+  static constexpr int kQuads = 4 * TF;                    // accumulator quads of a lane
+  static constexpr size_t kSlot = (size_t)512 * kQuads;    // of a workgroup, where its sums leave as they are
+};
+
+// Rows of either side where tile lin begins.
+// An XCD's 32 workgroups run at the same time on consecutive tiles: 4 tiles of the fp16 side x 8 of the codes, so that
+// both operands are shared in its L2 (an fp16 tile is four times the bytes of a codes tile)
+template <bool CODES_W>
+__device__ __forceinline__ void f16_tile_at(const GemmParams &p, int lin, int &c_base, int &f_base) {
+  using S = F16Shape<CODES_W>;
+  const int rows_c = CODES_W ? p.N : p.M, rows_f = CODES_W ? p.M : p.N;
+  const int tc = (rows_c + S::BC - 1) / S::BC, tf = (rows_f + S::BF - 1) / S::BF;
+  const int band = lin / (4 * tc), bw = min(4, tf - 4 * band), in_band = lin - band * 4 * tc;
+  c_base = (in_band / bw) * S::BC, f_base = (4 * band + in_band % bw) * S::BF;
+}
+
+// Tile lin of p, nk steps of 64 elements from step u0 on (both even): the tile of C, or with `partial` the fp32 sums.
+template <bool CODES_W>
+__device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, int nk, float4 *partial, uint8_t *smem, int tid) {
+  using S = F16Shape<CODES_W>;
+  constexpr int TF = S::TF, BC = S::BC, BF = S::BF, FI = S::FI, kF = S::kF, kC = S::kC, kRegion = S::kRegion;
+  const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int cpos = wave & 3, group = wave >> 2;
   const int kbytes = p.Kp >> 1, ksc = p.Kp >> 4, fbytes = p.Kp << 1;
-
-  int lin;
-  if (p.seg) {
-    if (!enter_segment<BM, BN, 16>(p, lin)) return;
-  } else {
-    const int total = ((p.M + BM - 1) / BM) * ((p.N + BN - 1) / BN);
-    lin = (blockIdx.x & 7) * ((total + 7) >> 3) + (blockIdx.x >> 3);
-    if (lin >= total) return;
-  }
   const int rows_c = CODES_W ? p.N : p.M, rows_f = CODES_W ? p.M : p.N;
-  const uint8_t *codes = CODES_W ? p.b_codes : p.a_codes, *scales = CODES_W ? p.b_scales : p.a_scales;
-  // An XCD's 32 workgroups run at the same time on consecutive tiles: 4 tiles of the fp16 side x 8 of the codes, so that
-  // both operands are shared in its L2 (an fp16 tile is four times the bytes of a codes tile)
-  const int tc = (rows_c + BC - 1) / BC, tf = (rows_f + BF - 1) / BF;
-  const int band = lin / (4 * tc), bw = min(4, tf - 4 * band), in_band = lin - band * 4 * tc;
-  const int c_base = (in_band / bw) * BC, f_base = (4 * band + in_band % bw) * BF;
-
-  const int nk = p.Kp >> 6;  // even
+  const uint8_t *codes = (CODES_W ? p.b_codes : p.a_codes) + u0 * 32, *scales = (CODES_W ? p.b_scales : p.a_scales) + u0 * 4;
+  int c_base, f_base;
+  f16_tile_at<CODES_W>(p, lin, c_base, f_base);
 
   // ---- global -> LDS: a wave-uniform base plus a 32-bit byte offset per lane
   uint32_t fvo[FI], cvo[2], svo;
@@ -102,7 +118,7 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
   }
   svo = (uint32_t)min(c_base + 64 * cpos + lane, rows_c - 1) * (uint32_t)ksc + 4 * group;
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(smem);
-  const uint8_t *f16 = reinterpret_cast<const uint8_t *>(p.f16);
+  const uint8_t *f16 = reinterpret_cast<const uint8_t *>(p.f16) + (size_t)u0 * 128;
   // (requests behind the last step fetch it again, into stages that nobody reads any more: the number of loads on their
   // way is the same in every step)
   auto request_f = [&](int u, int st, int i) {
@@ -228,8 +244,18 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
   }
   if (!group) barrier();
 
+  if (partial) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int t = 0; t < TF; ++t) {
+        const v4f a = CODES_W ? acc[i][t] : acc[t][i];
+        partial[(wave * S::kQuads + i * TF + t) * 64 + lane] = make_float4(a[0], a[1], a[2], a[3]);
+      }
+    return;
+  }
   const bool whole = c_base + BC <= rows_c && f_base + BF <= rows_f;
-  uint8_t *region = reinterpret_cast<uint8_t *>(smem) + wave * kRegion;
+  uint8_t *region = smem + wave * kRegion;
   if constexpr (CODES_W)
     store_wave_tile(p, Acc16<4, TF>{acc}, region, f_base + 16 * TF * group, c_base + 64 * cpos, whole, lane);
   else
@@ -237,9 +263,146 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
 }
 
 template <bool CODES_W>
-int launch(const GemmParams &p, hipStream_t st) {
+__global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
+  using S = F16Shape<CODES_W>;
+  __shared__ uint4 smem[(S::kF + S::kC + S::kS) / 16];
+  int lin;
+  if (p.seg) {
+    if (!enter_segment<S::BM, S::BN, 16>(p, lin)) return;
+  } else {
+    const int total = ((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN);
+    lin = (blockIdx.x & 7) * ((total + 7) >> 3) + (blockIdx.x >> 3);
+    if (lin >= total) return;
+  }
+  f16_tile<CODES_W>(p, lin, 0, p.Kp >> 6, nullptr, reinterpret_cast<uint8_t *>(smem), threadIdx.x);
+}
+
+// ---------------------------------------------------------------------------------------------
+// The same with its last round of tiles cut along K.  A round takes its time however few tiles it has, and with a long K that is
+// most of what a problem of one or two rounds costs.  The tiles of whole rounds run first, a workgroup each; the steps of
+// the other R tiles, one tile's behind the other's, are dealt out evenly to up to 256 workgroups.  A workgroup whose steps end
+// inside a tile, or begin there, leaves its fp32 sums in a slot of the workspace (two at most); a second launch adds a tile's up in
+// the order of K and stores it.  Every sum has a fixed place: the result does not depend on who is first.
+// The split and its edges follow from the number of tiles alone, which grouped launches only know on the device.
+// ---------------------------------------------------------------------------------------------
+struct LastRound {
+  int full, rest, groups;  // tiles of whole rounds, the other ones, workgroups that share those
+  int pairs;               // of steps, per tile
+  __device__ __forceinline__ LastRound(int total, int Kp) {
+    pairs = Kp >> 7;
+    full = total & ~255;
+    rest = total - full;
+    if (!last_round_cut(total, pairs)) full = total, rest = 0;
+    groups = min(256, rest * max(1, pairs / kSplitPairs));
+  }
+  __device__ __forceinline__ int begin(int w) const { return (int)((long)rest * pairs * w / groups); }
+  __device__ __forceinline__ int holder(int pair) const {  // the workgroup that has this pair
+    int w = (int)((long)pair * groups / ((long)rest * pairs));
+    while (begin(w + 1) <= pair) ++w;
+    return w;
+  }
+};
+
+// Tiles of the whole problem; with segments, p becomes the problem of the one that tile lin belongs to and lin its number there.
+template <bool CODES_W>
+__device__ __forceinline__ int f16_tiles(const GemmParams &p) {
+  using S = F16Shape<CODES_W>;
+  if (p.seg) return Segments<S::BM, S::BN, 16>(p).total;
+  return ((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN);
+}
+template <bool CODES_W>
+__device__ __forceinline__ bool f16_enter(GemmParams &p, int &lin) {
+  using S = F16Shape<CODES_W>;
+  if (!p.seg) return true;
+  Segments<S::BM, S::BN, 16> segments(p);
+  return segments.enter(p, lin);
+}
+
+template <bool CODES_W>
+__global__ __launch_bounds__(512) void gemm_nvfp4_f16_split(GemmParams p) {
+  using S = F16Shape<CODES_W>;
+  __shared__ uint4 smem[(S::kF + S::kC + S::kS) / 16];
+  const LastRound r(f16_tiles<CODES_W>(p), p.Kp);
+  const int full_grid = (r.full + 7) & ~7;
+  int at, end, w = -1;  // pairs of steps of the rest; a whole tile of the full rounds: its pairs, as if those were all
+  if ((int)blockIdx.x < full_grid) {
+    const int lin = (blockIdx.x & 7) * (full_grid >> 3) + (blockIdx.x >> 3);
+    if (lin >= r.full) return;
+    at = (lin - r.full) * r.pairs;  // negative: in front of the rest
+    end = at + r.pairs;
+  } else {
+    const int id = (int)blockIdx.x - full_grid;
+    if (id >= 256) return;
+    w = (id & 7) * 32 + (id >> 3);  // neighbours on one XCD
+    if (w >= r.groups) return;
+    at = r.begin(w);
+    end = r.begin(w + 1);
+  }
+  while (at < end) {
+    const int tile = (at + r.full * r.pairs) / r.pairs, first = at - (tile - r.full) * r.pairs, n = min(end - at, r.pairs - first);
+    GemmParams q = p;
+    int lin = tile;
+    if (!f16_enter<CODES_W>(q, lin)) return;
+    float4 *partial = n == r.pairs ? nullptr : p.split + (2 * w + (first + n == r.pairs ? 0 : 1)) * S::kSlot;
+    wait_dma_and_sync();  // the LDS of the part before this one
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // what follows from it is formed per part: hoisted out of this loop it would be spilled
+    f16_tile<CODES_W>(q, lin, 2 * first, 2 * n, partial, reinterpret_cast<uint8_t *>(smem), tid);
+    at += n;
+  }
+}
+
+// a wave per eighth of a tile
+template <bool CODES_W>
+__global__ __launch_bounds__(64) void f16_split_add_kernel(GemmParams p) {
+  using S = F16Shape<CODES_W>;
+  __shared__ uint4 smem[S::kRegion / 16];
+  constexpr int TF = S::TF;
+  const int lane = threadIdx.x, wave = blockIdx.x & 7, tile = blockIdx.x >> 3, cpos = wave & 3, group = wave >> 2;
+  const LastRound r(f16_tiles<CODES_W>(p), p.Kp);
+  if (tile >= r.rest) return;
+  const int w0 = r.holder(tile * r.pairs), w1 = r.holder((tile + 1) * r.pairs - 1);
+  int lin = r.full + tile;
+  if (w0 == w1 || !f16_enter<CODES_W>(p, lin)) return;  // (one workgroup had the whole tile and stored it)
+  v4f acc[CODES_W ? 4 : TF][CODES_W ? TF : 4];
+#pragma unroll
+  for (auto &a : acc)
+#pragma unroll
+    for (auto &b : a) b = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int w = w0; w <= w1; ++w) {
+    if (r.begin(w) == r.begin(w + 1)) continue;
+    const float4 *src = p.split + (2 * w + (w == w1 ? 0 : 1)) * S::kSlot + (size_t)wave * S::kQuads * 64 + lane;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int t = 0; t < TF; ++t) {
+        const float4 v = src[(i * TF + t) * 64];
+        (CODES_W ? acc[i][t] : acc[t][i]) += v4f{v.x, v.y, v.z, v.w};
+      }
+  }
+  const int rows_c = CODES_W ? p.N : p.M, rows_f = CODES_W ? p.M : p.N;
+  int c_base, f_base;
+  f16_tile_at<CODES_W>(p, lin, c_base, f_base);
+  const bool whole = c_base + S::BC <= rows_c && f_base + S::BF <= rows_f;
+  uint8_t *region = reinterpret_cast<uint8_t *>(smem);
+  if constexpr (CODES_W)
+    store_wave_tile(p, Acc16<4, TF>{acc}, region, f_base + 16 * TF * group, c_base + 64 * cpos, whole, lane);
+  else
+    store_wave_tile(p, Acc16<TF, 4>{acc}, region, c_base + 64 * cpos, f_base + 16 * TF * group, whole, lane);
+}
+
+template <bool CODES_W>
+int launch(const GemmParams &p, bool split, hipStream_t st) {
   const int total = ((p.M + 255) / 256 + (p.seg ? p.n_seg : 0)) * ((p.N + 255) / 256);
-  hipLaunchKernelGGL((gemm_nvfp4_f16<CODES_W>), dim3(((total + 7) / 8) * 8), dim3(512), 0, st, p);
+  const int grid = ((total + 7) / 8) * 8;
+  if (!split) {
+    hipLaunchKernelGGL((gemm_nvfp4_f16<CODES_W>), dim3(grid), dim3(512), 0, st, p);
+    ARCQ_HIP_TRY(hipGetLastError());
+    return ARCQ_OK;
+  }
+  hipLaunchKernelGGL((gemm_nvfp4_f16_split<CODES_W>), dim3(grid + 256), dim3(512), 0, st, p);
+  ARCQ_HIP_TRY(hipGetLastError());
+  hipLaunchKernelGGL((f16_split_add_kernel<CODES_W>), dim3(8 * std::min(total, 255)), dim3(64), 0, st, p);
   ARCQ_HIP_TRY(hipGetLastError());
   return ARCQ_OK;
 }
@@ -250,7 +413,20 @@ size_t nvfp4_f16_bytes(int M, int N, int Kp, bool grouped) {
   return (size_t)(grouped || M <= N ? M : N) * Kp * 2;
 }
 
-int run_nvfp4_f16(GemmParams p, void *workspace, hipStream_t st) {
+// (Experts: the tiles are known on the device alone; from 512 rows per expert on.  Eight of 4096 x 14464, 8192 rows skewed 912 -> 816 us
+// against 128x128 tiles, even 822 -> 713; 4096 rows skewed 495 -> 463; 64 of 2048 x 8320, 600 rows each, would lose 5 %.)
+size_t nvfp4_split_bytes(int M, int N, int Kp, int n_seg) {
+  if (Kp < 8192 || Kp % 128 != 0 || M <= 64) return 0;
+  if (n_seg == 0) {
+    const long total = (long)((M + 255) / 256) * ((N + 255) / 256);
+    if (!last_round_cut(total, Kp >> 7) || total > 6 * 256) return 0;
+  } else if (N <= 2048 || M / n_seg < 512 || ((M + 255) / 256 + n_seg / 2) * (long)((N + 255) / 256) > 6 * 256) {
+    return 0;
+  }
+  return 512 * F16Shape<true>::kSlot * sizeof(float4);
+}
+
+int run_nvfp4_f16(GemmParams p, void *workspace, hipStream_t st, bool split) {
   const bool codes_w = p.seg || p.M <= p.N;
   const int rows = codes_w ? p.M : p.N;
   const size_t dwords = (size_t)rows * (p.Kp >> 3);
@@ -259,7 +435,8 @@ int run_nvfp4_f16(GemmParams p, void *workspace, hipStream_t st) {
                      static_cast<uint4 *>(workspace), dwords);
   ARCQ_HIP_TRY(hipGetLastError());
   p.f16 = static_cast<const uint16_t *>(workspace);
-  return codes_w ? launch<true>(p, st) : launch<false>(p, st);
+  if (split) p.split = reinterpret_cast<float4 *>(static_cast<uint8_t *>(workspace) + nvfp4_f16_bytes(p.M, p.N, p.Kp, p.seg != nullptr));
+  return codes_w ? launch<true>(p, split, st) : launch<false>(p, split, st);
 }
 
 }  // namespace arcq

@@ -50,6 +50,8 @@ struct GemmParams {
   // gemm_nvfp4_f16: one operand decoded to fp16 [rows, K'] ahead of the launch (the activations, or the weights
   // where they have fewer rows)
   const uint16_t *f16 = nullptr;
+  // gemm_nvfp4_f16 with its last round of tiles cut along K: the workgroups' fp32 sums of parts of tiles, two slots each
+  float4 *split = nullptr;
   // weights made of several parts with a tensor scale each (q | k | v): rows part_end[k - 1] .. part_end[k] - 1 have *part_alpha[k]
   // in the place of *d_alpha_b.  Multiples of 32: a 16- or 32-column tile of accumulators lies in one part.
   int parts = 0;
@@ -59,7 +61,9 @@ struct GemmParams {
 
 // arcq_gemm_nv.hip: bytes of the decoded operand, and the GEMM on it
 size_t nvfp4_f16_bytes(int M, int N, int Kp, bool grouped);
-int run_nvfp4_f16(GemmParams p, void *workspace, hipStream_t st);
+int run_nvfp4_f16(GemmParams p, void *workspace, hipStream_t st, bool split);
+// scratch of the same with its last round cut along K, 0 where that does not pay
+size_t nvfp4_split_bytes(int M, int N, int Kp, int n_seg);
 
 // arcq_gemm_nv_stream.hip: decode batches, plain (n_seg = 0, M <= 64) and grouped
 bool nvfp4_stream_wanted(int M, int N, int Kp, int n_seg);
@@ -97,12 +101,12 @@ __device__ __forceinline__ int wave_prefix(int v) {
 // front of every tile (MXFP4, 64 experts of 2048 x 1536, 256 skewed rows each: 78 us with one walk, 104 with another one to count
 // the tiles, 68 so; NVFP4, 1024 rows: 457, 470, 426).
 template <int BM, int BN, int G>
-__device__ __forceinline__ bool enter_segment(GemmParams &p, int &lin) {
-  const int tiles_n = (p.N + BN - 1) / BN;
-  const int rows = p.M, lane = threadIdx.x & 63;
-  const int first = min(max(p.seg[0], 0), rows);
+struct Segments {
+  int tiles_n, rows, lane, first;
   int end, beg, tiles, upto;  // of segment e0 + lane: its rows, its tiles, the tiles up to its end
-  auto read = [&](int e0, int from) {
+  int total;                  // tiles of all segments
+
+  __device__ __forceinline__ void read(const GemmParams &p, int e0, int from) {
     const int e = e0 + lane;
     // offsets that do not grow or leave the tensor: empty segments
     end = min(wave_prefix<true>(max(e < p.n_seg ? p.seg[e + 1] : 0, from)), rows);
@@ -110,46 +114,63 @@ __device__ __forceinline__ bool enter_segment(GemmParams &p, int &lin) {
     if (lane == 0) beg = from;
     tiles = ((end - beg + BM - 1) / BM) * tiles_n;
     upto = wave_prefix<false>(tiles);
-  };
-  // contiguous runs of tiles per XCD, of the tiles that there are: cut from the upper bound, the last XCD would get the
-  // surplus workgroups and the others its tiles (8192 rows over 8 experts: 36 of 40 rows of tiles are real)
-  int total = 0;
-  for (int e0 = 0, from = first; e0 < p.n_seg; e0 += 64) {
-    read(e0, from);
-    total += __builtin_amdgcn_readlane(upto, 63);
-    from = __builtin_amdgcn_readlane(end, 63);
   }
-  const int per_xcd = (total + 7) >> 3;
-  if ((int)(blockIdx.x >> 3) >= per_xcd) return false;
-  lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
-  if (lin >= total) return false;
-  int e0 = 0;
-  if (p.n_seg > 64) {
-    for (int from = first; e0 < p.n_seg; e0 += 64) {
-      read(e0, from);
-      const int here = __builtin_amdgcn_readlane(upto, 63);
-      if (lin < here) break;
-      lin -= here;
+
+  __device__ __forceinline__ explicit Segments(const GemmParams &p) {
+    tiles_n = (p.N + BN - 1) / BN;
+    rows = p.M, lane = threadIdx.x & 63;
+    first = min(max(p.seg[0], 0), rows);
+    total = 0;
+    for (int e0 = 0, from = first; e0 < p.n_seg; e0 += 64) {
+      read(p, e0, from);
+      total += __builtin_amdgcn_readlane(upto, 63);
       from = __builtin_amdgcn_readlane(end, 63);
     }
-    if (e0 >= p.n_seg) return false;
   }
-  const int l = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lin < upto));  // the first segment that ends behind lin
-  lin -= __builtin_amdgcn_readlane(upto, l) - __builtin_amdgcn_readlane(tiles, l);
-  const int row0 = __builtin_amdgcn_readlane(beg, l), e = e0 + l;
-  const size_t kbytes = p.Kp >> 1, ksc = p.Kp / G;
-  p.a_codes += (size_t)row0 * kbytes;
-  p.a_scales += (size_t)row0 * ksc;
-  if (p.f16) p.f16 += (size_t)row0 * p.Kp;
-  p.c += (size_t)row0 * (p.swiglu ? p.N >> 1 : p.N);
-  if (p.residual) p.residual += (size_t)row0 * p.ld_residual;
-  p.b_codes += (size_t)e * p.seg_b_codes;
-  p.b_scales += (size_t)e * p.seg_b_scales;
-  if (p.d_alpha_a) p.d_alpha_a += e;
-  if (p.d_alpha_b) p.d_alpha_b += e;
-  p.M = __builtin_amdgcn_readlane(end, l) - row0;
-  p.seg_index = e;
-  return true;
+
+  // Turns p into the problem of the segment that tile lin belongs to, lin into the tile's number inside it; false past the end.
+  // (Up to 64 segments the constructor's one read still holds; beyond, p is read anew, so it has to be the launch's own.)
+  __device__ __forceinline__ bool enter(GemmParams &p, int &lin) {
+    if (lin >= total) return false;
+    int e0 = 0;
+    if (p.n_seg > 64) {
+      for (int from = first; e0 < p.n_seg; e0 += 64) {
+        read(p, e0, from);
+        const int here = __builtin_amdgcn_readlane(upto, 63);
+        if (lin < here) break;
+        lin -= here;
+        from = __builtin_amdgcn_readlane(end, 63);
+      }
+      if (e0 >= p.n_seg) return false;
+    }
+    const int l = __builtin_ctzll(__builtin_amdgcn_ballot_w64(lin < upto));  // the first segment that ends behind lin
+    lin -= __builtin_amdgcn_readlane(upto, l) - __builtin_amdgcn_readlane(tiles, l);
+    const int row0 = __builtin_amdgcn_readlane(beg, l), e = e0 + l;
+    const size_t kbytes = p.Kp >> 1, ksc = p.Kp / G;
+    p.a_codes += (size_t)row0 * kbytes;
+    p.a_scales += (size_t)row0 * ksc;
+    if (p.f16) p.f16 += (size_t)row0 * p.Kp;
+    p.c += (size_t)row0 * (p.swiglu ? p.N >> 1 : p.N);
+    if (p.residual) p.residual += (size_t)row0 * p.ld_residual;
+    p.b_codes += (size_t)e * p.seg_b_codes;
+    p.b_scales += (size_t)e * p.seg_b_scales;
+    if (p.d_alpha_a) p.d_alpha_a += e;
+    if (p.d_alpha_b) p.d_alpha_b += e;
+    p.M = __builtin_amdgcn_readlane(end, l) - row0;
+    p.seg_index = e;
+    return true;
+  }
+};
+
+template <int BM, int BN, int G>
+__device__ __forceinline__ bool enter_segment(GemmParams &p, int &lin) {
+  Segments<BM, BN, G> segments(p);
+  // contiguous runs of tiles per XCD, of the tiles that there are: cut from the upper bound, the last XCD would get the
+  // surplus workgroups and the others its tiles (8192 rows over 8 experts: 36 of 40 rows of tiles are real)
+  const int per_xcd = (segments.total + 7) >> 3;
+  if ((int)(blockIdx.x >> 3) >= per_xcd) return false;
+  lin = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  return segments.enter(p, lin);
 }
 
 // two bf16 pairs + two bf16 pairs, each sum rounded to bf16

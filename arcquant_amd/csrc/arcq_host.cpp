@@ -237,7 +237,7 @@ PyObject *matmul(PyObject *const *a) {
     res = &tensor(a[6], at::kBFloat16, 2);
     need(res->size(0) == M && res->size(1) == N && res->device() == A.device());
   }
-  need(!(M > 64 && fmt == ARCQ_FMT_NVFP4 && arcq_gemm_workspace_bytes(M, N, Kp, fmt, 0)));
+  need(!(M > 64 && fmt == ARCQ_FMT_NVFP4 && arcq_gemm_scratch_bytes(M, N, Kp, fmt, 0)));
   const at::Tensor C = empty({M, N}, A, at::kBFloat16);
   const void *ap = A.const_data_ptr(), *bp = B.const_data_ptr(), *asp = SFA.const_data_ptr(), *bsp = SFB.const_data_ptr();
   const float alpha = (float)(sa.host * sb.host);

@@ -231,6 +231,9 @@ typedef struct arcq_gemm_args {
 } arcq_gemm_args;
 int arcq_gemm(const arcq_gemm_args *args, void *stream);
 size_t arcq_gemm_workspace_bytes(int M, int N, int Kp, int fmt, int n_seg);
+/* Bytes with which arcq_gemm may also cut the last round of its tiles along K (NVFP4 with a long K': fp32 sums of parts of tiles behind
+ * the decoded operand, 128 MiB); arcq_gemm_workspace_bytes where it would not.  A workspace of either size is used for what it holds. */
+size_t arcq_gemm_scratch_bytes(int M, int N, int Kp, int fmt, int n_seg);
 
 /*
  * Several linears over one quantized input as one GEMM: their quantized weights lie behind one another in b_codes / b_scales

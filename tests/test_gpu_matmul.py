@@ -378,3 +378,42 @@ def test_matmul_parts(agemm, M, rows, fmt):
     assert torch.equal(agemm.matmul_parts(a, b, sfa, sfb, dgx, rows, scales, fmt=fmt, bias=bias), y + bias)
     with pytest.raises(RuntimeError):
         agemm.matmul_parts(a, b, sfa, sfb, dgx, (N - 16, 16), scales[:1] * 2, fmt=fmt)
+
+
+@pytest.mark.parametrize("M,N,kp,counts", [(4100, 4096, 8192, None), (3000, 6144, 8320, None), (6144, 3000, 8320, None), (5000, 4090, 10240, None),
+                                           (4096, 4352, 9088, [900, 2100, 0, 96, 1000]), (4096, 4360, 8192, [1, 4095])])
+def test_nvfp4_last_round_cut(agemm, oracle, M, N, kp, counts):
+    """NVFP4 problems of a few rounds of tiles with a long K': the last round's tiles shared by workgroups along K, either operand
+    decoded ahead, rows and columns ending inside a tile, experts without rows; against the kernels without a workspace (the
+    sum in another order: one bf16 rounding at most) and the 64-bit product of some rows."""
+    import ctypes
+    from arcquant_amd import _lib
+    L, E = _lib.lib(), len(counts) if counts else 0
+    g = torch.Generator(device="cuda").manual_seed(9)
+    codes = lambda rows: (torch.randint(0, 256, (rows, kp // 2), generator=g, device="cuda", dtype=torch.uint8),
+                          torch.randint(60, 90, (rows * (kp // 16),), generator=g, device="cuda", dtype=torch.uint8))
+    (a, sfa), (b, sfb) = codes(M), codes(N * max(E, 1))
+    seg = torch.tensor([0] + list(np.cumsum(counts)), dtype=torch.int32, device="cuda") if counts else None
+    res = torch.randn(M, N, generator=g, device="cuda").to(torch.bfloat16)
+    need = L.arcq_gemm_scratch_bytes(M, N, kp, 0, E)
+    if "ARCQ_GEMM_KERNEL" not in os.environ:
+        assert need >= 512 * 65536 * 4
+    out = []
+    for residual in (None, res):
+        for nbytes in (need, 0):
+            c = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+            work = torch.full((nbytes,), 0xff, dtype=torch.uint8, device="cuda") if nbytes else None
+            args = _lib.GemmArgs(a.data_ptr(), sfa.data_ptr(), b.data_ptr(), sfb.data_ptr(), M, N, kp, 0, 2.0 ** -9, 0, None, None,
+                                 None if residual is None else residual.data_ptr(), c.data_ptr(), None if seg is None else seg.data_ptr(), E,
+                                 None, None if work is None else work.data_ptr(), nbytes)
+            assert L.arcq_gemm(args, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+            out.append(c)
+    assert rel_fro(out[0].float(), out[1].float()) < 1e-3
+    assert torch.equal(out[2], out[0] + res)
+    rows = torch.tensor([0, 255, 256, M // 2, M - 1])
+    e = torch.bucketize(rows, seg.cpu()[1:].long(), right=True) if counts else torch.zeros(5, dtype=torch.long)
+    da = oracle_dq(oracle, a[rows.cuda()], sfa.view(M, -1)[rows.cuda()].reshape(-1), "NVFP4")
+    for i in range(5):
+        w = slice(int(e[i]) * N, (int(e[i]) + 1) * N)
+        want = da[i].double() @ oracle_dq(oracle, b[w], sfb.view(-1, kp // 16)[w].reshape(-1), "NVFP4").double().T * 2.0 ** -9
+        assert rel_fro(out[0][rows[i]].float(), want) < 2.5e-3
