@@ -1137,15 +1137,19 @@ GemmPlan plan_swiglu(int M, int N, int Kp, int fmt) {
   return plan;
 }
 
-// NVFP4 decode batches run as a stream of the weights, whichever tiles (and slices of K) the plan has for them, unless a kernel
-// or a number of slices is forced; plan 0 has operands that only the direct kernels take.
-bool takes_stream(const GemmPlan &plan, const GemmParams &p, int fmt) {
-  return fmt == ARCQ_FMT_NVFP4 && tuning().gemm_kernel < 0 && tuning().gemm_splitk == 0 && plan.kernel != 0 &&
-         nvfp4_stream_wanted(p.M, p.N, p.Kp, p.n_seg);
+// NVFP4 decode batches run as a stream of the weights, whichever tiles (and slices of K) the plan has for them, and plain problems
+// of a few hundred rows where that is faster than the plan's tiles, unless a kernel or a number of slices is forced; plan 0 has operands
+// that only the direct kernels take.  -1: by the plan; 0: as a stream; 1 + shape: that shape.
+int stream_way(const GemmPlan &plan, const GemmParams &p, int fmt) {
+  if (fmt != ARCQ_FMT_NVFP4 || tuning().gemm_kernel >= 0 || tuning().gemm_splitk != 0 || plan.kernel == 0) return -1;
+  if (nvfp4_stream_wanted(p.M, p.N, p.Kp, p.n_seg)) return 0;
+  const int shape = p.seg || p.swiglu ? -1 : nvfp4_mid_shape(p.M, p.N, p.Kp, plan.kernel, plan.slices);
+  return shape < 0 ? -1 : 1 + shape;
 }
 
 int run_gemm(GemmParams p, const GemmPlan &plan, int fmt, float *scratch, hipStream_t st) {
-  if (takes_stream(plan, p, fmt)) return run_nvfp4_stream(p, st);
+  const int way = stream_way(plan, p, fmt);
+  if (way >= 0) return way == 0 ? run_nvfp4_stream(p, st) : run_nvfp4_mid(p, way - 1, st);
   if (plan.slices > 1) {
     p.k_slices = plan.slices;
     p.partial = scratch;
@@ -1287,7 +1291,7 @@ int matmul_impl(const void *a_codes, const void *a_scales, const void *b_codes, 
   if (const int way = scales_aligned && workspace ? f16_way(M, N, Kp, fmt, 0, workspace_bytes) : 0) return run_nvfp4_f16(p, workspace, st, way == 2);
   const GemmPlan plan = plan_gemm(M, N, Kp, fmt, scales_aligned);
   float *scratch = nullptr;
-  if (plan.slices > 1 && !takes_stream(plan, p, fmt)) {
+  if (plan.slices > 1 && stream_way(plan, p, fmt) < 0) {
     int status = ARCQ_OK;
     scratch = static_cast<float *>(stream_workspace(kWsSplitK, st, &status));
     if (!scratch) return status;
@@ -1357,7 +1361,7 @@ extern "C" int arcq_matmul_noalloc(const void *a_codes, const void *a_scales, co
   const GemmPlan plan = plan_gemm(M, N, Kp, fmt, aligned16(a_scales) && aligned16(b_scales));
   if (plan.scratch_bytes() > kNoAllocScratchBytes) return ARCQ_ERR_WORKSPACE;  // beyond the fixed array: nothing is launched
   float *ws = nullptr;
-  if (plan.slices > 1 && !takes_stream(plan, p, fmt)) {
+  if (plan.slices > 1 && stream_way(plan, p, fmt) < 0) {
     int status = ARCQ_OK;
     ws = noalloc_scratch(&status);
     if (!ws) return status;

@@ -1,5 +1,5 @@
 // arcq_gemm_nv_stream.hip -- NVFP4 GEMM of decode batches (up to 64 rows, or experts of a few rows each): one pass over the
-// weights, all of whose bytes are on their way through many small workgroups.
+// weights, all of whose bytes are on their way through many small workgroups; and of a few hundred rows where tiles do not fill the chip.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -335,6 +335,59 @@ bool nvfp4_stream_wanted(int M, int N, int Kp, int n_seg) {
   if (Kp % 128 != 0 || Kp < 512 || Kp > (1 << 24)) return false;
   if (n_seg > 0) return M / n_seg < 96 && (M / n_seg <= 40 || Kp >= 2048);
   return M <= 64 && !(N <= 8192 && M <= 4) && !(N <= 4096 && M <= 8 && Kp < 8192);
+}
+
+// Beyond 64 rows the same kernel with 64 to 112 rows per workgroup: both operands are decoded in every workgroup, but only
+// once (its waves split K), which is about what the matrix instructions take, and small workgroups fill the chip where 128x128 tiles
+// do not.  A workgroup's time per K' = 4352 and its wait to start and end, measured (us; workgroups of 1 to 14 per CU):
+struct MidShape {
+  int mt, nt, wn, wk;
+  double us;
+};
+constexpr MidShape kMid[] = {{4, 3, 1, 8, 8.2}, {4, 4, 1, 8, 9.8}, {5, 3, 1, 8, 9.2}, {6, 4, 1, 8, 14.8}, {7, 3, 1, 8, 13.8},
+                             {5, 3, 2, 4, 16.6}, {4, 4, 2, 4, 18.0}, {6, 3, 2, 4, 22.5}, {5, 4, 2, 4, 25.0}};
+
+// The shape for a problem that the plan would give to 128x64 (21, K in `slices`), 128x128 (22) or 256x128 tiles (42), -1 where those
+// are faster by their own measured times.  us, before and now: 128 x 6144 x 4352 21.9 and 14.3, 333 rows 34.4 and 28.5, 512 rows 34.1
+// (kept); 256 x 4096 x 4352 23.3 and 16.3; 128 x 4096 x 14592 31 (kept), 333 rows 73.8 and 55.7; 80 x 28672 x 4352 43.6 and
+// 33, 256 rows 62 (kept).
+int nvfp4_mid_shape(int M, int N, int Kp, int kernel, int slices) {
+  if (M <= 64 || M > 1024 || Kp < 512 || Kp % 128 != 0 || Kp > (1 << 24)) return -1;
+  const double k = Kp / 4352.0;
+  auto rounds = [](long groups) { return (double)((groups + 255) / 256); };
+  auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  double tiled;
+  if (kernel == 21)
+    tiled = (slices > 1 ? 12 : 7) + 20 * k / slices * rounds(tiles(64, 128) * slices);
+  else if (kernel == 22)
+    tiled = 4 + (tiles(128, 128) <= 256 ? 30 : 27) * k * rounds(tiles(128, 128));
+  else if (kernel == 42)
+    tiled = 4 + 58 * k * rounds(tiles(128, 256));
+  else
+    return -1;
+  int best = -1;
+  double least = 0.97 * tiled;
+  for (int i = 0; i < (int)(sizeof(kMid) / sizeof(kMid[0])); ++i) {
+    const MidShape &s = kMid[i];
+    const double us = 6 + s.us * k * rounds(tiles(16 * s.mt, 16 * s.nt * s.wn));
+    if (us < least) best = i, least = us;
+  }
+  return best;
+}
+
+int run_nvfp4_mid(const GemmParams &p, int shape, hipStream_t st) {
+  switch (shape) {
+    case 0: return launch<4, 3, 1, 8, 2>(p, st);
+    case 1: return launch<4, 4, 1, 8, 2>(p, st);
+    case 2: return launch<5, 3, 1, 8, 2>(p, st);
+    case 3: return launch<6, 4, 1, 8, 2>(p, st);
+    case 4: return launch<7, 3, 1, 8, 2>(p, st);
+    case 5: return launch<5, 3, 2, 4, 2>(p, st);
+    case 6: return launch<4, 4, 2, 4, 2>(p, st);
+    case 7: return launch<6, 3, 2, 4, 2>(p, st);
+    case 8: return launch<5, 4, 2, 4, 2>(p, st);
+    default: return ARCQ_ERR_SHAPE;
+  }
 }
 
 int run_nvfp4_stream(const GemmParams &p, hipStream_t st) {

@@ -254,7 +254,7 @@ int arcq_gemm_parts(const arcq_gemm_args *args, const arcq_gemm_parts_args *part
  * ARCQ_GEMM_KERNEL environment variable forces (168 = one operand decoded ahead, 88 = MXFP4 ping-pong, ..., 1 = skinny,
  * 0 = direct); -1 for arguments arcq_gemm refuses.  NVFP4 problems of up to 64 rows, and experts of fewer than 96 on average, are
  * reported by the plan of tiles that they have where a kernel is forced (1, 11, 21, ...): unforced, most of them run as one pass
- * over the weights that cuts nothing.  Host only: for tests of the dispatch and for tuning. */
+ * over the weights that cuts nothing, and so do plain ones of up to 1024 rows whose tiles (21, 22, 42) would not fill the chip.  Host only: for tests of the dispatch and for tuning. */
 int arcq_gemm_kernel(int M, int N, int Kp, int fmt, int n_seg, int swiglu);
 
 /*
@@ -279,7 +279,7 @@ int arcq_matmul_noalloc(const void *a_codes, const void *a_scales, const void *b
                         void *stream);
 size_t arcq_matmul_noalloc_limit(void);
 /* bytes of split-K partial tiles that arcq_matmul's plan has for this problem (0: the plan does not cut K); an upper bound for
- * NVFP4 problems of up to 64 rows, most of which run as one pass over the weights without any */
+ * NVFP4 problems of up to 1024 rows, most of which run as one pass over the weights without any */
 size_t arcq_matmul_scratch_bytes(int M, int N, int Kp, int fmt);
 
 /*

@@ -417,3 +417,19 @@ def test_nvfp4_last_round_cut(agemm, oracle, M, N, kp, counts):
         w = slice(int(e[i]) * N, (int(e[i]) + 1) * N)
         want = da[i].double() @ oracle_dq(oracle, b[w], sfb.view(-1, kp // 16)[w].reshape(-1), "NVFP4").double().T * 2.0 ** -9
         assert rel_fro(out[0][rows[i]].float(), want) < 2.5e-3
+
+
+@pytest.mark.parametrize("M,N,K,S", [(65, 1000, 512, 0), (128, 6144, 576, 64), (100, 4096, 1024, 0), (200, 6144, 640, 0), (256, 4096, 1024, 128), (333, 6145, 1152, 0),
+                                     (333, 4096, 8192, 128), (400, 6144, 1024, 128), (400, 4100, 2048, 0), (80, 28672, 512, 128), (777, 6144, 1024, 128),
+                                     (1000, 4608, 1024, 0), (112, 20500, 640, 0), (512, 4096, 8192, 0), (1024, 3000, 512, 0)])
+def test_nvfp4_a_few_hundred_rows(agemm, oracle, M, N, K, S):
+    """NVFP4 problems of 65 to 1024 rows: shapes of up to 112 rows per workgroup in the place of the plan's tiles, rows and
+    columns ending inside them; exact products and fp32 sums as for decode batches."""
+    (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, K, S, "NVFP4", seed=71)
+    want = oracle_dq(oracle, a, sfa, "NVFP4") @ oracle_dq(oracle, b, sfb, "NVFP4").T * (gx * gw)
+    scale = (torch.tensor(gx, device="cuda"), torch.tensor(gw, device="cuda"))
+    y = agemm.matmul(a, b, sfa, sfb, scale)
+    assert rel_fro(y.float(), want) < 2.5e-3
+    assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
+    res = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
+    assert torch.equal(agemm.matmul(a, b, sfa, sfb, scale, residual=res), y + res)
