@@ -199,9 +199,7 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
     barrier();
   }
   if (!group) barrier();
-  const bool whole = m_base + BT <= p.M && n_base + BT <= p.N;
-  store_wave_tile(p, Acc16<8, 4>{acc}, reinterpret_cast<uint8_t *>(smem) + wave * kRegion, m_base + 64 * pos, n_base + 128 * group,
-                  whole, lane);
+  store_wave_tile(p, Acc16<8, 4>{acc}, reinterpret_cast<uint8_t *>(smem) + wave * kRegion, m_base + 64 * pos, n_base + 128 * group, lane);
 }
 
 }  // namespace

@@ -254,12 +254,11 @@ __device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, i
       }
     return;
   }
-  const bool whole = c_base + BC <= rows_c && f_base + BF <= rows_f;
   uint8_t *region = smem + wave * kRegion;
   if constexpr (CODES_W)
-    store_wave_tile(p, Acc16<4, TF>{acc}, region, f_base + 16 * TF * group, c_base + 64 * cpos, whole, lane);
+    store_wave_tile(p, Acc16<4, TF>{acc}, region, f_base + 16 * TF * group, c_base + 64 * cpos, lane);
   else
-    store_wave_tile(p, Acc16<TF, 4>{acc}, region, c_base + 64 * cpos, f_base + 16 * TF * group, whole, lane);
+    store_wave_tile(p, Acc16<TF, 4>{acc}, region, c_base + 64 * cpos, f_base + 16 * TF * group, lane);
 }
 
 template <bool CODES_W>
@@ -380,15 +379,13 @@ __global__ __launch_bounds__(64) void f16_split_add_kernel(GemmParams p) {
         (CODES_W ? acc[i][t] : acc[t][i]) += v4f{v.x, v.y, v.z, v.w};
       }
   }
-  const int rows_c = CODES_W ? p.N : p.M, rows_f = CODES_W ? p.M : p.N;
   int c_base, f_base;
   f16_tile_at<CODES_W>(p, lin, c_base, f_base);
-  const bool whole = c_base + S::BC <= rows_c && f_base + S::BF <= rows_f;
   uint8_t *region = reinterpret_cast<uint8_t *>(smem);
   if constexpr (CODES_W)
-    store_wave_tile(p, Acc16<4, TF>{acc}, region, f_base + 16 * TF * group, c_base + 64 * cpos, whole, lane);
+    store_wave_tile(p, Acc16<4, TF>{acc}, region, f_base + 16 * TF * group, c_base + 64 * cpos, lane);
   else
-    store_wave_tile(p, Acc16<TF, 4>{acc}, region, c_base + 64 * cpos, f_base + 16 * TF * group, whole, lane);
+    store_wave_tile(p, Acc16<TF, 4>{acc}, region, c_base + 64 * cpos, f_base + 16 * TF * group, lane);
 }
 
 template <bool CODES_W>

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "arcq_gemm_tile.h"
 
@@ -59,7 +60,7 @@ struct StreamShape {
   static_assert(NW * kBatch * 1024 <= kLds, "a batch of sums fits");
 };
 
-template <int MT, int NT, int WN, int WK, int NS>
+template <int MT, int NT, int WN, int WK, int NS, bool GROUPED>
 __device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, int m_base, uint8_t *smem) {
   using S = StreamShape<MT, NT, WN, WK, NS>;
   constexpr int NW = S::NW, BN = S::BN, BM = S::BM, RB = S::RB, SB = S::SB, NB = S::NB;
@@ -195,7 +196,10 @@ __device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, 
 
   // the sums of the waves that share a tile meet in LDS, added in the order of K
   float4 *red = reinterpret_cast<float4 *>(smem);
-  const Alpha by_column(p);
+  // (a grouped launch has one alpha and a residual of C's shape; with the parts' code in it, too, a decode step
+  // over eight experts of 28672 x 4224 and 4096 x 14464 takes 288 us instead of 253)
+  const std::conditional_t<GROUPED, OneAlpha, Alpha> by_column(p);
+  const size_t ld_residual = GROUPED ? p.N : p.ld_residual;
   uint32_t amax = 0u;
   constexpr int Q = NT * MT, QB = S::kBatch;
 #pragma unroll
@@ -229,7 +233,7 @@ __device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, 
       }
       if (m >= p.M || n >= p.N) continue;
       uint16_t *dst = p.c + (size_t)m * p.N + n;
-      const uint16_t *res = p.residual ? p.residual + (size_t)m * p.ld_residual + n : nullptr;
+      const uint16_t *res = p.residual ? p.residual + (size_t)m * ld_residual + n : nullptr;
       if ((p.N & 3) == 0) {
         uint2 o = make_uint2(pack_bf16_rne(v.x * alpha, v.y * alpha), pack_bf16_rne(v.z * alpha, v.w * alpha));
         if (res) o = add_bf16_x4(o, *reinterpret_cast<const uint2 *>(res));
@@ -282,11 +286,11 @@ __global__ __launch_bounds__(64 * WN * WK) void gemm_nvfp4_stream(GemmParams p) 
   const int n_base = (lin / tiles_m) * S::BN, m_base = (lin % tiles_m) * S::BM;
   if constexpr (GROUPED && MT > 1) {  // experts of few rows: no matrix instructions for rows that are not there
     const int rows = p.M - m_base;
-    if (rows <= 16) return nv_stream_tile<1, NT, WN, WK, NS>(p, n_base, m_base, lds);
-    if (MT > 2 && rows <= 32) return nv_stream_tile<2, NT, WN, WK, NS>(p, n_base, m_base, lds);
-    if (MT > 3 && rows <= 48) return nv_stream_tile<3, NT, WN, WK, NS>(p, n_base, m_base, lds);
+    if (rows <= 16) return nv_stream_tile<1, NT, WN, WK, NS, GROUPED>(p, n_base, m_base, lds);
+    if (MT > 2 && rows <= 32) return nv_stream_tile<2, NT, WN, WK, NS, GROUPED>(p, n_base, m_base, lds);
+    if (MT > 3 && rows <= 48) return nv_stream_tile<3, NT, WN, WK, NS, GROUPED>(p, n_base, m_base, lds);
   }
-  nv_stream_tile<MT, NT, WN, WK, NS>(p, n_base, m_base, lds);
+  nv_stream_tile<MT, NT, WN, WK, NS, GROUPED>(p, n_base, m_base, lds);
 }
 
 template <int MT, int NT, int WN, int WK, int NS, bool GROUPED = false>
@@ -362,7 +366,7 @@ int nvfp4_mid_shape(int M, int N, int Kp, int kernel, int slices) {
   else if (kernel == 22)
     tiled = 4 + (tiles(128, 128) <= 256 ? 30 : 27) * k * rounds(tiles(128, 128));
   else if (kernel == 42)
-    tiled = 4 + 58 * k * rounds(tiles(128, 256));
+    tiled = 4 + 28 * k * (1 + rounds(tiles(128, 256)));  // (further rounds: half the first one's and more)
   else
     return -1;
   int best = -1;

@@ -218,6 +218,12 @@ struct Alpha {
   }
 };
 
+struct OneAlpha {
+  float a;
+  __device__ __forceinline__ explicit OneAlpha(const GemmParams &p) : a(effective_alpha(p)) {}
+  __device__ __forceinline__ float at(const GemmParams &, int) const { return a; }
+};
+
 // These write M0.  The compiler reserves M0 and refuses it on a clobber list ("may lead to undefined
 // behaviour"), so the contract is kept by hand: the kernels that use these helpers contain nothing for
 // which the compiler would set or read M0 itself (no LDS-direct builtins, no indirect register
@@ -283,13 +289,11 @@ struct Acc16 {  // v_mfma_*_16x16x*: element e of a lane is n = 4 (lane / 16) + 
   __device__ __forceinline__ float4 quad(int q, int j) const { return make_float4(a[q][j][0], a[q][j][1], a[q][j][2], a[q][j][3]); }
 };
 
-// Fused SwiGLU epilogue of the tiled kernels (p.swiglu): a lane's four consecutive columns of one row are
+// Fused SwiGLU epilogue of the tiled kernels (p.swiglu; N is a multiple of 16): a lane's four consecutive columns of one row are
 // (gate_j, up_j, gate_j+1, up_j+1); each is rounded to bf16 as the plain epilogue would store it, and the two
-// products act_fn(gate) * up leave as one dword.  Whole tiles go through LDS so that every store
-// instruction writes 16 bytes per lane along output rows; ragged tiles store dwords with bounds checks.
+// products act_fn(gate) * up leave through LDS, so that every store instruction writes 16 bytes per lane along output rows.
 template <class Acc>
-__device__ __forceinline__ void store_wave_tile_swiglu(const GemmParams &p, const Acc &acc, uint8_t *region, int m0, int n0,
-                                                       bool whole, int lane) {
+__device__ __forceinline__ void store_wave_tile_swiglu(const GemmParams &p, const Acc &acc, uint8_t *region, int m0, int n0, int lane) {
   const float alpha = effective_alpha(p);
   const int No = p.N >> 1;  // output columns
   uint32_t amax = 0u;       // max |t| of this lane as bf16 bits without the sign
@@ -297,47 +301,35 @@ __device__ __forceinline__ void store_wave_tile_swiglu(const GemmParams &p, cons
     const float4 v = acc.quad(q, j);
     return swiglu_pair(pack_bf16_rne(v.x * alpha, v.z * alpha), pack_bf16_rne(v.y * alpha, v.w * alpha));
   };
-  auto track = [&](uint32_t t) {
-    const uint32_t lo = t & 0x7fffu, hi = (t >> 16) & 0x7fffu;
-    amax = lo > amax ? lo : amax;
-    amax = hi > amax ? hi : amax;
-  };
-  if (whole && (No & 7) == 0) {
-    wait_dma_and_sync();  // every wave is done reading operands
-    constexpr int RB = Acc::kN;        // bytes per row of the wave tile: kN / 2 products
-    constexpr int LPR = Acc::kN / 16;  // lanes per row when reading 16 bytes each
-    static_assert((LPR & (LPR - 1)) == 0, "the swizzle needs a power of two");
+  wait_dma_and_sync();  // every wave is done reading operands
+  const int rows = p.M - m0;  // of this wave's tile inside C
+  if (rows <= 0) return;
+  constexpr int RB = Acc::kN;        // bytes per row of the wave tile: kN / 2 products
+  constexpr int LPR = Acc::kN / 16;  // lanes per row when reading 16 bytes each
+  static_assert((LPR & (LPR - 1)) == 0, "the swizzle needs a power of two");
 #pragma unroll
-    for (int q = 0; q < Acc::kQuads; ++q)
+  for (int q = 0; q < Acc::kQuads; ++q)
 #pragma unroll
-      for (int j = 0; j < Acc::kTiles; ++j) {
-        const int m = Acc::m(j, lane), c = Acc::n(q, lane) >> 2;  // row and dword of the row
-        const int sw = m & (LPR - 1);                             // swizzle of the row's 16-byte groups
-        const uint32_t t = product(q, j);
-        track(t);
-        *reinterpret_cast<uint32_t *>(region + m * RB + ((((c >> 2) ^ sw) << 2) | (c & 3)) * 4) = t;
+    for (int j = 0; j < Acc::kTiles; ++j) {
+      const int m = Acc::m(j, lane), c = Acc::n(q, lane) >> 2;  // row and dword of the row
+      const int sw = m & (LPR - 1);                             // swizzle of the row's 16-byte groups
+      const uint32_t t = product(q, j);  // (every lane: the special-value test of the activation is a vote of the whole wave)
+      if (m < rows && n0 + Acc::n(q, lane) < p.N) {
+        const uint32_t lo = t & 0x7fffu, hi = (t >> 16) & 0x7fffu;
+        amax = lo > amax ? lo : amax;
+        amax = hi > amax ? hi : amax;
       }
-    const int rr = lane / LPR, tq = lane % LPR;
-    uint16_t *cbase = p.c + (size_t)m0 * No + (n0 >> 1) + 8 * tq;
-#pragma unroll
-    for (int it = 0; it < (Acc::kM * LPR) / 64; ++it) {
-      const int m = it * (64 / LPR) + rr;
-      const int sw = m & (LPR - 1);
-      const uint4 v = *reinterpret_cast<const uint4 *>(region + m * RB + ((tq ^ sw) << 4));
-      *reinterpret_cast<uint4 *>(cbase + (size_t)m * No) = v;
+      *reinterpret_cast<uint32_t *>(region + m * RB + ((((c >> 2) ^ sw) << 2) | (c & 3)) * 4) = t;
     }
-  } else {
+  const int rr = lane / LPR, tq = lane % LPR, col = (n0 >> 1) + 8 * tq;
+  uint16_t *cbase = p.c + (size_t)m0 * No + col;
+  const int lane_rows = col < No ? rows : 0;
 #pragma unroll
-    for (int q = 0; q < Acc::kQuads; ++q)
-#pragma unroll
-      for (int j = 0; j < Acc::kTiles; ++j) {
-        const int m = m0 + Acc::m(j, lane), n = n0 + Acc::n(q, lane);
-        const uint32_t t = product(q, j);   // every lane computes (the special-value test of the
-        if (m < p.M && n + 3 < p.N) {       // activation function is a vote of the whole wave)
-          track(t);
-          *reinterpret_cast<uint32_t *>(p.c + (size_t)m * No + (n >> 1)) = t;
-        }
-      }
+  for (int it = 0; it < (Acc::kM * LPR) / 64; ++it) {
+    const int m = it * (64 / LPR) + rr;
+    const int sw = m & (LPR - 1);
+    const uint4 v = *reinterpret_cast<const uint4 *>(region + m * RB + ((tq ^ sw) << 4));
+    if (m < lane_rows) *reinterpret_cast<uint4 *>(cbase + (size_t)m * No) = v;
   }
   if (p.absmax_bits) {
 #pragma unroll
@@ -392,13 +384,12 @@ __device__ __forceinline__ void store_tile(const GemmParams &p, const Acc &acc, 
   }
 }
 
-// Epilogue shared by the tiled kernels, called by every wave of the workgroup.  m0 / n0: first row / column of C of this
-// wave's tile.  whole: the whole WORKGROUP tile lies inside C (the same for every wave: there is a barrier behind it).
-// region: 2 * kM * kN bytes of LDS of this wave's own, free for reuse once every wave is done reading operands.
+// Epilogue shared by the tiled kernels, called by every wave of the workgroup (there is a barrier in it).  m0 / n0: first row /
+// column of C of this wave's tile.  region: 2 * kM * kN bytes of LDS of this wave's own, free for reuse once every wave is done
+// reading operands.
 template <class Acc>
-__device__ __forceinline__ void store_wave_tile(const GemmParams &p, const Acc &acc, uint8_t *region, int m0, int n0,
-                                                bool whole, int lane) {
-  if (p.swiglu) return store_wave_tile_swiglu(p, acc, region, m0, n0, whole, lane);
+__device__ __forceinline__ void store_wave_tile(const GemmParams &p, const Acc &acc, uint8_t *region, int m0, int n0, int lane) {
+  if (p.swiglu) return store_wave_tile_swiglu(p, acc, region, m0, n0, lane);
   if (p.partial) {  // split-K: the unscaled fp32 tile of this K range
     float *part = p.partial + (size_t)blockIdx.y * p.M * p.N;
     const bool quads = (p.N & 3) == 0, inside = quads && n0 + Acc::kN <= p.N;
@@ -429,59 +420,94 @@ __device__ __forceinline__ void store_wave_tile(const GemmParams &p, const Acc &
     }
     return;
   }
-  const Alpha by_column(p);
+  // Each wave's tile is transposed through LDS (free now) so that every store instruction writes whole rows of the wave tile, 16
+  // bytes per lane; what lies behind C's last row or column is left out there.  (Tiles that reach
+  // beyond C stored from the registers, 8 bytes per lane and with tests per quad: 1500 x 6144 x 4352 MXFP4 37.0 us, so 32.7; 4090
+  // rows 78.0, so 73.0; NVFP4 192.0, so 187.2.  And that code made half of each kernel: 112 KB of <4,2,2>, more than the
+  // instruction cache holds.)
   constexpr int RB = 2 * Acc::kN;   // bytes per row of the wave tile
   constexpr int LPR = Acc::kN / 8;  // lanes per row when reading 16 bytes each
+  constexpr int IT = (Acc::kM * LPR) / 64;
   static_assert((LPR & (LPR - 1)) == 0, "the swizzle needs a power of two");
-  if (whole && (p.N & 7) == 0) {
-    // Whole tile inside C: transpose each wave's tile through LDS (free now) so that every store
-    // instruction writes whole rows of the wave tile, 16 bytes per lane.
-    const int rr = lane / LPR, t = lane % LPR;
-    uint16_t *cbase = p.c + (size_t)m0 * p.N + n0 + 8 * t;
-    constexpr int IT = (Acc::kM * LPR) / 64, RI = IT < 16 ? IT : 16;
-    // The residual is asked for ahead of the stores, sixteen pieces per lane at a time, the first ones before the transpose: one
-    // by one, each is a round trip to memory that the store before it holds up (16384 x 4096 x 4352 with a residual, four
-    // rounds of tiles: 439 us, so 397).
-    uint4 res[RI];
-    auto read_residual = [&](int first) {
+  float alpha[Acc::kQuads / Acc::kTileQuads];
+  {
+    const Alpha by_column(p);
 #pragma unroll
-      for (int k = 0; k < RI; ++k)
-        res[k] = *reinterpret_cast<const uint4 *>(p.residual + (size_t)(m0 + (first + k) * (64 / LPR) + rr) * p.ld_residual + n0 + 8 * t);
-    };
-    wait_dma_and_sync();  // every wave is done reading operands
-    if (p.residual) read_residual(0);
+    for (int i = 0; i < Acc::kQuads / Acc::kTileQuads; ++i) alpha[i] = by_column.at(p, n0 + Acc::kSide * i);
+  }
+  wait_dma_and_sync();  // every wave is done reading operands
+  if (m0 >= p.M) return;
 #pragma unroll
-    for (int q = 0; q < Acc::kQuads; ++q) {
-      const float alpha = by_column.at(p, n0 + Acc::kSide * (q / Acc::kTileQuads));
+  for (int q = 0; q < Acc::kQuads; ++q)
 #pragma unroll
-      for (int j = 0; j < Acc::kTiles; ++j) {
-        const int m = Acc::m(j, lane), c = Acc::n(q, lane) >> 2;  // row and 8-byte chunk of the row
-        const int sw = (m & (LPR - 1)) << 1;                      // even: keeps 8-byte chunk pairs adjacent
-        const float4 v = acc.quad(q, j);                          // the hardware's round-to-nearest-even convert
-        *reinterpret_cast<uint2 *>(region + m * RB + ((c ^ sw) << 3)) =
-            make_uint2(pack_bf16_rne(v.x * alpha, v.y * alpha), pack_bf16_rne(v.z * alpha, v.w * alpha));
-      }
+    for (int j = 0; j < Acc::kTiles; ++j) {
+      const int m = Acc::m(j, lane), c = Acc::n(q, lane) >> 2;  // row and 8-byte chunk of the row
+      const int sw = (m & (LPR - 1)) << 1;                      // even: keeps 8-byte chunk pairs adjacent
+      const float4 v = acc.quad(q, j);                          // the hardware's round-to-nearest-even convert
+      const float a = alpha[q / Acc::kTileQuads];
+      *reinterpret_cast<uint2 *>(region + m * RB + ((c ^ sw) << 3)) = make_uint2(pack_bf16_rne(v.x * a, v.y * a), pack_bf16_rne(v.z * a, v.w * a));
     }
+  const int rr = lane / LPR, n = n0 + 8 * (lane % LPR);
+  const int rows = n < p.N ? p.M - m0 : 0;  // of this lane's columns inside C
+  uint16_t *cbase = p.c + (size_t)m0 * p.N + n;
+  const uint16_t *rbase = p.residual ? p.residual + (size_t)m0 * p.ld_residual + n : nullptr;
+  auto row = [&](int it) { return it * (64 / LPR) + rr; };
+  auto piece = [&](int it) {
+    const int m = row(it), sw = (m & (LPR - 1)) << 1;
+    return *reinterpret_cast<const uint4 *>(region + m * RB + (((2 * (lane % LPR)) ^ sw) << 3));
+  };
+  auto put = [&](int it, const uint4 &v) {
+    if (row(it) < rows) *reinterpret_cast<uint4 *>(cbase + (size_t)row(it) * p.N) = v;
+  };
+  if ((p.N & 7) != 0) {  // rows of C that are not 16-byte aligned, and columns that end inside a lane's eight
+#pragma unroll 1
+    for (int it = 0; it < IT; ++it) {
+      if (row(it) >= rows) continue;
+      const uint4 v = piece(it);
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+      uint16_t *dst = cbase + (size_t)row(it) * p.N;
+      const uint16_t *res = rbase ? rbase + (size_t)row(it) * p.ld_residual : nullptr;
+      if ((p.N & 3) == 0) {  // quads are 8-byte aligned, and inside C or outside as a whole
 #pragma unroll
-    for (int it0 = 0; it0 < IT; it0 += RI) {
-      if (p.residual && it0 > 0) read_residual(it0);
-#pragma unroll
-      for (int k = 0; k < RI; ++k) {
-        const int m = (it0 + k) * (64 / LPR) + rr;
-        const int sw = (m & (LPR - 1)) << 1;
-        uint4 v = *reinterpret_cast<const uint4 *>(region + m * RB + (((2 * t) ^ sw) << 3));
-        if (p.residual)
-          v = make_uint4(add_bf16_pair(v.x, res[k].x), add_bf16_pair(v.y, res[k].y), add_bf16_pair(v.z, res[k].z),
-                         add_bf16_pair(v.w, res[k].w));
-        *reinterpret_cast<uint4 *>(cbase + (size_t)m * p.N) = v;
+        for (int h = 0; h < 2; ++h)
+          if (n + 4 * h < p.N) {
+            uint2 x = make_uint2(w[2 * h], w[2 * h + 1]);
+            if (res) x = add_bf16_x4(x, reinterpret_cast<const uint2 *>(res)[h]);
+            reinterpret_cast<uint2 *>(dst)[h] = x;
+          }
+        continue;
       }
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (n + e < p.N) {
+          uint32_t h = (w[e >> 1] >> (16 * (e & 1))) & 0xffffu;
+          if (res) h = f32_to_bf16_bits(bf16_bits_to_f32(h) + bf16_bits_to_f32(res[e]));
+          dst[e] = (uint16_t)h;
+        }
     }
     return;
   }
+  if (!rbase) {
 #pragma unroll
-  for (int i = 0; i < Acc::kQuads / Acc::kTileQuads; ++i)
+    for (int it = 0; it < IT; ++it) put(it, piece(it));
+    return;
+  }
+  // The residual is asked for sixteen pieces per lane at a time: one by one, each is a round trip to memory that the store
+  // before it holds up (16384 x 4096 x 4352 with a residual, four rounds of tiles: 439 us, so 397).
+  constexpr int RI = IT < 16 ? IT : 16;
 #pragma unroll
-    for (int j = 0; j < Acc::kTiles; ++j) store_tile(p, acc, i, j, m0, n0, lane, by_column);
+  for (int it0 = 0; it0 < IT; it0 += RI) {
+    uint4 res[RI];
+#pragma unroll
+    for (int k = 0; k < RI; ++k)
+      if (row(it0 + k) < rows) res[k] = *reinterpret_cast<const uint4 *>(rbase + (size_t)row(it0 + k) * p.ld_residual);
+#pragma unroll
+    for (int k = 0; k < RI; ++k) {
+      const uint4 v = piece(it0 + k);
+      put(it0 + k, make_uint4(add_bf16_pair(v.x, res[k].x), add_bf16_pair(v.y, res[k].y), add_bf16_pair(v.z, res[k].z),
+                              add_bf16_pair(v.w, res[k].w)));
+    }
+  }
 }
 
 // The same for the kernels whose waves form a 2 (along N) x NWM (along M) grid, wave = n + 2 * m, of 32x32 tiles.
@@ -489,10 +515,8 @@ __device__ __forceinline__ void store_wave_tile(const GemmParams &p, const Acc &
 template <int WN, int WM, int NWM = 2>
 __device__ __forceinline__ void store_workgroup_tile(const GemmParams &p, v16f (&acc)[WN][WM], uint8_t *ldsA,
                                                      uint8_t *ldsB, int m_base, int n_base, int wave, int lane) {
-  constexpr int BN = 64 * WN, BM = 32 * WM * NWM;
-  const bool whole = m_base + BM <= p.M && n_base + BN <= p.N;
   uint8_t *region = (wave < NWM ? ldsA : ldsB) + (wave % NWM) * (32 * WM * 64 * WN);
-  store_wave_tile(p, Acc32<WN, WM>{acc}, region, m_base + (wave >> 1) * 32 * WM, n_base + (wave & 1) * 32 * WN, whole, lane);
+  store_wave_tile(p, Acc32<WN, WM>{acc}, region, m_base + (wave >> 1) * 32 * WM, n_base + (wave & 1) * 32 * WN, lane);
 }
 
 // Swizzle of staged rows of eight 16-byte chunks for the 16x16 matrix instructions.  A 16-byte LDS read is served in groups of 16 lanes that are not
