@@ -998,8 +998,8 @@ constexpr size_t kSplitMaxBytes = kWorkspaceBytes[kWsSplitK];
 // The 256x256 MXFP4 tile: with a long K the ping-pong kernel (88, arcq_gemm_mx.hip), whose main loop is faster, else the one
 // that requests the next stage from one wave per SIMD (84), which gets in and out of a tile faster where that decides (grouped
 // launches; 2048 x 28672).  88's time against 84's, each forced for the whole of a process, whole and ragged problems of 2048 to
-// 16384 rows: K' = 19072 0.83-0.93, 14592 0.87-1.01, 11264 0.84-1.01, 9216 0.83-1.01, 8192 0.82-1.01, 4352 0.77 (4000 x 4090, which
-// 84 cannot run as persistent workgroups) to 1.03 (2048 x 28672).
+// 16384 rows: K' = 19072 0.83-0.93, 14592 0.87-1.01, 11264 0.84-1.01, 9216 0.83-1.01, 8192 0.82-1.01, 2176 to 5248, ragged ones
+// (700 to 7300 rows), 0.93-1.10.
 int large_mx_tile(int kernel, int Kp) { return kernel == 84 && Kp >= 8192 ? 88 : kernel; }
 
 // The eight-wave MXFP4 kernels address an operand's rows with 32-bit byte offsets from its base; beyond, the four-wave tile
