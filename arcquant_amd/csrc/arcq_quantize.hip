@@ -1541,6 +1541,45 @@ __global__ __launch_bounds__(1024) void rmsnorm_rows_kernel(const uint16_t *x, c
   meet_for_scale(top, divisor, ws, out);
 }
 
+// Few rows: the scales of all segments in one launch, a workgroup per segment and a wave per row, instead of clearing the words,
+// maxima by atomics and the division as three, which are bound by their launches.  A segment's rows all pass one CU, at about 100 GB/s, so
+// only while there are few: 4096 channels, eight even segments, 16 / 64 / 128 / 256 / 512 rows 2.9 / 3.3 / 4.0 / 5.4 / 8.3 us, all rows in
+// one segment 3.9 / 8.1 / 13.5 / 24.7 / 49; as three launches 7.1 to 7.6.  (Rows routed to two experts each: at most half of them in one.)
+constexpr size_t kGroupedScaleElems = (size_t)1 << 19;
+
+__global__ __launch_bounds__(1024) void grouped_scale_kernel(const uint16_t *x, size_t ld, int rows, int K, const int *seg, float divisor,
+                                                             float *out) {
+  __shared__ uint32_t wave_max[16];
+  const int e = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cpr = K >> 3;
+  int beg = 0;  // a segment begins where all before it have ended
+  for (int i = 1 + lane; i <= e; i += 64) beg = max(beg, seg[i]);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) beg = max(beg, __shfl_xor(beg, o));
+  const int end = min(seg[e + 1], rows);
+  uint32_t m = 0u;
+  for (int r = beg + wave; r < end; r += 16)
+    for (int c0 = lane; c0 < cpr; c0 += 512) {
+      uint4 q[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        q[j] = c0 + 64 * j < cpr ? *reinterpret_cast<const uint4 *>(x + (size_t)r * ld + 8 * (c0 + 64 * j)) : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t t[4] = {q[j].x, q[j].y, q[j].z, q[j].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m = max(m, max((t[i] << 16) & 0x7fffffffu, t[i] & 0x7fff0000u));
+      }
+    }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o));
+  if (lane == 0) wave_max[wave] = m;
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  for (int w = 1; w < 16; ++w) m = max(m, wave_max[w]);
+  const float scale = u2f(m) / divisor;
+  out[e] = scale == 0.0f ? 1.0f : scale;
+}
+
 // Per-segment maxima for grouped launches (rows sorted by segment): max |x|, or max |act_fn(gate) * up|,
 // over the rows of each segment, accumulated as the bits of a non-negative float in bits[segment] (zeroed
 // by the caller's launch in front).  A workgroup takes a contiguous run of rows and flushes its running
@@ -2157,6 +2196,12 @@ int arcq_grouped_tensor_scale(const void *x, const void *up, int ld, int M, int 
   if (!d_scales || !seg_offsets || (M > 0 && !x)) return ARCQ_ERR_NULL;
   if (M > 0 && (!arcq::aligned16(x) || (up && !arcq::aligned16(up)))) return ARCQ_ERR_ALIGN;
   hipStream_t st = static_cast<hipStream_t>(stream);
+  if (!up && M > 0 && n_seg <= 256 && (size_t)M * K <= arcq::kGroupedScaleElems) {
+    hipLaunchKernelGGL(arcq::grouped_scale_kernel, dim3(n_seg), dim3(1024), 0, st, static_cast<const uint16_t *>(x), (size_t)ld, M, K,
+                       seg_offsets, divisor, d_scales);
+    ARCQ_HIP_TRY(hipGetLastError());
+    return ARCQ_OK;
+  }
   uint32_t *bits = reinterpret_cast<uint32_t *>(d_scales);
   const int fin = (n_seg + 255) / 256;
   hipLaunchKernelGGL(arcq::zero_words_kernel, dim3(fin), dim3(256), 0, st, bits, n_seg);
