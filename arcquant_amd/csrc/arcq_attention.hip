@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "arcq_gemm_tile.h"
 
@@ -207,6 +208,8 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(AttentionPara
 extern "C" int arcq_attention_prefill(const void *q, int ldq, const void *k, int ldk, const void *v, int ldv, int batch, int seq,
                                       int num_qo_heads, int num_kv_heads, int head_dim, float sm_scale, void *o, int ldo, void *stream) {
   using namespace arcq;
+  const float scale = sm_scale * 1.44269504088896341f;
+  if (!(scale > 0.0f) || std::isinf(scale)) return ARCQ_ERR_SHAPE;  // the maximum is taken, and masked, ahead of the scale
   if (batch < 0 || seq < 0 || head_dim != 128 || num_kv_heads < 1 || num_qo_heads < num_kv_heads || num_qo_heads % num_kv_heads != 0)
     return ARCQ_ERR_SHAPE;
   const int need_q = num_qo_heads * 128, need_kv = num_kv_heads * 128;
@@ -220,7 +223,7 @@ extern "C" int arcq_attention_prefill(const void *q, int ldq, const void *k, int
   if (total > (1l << 30)) return ARCQ_ERR_SHAPE;
   AttentionParams p{static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k), static_cast<const uint16_t *>(v),
                     static_cast<uint16_t *>(o), ldq, ldk, ldv, ldo, batch, seq, num_qo_heads, num_kv_heads,
-                    sm_scale * 1.44269504088896341f};
+                    scale};
   hipLaunchKernelGGL(attention_prefill_kernel, dim3((unsigned)(((total + 7) / 8) * 8)), dim3(256), 0, static_cast<hipStream_t>(stream), p);
   ARCQ_HIP_TRY(hipGetLastError());
   return ARCQ_OK;

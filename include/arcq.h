@@ -349,8 +349,8 @@ int arcq_scales_from_absmax(float *d_values, int n, float divisor, void *stream)
  * Causal attention of whole prompts (model/qLlamaLayer.py:340-370): o = softmax(q k^T * sm_scale) v over a sequence's own keys,
  * query i of a sequence seeing keys 0 .. i.  bf16, head_dim 128; query heads a multiple of the KV heads.  Rows are tokens (sequence b's
  * token t is row b * seq + t), a head's 128 values contiguous, ld* elements from row to row (multiples of 8; a fused projection's
- * output is read in place); every operand 16-byte aligned and a sequence's keys below 4 GiB.  Scores, weights' sums and outputs
- * accumulate in fp32, the weights enter the second product in bf16.
+ * output is read in place); every operand 16-byte aligned and a sequence's keys below 4 GiB; sm_scale above 0 and finite
+ * (ARCQ_ERR_SHAPE).  Scores, weights' sums and outputs accumulate in fp32, the weights enter the second product in bf16.
  */
 int arcq_attention_prefill(const void *q, int ldq, const void *k, int ldk, const void *v, int ldv, int batch, int seq,
                            int num_qo_heads, int num_kv_heads, int head_dim, float sm_scale, void *o, int ldo, void *stream);

@@ -70,4 +70,6 @@ def test_attention_prefill_refuses():
     call = lambda **kw: f(*{**good, **kw}.values(), None)
     assert call() == 0 and call(b=1, s=0) == 0
     assert call(d=64) == 2 and call(h=3) == 2 and call(ldq=511) == 2 and call(ldv=260) == 2 and call(ldk=128) == 2 and call(g=0) == 2
+    for c in (0.0, -0.1, float("inf"), float("-inf"), float("nan"), 3e38):             # 3e38 log2 e is not finite
+        assert call(c=c) == 2
     assert call(b=1, q=None) == 1 and call(b=1, v=0x1008) == 4 and call(b=1, s=1 << 23, ldk=512) == 2
