@@ -132,8 +132,9 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(AttentionPara
 #pragma unroll
       for (int e = 0; e < 16; ++e) top = __builtin_fmaxf(top, s[u][e]);
     top = __builtin_fmaxf(top, __shfl_xor(top, 32));
+    // (a query whose scores have all been -inf so far, by an infinity among its keys: weights of 0, not exp2(-inf + inf))
     if (__builtin_amdgcn_ballot_w64(top > m) != 0) {
-      const float next = __builtin_fmaxf(m, top), down = __builtin_amdgcn_exp2f((m - next) * c);
+      const float next = __builtin_fmaxf(m, top), down = next == -__builtin_inff() ? 0.0f : __builtin_amdgcn_exp2f((m - next) * c);
       m = next;
       l *= down;
 #pragma unroll
@@ -141,7 +142,7 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(AttentionPara
 #pragma unroll
         for (int e = 0; e < 16; ++e) o[t][e] *= down;
     }
-    const float mc = m * c;
+    const float mc = m == -__builtin_inff() ? 0.0f : m * c;
     v8bf pf[4];
 #pragma unroll
     for (int u = 0; u < 2; ++u)

@@ -350,7 +350,9 @@ int arcq_scales_from_absmax(float *d_values, int n, float divisor, void *stream)
  * query i of a sequence seeing keys 0 .. i.  bf16, head_dim 128; query heads a multiple of the KV heads.  Rows are tokens (sequence b's
  * token t is row b * seq + t), a head's 128 values contiguous, ld* elements from row to row (multiples of 8; a fused projection's
  * output is read in place); every operand 16-byte aligned and a sequence's keys below 4 GiB; sm_scale above 0 and finite
- * (ARCQ_ERR_SHAPE).  Scores, weights' sums and outputs accumulate in fp32, the weights enter the second product in bf16.
+ * (ARCQ_ERR_SHAPE).  Scores, weights' sums and outputs accumulate in fp32, the weights enter the second product in bf16.  A query
+ * with a visible score of +inf or NaN, or none but -inf, is NaN; an infinity or a NaN in a token's v also reaches the queries
+ * ahead of it in its tile of 64 tokens (0 * inf).
  */
 int arcq_attention_prefill(const void *q, int ldq, const void *k, int ldk, const void *v, int ldv, int batch, int seq,
                            int num_qo_heads, int num_kv_heads, int head_dim, float sm_scale, void *o, int ldo, void *stream);

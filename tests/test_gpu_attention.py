@@ -56,6 +56,24 @@ def test_attention_prefill_large_scores_and_order():
         assert float((got - want).norm() / want.norm()) < 2.3e-3
 
 
+def test_attention_prefill_minus_infinite_scores():
+    """An infinity among the keys that makes a query's scores -inf: no weight for that key, also where it is all that a query has seen
+    in its first tile of 64 keys; no other query of the wave is touched, and a query that sees nothing else is NaN"""
+    from arcquant_amd import kv_cache
+    seq, heads, hidden = 200, 2, 70
+    q, k, qkv = operands(1, seq, heads, heads)
+    q[..., 5] = torch.where(torch.arange(seq).view(-1, 1) % 2 == 0, 1.0, -1.0)      # even queries see -inf, odd ones +inf
+    for first in (0, 3):
+        kk = k.clone()
+        kk[first:hidden, :, 5] = float("-inf")
+        got = kv_cache.attention_prefill(q.cuda(), kk.cuda(), qkv.cuda()[:, 2 * heads * 128:], seq).cpu().double().view(seq, -1)
+        want = reference(q, kk, qkv[:, 2 * heads * 128:], seq).view(seq, -1)        # (NaN where the kernel documents it)
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        ok = ~torch.isnan(want).any(1)
+        assert int(ok.sum()) == (65 if first == 0 else 65 + 3 + 33) and bool(ok[198]) and not bool(ok[199])
+        assert float((got[ok] - want[ok]).norm() / want[ok].norm()) < 2.3e-3
+
+
 def test_attention_prefill_refuses():
     """what the kernel does not take is left to torch, and refused by the entry point"""
     from arcquant_amd import _lib, kv_cache
