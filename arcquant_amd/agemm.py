@@ -219,26 +219,30 @@ def _infer_fmt(A, SFA, fmt):
 
 
 @functools.lru_cache(maxsize=4096)
-def _workspace_bytes(M, N, Kp, f, n_seg):
-    """arcq_gemm_scratch_bytes, a function of these numbers alone (0.9 us a call through ctypes)"""
-    return _lib.lib().arcq_gemm_scratch_bytes(M, N, Kp, f, n_seg)
+def _workspace_sizes(M, N, Kp, f, n_seg):
+    """the sizes of workspace that arcq_gemm has a use for, the larger one first: arcq_gemm_scratch_bytes and
+    arcq_gemm_workspace_bytes, functions of these numbers alone (0.9 us a call through ctypes)"""
+    L = _lib.lib()
+    sizes = {ask(M, N, Kp, f, n_seg) for ask in (L.arcq_gemm_scratch_bytes, L.arcq_gemm_workspace_bytes)}
+    return tuple(sorted(sizes - {0}, reverse=True))
 
 
 def _gemm(A, SFA, B, SFB, M, N, Kp, f, c, *, alpha=1.0, da=None, db=None, residual=None, swiglu=0, seg=None, n_seg=0,
           absmax=None, parts=None):
     """arcq_gemm with the scratch memory its fastest kernel for the problem takes (up to 4 GiB, for the call), from torch's
-    allocator; where there is none, by the kernel that takes none"""
+    allocator; where there is none, by the kernel that takes less, or none"""
     L = _lib.lib()
-    nbytes, work = _workspace_bytes(M, N, Kp, f, n_seg) if f == _lib.NVFP4 else 0, None
-    if nbytes:
+    work = None
+    for size in _workspace_sizes(M, N, Kp, f, n_seg) if f == _lib.NVFP4 else ():
         try:
-            work = torch.empty(nbytes, dtype=torch.uint8, device=A.device)
+            work = torch.empty(size, dtype=torch.uint8, device=A.device)
+            break
         except torch.OutOfMemoryError:
-            nbytes = 0
+            pass
     args = _lib.GemmArgs(A.data_ptr(), SFA.data_ptr(), B.data_ptr(), SFB.data_ptr(), M, N, Kp, f, alpha, swiglu, da, db,
                          None if residual is None else residual.data_ptr(), c.data_ptr(),
                          None if seg is None else seg.data_ptr(), n_seg, None if absmax is None else absmax.data_ptr(),
-                         None if work is None else work.data_ptr(), nbytes)
+                         None if work is None else work.data_ptr(), 0 if work is None else work.numel())
     with _on_device(A):
         if parts is None:
             _lib.check(L.arcq_gemm(args, _stream(A)), "arcq_gemm")
@@ -289,7 +293,7 @@ def matmul(A, B, SFA, SFB, scale, *, fmt=None, residual=None):
         _require(residual, "residual", torch.bfloat16, 2)
         if tuple(residual.shape) != (M, N) or residual.device != A.device:
             raise RuntimeError(f"residual must be bf16 [{M}, {N}] on A's device")
-    if M > 64 and f == _lib.NVFP4 and _workspace_bytes(M, N, Kp, f, 0):
+    if M > 64 and f == _lib.NVFP4 and _workspace_sizes(M, N, Kp, f, 0):
         _gemm(A, SFA, B, SFB, M, N, Kp, f, C, alpha=alpha, da=da, db=db, residual=residual)
         return C
     with _on_device(A):

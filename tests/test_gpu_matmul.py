@@ -315,6 +315,40 @@ def test_gemm_without_memory_for_the_workspace(agemm, monkeypatch, form):
     assert rel_fro(got.float(), want.float()) < 1e-3
 
 
+def test_gemm_with_memory_for_the_smaller_workspace(agemm, monkeypatch):
+    """Memory for the decoded operand, but not for the sums of the last round's parts beside it: the kernel that takes that much,
+    bit for bit, and not the ones that take none"""
+    import ctypes
+    from arcquant_amd import _lib
+    L, (M, N, kp) = _lib.lib(), (4100, 4096, 8192)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    codes = lambda rows: (torch.randint(0, 256, (rows, kp // 2), generator=g, device="cuda", dtype=torch.uint8),
+                          torch.randint(60, 90, (rows * (kp // 16),), generator=g, device="cuda", dtype=torch.uint8))
+    (a, sfa), (b, sfb) = codes(M), codes(N)
+    sizes = [L.arcq_gemm_scratch_bytes(M, N, kp, 0, 0), L.arcq_gemm_workspace_bytes(M, N, kp, 0, 0)]
+    if "ARCQ_GEMM_KERNEL" in os.environ:
+        pytest.skip("another kernel is forced")
+    assert sizes[0] > sizes[1] > 0
+    want = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    work = torch.empty(sizes[1], dtype=torch.uint8, device="cuda")
+    args = _lib.GemmArgs(a.data_ptr(), sfa.data_ptr(), b.data_ptr(), sfb.data_ptr(), M, N, kp, 0, 2.0 ** -9, 0, None, None, None, want.data_ptr(),
+                         None, 0, None, work.data_ptr(), sizes[1])
+    assert L.arcq_gemm(args, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    asked, empty = [], torch.empty
+
+    def scarce(*size, **kw):
+        if kw.get("dtype") is torch.uint8:
+            asked.append(size[0])
+            if size[0] > sizes[1]:
+                raise torch.OutOfMemoryError("no memory for the larger workspace")
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(torch, "empty", scarce)
+    got = agemm.matmul(a, b, sfa, sfb, 2.0 ** -9)
+    monkeypatch.undo()
+    assert asked == sizes and torch.equal(got, want)
+
+
 def test_gemm_workspace_too_small(agemm):
     """A workspace one byte short of what arcq_gemm_workspace_bytes says is not used: the result of the call without one,
     bit for bit, and not a byte of it written."""
