@@ -1542,10 +1542,22 @@ __global__ __launch_bounds__(1024) void rmsnorm_rows_kernel(const uint16_t *x, c
 }
 
 // Few rows: the scales of all segments in one launch, a workgroup per segment and a wave per row, instead of clearing the words,
-// maxima by atomics and the division as three, which are bound by their launches.  A segment's rows all pass one CU, at about 100 GB/s, so
-// only while there are few: 4096 channels, eight even segments, 16 / 64 / 128 / 256 / 512 rows 2.9 / 3.3 / 4.0 / 5.4 / 8.3 us, all rows in
-// one segment 3.9 / 8.1 / 13.5 / 24.7 / 49; as three launches 7.1 to 7.6.  (Rows routed to two experts each: at most half of them in one.)
-constexpr size_t kGroupedScaleElems = (size_t)1 << 19;
+// maxima by atomics and the division as three, which are bound by their launches (7.0 to 7.6 us with 1 to 8 segments of 4096
+// channels, 11 with 14336 or with 64 segments, 6.4 with 8 to 64 channels).  A segment's rows all pass one CU, at about 90 GB/s from 512
+// channels on and a wave's load at a time below, so the time is the longest segment's, which only the device knows.
+constexpr int kGroupedScaleSegments = 256;
+
+// So that rows dealt out evenly are one to a wave, and few enough that a skewed segment costs little: 4096 channels, eight
+// segments, us even / half of the rows in one segment (the most that routing to two experts each can give) / all of them: 32 rows
+// 3.0 / 3.8 / 5.1, 64 rows 3.2 / 5.0 / 7.9, 128 rows 4.0 / 8.0 / 13.5 (three launches 7.5 / 7.6 / 7.4), 256 rows would be 5.4 / 13 / 25.
+// One segment: 16 rows 3.7 (7.0), 128 would be 13.4.  64 segments of 2048 channels: 128 rows 3.0 / 7.4 / 12.7, 256 rows 3.0 / 12.6 / 23
+// (three launches 12 / 11.6 / 9; tokens that go to eight of 64 experts leave an eighth of the rows to one at most).  Short rows: 32
+// of 64 channels 3.3 / 3.8 / 6.5 (6.9 / 6.5 / 6.4), 128 would be 4.1 / 12 / 18.
+bool grouped_scale_in_one_launch(int M, int K, int n_seg) {
+  const size_t n = (size_t)M * K;
+  return n_seg <= kGroupedScaleSegments && M <= 16 * n_seg && M <= (K < 512 ? 32 : n_seg < 32 ? 128 : 256) &&
+         n <= (size_t)n_seg << 16 && n <= (size_t)1 << 19;
+}
 
 __global__ __launch_bounds__(1024) void grouped_scale_kernel(const uint16_t *x, size_t ld, int rows, int K, const int *seg, float divisor,
                                                              float *out) {
@@ -2196,7 +2208,7 @@ int arcq_grouped_tensor_scale(const void *x, const void *up, int ld, int M, int 
   if (!d_scales || !seg_offsets || (M > 0 && !x)) return ARCQ_ERR_NULL;
   if (M > 0 && (!arcq::aligned16(x) || (up && !arcq::aligned16(up)))) return ARCQ_ERR_ALIGN;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  if (!up && M > 0 && n_seg <= 256 && (size_t)M * K <= arcq::kGroupedScaleElems) {
+  if (!up && M > 0 && arcq::grouped_scale_in_one_launch(M, K, n_seg)) {
     hipLaunchKernelGGL(arcq::grouped_scale_kernel, dim3(n_seg), dim3(1024), 0, st, static_cast<const uint16_t *>(x), (size_t)ld, M, K,
                        seg_offsets, divisor, d_scales);
     ARCQ_HIP_TRY(hipGetLastError());
