@@ -53,6 +53,13 @@ def _no_grad(forward):
     return run
 
 
+def _own(module, name):
+    """module.name where it is a buffer, without the search through three dictionaries that an access through the module begins
+    with; what has taken a buffer's place since (a Parameter, a parametrization) as the module has it"""
+    t = module._buffers.get(name)
+    return getattr(module, name) if t is None else t
+
+
 def _tensor_scale(t: torch.Tensor, signed: bool) -> torch.Tensor:
     """NVFP4 tensor scale as a 0-dim fp32 device tensor.  Activations: max|x| / 2688
     (model/qLlamaLayer.py:74); weights: the signed max (model/qLinearLayer.py:26).  A zero tensor
@@ -147,11 +154,10 @@ class QLinearLayer(nn.Module):
         """residual [..., out_features]: added to the output (in the GEMM's epilogue when the layer has
         no bias), same bits as `self(x) + residual`"""
         qx, scale_x, scale, bsz, q_len = x
-        own = self._buffers                # (each access through the module would search three dictionaries first)
-        alpha = (scale if isinstance(scale, torch.Tensor) else float(scale), own["scale"])
-        bias = self.bias if "bias" not in own else own["bias"]
+        alpha = (scale if isinstance(scale, torch.Tensor) else float(scale), _own(self, "scale"))
+        bias = _own(self, "bias")
         fused = residual is not None and bias is None
-        y = agemm.matmul(qx, own["W"], scale_x, own["scale_w"], alpha, fmt=self.quant_type,
+        y = agemm.matmul(qx, _own(self, "W"), scale_x, _own(self, "scale_w"), alpha, fmt=self.quant_type,
                          residual=residual.reshape(-1, self.out_features).contiguous() if fused else None)
         if bias is not None:
             y = y + bias
@@ -188,8 +194,7 @@ class RMSNormQuant(nn.Module):
     def forward(self, hidden_states):
         bsz, q_len, _ = hidden_states.shape
         flat = hidden_states.reshape(bsz * q_len, -1).contiguous()
-        own = self._buffers
-        A, SFA = agemm.rmsnorm_quantize_x(flat, own["weight"], self.variance_epsilon, own["reorder_index"],
+        A, SFA = agemm.rmsnorm_quantize_x(flat, _own(self, "weight"), self.variance_epsilon, _own(self, "reorder_index"),
                                           self.select_num, fmt=self.quant_type)
         return A, SFA, 1.0, bsz, q_len
 
@@ -443,7 +448,7 @@ class SplitQLinear(nn.Module):
             if bias is None or bias.dtype != torch.bfloat16:
                 return None
         W, scale_w = self._joint("W"), self._joint("scale_w")
-        scales = [p._buffers["scale"] for p in ps]
+        scales = [_own(p, "scale") for p in ps]
         if W is None or scale_w is None or any(s.dtype != torch.float32 or s.device != W.device for s in scales):
             return None
         return agemm.matmul_parts(qx, W, scale_x, scale_w, scale, [p.out_features for p in ps], scales, fmt=ps[0].quant_type,
@@ -471,7 +476,7 @@ class LlamaRMSNorm(nn.Module):
 
     def _in_one_launch(self, hidden_states):
         """bf16 rows that arcq_rmsnorm takes, as [rows, K]; None for others"""
-        w, x = self._buffers["weight"], hidden_states
+        w, x = _own(self, "weight"), hidden_states
         k = x.shape[-1] if x.dim() else 0
         if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not x.is_cuda or x.device != w.device or x.dim() < 2 or \
                 w.shape != (k,) or k % 8 or not 8 <= k <= 16384 or not self.variance_epsilon >= 0:

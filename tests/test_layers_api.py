@@ -40,3 +40,43 @@ def test_rotary_matches_closed_form():
     for i, p in enumerate((2, 3, 4)):
         assert qe[0, 0, i, 0].item() == pytest.approx(torch.cos(torch.tensor(float(p))).item(), abs=1e-6)
         assert qe[0, 0, i, 2].item() == pytest.approx(torch.sin(torch.tensor(float(p))).item(), abs=1e-6)
+
+
+def _quantized_linear(out_features, half, bias=None):
+    """a QLinearLayer over given codes (its constructor quantizes on the GPU)"""
+    lin = layers.QLinearLayer.__new__(layers.QLinearLayer)
+    nn.Module.__init__(lin)
+    lin.in_features, lin.out_features, lin.select_num, lin.quant_type = 2 * half, out_features, 0, "NVFP4"
+    g = torch.Generator().manual_seed(out_features)
+    lin.register_buffer("W", torch.randint(0, 256, (out_features, half), generator=g, dtype=torch.uint8))
+    lin.register_buffer("scale_w", torch.randint(0, 256, (out_features * half // 8,), generator=g, dtype=torch.uint8))
+    lin.register_buffer("scale", torch.tensor(0.5))
+    if bias is None:
+        lin.bias = None
+    else:
+        lin.register_buffer("bias", bias)
+    return lin
+
+
+def test_buffers_replaced_by_parameters(monkeypatch):
+    """torch moves a name out of the buffers when a Parameter is assigned to it: the layers find it all the same"""
+    seen = []
+    monkeypatch.setattr(layers.agemm, "matmul", lambda *a, **kw: seen.append(a) or torch.zeros(2, 32, dtype=torch.bfloat16))
+    monkeypatch.setattr(layers.agemm, "rmsnorm_quantize_x", lambda *a, **kw: seen.append(a) or (None, None))
+    param = lambda t: nn.Parameter(t, requires_grad=False)
+    x = torch.randn(1, 2, 64).to(torch.bfloat16)
+    lin = _quantized_linear(32, 32, torch.ones(32, dtype=torch.bfloat16))
+    quantized = (torch.zeros(2, 32, dtype=torch.uint8), torch.zeros(8, dtype=torch.uint8), 0.25, 1, 2)
+    want = lin(quantized)
+    for name in ("W", "scale_w", "scale", "bias"):
+        setattr(lin, name, param(getattr(lin, name)))
+    assert torch.equal(lin(quantized), want) and not lin._buffers
+    assert all(a is b for a, b in zip((seen[1][1], seen[1][3], seen[1][4][1]), (lin.W, lin.scale_w, lin.scale)))
+    norm = layers.RMSNormQuant(torch.ones(64), 1e-5, 0, torch.arange(64))
+    norm.weight, norm.reorder_index = param(norm.weight), param(norm.reorder_index)
+    norm(x)
+    assert seen[2][1] is norm.weight and seen[2][3] is norm.reorder_index
+    plain = layers.LlamaRMSNorm(torch.linspace(0.5, 1.5, 64), 1e-5)
+    want = plain(x)
+    plain.weight = param(plain.weight)
+    assert torch.equal(plain(x), want)
