@@ -406,21 +406,33 @@ class SplitQLinear(nn.Module):
     (model/qLinearLayer.py:25-28), where the fused layers above have one scale for the stacked weight.
 
     The parts' quantized weights (and biases) are put one behind the other in one allocation, of which the parts hold
-    their pieces, and run as one GEMM that scales the columns by part, as long as they still lie so."""
+    their pieces, and run as one GEMM that scales the columns by part, as long as they still lie so.  Parts that such a GEMM does not take stay as they are and run one by one."""
 
     def __init__(self, parts):
         super().__init__()
         self.parts = nn.ModuleList(parts)
         self.select_num = parts[0].select_num
         self.out_features = sum(p.out_features for p in parts)
-        names = ["W", "scale_w"] + (["bias"] if all(p.bias is not None for p in parts) else [])
-        if len({p.W.shape[1] for p in parts}) == 1:
-            for name in names:
-                joint, at = torch.cat([getattr(p, name) for p in parts]), 0
-                for p in parts:
-                    n = getattr(p, name).shape[0]
-                    setattr(p, name, joint[at:at + n])
-                    at += n
+        self._join()
+
+    def _join(self):
+        """puts the parts' tensors one behind the other, if one GEMM takes them"""
+        ps, held = list(self.parts), {}
+        if not 2 <= len(ps) <= 4 or len(set(ps)) != len(ps) or \
+                any(type(p) is not QLinearLayer or p.quant_type != ps[0].quant_type or p.out_features % 32 for p in ps):
+            return
+        for name in ["W", "scale_w"] + (["bias"] if any(_own(p, "bias") is not None for p in ps) else []):
+            held[name] = ts = [p._buffers.get(name) for p in ps]
+            if any(type(t) is not torch.Tensor or t.is_meta or t.dtype != ts[0].dtype or
+                   t.device != ts[0].device or t.shape[1:] != ts[0].shape[1:] for t in ts):
+                return
+        try:
+            joint = {name: torch.cat(ts) for name, ts in held.items() if self._joint(name) is None}
+        except torch.OutOfMemoryError:
+            return
+        for name, whole in joint.items():
+            for p, piece in zip(ps, whole.split([t.shape[0] for t in held[name]])):
+                p._buffers[name] = piece
 
     def _joint(self, name):
         """the parts' tensors as the one that they are pieces of; None if they are not"""
@@ -429,6 +441,8 @@ class SplitQLinear(nn.Module):
             return None
         base = ts[0].untyped_storage().data_ptr()
         at = ts[0].data_ptr()
+        if at % 16:
+            return None
         for t in ts:
             if t.data_ptr() != at or t.untyped_storage().data_ptr() != base or t.dtype != ts[0].dtype or t.shape[1:] != ts[0].shape[1:]:
                 return None

@@ -80,3 +80,56 @@ def test_buffers_replaced_by_parameters(monkeypatch):
     want = plain(x)
     plain.weight = param(plain.weight)
     assert torch.equal(plain(x), want)
+
+
+def test_split_linear_leaves_other_parts_as_they_are(monkeypatch):
+    """parts that one GEMM does not take: odd row counts (whose scale bytes would lie unaligned), Parameters, biases of two types, one
+    part twice, other modules; each is built, keeps its tensors, and runs part by part"""
+    class Other(nn.Module):
+        select_num, out_features = 0, 8
+
+        def forward(self, x):
+            return torch.ones(x[0].shape[0], 8, dtype=torch.bfloat16)
+
+    monkeypatch.setattr(layers.agemm, "matmul", lambda A, B, *a, **kw: torch.ones(A.shape[0], B.shape[0], dtype=torch.bfloat16))
+    monkeypatch.setattr(layers.agemm, "matmul_parts", lambda *a, **kw: pytest.fail("run as one"))
+    bf = lambda n, t=torch.bfloat16: torch.ones(n, dtype=t)
+    held = _quantized_linear(32, 32)
+    held.W = nn.Parameter(held.W, requires_grad=False)
+    mixed = [_quantized_linear(32, 32, bf(32)), _quantized_linear(32, 32, bf(32, torch.float32))]
+    one = _quantized_linear(32, 32)
+    for parts in ([_quantized_linear(33, 32), _quantized_linear(40, 32)], [held, _quantized_linear(64, 32)], mixed,
+                  [one, one], [_quantized_linear(32, 32, bf(32)), _quantized_linear(32, 32)], [Other(), one],
+                  [_quantized_linear(32, 32) for _ in range(5)], [_quantized_linear(32, 32), _quantized_linear(32, 64)]):
+        before = [dict(p._buffers) for p in parts]
+        split = layers.SplitQLinear(parts)
+        assert all(p._buffers[k] is v for p, b in zip(parts, before) for k, v in b.items())
+        y = split((torch.zeros(2, 32, dtype=torch.uint8), torch.zeros(8, dtype=torch.uint8), 1.0, None, 2))
+        assert y.shape == (2, split.out_features)
+    assert mixed[1].bias.dtype == torch.float32
+
+
+def test_split_linear_runs_part_by_part_where_a_part_is_not_itself(monkeypatch):
+    """hooks, a replaced forward and tensors put in the joint ones' place: the parts are called as the modules that they are"""
+    ran = []
+    monkeypatch.setattr(layers.agemm, "matmul", lambda A, B, *a, **kw: ran.append("part") or torch.ones(A.shape[0], B.shape[0], dtype=torch.bfloat16))
+    monkeypatch.setattr(layers.agemm, "matmul_parts", lambda A, B, *a, **kw: ran.append("one") or torch.ones(A.shape[0], B.shape[0], dtype=torch.bfloat16))
+    x = (torch.zeros(2, 32, dtype=torch.uint8), torch.zeros(8, dtype=torch.uint8), 1.0, 1, 2)
+
+    def run(change):
+        split = layers.SplitQLinear([_quantized_linear(64, 32), _quantized_linear(32, 32)])
+        undo = change(split)
+        ran.clear()
+        assert split(x).shape == (1, 2, 96)
+        if undo is not None:
+            undo.remove()
+        return ran == ["one"]
+
+    assert run(lambda s: None)
+    assert not run(lambda s: s.parts[1].register_forward_hook(lambda *a: None))
+    assert not run(lambda s: s.parts[0].register_forward_pre_hook(lambda *a: None))
+    assert not run(lambda s: nn.modules.module.register_module_forward_hook(lambda *a: None))
+    assert not run(lambda s: setattr(s.parts[0], "forward", s.parts[0].forward))
+    assert not run(lambda s: setattr(s.parts[1], "W", s.parts[1].W.clone()))
+    assert not run(lambda s: setattr(s.parts[0], "scale_w", nn.Parameter(s.parts[0].scale_w, requires_grad=False)))
+    assert not run(lambda s: setattr(s.parts[0], "scale", s.parts[0].scale.double()))
