@@ -406,7 +406,8 @@ class SplitQLinear(nn.Module):
     (model/qLinearLayer.py:25-28), where the fused layers above have one scale for the stacked weight.
 
     The parts' quantized weights (and biases) are put one behind the other in one allocation, of which the parts hold
-    their pieces, and run as one GEMM that scales the columns by part, as long as they still lie so.  Parts that such a GEMM does not take stay as they are and run one by one."""
+    their pieces, and run as one GEMM that scales the columns by part, as long as they still lie so.  Moving the module
+    joins them again.  Parts that such a GEMM does not take stay as they are and run one by one."""
 
     def __init__(self, parts):
         super().__init__()
@@ -414,6 +415,11 @@ class SplitQLinear(nn.Module):
         self.select_num = parts[0].select_num
         self.out_features = sum(p.out_features for p in parts)
         self._join()
+
+    def _apply(self, fn, recurse=True):
+        super()._apply(fn, recurse)
+        self._join()
+        return self
 
     def _join(self):
         """puts the parts' tensors one behind the other, if one GEMM takes them"""
@@ -423,7 +429,7 @@ class SplitQLinear(nn.Module):
             return
         for name in ["W", "scale_w"] + (["bias"] if any(_own(p, "bias") is not None for p in ps) else []):
             held[name] = ts = [p._buffers.get(name) for p in ps]
-            if any(type(t) is not torch.Tensor or t.is_meta or t.dtype != ts[0].dtype or
+            if any(type(t) is not torch.Tensor or not (t.is_cuda or t.is_cpu and not t.is_shared()) or t.dtype != ts[0].dtype or
                    t.device != ts[0].device or t.shape[1:] != ts[0].shape[1:] for t in ts):
                 return
         try:

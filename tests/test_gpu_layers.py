@@ -624,3 +624,34 @@ def test_mixtral_block_from_calibration_files(layers, oracle, fmt, grouped, tmp_
     bad[cal.MOE_NAME_TEMPLATE.format(li, 0, "w3")] = torch.flip(ri[cal.MOE_NAME_TEMPLATE.format(li, 0, "w3")], [0])
     with pytest.raises(ValueError):
         layers.QMixtralSparseMoeBlock(gate, experts, sn, bad, li, quant_type=fmt)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("bias", [False, True])
+def test_split_linear_after_a_move(layers, monkeypatch, fmt, bias):
+    """to the CPU and back: the parts are one GEMM again, with the same result, and the first copy's memory is given back; a part
+    with a hook, or moved by itself, makes it run part by part: the same products, one bf16 rounding apart at most"""
+    idx = torch.randperm(512, generator=torch.Generator().manual_seed(3)).to(torch.int16).cuda()
+    parts = []
+    for n in (1024, 256, 288):
+        lin = nn.Linear(512, n, bias=bias, device="cuda", dtype=torch.bfloat16)
+        parts.append(layers.QLinearLayer(lin, 64, idx, quant_type=fmt))
+    split = layers.SplitQLinear(parts)
+    x = layers.quantize_tokens(torch.randn(1, 37, 512, device="cuda").to(torch.bfloat16), idx, 64, fmt)
+    ran, as_parts = [], layers.agemm.matmul_parts
+    monkeypatch.setattr(layers.agemm, "matmul_parts", lambda *a, **kw: ran.append(1) or as_parts(*a, **kw))
+    want = split(x)
+    used = torch.cuda.memory_allocated()
+    split.cpu()
+    assert torch.cuda.memory_allocated() < used - sum(p.W.numel() for p in parts)
+    split.cuda()
+    assert torch.cuda.memory_allocated() <= used
+    assert torch.equal(split(x), want) and len(ran) == 2
+    handle = parts[1].register_forward_hook(lambda *a: None)
+    hooked = split(x)
+    handle.remove()
+    parts[1].cpu().cuda()
+    moved = split(x)
+    assert len(ran) == 2 and torch.equal(hooked, moved) and torch.equal(hooked, torch.cat([p(x) for p in parts], dim=-1))
+    assert float((hooked.float() - want.float()).norm() / want.float().norm()) < 1e-3
+    assert torch.equal(split.cuda()(x), want) and len(ran) == 3

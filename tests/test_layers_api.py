@@ -1,5 +1,6 @@
 """Host-side checks of arcquant_amd.layers that need no GPU: the module imports, its callers keep the
 reference's names and argument order, and building a layer from CPU weights fails loudly."""
+import copy
 import inspect
 
 import pytest
@@ -80,6 +81,31 @@ def test_buffers_replaced_by_parameters(monkeypatch):
     want = plain(x)
     plain.weight = param(plain.weight)
     assert torch.equal(plain(x), want)
+
+
+def _one_behind_the_other(split, name):
+    ts = [p._buffers[name] for p in split.parts]
+    return all(a.data_ptr() + a.numel() * a.element_size() == b.data_ptr() for a, b in zip(ts, ts[1:])) and \
+        torch.equal(split._joint(name), torch.cat(ts))
+
+
+def test_split_linear_joins_its_parts_again_when_moved():
+    parts = [_quantized_linear(n, 64, torch.full((n,), float(n), dtype=torch.bfloat16)) for n in (96, 32, 64)]
+    want = [{k: v.clone() for k, v in p.state_dict().items()} for p in parts]
+    split = layers.SplitQLinear(parts)
+    names = ("W", "scale_w", "bias")
+    assert all(_one_behind_the_other(split, n) for n in names)
+    held = split._joint("W").data_ptr()
+    split.to(torch.device("cpu"))                                 # nothing moves: nothing is copied
+    assert split._joint("W").data_ptr() == held
+    shared = copy.deepcopy(split).share_memory()                  # not joined anew, which would take them out of the shared memory
+    assert all(p.W.is_shared() for p in shared.parts)
+    for moved in (split._apply(torch.clone), copy.deepcopy(split), nn.Sequential(parts[1], split)._apply(torch.clone)[1]):
+        assert all(_one_behind_the_other(moved, n) and moved._joint(n) is not None for n in names)
+        assert all(torch.equal(v, w[k]) for p, w in zip(moved.parts, want) for k, v in p.state_dict().items())
+    split.load_state_dict({k: v + 1 for k, v in split.state_dict().items()})
+    assert all(_one_behind_the_other(split, n) for n in names) and torch.equal(split.parts[2].bias, want[2]["bias"] + 1)
+    assert split._apply(torch.empty_like).to("meta").parts[0].W.is_meta
 
 
 def test_split_linear_leaves_other_parts_as_they_are(monkeypatch):
