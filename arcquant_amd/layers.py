@@ -29,6 +29,7 @@ from __future__ import annotations
 
 import functools
 import math
+import weakref
 from typing import Optional
 
 import torch
@@ -406,20 +407,29 @@ class SplitQLinear(nn.Module):
     (model/qLinearLayer.py:25-28), where the fused layers above have one scale for the stacked weight.
 
     The parts' quantized weights (and biases) are put one behind the other in one allocation, of which the parts hold
-    their pieces, and run as one GEMM that scales the columns by part, as long as they still lie so.  Moving the module
-    joins them again.  Parts that such a GEMM does not take stay as they are and run one by one."""
+    their pieces, and run as one GEMM that scales the columns by part, as long as they still lie so.  Moving or copying the
+    module joins them again.  Parts that such a GEMM does not take stay as they are and run one by one.  (A piece has a storage
+    of its own, which Tensor.record_stream does not see through: a module is given up when the streams that ran it are done.)"""
 
     def __init__(self, parts):
         super().__init__()
         self.parts = nn.ModuleList(parts)
         self.select_num = parts[0].select_num
         self.out_features = sum(p.out_features for p in parts)
+        self._first = {}                     # by name, the first piece of a joint tensor, for as long as a part holds it
         self._join()
 
     def _apply(self, fn, recurse=True):
         super()._apply(fn, recurse)
         self._join()
         return self
+
+    def __getstate__(self):
+        return {**self.__dict__, "_first": {}}
+
+    def __setstate__(self, state):
+        super().__setstate__({"_first": {}, **state})
+        self._join()
 
     def _join(self):
         """puts the parts' tensors one behind the other, if one GEMM takes them"""
@@ -437,23 +447,27 @@ class SplitQLinear(nn.Module):
         except torch.OutOfMemoryError:
             return
         for name, whole in joint.items():
-            for p, piece in zip(ps, whole.split([t.shape[0] for t in held[name]])):
-                p._buffers[name] = piece
+            pieces = whole.split([t.shape[0] for t in held[name]])
+            # (the first piece stays referenced below the first part's tensor and is gone with it)
+            self._first[name] = weakref.ref(pieces[0])
+            for p, piece in zip(ps, pieces):
+                # a storage of its own size, so that the piece is saved, shared and copied as any tensor is
+                p._buffers[name] = torch.utils.dlpack.from_dlpack(torch.utils.dlpack.to_dlpack(piece))
 
     def _joint(self, name):
         """the parts' tensors as the one that they are pieces of; None if they are not"""
-        ts = [p._buffers.get(name) for p in self.parts]
-        if any(t is None or not t.is_contiguous() for t in ts):
+        first = self._first.get(name)
+        first = None if first is None else first()
+        if first is None:
             return None
-        base = ts[0].untyped_storage().data_ptr()
-        at = ts[0].data_ptr()
-        if at % 16:
-            return None
-        for t in ts:
-            if t.data_ptr() != at or t.untyped_storage().data_ptr() != base or t.dtype != ts[0].dtype or t.shape[1:] != ts[0].shape[1:]:
+        at, rows = first.data_ptr(), 0
+        for p in self.parts:
+            t = p._buffers.get(name)
+            if t is None or t.data_ptr() != at or not t.is_contiguous() or t.dtype != first.dtype or t.shape[1:] != first.shape[1:]:
                 return None
             at += t.numel() * t.element_size()
-        return torch.as_strided(ts[0], (sum(t.shape[0] for t in ts), *ts[0].shape[1:]), ts[0].stride())
+            rows += t.shape[0]
+        return torch.as_strided(first, (rows, *first.shape[1:]), first.stride())
 
     def _as_one(self, x):
         """one GEMM over all parts, or None where they have to run one by one"""

@@ -85,6 +85,7 @@ def test_buffers_replaced_by_parameters(monkeypatch):
 
 def _one_behind_the_other(split, name):
     ts = [p._buffers[name] for p in split.parts]
+    assert all(t.untyped_storage().nbytes() == t.numel() * t.element_size() for t in ts)
     return all(a.data_ptr() + a.numel() * a.element_size() == b.data_ptr() for a, b in zip(ts, ts[1:])) and \
         torch.equal(split._joint(name), torch.cat(ts))
 
@@ -99,13 +100,43 @@ def test_split_linear_joins_its_parts_again_when_moved():
     split.to(torch.device("cpu"))                                 # nothing moves: nothing is copied
     assert split._joint("W").data_ptr() == held
     shared = copy.deepcopy(split).share_memory()                  # not joined anew, which would take them out of the shared memory
-    assert all(p.W.is_shared() for p in shared.parts)
+    assert all(p.W.is_shared() for p in shared.parts) and shared._joint("W") is None
     for moved in (split._apply(torch.clone), copy.deepcopy(split), nn.Sequential(parts[1], split)._apply(torch.clone)[1]):
         assert all(_one_behind_the_other(moved, n) and moved._joint(n) is not None for n in names)
         assert all(torch.equal(v, w[k]) for p, w in zip(moved.parts, want) for k, v in p.state_dict().items())
     split.load_state_dict({k: v + 1 for k, v in split.state_dict().items()})
     assert all(_one_behind_the_other(split, n) for n in names) and torch.equal(split.parts[2].bias, want[2]["bias"] + 1)
+    first = split._first["W"]
+    split.parts[0].W = split.parts[0].W.clone()                   # the joint tensor goes with the pieces
+    assert first() is None and split._joint("W") is None
     assert split._apply(torch.empty_like).to("meta").parts[0].W.is_meta
+
+
+class _TwoNames(nn.Module):
+    """its parts under two names, as the attention layers have them"""
+
+    def __init__(self, parts):
+        super().__init__()
+        self.qkv_proj = layers.SplitQLinear(parts)
+        self.q_proj, self.k_proj = parts
+
+
+def test_split_linear_is_saved_as_its_parts_are(tmp_path):
+    """the pieces of a joint allocation are tensors of their own for whoever saves them: no part carries the others' bytes, and
+    safetensors finds a name for each where a part has two"""
+    model = _TwoNames([_quantized_linear(96, 64), _quantized_linear(32, 64)])
+    state = {k: v.clone() for k, v in model.state_dict().items()}
+    torch.save(model.k_proj.state_dict(), tmp_path / "k.pt")
+    assert (tmp_path / "k.pt").stat().st_size < 96 * 64
+    torch.save(model, tmp_path / "model.pt")
+    again = torch.load(tmp_path / "model.pt", weights_only=False)
+    assert again.q_proj is again.qkv_proj.parts[0] and _one_behind_the_other(again.qkv_proj, "W")
+    safetensors = pytest.importorskip("safetensors.torch")
+    safetensors.save_model(model, str(tmp_path / "model.safetensors"))
+    model.load_state_dict({k: torch.zeros_like(v) for k, v in state.items()})
+    safetensors.load_model(model, str(tmp_path / "model.safetensors"))
+    for m in (model, again):
+        assert all(torch.equal(v, state[k]) for k, v in m.state_dict().items()) and _one_behind_the_other(m.qkv_proj, "scale_w")
 
 
 def test_split_linear_leaves_other_parts_as_they_are(monkeypatch):
