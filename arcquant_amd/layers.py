@@ -61,6 +61,17 @@ def _own(module, name):
     return getattr(module, name) if t is None else t
 
 
+def _plain(*tensors):
+    """Ordinary tensors, and nothing around this call that has to see every operator on them: traces, compilation, modes, vmap and
+    the other transforms, and forward-mode gradients are left to torch's own operators."""
+    C = torch._C
+    return not (torch.compiler.is_compiling() or C._get_tracing_state() is not None or torch.autograd.forward_ad._current_level >= 0 or
+                C._len_torch_dispatch_stack() > 0 or C._functorch.peek_interpreter_stack() is not None or
+                C._is_torch_function_mode_enabled() and not all(isinstance(m, torch.utils._device.DeviceContext) for m in
+                                                                torch.overrides._get_current_function_mode_stack())) and \
+        all(type(t) is torch.Tensor or type(t) is nn.Parameter for t in tensors)
+
+
 def _tensor_scale(t: torch.Tensor, signed: bool) -> torch.Tensor:
     """NVFP4 tensor scale as a 0-dim fp32 device tensor.  Activations: max|x| / 2688
     (model/qLlamaLayer.py:74); weights: the signed max (model/qLinearLayer.py:26).  A zero tensor
@@ -335,7 +346,7 @@ class LlamaAttention(nn.Module):
             kc[:, :, past_len:past_len + q_len] = k
             vc[:, :, past_len:past_len + q_len] = v
             k, v = kc[:, :, :past_len + q_len], vc[:, :, :past_len + q_len]
-        if rows is not None and kv_cache is None and past_len == 0:
+        if rows is not None and kv_cache is None and past_len == 0 and _plain(*rows):
             out = _kvc.attention_prefill(*rows, q_len)          # a prompt's own keys, read where they are
             if out is not None:
                 return self.o_proj(quantize_tokens(out.view(bsz, q_len, nh * d), self.o_reorder_index, self.o_proj.select_num,
@@ -510,7 +521,9 @@ class LlamaRMSNorm(nn.Module):
 
     def _in_one_launch(self, hidden_states):
         """bf16 rows that arcq_rmsnorm takes, as [rows, K]; None for others"""
-        w, x = _own(self, "weight"), hidden_states
+        if not _plain(hidden_states, self.weight):
+            return None
+        w, x = self.weight, hidden_states
         k = x.shape[-1] if x.dim() else 0
         if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or not x.is_cuda or x.device != w.device or x.dim() < 2 or \
                 w.shape != (k,) or k % 8 or not 8 <= k <= 16384 or not self.variance_epsilon >= 0:

@@ -655,3 +655,41 @@ def test_split_linear_after_a_move(layers, monkeypatch, fmt, bias):
     assert len(ran) == 2 and torch.equal(hooked, moved) and torch.equal(hooked, torch.cat([p(x) for p in parts], dim=-1))
     assert float((hooked.float() - want.float()).norm() / want.float().norm()) < 1e-3
     assert torch.equal(split.cuda()(x), want) and len(ran) == 3
+
+
+def test_rmsnorm_under_traces_and_transforms(layers, monkeypatch):
+    """What records or transforms torch's operators finds them in LlamaRMSNorm, whose own launch it could not see: a trace that is run on
+    other rows, vmap, forward-mode gradients, a compiled graph, a dispatch mode.  A default device is no reason to leave it."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils._python_dispatch import TorchDispatchMode
+    g = torch.Generator().manual_seed(8)
+    norm = layers.LlamaRMSNorm(torch.rand(512, generator=g).cuda() + 0.5, 1e-5)
+    x, other = (torch.randn(2, 5, 512, generator=g).to(torch.bfloat16).cuda() for _ in range(2))
+
+    def torchs(t):
+        h = t.float()
+        return norm.weight * (h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + 1e-5)).to(torch.bfloat16)
+
+    ran, own = [], layers.agemm.rmsnorm
+    monkeypatch.setattr(layers.agemm, "rmsnorm", lambda *a, **kw: ran.append(1) or own(*a, **kw))
+    assert rel_fro(torch.jit.trace(norm, x)(other), torchs(other)) < 5e-3    # (torch's fuser leaves out the rounding in between)
+    ran.clear()                                                              # (the trace's check runs the module by itself, too)
+    assert torch.equal(make_fx(lambda t: norm(t))(x)(other), torchs(other))
+    assert torch.equal(torch.vmap(norm)(torch.stack([x, other])), torch.stack([torchs(x), torchs(other)]))
+    assert torch.equal(torch.compile(norm, backend="eager", fullgraph=True)(x), torchs(x))
+    with torch.autograd.forward_ad.dual_level():
+        dual = lambda f: torch.autograd.forward_ad.unpack_dual(f(torch.autograd.forward_ad.make_dual(x, other)))
+        assert torch.equal(dual(norm).tangent, dual(torchs).tangent)
+
+    class Names(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    seen = []
+    with Names():
+        norm(x)
+    assert any("rsqrt" in s for s in seen) and not ran
+    with torch.device("cuda"):
+        y = norm(x)
+    assert len(ran) == 1 and torch.equal(norm(x), y) and rel_fro(y, torchs(x)) < 1e-3

@@ -190,3 +190,13 @@ def test_split_linear_runs_part_by_part_where_a_part_is_not_itself(monkeypatch):
     assert not run(lambda s: setattr(s.parts[1], "W", s.parts[1].W.clone()))
     assert not run(lambda s: setattr(s.parts[0], "scale_w", nn.Parameter(s.parts[0].scale_w, requires_grad=False)))
     assert not run(lambda s: setattr(s.parts[0], "scale", s.parts[0].scale.double()))
+
+
+def test_rmsnorm_of_tensors_without_memory():
+    """GPU tensors that only stand for some (a shape propagation ahead of a compilation): torch's operators, not an address"""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    norm = layers.LlamaRMSNorm(torch.ones(64), 1e-5)
+    with FakeTensorMode(allow_non_fake_inputs=True) as mode:
+        norm.weight = torch.empty(64, dtype=torch.bfloat16, device="cuda")
+        y = norm(torch.empty(2, 3, 64, dtype=torch.bfloat16, device="cuda"))
+        assert y.shape == (2, 3, 64) and y.dtype == torch.bfloat16 and y.fake_mode is mode
