@@ -406,10 +406,14 @@ class LlamaDecoderLayer(nn.Module):
 
 
 def _unhooked(module, cls):
-    """a call of the module is cls.forward and nothing else"""
-    return type(module) is cls and "forward" not in module.__dict__ and not (
-        module._forward_hooks or module._forward_pre_hooks or nn.modules.module._global_forward_hooks or
-        nn.modules.module._global_forward_pre_hooks)
+    """a call of the module is cls.forward as it stands here and nothing else"""
+    return type(module) is cls and cls.forward is _FORWARD[cls] and "forward" not in module.__dict__ and \
+        module._compiled_call_impl is None and not (
+            module._forward_hooks or module._forward_pre_hooks or nn.modules.module._global_forward_hooks or
+            nn.modules.module._global_forward_pre_hooks)
+
+
+_FORWARD = {QLinearLayer: QLinearLayer.forward}       # and LlamaRMSNorm, below
 
 
 class SplitQLinear(nn.Module):
@@ -546,6 +550,9 @@ class LlamaRMSNorm(nn.Module):
         h = hidden_states.to(torch.float32)
         h = h * torch.rsqrt(h.pow(2).mean(-1, keepdim=True) + self.variance_epsilon)
         return self.weight * h.to(dt)
+
+
+_FORWARD[LlamaRMSNorm] = LlamaRMSNorm.forward
 
 
 CALIBRATION_KEY = "layers.{}.{}.{}.{}"     # model/qLlamaLayer.py:236: layer, block, projection, 'input'

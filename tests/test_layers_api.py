@@ -187,9 +187,33 @@ def test_split_linear_runs_part_by_part_where_a_part_is_not_itself(monkeypatch):
     assert not run(lambda s: s.parts[0].register_forward_pre_hook(lambda *a: None))
     assert not run(lambda s: nn.modules.module.register_module_forward_hook(lambda *a: None))
     assert not run(lambda s: setattr(s.parts[0], "forward", s.parts[0].forward))
+    assert not run(lambda s: setattr(s.parts[0], "_compiled_call_impl", s.parts[0].forward))     # what .compile() sets
     assert not run(lambda s: setattr(s.parts[1], "W", s.parts[1].W.clone()))
     assert not run(lambda s: setattr(s.parts[0], "scale_w", nn.Parameter(s.parts[0].scale_w, requires_grad=False)))
     assert not run(lambda s: setattr(s.parts[0], "scale", s.parts[0].scale.double()))
+    own = layers.QLinearLayer.forward
+    monkeypatch.setattr(layers.QLinearLayer, "forward", lambda self, *a, **kw: own(self, *a, **kw))
+    assert not run(lambda s: None)
+
+
+def test_norm_ahead_of_a_quantizer_is_the_module(monkeypatch):
+    """the norm's launch that also forms the tensor scale stands in for LlamaRMSNorm's own forward alone"""
+    layer = layers.QLlamaDecoderLayer.__new__(layers.QLlamaDecoderLayer)
+    nn.Module.__init__(layer)
+    layer.fuse_norm, layer.quant_type = False, "NVFP4"
+    norm, x = layers.LlamaRMSNorm(torch.ones(64), 1e-5), torch.randn(1, 2, 64).to(torch.bfloat16)
+    monkeypatch.setattr(layers, "quantize_tokens", lambda t, *a: t)
+    monkeypatch.setattr(layers.agemm, "reorder_quantize_x", lambda t, *a, **kw: ("codes", "scales"))
+    monkeypatch.setattr(layers.LlamaRMSNorm, "forward_with_scale", lambda self, t: (t, 1.0))
+    quantize = lambda: layer._norm_and_quantize(norm, x, None, 0)
+    want = norm(x)
+    assert quantize() == ("codes", "scales", 1.0, 1, 2)
+    handle = norm.register_forward_hook(lambda m, i, y: y + 1)
+    assert torch.equal(quantize(), want + 1)
+    handle.remove()
+    own = layers.LlamaRMSNorm.forward
+    monkeypatch.setattr(layers.LlamaRMSNorm, "forward", lambda self, t: own(self, t) + 2)
+    assert torch.equal(quantize(), want + 2)
 
 
 def test_rmsnorm_of_tensors_without_memory():
