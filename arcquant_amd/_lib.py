@@ -131,22 +131,44 @@ def lib() -> ctypes.CDLL:
 HOST_LIB_PATH = os.path.join(_HERE, "csrc", "_arcq_host.so")
 
 
+def host_lib_mark() -> bytes:
+    """what _arcq_host.so holds if it was built against this torch"""
+    import torch
+    return b"built against torch " + torch.__version__.encode() + b"\0"
+
+
+def host_lib_is_current() -> bool:
+    if not os.path.exists(HOST_LIB_PATH):
+        return False
+    with open(HOST_LIB_PATH, "rb") as f:
+        return host_lib_mark() in f.read()
+
+
 class _Host:
     """_arcq_host.so (csrc/arcq_host.cpp), loaded on the first call: the ordinary case of an operator in one native call
-    that returns None for arguments it does not take."""
+    that returns None for arguments it does not take.  Where it is missing or belongs to another torch, that is all of them:
+    the general route over libarcq_hip.so needs nothing of it."""
+    _ENTRIES = ("quantize", "swiglu_quantize", "matmul", "decode_step")
 
     def __getattr__(self, name):
+        if name not in self._ENTRIES:
+            raise AttributeError(name)
         lib()
-        if not os.path.exists(HOST_LIB_PATH):
-            raise RuntimeError(f"{HOST_LIB_PATH} is missing: build it with `python -m arcquant_amd.build`")
         import importlib.util
-        import torch  # noqa: F401  (its libraries first: the module is linked against them)
-        spec = importlib.util.spec_from_file_location("_arcq_host", HOST_LIB_PATH)
-        module = importlib.util.module_from_spec(spec)
-        spec.loader.exec_module(module)
-        for f in ("quantize", "swiglu_quantize", "matmul", "decode_step"):
-            self.__dict__[f] = getattr(module, f)
-        return self.__dict__[name]
+        try:
+            if not host_lib_is_current():
+                raise ImportError(f"{HOST_LIB_PATH} is missing or was built against another torch")
+            spec = importlib.util.spec_from_file_location("_arcq_host", HOST_LIB_PATH)
+            module = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(module)
+            found = {f: getattr(module, f) for f in self._ENTRIES}
+        except (ImportError, OSError) as e:
+            import warnings
+            warnings.warn(f"{e}: operators take their general route, which costs the host more per call "
+                          "(`python -m arcquant_amd.build` builds it)", RuntimeWarning, stacklevel=2)
+            found = {f: lambda *args: None for f in self._ENTRIES}
+        self.__dict__.update(found)
+        return found[name]
 
 
 host = _Host()

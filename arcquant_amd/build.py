@@ -77,13 +77,15 @@ def build_host(force: bool = False, verbose: bool = False) -> str:
     import torch
     from torch.utils import cpp_extension
 
+    from . import _lib
+
     src = os.path.join(CSRC, "arcq_host.cpp")
-    if force or _stale(HOST_LIB, [src, os.path.join(HERE, "..", "include", "arcq.h"), HIP_LIB]):
+    if force or _stale(HOST_LIB, [src, os.path.join(HERE, "..", "include", "arcq.h"), HIP_LIB]) or not _lib.host_lib_is_current():
         rocm = os.path.dirname(os.path.dirname(_hipcc()))
         includes = [f"-isystem{d}" for d in (*cpp_extension.include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"])]
         libs = [f"-L{d}" for d in cpp_extension.library_paths()]
         cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
-               f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *includes, "-o", HOST_LIB, src, *libs, "-lc10",
+               f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f'-DARCQ_TORCH_VERSION="{torch.__version__}"', *includes, "-o", HOST_LIB, src, *libs, "-lc10",
                "-lc10_hip", "-ltorch_cpu", "-ltorch_python", f"-L{CSRC}", "-l:libarcq_hip.so", "-Wl,-rpath,$ORIGIN"]
         if verbose:
             print(" ".join(cmd), flush=True)

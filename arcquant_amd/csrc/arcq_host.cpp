@@ -304,4 +304,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_arcq_host", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__arcq_host(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__arcq_host(void) {
+  PyObject *m = PyModule_Create(&module);
+  // (looked for in the file ahead of loading it: a library of another torch is not loaded)
+  if (m && PyModule_AddStringConstant(m, "built", "built against torch " ARCQ_TORCH_VERSION) < 0) Py_CLEAR(m);
+  return m;
+}

@@ -27,6 +27,30 @@ def test_what_is_not_taken_on_the_cpu():
         agemm.matmul(codes, codes, sf, sf, 1.0)
 
 
+@pytest.mark.parametrize("how", ["missing", "another torch", "not a library"])
+def test_without_the_native_host_path(monkeypatch, tmp_path, how):
+    """no _arcq_host.so, one of another torch, one that does not load: a warning, and every operator by its general route"""
+    from arcquant_amd import _lib, agemm
+    assert _lib.host_lib_is_current()
+    path = tmp_path / "_arcq_host.so"
+    if how == "another torch":
+        with open(_lib.HOST_LIB_PATH, "rb") as f:
+            path.write_bytes(f.read().replace(_lib.host_lib_mark(), b"x" * len(_lib.host_lib_mark())))
+    elif how == "not a library":
+        path.write_bytes(_lib.host_lib_mark())
+    monkeypatch.setattr(_lib, "HOST_LIB_PATH", str(path))
+    h = _lib._Host()
+    with pytest.warns(RuntimeWarning, match="general route"):
+        assert h.matmul() is None
+    assert h.quantize(1, 2) is None and h.swiglu_quantize() is None and h.decode_step() is None
+    monkeypatch.setattr(agemm, "_host", h)
+    codes, sf = torch.zeros(4, 32, dtype=torch.uint8), torch.zeros(16, dtype=torch.uint8)
+    with pytest.raises(RuntimeError, match="must be on the GPU"):
+        agemm.matmul(codes, codes, sf, sf, 1.0)
+    with pytest.raises(AttributeError):
+        h.nothing
+
+
 def _general(monkeypatch, call):
     """the call by the general route"""
     from arcquant_amd import _lib, agemm
