@@ -410,15 +410,19 @@ size_t nvfp4_f16_bytes(int M, int N, int Kp, bool grouped) {
   return (size_t)(grouped || M <= N ? M : N) * Kp * 2;
 }
 
-// (Experts: the tiles are known on the device alone; from 512 rows per expert on.  Eight of 4096 x 14464, 8192 rows skewed 912 -> 816 us
-// against 128x128 tiles, even 822 -> 713; 4096 rows skewed 495 -> 463; 64 of 2048 x 8320, 600 rows each, would lose 5 %.)
+// (Experts: the tiles are known on the device alone; from 512 rows per expert on, and where the most tiles that the rows can make are
+// more than a round -- with no more of them nothing is ever cut, and 256x256 tiles leave CUs idle: 4096 x 14464, four experts of 512
+// rows 274 us, two 240, the kernels without a workspace 242 and 126.  Eight of 4096 x 14464, 8192 rows skewed 912 -> 825 us against
+// 128x128 tiles, even 840 -> 732; 4096 rows skewed 496 -> 464, even (256 tiles: one round) 439 -> 386; 5000 rows skewed 598 -> 552, but
+// even (625 rows each, three tiles) 539 -> 564; 64 of 2048 x 8320, 600 rows each, would lose 5 %.)
 size_t nvfp4_split_bytes(int M, int N, int Kp, int n_seg) {
   if (Kp < 8192 || Kp % 128 != 0 || M <= 64) return 0;
   if (n_seg == 0) {
     const long total = (long)((M + 255) / 256) * ((N + 255) / 256);
     if (!last_round_cut(total, Kp >> 7) || total > 6 * 256) return 0;
-  } else if (N <= 2048 || M / n_seg < 512 || ((M + 255) / 256 + n_seg / 2) * (long)((N + 255) / 256) > 6 * 256) {
-    return 0;
+  } else {
+    const long tiles_n = (N + 255) / 256, tiles_m = (M + 255) / 256;
+    if (N <= 2048 || M / n_seg < 512 || (tiles_m + n_seg) * tiles_n <= 256 || (tiles_m + n_seg / 2) * tiles_n > 6 * 256) return 0;
   }
   return 512 * F16Shape<true>::kSlot * sizeof(float4);
 }

@@ -149,6 +149,20 @@ def test_grouped_gemm_workspace(rows, n, kp, n_seg, decoded_rows):
     assert ask(rows, n, kp, 1, n_seg) == 0  # MXFP4 decodes nothing
 
 
+@pytest.mark.parametrize("rows,n,kp,n_seg,cut", [
+    (4 * 512, 4096, 14464, 4, False), (2 * 512, 4096, 14464, 2, False), (3072, 4096, 8192, 4, False),   # never more than a round of tiles
+    (3073, 4096, 8192, 4, True), (8 * 512, 4096, 14464, 8, True), (2 * 650, 14336, 8320, 2, True), (8 * 1024, 4096, 14464, 8, True),
+    (8 * 511, 4096, 14464, 8, False), (8 * 1024, 2048, 14464, 8, False), (8 * 1024, 4096, 8064, 8, False), (16 * 4096, 4096, 8192, 16, False),
+    (3000, 6144, 10240, 0, True), (4096, 4096, 14592, 0, False), (2331, 4096, 14592, 0, False),        # whole rounds; less than one
+])
+def test_gemm_scratch_for_a_cut_round(rows, n, kp, n_seg, cut):
+    """which NVFP4 problems take 128 MiB behind the decoded operand, to cut their last round of tiles along K': only where more than
+    a round of 256 is possible at all"""
+    L = _lib.lib()
+    operand = 2 * kp * (rows if n_seg else min(rows, n))
+    assert L.arcq_gemm_scratch_bytes(rows, n, kp, 0, n_seg) == (operand + (128 << 20) if cut else L.arcq_gemm_workspace_bytes(rows, n, kp, 0, n_seg))
+
+
 @pytest.mark.parametrize("M,N,kp,decoded_rows", [
     (2049, 4096, 4352, 2049), (257, 28672, 4352, 257), (33000, 64, 1152, 64), (65, 70000, 1152, 65),
     (2048, 4096, 4352, 0), (256, 28672, 4352, 0),                                 # one round of 256x128 tiles
