@@ -107,6 +107,8 @@ def lib() -> ctypes.CDLL:
     L.arcq_gemm_scratch_bytes.restype = sz
     L.arcq_gemm_kernel.argtypes = [i, i, i, i, i, i]
     L.arcq_gemm_kernel.restype = i
+    L.arcq_gemm_route.argtypes = [i, i, i, i, i, i]
+    L.arcq_gemm_route.restype = i
     for name in ("arcq_grouped_matmul_swiglu", "arcq_matmul_swiglu", "arcq_scales_from_absmax"):
         getattr(L, name).restype = i
     L.arcq_moe_combine.argtypes = [vp, vp, vp, i, i, i, i, vp, vp]

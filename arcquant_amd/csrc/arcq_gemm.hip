@@ -1137,19 +1137,19 @@ GemmPlan plan_swiglu(int M, int N, int Kp, int fmt) {
   return plan;
 }
 
-// NVFP4 decode batches run as a stream of the weights, whichever tiles (and slices of K) the plan has for them, and plain problems
-// of a few hundred rows where that is faster than the plan's tiles, unless a kernel or a number of slices is forced; plan 0 has operands
-// that only the direct kernels take.  -1: by the plan; 0: as a stream; 1 + shape: that shape.
-int stream_way(const GemmPlan &plan, const GemmParams &p, int fmt) {
-  if (fmt != ARCQ_FMT_NVFP4 || tuning().gemm_kernel >= 0 || tuning().gemm_splitk != 0 || plan.kernel == 0) return -1;
-  if (nvfp4_stream_wanted(p.M, p.N, p.Kp, p.n_seg)) return 0;
-  const int shape = p.seg || p.swiglu ? -1 : nvfp4_mid_shape(p.M, p.N, p.Kp, plan.kernel, plan.slices);
-  return shape < 0 ? -1 : 1 + shape;
+// NVFP4 decode batches run as a stream of the weights where that is faster than what the plan has for them, and so do plain problems
+// of a few hundred rows, unless a kernel or a number of slices is forced; plan 0 has operands that only the direct kernels take.
+// By the plan, as a stream, or kMidRows + a shape of it.
+constexpr int kByPlan = -1, kAsStream = 0, kMidRows = 1;
+int stream_way(const GemmPlan &plan, int M, int N, int Kp, int fmt, int n_seg, bool swiglu) {
+  if (fmt != ARCQ_FMT_NVFP4 || tuning().gemm_kernel >= 0 || tuning().gemm_splitk != 0 || plan.kernel == 0) return kByPlan;
+  if (nvfp4_stream_wanted(M, N, Kp, n_seg)) return kAsStream;
+  const int shape = n_seg > 0 || swiglu ? -1 : nvfp4_mid_shape(M, N, Kp, plan.kernel, plan.slices);
+  return shape < 0 ? kByPlan : kMidRows + shape;
 }
 
-int run_gemm(GemmParams p, const GemmPlan &plan, int fmt, float *scratch, hipStream_t st) {
-  const int way = stream_way(plan, p, fmt);
-  if (way >= 0) return way == 0 ? run_nvfp4_stream(p, st) : run_nvfp4_mid(p, way - 1, st);
+int run_gemm(GemmParams p, const GemmPlan &plan, int fmt, float *scratch, hipStream_t st, int way) {
+  if (way != kByPlan) return way == kAsStream ? run_nvfp4_stream(p, st) : run_nvfp4_mid(p, way - kMidRows, st);
   if (plan.slices > 1) {
     p.k_slices = plan.slices;
     p.partial = scratch;
@@ -1290,13 +1290,14 @@ int matmul_impl(const void *a_codes, const void *a_scales, const void *b_codes, 
   const bool scales_aligned = aligned16(a_scales) && aligned16(b_scales);
   if (const int way = scales_aligned && workspace ? f16_way(M, N, Kp, fmt, 0, workspace_bytes) : 0) return run_nvfp4_f16(p, workspace, st, way == 2);
   const GemmPlan plan = plan_gemm(M, N, Kp, fmt, scales_aligned);
+  const int way = stream_way(plan, M, N, Kp, fmt, 0, false);
   float *scratch = nullptr;
-  if (plan.slices > 1 && stream_way(plan, p, fmt) < 0) {
+  if (plan.slices > 1 && way == kByPlan) {
     int status = ARCQ_OK;
     scratch = static_cast<float *>(stream_workspace(kWsSplitK, st, &status));
     if (!scratch) return status;
   }
-  return run_gemm(p, plan, fmt, scratch, st);
+  return run_gemm(p, plan, fmt, scratch, st, way);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1361,14 +1362,15 @@ extern "C" int arcq_matmul_noalloc(const void *a_codes, const void *a_scales, co
   const GemmPlan plan = plan_gemm(M, N, Kp, fmt, aligned16(a_scales) && aligned16(b_scales));
   if (plan.scratch_bytes() > kNoAllocScratchBytes) return ARCQ_ERR_WORKSPACE;  // beyond the fixed array: nothing is launched
   float *ws = nullptr;
-  if (plan.slices > 1 && stream_way(plan, p, fmt) < 0) {
+  const int way = stream_way(plan, M, N, Kp, fmt, 0, false);
+  if (plan.slices > 1 && way == kByPlan) {
     int status = ARCQ_OK;
     ws = noalloc_scratch(&status);
     if (!ws) return status;
     // every word of the partial tiles that the reduction reads is written by this call's first
     // launch, so nothing of the previous call's contents has to be cleared
   }
-  return run_gemm(p, plan, fmt, ws, static_cast<hipStream_t>(stream));
+  return run_gemm(p, plan, fmt, ws, static_cast<hipStream_t>(stream), way);
 }
 
 extern "C" size_t arcq_matmul_noalloc_limit(void) { return arcq::kNoAllocScratchBytes; }
@@ -1418,7 +1420,8 @@ int grouped_matmul_impl(const void *a_codes, const void *a_scales, const void *b
   p.absmax_bits = reinterpret_cast<uint32_t *>(d_absmax);
   if (const int way = workspace ? f16_way(M, N, Kp, fmt, n_seg, workspace_bytes) : 0)
     return run_nvfp4_f16(p, workspace, static_cast<hipStream_t>(stream), way == 2);
-  return run_gemm(p, plan_grouped(M, Kp, fmt, n_seg), fmt, nullptr, static_cast<hipStream_t>(stream));
+  const GemmPlan plan = plan_grouped(M, Kp, fmt, n_seg);
+  return run_gemm(p, plan, fmt, nullptr, static_cast<hipStream_t>(stream), stream_way(plan, M, N, Kp, fmt, n_seg, swiglu));
 }
 
 __global__ void scales_from_absmax_kernel(float *v, int n, float divisor) {
@@ -1462,7 +1465,8 @@ int matmul_swiglu_impl(const void *a_codes, const void *a_scales, const void *b_
   p.absmax_bits = reinterpret_cast<uint32_t *>(d_absmax);
   if (const int way = workspace ? f16_way(M, N, Kp, fmt, 0, workspace_bytes) : 0)
     return run_nvfp4_f16(p, workspace, static_cast<hipStream_t>(stream), way == 2);
-  return run_gemm(p, plan_swiglu(M, N, Kp, fmt), fmt, nullptr, static_cast<hipStream_t>(stream));
+  const GemmPlan plan = plan_swiglu(M, N, Kp, fmt);
+  return run_gemm(p, plan, fmt, nullptr, static_cast<hipStream_t>(stream), stream_way(plan, M, N, Kp, fmt, 0, true));
 }
 }  // namespace
 }  // namespace arcq
@@ -1523,6 +1527,17 @@ extern "C" int arcq_gemm_kernel(int M, int N, int Kp, int fmt, int n_seg, int sw
   const GemmPlan plan = n_seg > 0 ? plan_grouped(M, Kp, fmt, n_seg)
                         : swiglu ? plan_swiglu(M, N, Kp, fmt) : plan_gemm(M, N, Kp, fmt, true);
   return fmt == ARCQ_FMT_MXFP4 ? addressable_tile(plan.kernel, M, N, Kp) : plan.kernel;
+}
+
+extern "C" int arcq_gemm_route(int M, int N, int Kp, int fmt, int n_seg, int swiglu) {
+  using namespace arcq;
+  if (arcq_gemm_kernel(M, N, Kp, fmt, n_seg, swiglu) < 0) return -1;
+  if (const int ahead = f16_way(M, N, Kp, fmt, n_seg, arcq_gemm_scratch_bytes(M, N, Kp, fmt, n_seg)))
+    return ahead == 2 ? ARCQ_ROUTE_AHEAD_CUT : ARCQ_ROUTE_AHEAD;
+  const GemmPlan plan = n_seg > 0 ? plan_grouped(M, Kp, fmt, n_seg)
+                        : swiglu ? plan_swiglu(M, N, Kp, fmt) : plan_gemm(M, N, Kp, fmt, true);
+  const int way = stream_way(plan, M, N, Kp, fmt, n_seg, swiglu != 0);
+  return way == kByPlan ? ARCQ_ROUTE_PLAN : way == kAsStream ? ARCQ_ROUTE_STREAM : ARCQ_ROUTE_STREAM_SHAPE + way - kMidRows;
 }
 
 extern "C" int arcq_scales_from_absmax(float *d_values, int n, float divisor, void *stream) {

@@ -213,6 +213,20 @@ def test_gemm_kernel_of_a_problem():
         assert k(*bad) == -1
 
 
+PLAN, AHEAD, CUT, STREAM, SHAPE = 0, 1, 2, 3, 16
+
+
+@pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
+def test_route_of_other_nvfp4_problems():
+    """as arcq_gemm launches them, given the scratch that it asks for"""
+    route = _lib.lib().arcq_gemm_route
+    for (M, N, kp, E), want in {
+            (4096, 4096, 4352, 0): AHEAD, (3000, 6144, 10240, 0): CUT, (2048, 4096, 4352, 0): PLAN,
+            (8 * 1024, 4096, 14464, 8): CUT, (8 * 1024, 28672, 4224, 8): AHEAD, (4 * 512, 4096, 14464, 4): PLAN}.items():
+        assert route(M, N, kp, 0, E, 0) == want, (M, N, kp, E)
+    assert route(0, 4096, 4352, 0, 0, 0) == route(64, 256, 448, 0, 2, 0) == route(64, 256, 512, 2, 0, 0) == -1
+
+
 def test_release_stream_without_buffers_needs_no_gpu_work():
     assert hasattr(_lib.lib(), "arcq_release_stream")
 
