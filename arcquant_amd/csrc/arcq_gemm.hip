@@ -724,7 +724,7 @@ __global__ __launch_bounds__(128 * NWM) void gemm_nvfp4_tiled(GemmParams p) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// Skinny kernels for M <= 64 (decode batches; NVFP4: a few rows on a narrow layer, see nvfp4_stream_wanted, and K' < 512): the GEMM is a stream of the weight matrix, read
+// Skinny kernels for M <= 64 (decode batches; NVFP4: few rows, narrow layers and a short K', see kStreamFrom): the GEMM is a stream of the weight matrix, read
 // exactly once, so nothing is staged through LDS.  A workgroup owns 16 weight rows; its NW waves
 // take the K steps of 128 round-robin in pairs (split-K: with four waves wave w does steps 2w, 2w+1, 2w+8, 2w+9, ...:
 // a pair of steps is one whole 128-byte line of every row, and the four waves walk neighbouring lines) and their partial sums meet in LDS.  A lane loads
@@ -1143,8 +1143,16 @@ GemmPlan plan_swiglu(int M, int N, int Kp, int fmt) {
 constexpr int kByPlan = -1, kAsStream = 0, kMidRows = 1;
 int stream_way(const GemmPlan &plan, int M, int N, int Kp, int fmt, int n_seg, bool swiglu) {
   if (fmt != ARCQ_FMT_NVFP4 || tuning().gemm_kernel >= 0 || tuning().gemm_splitk != 0 || plan.kernel == 0) return kByPlan;
-  if (nvfp4_stream_wanted(M, N, Kp, n_seg)) return kAsStream;
-  const int shape = n_seg > 0 || swiglu ? -1 : nvfp4_mid_shape(M, N, Kp, plan.kernel, plan.slices);
+  if (nvfp4_stream_wanted(M, N, Kp, n_seg, swiglu)) return kAsStream;
+  const int shape = n_seg > 0 || swiglu ? -1 : nvfp4_mid_shape(M, N, Kp, plan.kernel, plan.slices, false);
+  return shape < 0 ? kByPlan : kMidRows + shape;
+}
+
+// For a plain problem whose plan has slices of K and no memory for them: the stream all the same, where it takes the problem.
+int way_without_scratch(const GemmPlan &plan, int M, int N, int Kp, int fmt) {
+  if (fmt != ARCQ_FMT_NVFP4 || tuning().gemm_kernel >= 0 || tuning().gemm_splitk != 0) return kByPlan;
+  if (nvfp4_stream_able(M, Kp, 0)) return kAsStream;
+  const int shape = nvfp4_mid_shape(M, N, Kp, plan.kernel, plan.slices, true);
   return shape < 0 ? kByPlan : kMidRows + shape;
 }
 
@@ -1290,12 +1298,15 @@ int matmul_impl(const void *a_codes, const void *a_scales, const void *b_codes, 
   const bool scales_aligned = aligned16(a_scales) && aligned16(b_scales);
   if (const int way = scales_aligned && workspace ? f16_way(M, N, Kp, fmt, 0, workspace_bytes) : 0) return run_nvfp4_f16(p, workspace, st, way == 2);
   const GemmPlan plan = plan_gemm(M, N, Kp, fmt, scales_aligned);
-  const int way = stream_way(plan, M, N, Kp, fmt, 0, false);
+  int way = stream_way(plan, M, N, Kp, fmt, 0, false);
   float *scratch = nullptr;
   if (plan.slices > 1 && way == kByPlan) {
     int status = ARCQ_OK;
     scratch = static_cast<float *>(stream_workspace(kWsSplitK, st, &status));
-    if (!scratch) return status;
+    if (!scratch) {  // (none while the stream is being captured, unless it was prepared)
+      way = status == ARCQ_ERR_WORKSPACE ? way_without_scratch(plan, M, N, Kp, fmt) : kByPlan;
+      if (way == kByPlan) return status;
+    }
   }
   return run_gemm(p, plan, fmt, scratch, st, way);
 }

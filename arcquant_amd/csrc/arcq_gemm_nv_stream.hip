@@ -1,6 +1,8 @@
 // arcq_gemm_nv_stream.hip -- NVFP4 GEMM of decode batches (up to 64 rows, or experts of a few rows each): one pass over the
 // weights, all of whose bytes are on their way through many small workgroups; and of a few hundred rows where tiles do not fill the chip.
 #include <hip/hip_runtime.h>
+#include <limits.h>
+#include <math.h>
 
 #include <algorithm>
 #include <type_traits>
@@ -305,9 +307,9 @@ int launch(const GemmParams &p, hipStream_t st) {
 // Rows per workgroup.  Up to 12288 rows of weights make at most one workgroup per CU of 16, 32 or 48 rows, which then has
 // sixteen waves (us at 16 rows: 6144 x 4352 7.8, eight waves 8.9; 10240 x 8320 15.0 and 17.6).  Beyond, eight waves, and the
 // rows per workgroup by how many rounds of 256 workgroups they make: the rows and activation rows of a CU's workgroups
-// together, a quarter more where up to 32 rows have a single workgroup per CU to themselves (nothing else asks for weights
-// while it starts, waits and ends): 28672 rows take 64 per workgroup up to 32 rows and 112 above (64 rows: 24.7 us against
-// 25.4), 18944 rows 48 and 80.
+// together, a quarter more where up to 32 rows, or a K' of one or two steps, have a single workgroup per CU to themselves (nothing else
+// asks for weights while it starts, waits and ends): 28672 rows take 64 per workgroup up to 32 rows and 112 above (64 rows, K' = 4352:
+// 24.7 us against 25.4; K' = 512: 64 per workgroup 8.2 against 9.3), 18944 rows 48 and 80.
 template <int MT>
 int launch_plain(const GemmParams &p, hipStream_t st) {
   if (p.N <= 4096) return launch<MT, 1, 1, 16, (MT == 1 ? 3 : 2)>(p, st);
@@ -317,7 +319,7 @@ int launch_plain(const GemmParams &p, hipStream_t st) {
   double least = 0;
   for (const int nt : {2, 3, 4, 5, 7}) {
     const int groups = (p.N + 16 * nt - 1) / (16 * nt);
-    const double cost = (groups + 255) / 256 * (nt + 0.25 * MT) * (groups <= 256 && MT <= 2 ? 1.25 : 1.0);
+    const double cost = (groups + 255) / 256 * (nt + 0.25 * MT) * (groups <= 256 && (MT <= 2 || p.Kp < 1024) ? 1.25 : 1.0);
     if (!best || cost < least) best = nt, least = cost;
   }
   switch (best) {
@@ -331,14 +333,44 @@ int launch_plain(const GemmParams &p, hipStream_t st) {
 
 }  // namespace
 
-// Plain problems of up to 64 rows, but for a few rows on a narrow layer, where the kernel that reads its operands straight
-// into registers gets in and out faster (4 rows: 3584 x 3712 4.9 against 5.7 us; 1 row: 4096 x 14592 10.8 against 12.0, 8 rows
-// 12.8 against 12.0).  Experts: an average of fewer than 96 rows; from 40 rows on the 128x64 tiles
-// are as good where K is short (64 experts of 2048 x 1536, 64 rows each: 37 against 43 us).
-bool nvfp4_stream_wanted(int M, int N, int Kp, int n_seg) {
-  if (Kp % 128 != 0 || Kp < 512 || Kp > (1 << 24)) return false;
+// What the kernel takes: whole 128s of K', one step at least, 32-bit offsets inside a workgroup's rows.
+bool nvfp4_stream_able(int M, int Kp, int n_seg) { return Kp % 128 == 0 && Kp >= 512 && Kp <= (1 << 24) && (n_seg > 0 || M <= 64); }
+
+// The shortest K' from which on plain problems of up to 64 rows run as such a stream.  Below, the kernel that reads its operands
+// straight into registers, which has nothing to fill, wait for and add up, gets in and out faster (the stream's waves take 512 to 1024
+// elements at a time, and a last step that is mostly empty costs as much as a whole one), and 64 rows of a short K' on 32769 to 49151 rows
+// of weights are as fast in 128x64 tiles.  us as a stream and so: 16 rows, 2048 x 1152 4.4 / 3.3, 4096 x 2176 5.3 / 4.4, 4096 x 8320 8.0
+// / 9.4, 8192 x 1152 4.9 / 4.3, 12288 x 1152 5.6 / 4.9; 32 rows, 4096 x 1152 4.8 / 4.4, 4096 x 4352 6.9 / 8.8; 8 rows, 2048 x 8320 8.5 / 7.1,
+// 3584 x 14592 10.8 / 11.6; 4 rows, 18944 x 1152 6.7 / 5.5, 18944 x 4352 13.0 / 16.4; 64 rows, 37888 x 512 13.0 / 9.6, 37888 x 2176 26.7 / 28.4.
+constexpr int kNever = 1 << 30;
+constexpr int kStreamRows[7] = {4, 7, 8, 16, 32, 48, 64};
+constexpr struct {
+  int N;           // up to this many rows of weights
+  int from[7];     // K', by activation rows
+} kStreamFrom[] = {{2048, {kNever, kNever, kNever, 10240, 4096, 0, 0}},
+                   {4096, {kNever, 10240, 10240, 8192, 4096, 0, 0}},
+                   {8192, {kNever, 4096, 4096, 4096, 2048, 0, 0}},
+                   {12288, {2560, 2560, 2560, 2560, 0, 0, 0}},
+                   {16383, {2560, 2560, 2560, 1536, 0, 0, 0}},
+                   {24576, {2560, 2048, 0, 0, 0, 0, 0}},
+                   {32768, {2048, 2048, 0, 0, 0, 0, 0}},
+                   {49151, {2048, 2048, 0, 0, 0, 0, 1536}},
+                   {INT_MAX, {2048, 2048, 0, 0, 0, 0, 0}}};
+
+bool nvfp4_stream_wanted(int M, int N, int Kp, int n_seg, bool swiglu) {
+  if (!nvfp4_stream_able(M, Kp, n_seg)) return false;
+  // Experts: an average of fewer than 96 rows; from 40 rows on the 128x64 tiles are as good where K is short (64 experts of
+  // 2048 x 1536, 64 rows each: 37 against 43 us).
   if (n_seg > 0) return M / n_seg < 96 && (M / n_seg <= 40 || Kp >= 2048);
-  return M <= 64 && !(N <= 8192 && M <= 4) && !(N <= 4096 && M <= 8 && Kp < 8192);
+  // The kernels above have no SwiGLU epilogue: the 128x64 tiles, which would take 1.05 (4096 x 512) to 5 (1024 x 14592) times as long.
+  if (swiglu) return true;
+  // (64 rows of a long K' on a narrow layer: 128x64 tiles with K in eight slices, 2048 x 19072 25.6 / 23.0 us, 1024 x 14592 20.2 / 19.5)
+  if (M > 48 && N <= 4096 && Kp >= (N <= 1024 ? 12288 : 16384)) return false;
+  if (M <= 7 && N > 20480 && Kp <= 512) return true;  // one step: 4 rows, 28672 x 512 5.3 / 6.1
+  int n = 0, m = 0;
+  while (N > kStreamFrom[n].N) ++n;
+  while (M > kStreamRows[m]) ++m;
+  return Kp >= kStreamFrom[n].from[m];
 }
 
 // Beyond 64 rows the same kernel with 64 to 112 rows per workgroup: both operands are decoded in every workgroup, but only
@@ -352,10 +384,10 @@ constexpr MidShape kMid[] = {{4, 3, 1, 8, 8.2}, {4, 4, 1, 8, 9.8}, {5, 3, 1, 8, 
                              {5, 3, 2, 4, 16.6}, {4, 4, 2, 4, 18.0}, {6, 3, 2, 4, 22.5}, {5, 4, 2, 4, 25.0}};
 
 // The shape for a problem that the plan would give to 128x64 (21, K in `slices`), 128x128 (22) or 256x128 tiles (42), -1 where those
-// are faster by their own measured times.  us, before and now: 128 x 6144 x 4352 21.9 and 14.3, 333 rows 34.4 and 28.5, 512 rows 34.1
+// are faster by their own measured times (`always`: the best one whatever theirs are).  us, before and now: 128 x 6144 x 4352 21.9 and 14.3, 333 rows 34.4 and 28.5, 512 rows 34.1
 // (kept); 256 x 4096 x 4352 23.3 and 16.3; 128 x 4096 x 14592 31 (kept), 333 rows 73.8 and 55.7; 80 x 28672 x 4352 43.6 and
 // 33, 256 rows 62 (kept).
-int nvfp4_mid_shape(int M, int N, int Kp, int kernel, int slices) {
+int nvfp4_mid_shape(int M, int N, int Kp, int kernel, int slices, bool always) {
   if (M <= 64 || M > 1024 || Kp < 512 || Kp % 128 != 0 || Kp > (1 << 24)) return -1;
   const double k = Kp / 4352.0;
   auto rounds = [](long groups) { return (double)((groups + 255) / 256); };
@@ -370,7 +402,7 @@ int nvfp4_mid_shape(int M, int N, int Kp, int kernel, int slices) {
   else
     return -1;
   int best = -1;
-  double least = 0.97 * tiled;
+  double least = always ? HUGE_VAL : 0.97 * tiled;
   for (int i = 0; i < (int)(sizeof(kMid) / sizeof(kMid[0])); ++i) {
     const MidShape &s = kMid[i];
     const double us = 6 + s.us * k * rounds(tiles(16 * s.mt, 16 * s.nt * s.wn));

@@ -66,10 +66,11 @@ int run_nvfp4_f16(GemmParams p, void *workspace, hipStream_t st, bool split);
 size_t nvfp4_split_bytes(int M, int N, int Kp, int n_seg);
 
 // arcq_gemm_nv_stream.hip: decode batches, plain (n_seg = 0, M <= 64) and grouped
-bool nvfp4_stream_wanted(int M, int N, int Kp, int n_seg);
+bool nvfp4_stream_able(int M, int Kp, int n_seg);
+bool nvfp4_stream_wanted(int M, int N, int Kp, int n_seg, bool swiglu);
 int run_nvfp4_stream(const GemmParams &p, hipStream_t st);
 // 65 to 1024 rows: a shape of the same kernel in the place of the plan's tiles, or -1
-int nvfp4_mid_shape(int M, int N, int Kp, int kernel, int slices);
+int nvfp4_mid_shape(int M, int N, int Kp, int kernel, int slices, bool always);
 int run_nvfp4_mid(const GemmParams &p, int shape, hipStream_t st);
 
 // arcq_gemm_mx.hip

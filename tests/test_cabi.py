@@ -217,6 +217,32 @@ PLAN, AHEAD, CUT, STREAM, SHAPE = 0, 1, 2, 3, 16
 
 
 @pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
+@pytest.mark.parametrize("N,edges", [
+    # by rows: the K' below which the weights are not streamed (0: always, None: never)
+    (2048, {1: None, 8: None, 9: 10240, 16: 10240, 17: 4096, 32: 4096, 33: 0, 48: 0}),
+    (4096, {4: None, 5: 10240, 8: 10240, 9: 8192, 16: 8192, 17: 4096, 33: 0}),
+    (8192, {4: None, 5: 4096, 16: 4096, 17: 2048, 32: 2048, 33: 0, 64: 0}),
+    (12288, {1: 2560, 16: 2560, 17: 0, 64: 0}), (14336, {8: 2560, 9: 1536, 16: 1536, 17: 0}),
+    (18944, {4: 2560, 5: 2048, 7: 2048, 8: 0, 64: 0}), (28672, {8: 0, 64: 0}), (37888, {8: 0, 48: 0, 49: 1536, 64: 1536}),
+    (49152, {8: 0, 64: 0}),
+])
+def test_route_of_nvfp4_decode_batches(N, edges):
+    """where a decode batch is a stream of the weights, and where the kernels that begin and end sooner have it; a fused SwiGLU
+    epilogue, which those have not, always is one"""
+    route = _lib.lib().arcq_gemm_route
+    for M, edge in edges.items():
+        for kp in ((512, 8192) if edge == 0 else (512, 16256) if edge is None else (edge - 128, edge)):
+            want = STREAM if edge is not None and kp >= edge else PLAN
+            assert route(M, N, kp, 0, 0, 0) == want, (M, kp)
+            assert route(M, N, kp, 0, 0, 1) == STREAM
+            assert route(M, N, kp, 1, 0, 0) == PLAN                         # MXFP4
+    assert route(4, 28672, 512, 0, 0, 0) == STREAM and route(4, 28672, 640, 0, 0, 0) == PLAN   # one step of a wide layer
+    for (M, N, kp), want in {(64, 1024, 12160): STREAM, (64, 1024, 12288): PLAN, (64, 4096, 16256): STREAM, (64, 4096, 16384): PLAN,
+                             (48, 4096, 16384): STREAM, (64, 4096, 448): PLAN, (64, 4096, 4160): PLAN}.items():
+        assert route(M, N, kp, 0, 0, 0) == want, (M, N, kp)
+
+
+@pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
 def test_route_of_other_nvfp4_problems():
     """as arcq_gemm launches them, given the scratch that it asks for"""
     route = _lib.lib().arcq_gemm_route

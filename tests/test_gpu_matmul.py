@@ -467,3 +467,38 @@ def test_nvfp4_a_few_hundred_rows(agemm, oracle, M, N, K, S):
     assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
     res = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
     assert torch.equal(agemm.matmul(a, b, sfa, sfb, scale, residual=res), y + res)
+
+
+@pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
+@pytest.mark.parametrize("M,N,kp,route", [
+    (5, 4096, 10240, 3), (5, 4096, 10112, 0), (16, 2048, 10240, 3), (16, 2048, 10112, 0), (9, 4096, 8192, 3), (17, 2048, 4096, 3),
+    (17, 2048, 3968, 0), (5, 8192, 4096, 3), (5, 8192, 3968, 0), (1, 12288, 2560, 3), (1, 12288, 2432, 0), (4, 28672, 512, 3),
+    (64, 1024, 12288, 0), (64, 1024, 12160, 3), (64, 4096, 16384, 0), (64, 37888, 1408, 0), (64, 28672, 512, 3)])
+def test_nvfp4_decode_batches_at_the_edges_of_the_stream(agemm, oracle, M, N, kp, route):
+    """both sides of the lines between the stream of the weights and the kernels that begin and end sooner"""
+    from arcquant_amd import _lib
+    assert _lib.lib().arcq_gemm_route(M, N, kp, 0, 0, 0) == route
+    (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, kp - 64, 64, "NVFP4", seed=85)
+    want = oracle_dq(oracle, a, sfa, "NVFP4") @ oracle_dq(oracle, b, sfb, "NVFP4").T * (gx * gw)
+    y = agemm.matmul(a, b, sfa, sfb, gx * gw)
+    assert rel_fro(y.float(), want) < 2.5e-3
+    assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
+
+
+@pytest.mark.parametrize("M,N,kp", [(64, 1024, 12288), (64, 2048, 16384), (130, 256, 8320)])
+def test_nvfp4_captured_without_scratch(agemm, oracle, M, N, kp):
+    """a plan with slices of K on a stream that is captured and was not prepared: there is no memory for their sums, and a kernel
+    that needs none has the problem (M = 130: the plan's slices, or a shape that needs none, by their times)"""
+    (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, kp - 64, 64, "NVFP4", seed=87)
+    want = oracle_dq(oracle, a, sfa, "NVFP4") @ oracle_dq(oracle, b, sfb, "NVFP4").T * (gx * gw)
+    if "ARCQ_GEMM_KERNEL" in os.environ:
+        pytest.skip("another kernel is forced")
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        y = agemm.matmul(a, b, sfa, sfb, gx * gw)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert rel_fro(y.float(), want) < 2.5e-3
+        assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
