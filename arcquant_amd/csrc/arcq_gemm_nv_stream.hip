@@ -359,9 +359,19 @@ constexpr struct {
 
 bool nvfp4_stream_wanted(int M, int N, int Kp, int n_seg, bool swiglu) {
   if (!nvfp4_stream_able(M, Kp, n_seg)) return false;
-  // Experts: an average of fewer than 96 rows; from 40 rows on the 128x64 tiles are as good where K is short (64 experts of
-  // 2048 x 1536, 64 rows each: 37 against 43 us).
-  if (n_seg > 0) return M / n_seg < 96 && (M / n_seg <= 40 || Kp >= 2048);
+  // Experts: few rows on average, so that the weights are the work; a workgroup has at most 48 rows of its expert, and what they
+  // decode of the weights is decoded again for the next 48.  us as a stream and in 128x64 tiles, even and skewed sizes, eight experts of
+  // 4096 x 14464: 40 rows each 61, 86 / 85, 126; 48 rows 68, 148 / 84, 129; 64 rows 80, 150 / 85, 133; 8192 x 2176, 40 rows 26, 31 / 27, 38; 64
+  // rows 34, 45 / 28, 39.  Wide layers take workgroups of 96 weight rows there, which decode less: 28672 x 4224, 64 rows 185, 220 / 185,
+  // 237, 95 rows 290, 299 / 321, 322; so do a few narrow experts, all of whose tiles together are less than a round: 8 of 2048 x 8320, 64
+  // rows 45, 45 / 49, 49.  K' < 2048: 64 of 2048 x 1536, 24 rows 31, 40 / 34, 40, 40 rows 38, 47 / 34, 42; 8 of 1536 x 1536, 40 rows 8.4, 8.7 /
+  // 12.4, 12.4.
+  if (n_seg > 0) {
+    const int rows = M / n_seg;
+    const bool few = (long)n_seg * N <= 16384;
+    if (Kp < 2048) return rows <= (few ? 40 : 32);
+    return rows <= 40 || (rows < 96 && (N > 8192 || few));
+  }
   // The kernels above have no SwiGLU epilogue: the 128x64 tiles, which would take 1.05 (4096 x 512) to 5 (1024 x 14592) times as long.
   if (swiglu) return true;
   // (64 rows of a long K' on a narrow layer: 128x64 tiles with K in eight slices, 2048 x 19072 25.6 / 23.0 us, 1024 x 14592 20.2 / 19.5)

@@ -250,6 +250,12 @@ def test_route_of_other_nvfp4_problems():
             (4096, 4096, 4352, 0): AHEAD, (3000, 6144, 10240, 0): CUT, (2048, 4096, 4352, 0): PLAN,
             (8 * 1024, 4096, 14464, 8): CUT, (8 * 1024, 28672, 4224, 8): AHEAD, (4 * 512, 4096, 14464, 4): PLAN}.items():
         assert route(M, N, kp, 0, E, 0) == want, (M, N, kp, E)
+    # experts: 40 rows on average, 95 where a layer is wide or all experts together are small, 32 where K' is short
+    for (rows, N, kp, E), want in {
+            (40, 4096, 14464, 8): STREAM, (41, 4096, 14464, 8): PLAN, (95, 8208, 2048, 8): STREAM, (96, 8208, 2048, 8): PLAN,
+            (95, 2048, 8320, 8): STREAM, (41, 2064, 8320, 8): PLAN, (32, 2048, 1536, 64): STREAM, (33, 2048, 1536, 64): PLAN,
+            (40, 2048, 1536, 8): STREAM, (41, 2048, 1536, 8): PLAN, (40, 28672, 1920, 8): PLAN}.items():
+        assert route(rows * E, N, kp, 0, E, 0) == route(rows * E, N, kp, 0, E, 1) == want, (rows, N, kp, E)
     assert route(0, 4096, 4352, 0, 0, 0) == route(64, 256, 448, 0, 2, 0) == route(64, 256, 512, 2, 0, 0) == -1
 
 
