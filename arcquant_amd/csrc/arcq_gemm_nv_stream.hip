@@ -385,13 +385,18 @@ bool nvfp4_stream_wanted(int M, int N, int Kp, int n_seg, bool swiglu) {
 
 // Beyond 64 rows the same kernel with 64 to 112 rows per workgroup: both operands are decoded in every workgroup, but only
 // once (its waves split K), which is about what the matrix instructions take, and small workgroups fill the chip where 128x128 tiles
-// do not.  A workgroup's time per K' = 4352 and its wait to start and end, measured (us; workgroups of 1 to 14 per CU):
+// do not.  A workgroup's time per K' = 4352 and its wait to start and end (6 us; less for the smallest shapes, as long as they make one
+// round), measured, by shape; where workgroups have a CU to themselves, each of several rounds takes an eighth more (us; workgroups of 1
+// to 14 per CU; 1900 problems of 65 to 1024 rows, 256 to 28672 weight rows and K' = 512 to 14592 to within 10 % in one round):
 struct MidShape {
   int mt, nt, wn, wk;
-  double us;
+  double us, rounds;
+  double short_start, short_us;
 };
-constexpr MidShape kMid[] = {{4, 3, 1, 8, 8.2}, {4, 4, 1, 8, 9.8}, {5, 3, 1, 8, 9.2}, {6, 4, 1, 8, 14.8}, {7, 3, 1, 8, 13.8},
-                             {5, 3, 2, 4, 16.6}, {4, 4, 2, 4, 18.0}, {6, 3, 2, 4, 22.5}, {5, 4, 2, 4, 25.0}};
+constexpr double kMidStart = 6;
+constexpr MidShape kMid[] = {{4, 3, 1, 8, 8.2, 1.0, 4.0, 10.0}, {4, 4, 1, 8, 9.8, 1.0, 4.7, 11.8},   {5, 3, 1, 8, 9.2, 1.0, 4.7, 11.3},
+                             {6, 4, 1, 8, 14.8, 1.12, 6, 14.8}, {7, 3, 1, 8, 13.8, 1.12, 6, 13.8},   {5, 3, 2, 4, 16.6, 1.0, 6, 16.6},
+                             {4, 4, 2, 4, 18.0, 1.0, 6, 18.0},  {6, 3, 2, 4, 22.5, 1.0, 6, 22.5},    {5, 4, 2, 4, 25.0, 1.0, 6, 25.0}};
 
 // The shape for a problem that the plan would give to 128x64 (21, K in `slices`), 128x128 (22) or 256x128 tiles (42), -1 where those
 // are faster by their own measured times (`always`: the best one whatever theirs are).  us, before and now: 128 x 6144 x 4352 21.9 and 14.3, 333 rows 34.4 and 28.5, 512 rows 34.1
@@ -403,9 +408,10 @@ int nvfp4_mid_shape(int M, int N, int Kp, int kernel, int slices, bool always) {
   auto rounds = [](long groups) { return (double)((groups + 255) / 256); };
   auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
   double tiled;
-  if (kernel == 21)
-    tiled = (slices > 1 ? 12 : 7) + 20 * k / slices * rounds(tiles(64, 128) * slices);
-  else if (kernel == 22)
+  if (kernel == 21) {
+    const double r = rounds(tiles(64, 128) * slices);
+    tiled = slices > 1 ? 12 + 20 * k / slices * r : std::min(7 + 20 * k * r, 3.6 + 26 * k * r);  // (a short K' is little but its first step)
+  } else if (kernel == 22)
     tiled = 4 + (tiles(128, 128) <= 256 ? 30 : 27) * k * rounds(tiles(128, 128));
   else if (kernel == 42)
     tiled = 4 + 28 * k * (1 + rounds(tiles(128, 256)));  // (further rounds: half the first one's and more)
@@ -415,7 +421,8 @@ int nvfp4_mid_shape(int M, int N, int Kp, int kernel, int slices, bool always) {
   double least = always ? HUGE_VAL : 0.97 * tiled;
   for (int i = 0; i < (int)(sizeof(kMid) / sizeof(kMid[0])); ++i) {
     const MidShape &s = kMid[i];
-    const double us = 6 + s.us * k * rounds(tiles(16 * s.mt, 16 * s.nt * s.wn));
+    const double r = rounds(tiles(16 * s.mt, 16 * s.nt * s.wn));
+    const double us = r > 1 ? kMidStart + s.us * k * r * s.rounds : std::min(kMidStart + s.us * k, s.short_start + s.short_us * k);
     if (us < least) best = i, least = us;
   }
   return best;

@@ -470,6 +470,28 @@ def test_nvfp4_a_few_hundred_rows(agemm, oracle, M, N, K, S):
 
 
 @pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
+@pytest.mark.parametrize("M,N,kp,shape", [
+    (65, 4101, 512, 0), (83, 6145, 512, 1), (79, 6145, 640, 2), (137, 6145, 1152, 3), (197, 4101, 1152, 4), (197, 6145, 2176, 5),
+    (902, 4101, 640, 6), (449, 4101, 2176, 7), (323, 6145, 4352, 8),                   # N % 4 != 0
+    (65, 256, 512, 0), (100, 8192, 1152, 1), (144, 4096, 4352, 2), (113, 6144, 1152, 0), (520, 2048, 640, 4), (65, 18944, 512, 5), (161, 18944, 640, 6),
+    (333, 6144, 4352, 7), (83, 18944, 640, 7), (65, 28672, 512, 8), (333, 4096, 8192, 3)])
+def test_nvfp4_every_shape_of_a_few_hundred_rows(agemm, oracle, M, N, kp, shape):
+    """Each shape of the kernel for 65 to 1024 rows, on problems that are given to it: rows and columns ending inside its tile, columns
+    that are no multiple of four, plain and with a residual; exact products and fp32 sums."""
+    from arcquant_amd import _lib
+    assert _lib.lib().arcq_gemm_route(M, N, kp, 0, 0, 0) == 16 + shape
+    S = 64 if kp % 256 else 0
+    (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, kp - S, S, "NVFP4", seed=83)
+    want = oracle_dq(oracle, a, sfa, "NVFP4") @ oracle_dq(oracle, b, sfb, "NVFP4").T * (gx * gw)
+    scale = (torch.tensor(gx, device="cuda"), torch.tensor(gw, device="cuda"))
+    y = agemm.matmul(a, b, sfa, sfb, scale)
+    assert rel_fro(y.float(), want) < 2.5e-3
+    assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
+    res = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
+    assert torch.equal(agemm.matmul(a, b, sfa, sfb, scale, residual=res), y + res)
+
+
+@pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
 @pytest.mark.parametrize("M,N,kp,route", [
     (5, 4096, 10240, 3), (5, 4096, 10112, 0), (16, 2048, 10240, 3), (16, 2048, 10112, 0), (9, 4096, 8192, 3), (17, 2048, 4096, 3),
     (17, 2048, 3968, 0), (5, 8192, 4096, 3), (5, 8192, 3968, 0), (1, 12288, 2560, 3), (1, 12288, 2432, 0), (4, 28672, 512, 3),
