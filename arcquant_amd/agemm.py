@@ -346,6 +346,24 @@ def matmul_parts(A, B, SFA, SFB, scale, part_rows, part_scales, *, fmt, bias=Non
     return C
 
 
+@functools.lru_cache(maxsize=4096)
+def parts_pay(M, part_rows, Kp, fmt):
+    """Whether matmul_parts over part_rows (a tuple) is faster than a GEMM per part and a concatenation: nearly always, 0.6 of the time on
+    average.  Not where the parts by themselves fit smaller NVFP4 tiles and all of them together make 256x256 ones, whose last round
+    is nearly empty (two parts of 18944 x 4352, 300 rows, 296 tiles: 171 against 133 us; 11008, 600 rows, 258 tiles: 174 / 141) or whose rows
+    are (28672 x 4352, 80 rows: 101 / 71, 128 rows 103 / 90)."""
+    f = _fmt_id(fmt)
+    if f != _lib.NVFP4 or M <= 64:
+        return True
+    L, N = _lib.lib(), sum(part_rows)
+    large = lambda n: L.arcq_gemm_route(M, n, Kp, f, 0, 0) in (1, 2) or \
+        (L.arcq_gemm_route(M, n, Kp, f, 0, 0) == 0 and L.arcq_gemm_kernel(M, n, Kp, f, 0, 0) == 44)
+    if not large(N) or any(large(n) for n in part_rows):
+        return True
+    tiles = -(-M // 256) * -(-N // 256)
+    return M > 128 and not (tiles > 256 and 0 < tiles % 256 <= 64)
+
+
 def rmsnorm(X, W, eps, *, tensor_scale=False):
     """RMSNorm as HF's LlamaRMSNorm has it (benchmarks/modeling_arc.py:237-242): bf16(W * bf16(X / sqrt(mean(X^2) + eps))) of bf16
     X [M, K], W [K]; tensor_scale=True also returns the result's NVFP4 tensor scale max|Y| / 2688 (0-dim fp32 device tensor)."""

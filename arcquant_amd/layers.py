@@ -491,6 +491,9 @@ class SplitQLinear(nn.Module):
         if not 2 <= len(ps) <= 4 or not all(_unhooked(p, QLinearLayer) and p.quant_type == ps[0].quant_type for p in ps) or \
                 any(p.out_features % 32 for p in ps) or not isinstance(scale, (float, int, torch.Tensor)):
             return None
+        rows = tuple(p.out_features for p in ps)
+        if qx.dim() != 2 or not agemm.parts_pay(qx.shape[0], rows, 2 * qx.shape[1], ps[0].quant_type):
+            return None
         bias = None
         if any(p.bias is not None for p in ps):
             bias = self._joint("bias")
@@ -500,8 +503,7 @@ class SplitQLinear(nn.Module):
         scales = [_own(p, "scale") for p in ps]
         if W is None or scale_w is None or any(s.dtype != torch.float32 or s.device != W.device for s in scales):
             return None
-        return agemm.matmul_parts(qx, W, scale_x, scale_w, scale, [p.out_features for p in ps], scales, fmt=ps[0].quant_type,
-                                  bias=bias)
+        return agemm.matmul_parts(qx, W, scale_x, scale_w, scale, rows, scales, fmt=ps[0].quant_type, bias=bias)
 
     @_no_grad
     def forward(self, x, residual=None):

@@ -2,6 +2,7 @@
 reference's names and argument order, and building a layer from CPU weights fails loudly."""
 import copy
 import inspect
+import os
 
 import pytest
 import torch
@@ -194,6 +195,26 @@ def test_split_linear_runs_part_by_part_where_a_part_is_not_itself(monkeypatch):
     own = layers.QLinearLayer.forward
     monkeypatch.setattr(layers.QLinearLayer, "forward", lambda self, *a, **kw: own(self, *a, **kw))
     assert not run(lambda s: None)
+
+
+@pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
+def test_split_linear_runs_part_by_part_where_that_is_faster(monkeypatch):
+    """one GEMM over all parts, but for the sizes at which its 256x256 tiles leave most of a round, or most of their rows, empty"""
+    for M, rows, kp, one in ((300, (18944, 18944), 4352, False), (384, (18944, 18944), 4352, False), (600, (11008, 11008), 4352, False),
+                             (80, (28672, 28672), 8320, False), (128, (28672, 28672), 8320, False), (129, (28672, 28672), 8320, True),
+                             (64, (28672, 28672), 8320, True), (200, (18944, 18944), 4352, True), (300, (14336, 14336), 4352, True),
+                             (2331, (3584, 512, 512), 3712, True), (2331, (18944, 18944), 3712, True)):
+        assert layers.agemm.parts_pay(M, rows, kp, "NVFP4") == one, (M, rows)
+        assert layers.agemm.parts_pay(M, rows, kp, "MXFP4")
+    ran = []
+    monkeypatch.setattr(layers.agemm, "matmul", lambda A, B, *a, **kw: ran.append("part") or torch.ones(A.shape[0], B.shape[0], dtype=torch.bfloat16))
+    monkeypatch.setattr(layers.agemm, "matmul_parts", lambda A, B, *a, **kw: ran.append("one") or torch.ones(A.shape[0], B.shape[0], dtype=torch.bfloat16))
+    split = layers.SplitQLinear([_quantized_linear(64, 32), _quantized_linear(32, 32)])
+    x = (torch.zeros(2, 32, dtype=torch.uint8), torch.zeros(8, dtype=torch.uint8), 1.0, 1, 2)
+    split(x)
+    monkeypatch.setattr(layers.agemm, "parts_pay", lambda M, rows, kp, fmt: (M, rows, kp, fmt) != (2, (64, 32), 64, "NVFP4"))
+    split(x)
+    assert ran == ["one", "part", "part"]
 
 
 def test_norm_ahead_of_a_quantizer_is_the_module(monkeypatch):
