@@ -693,3 +693,16 @@ def test_rmsnorm_under_traces_and_transforms(layers, monkeypatch):
     with torch.device("cuda"):
         y = norm(x)
     assert len(ran) == 1 and torch.equal(norm(x), y) and rel_fro(y, torchs(x)) < 1e-3
+
+
+def test_prompts_of_one_token_and_more(layers, monkeypatch):
+    """the attention of whole prompts has its own kernel from two tokens on; a token by itself is its own value, by torch's"""
+    nh, nkv, hidden = 4, 2, 512
+    layer = layers.LlamaDecoderLayer(hidden, 1024, nh, nkv, select_num=64, select_num_down=64, quant_type="MXFP4", seed=35)
+    ran, own = [], layers._kvc.attention_prefill
+    monkeypatch.setattr(layers._kvc, "attention_prefill", lambda q, k, v, n: ran.append(n) or own(q, k, v, n))
+    x = torch.randn(3, 2, hidden, generator=torch.Generator().manual_seed(36)).to(torch.bfloat16).cuda()
+    two = layer(x)
+    assert ran == [2]
+    one = layer(x[:, :1].contiguous())
+    assert ran == [2] and torch.equal(one, two[:, :1])
