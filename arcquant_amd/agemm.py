@@ -526,7 +526,8 @@ def _absmax_to_scales(buf, divisor):
 def matmul_swiglu(A, B, SFA, SFB, scale, *, fmt=None, tensor_scale=False):
     """matmul for a fused gate/up projection whose weight rows alternate gate, up (interleave_gate_up), with
     act_fn(gate) * up formed in the epilogue: returns t bf16 [M, N/2], bit-identical to
-    ``h = matmul(...); F.silu(h_gate) * h_up`` in bf16, without h going through memory.  tensor_scale=True
+    ``h = matmul(...); F.silu(h_gate) * h_up`` in bf16 (where matmul takes another kernel, NVFP4 decode batches, h's sums are in
+    another order), without h going through memory.  tensor_scale=True
     also returns the NVFP4 tensor scale max|t| / 2688 of t (0-dim fp32 device tensor, 1 for all zeros)."""
     _require(A, "A", torch.uint8, 2)
     _require(B, "B", torch.uint8, 2)

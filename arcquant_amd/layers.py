@@ -54,13 +54,6 @@ def _no_grad(forward):
     return run
 
 
-def _own(module, name):
-    """module.name where it is a buffer, without the search through three dictionaries that an access through the module begins
-    with; what has taken a buffer's place since (a Parameter, a parametrization) as the module has it"""
-    t = module._buffers.get(name)
-    return getattr(module, name) if t is None else t
-
-
 def _plain(*tensors):
     """Ordinary tensors, and nothing around this call that has to see every operator on them: traces, compilation, modes, vmap and
     the other transforms, and forward-mode gradients are left to torch's own operators."""
@@ -166,10 +159,15 @@ class QLinearLayer(nn.Module):
         """residual [..., out_features]: added to the output (in the GEMM's epilogue when the layer has
         no bias), same bits as `self(x) + residual`"""
         qx, scale_x, scale, bsz, q_len = x
-        alpha = (scale if isinstance(scale, torch.Tensor) else float(scale), _own(self, "scale"))
-        bias = _own(self, "bias")
+        own = self._buffers                # (each access through the module would search three dictionaries first)
+        try:
+            W, scale_w, own_scale = own["W"], own["scale_w"], own["scale"]
+        except KeyError:                   # a Parameter, or a parametrization, has taken a buffer's place
+            W, scale_w, own_scale = self.W, self.scale_w, self.scale
+        bias = own["bias"] if "bias" in own else self.bias
+        alpha = (scale if isinstance(scale, torch.Tensor) else float(scale), own_scale)
         fused = residual is not None and bias is None
-        y = agemm.matmul(qx, _own(self, "W"), scale_x, _own(self, "scale_w"), alpha, fmt=self.quant_type,
+        y = agemm.matmul(qx, W, scale_x, scale_w, alpha, fmt=self.quant_type,
                          residual=residual.reshape(-1, self.out_features).contiguous() if fused else None)
         if bias is not None:
             y = y + bias
@@ -206,8 +204,12 @@ class RMSNormQuant(nn.Module):
     def forward(self, hidden_states):
         bsz, q_len, _ = hidden_states.shape
         flat = hidden_states.reshape(bsz * q_len, -1).contiguous()
-        A, SFA = agemm.rmsnorm_quantize_x(flat, _own(self, "weight"), self.variance_epsilon, _own(self, "reorder_index"),
-                                          self.select_num, fmt=self.quant_type)
+        own = self._buffers
+        try:
+            weight, index = own["weight"], own["reorder_index"]
+        except KeyError:
+            weight, index = self.weight, self.reorder_index
+        A, SFA = agemm.rmsnorm_quantize_x(flat, weight, self.variance_epsilon, index, self.select_num, fmt=self.quant_type)
         return A, SFA, 1.0, bsz, q_len
 
 
@@ -454,7 +456,7 @@ class SplitQLinear(nn.Module):
         if not 2 <= len(ps) <= 4 or len(set(ps)) != len(ps) or \
                 any(type(p) is not QLinearLayer or p.quant_type != ps[0].quant_type or p.out_features % 32 for p in ps):
             return
-        for name in ["W", "scale_w"] + (["bias"] if any(_own(p, "bias") is not None for p in ps) else []):
+        for name in ["W", "scale_w"] + (["bias"] if any(p.bias is not None for p in ps) else []):
             held[name] = ts = [p._buffers.get(name) for p in ps]
             if any(type(t) is not torch.Tensor or not (t.is_cuda or t.is_cpu and not t.is_shared()) or t.dtype != ts[0].dtype or
                    t.device != ts[0].device or t.shape[1:] != ts[0].shape[1:] for t in ts):
@@ -502,7 +504,7 @@ class SplitQLinear(nn.Module):
             if bias is None or bias.dtype != torch.bfloat16:
                 return None
         W, scale_w = self._joint("W"), self._joint("scale_w")
-        scales = [_own(p, "scale") for p in ps]
+        scales = [p.scale for p in ps]
         if W is None or scale_w is None or any(s.dtype != torch.float32 or s.device != W.device for s in scales):
             return None
         return agemm.matmul_parts(qx, W, scale_x, scale_w, scale, rows, scales, fmt=ps[0].quant_type, bias=bias)

@@ -266,12 +266,12 @@ int arcq_gemm_route(int M, int N, int Kp, int fmt, int n_seg, int swiglu);
 /*
  * arcq_matmul for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same arguments, same kernel
- * choice and the same bits as arcq_matmul (arcq_gemm with a workspace may differ by one rounding), but the split-K partial tiles live in a fixed 8 MiB array inside
- * the library's code object (one copy per GPU, held until the process ends) instead of a stream's scratch
- * buffer, and the call contains no allocation of any kind.
+ * choice and the same bits as arcq_matmul (arcq_gemm with a workspace may differ by one rounding; so may a captured arcq_matmul
+ * whose stream was not prepared), but the split-K partial tiles live in a fixed 8 MiB array inside the library's code object (one
+ * copy per GPU, held until the process ends) instead of a stream's scratch buffer, and the call contains no allocation of any kind.
  *   - A problem whose plan needs more than arcq_matmul_noalloc_limit() bytes of partial tiles
  *     (arcq_matmul_scratch_bytes tells, 0 = none needed) is refused with ARCQ_ERR_WORKSPACE and nothing is
- *     launched: e.g. the NVFP4 4096 x 14336 down projection at 512 rows (two K slices, 16 MiB).  Every decode batch
+ *     launched, also where arcq_gemm_route would run it without any: e.g. the NVFP4 4096 x 14336 down projection at 512 rows (two K slices, 16 MiB).  Every decode batch
  *     (M <= 64) of the Llama-3-8B shapes fits.
  *   - All calls on one GPU share that GPU's array: calls that overlap in time on one GPU (two streams,
  *     two threads) race.  The array keeps the last call's contents; every word a call reads back it has
@@ -334,8 +334,8 @@ int arcq_grouped_matmul(const void *a_codes, const void *a_scales, const void *b
  * arcq_reorder_quantize_w): output columns 2j and 2j+1 of a token then sit in one lane, and instead of the
  * [M, N] projection output the kernel writes t [M, N/2] = act_fn(gate) * up, formed from the bf16-rounded
  * GEMM outputs exactly as the reference's layers form it from the projection output in bf16
- * (model/qLlamaLayer.py:432, model/qMixtralLayer.py:531): the same bits as the unfused sequence, without the
- * projection output passing through memory.  No counterpart in the reference (it names the fusion,
+ * (model/qLlamaLayer.py:432, model/qMixtralLayer.py:531): the same bits as the unfused sequence (the order of the sums aside where
+ * that takes another kernel: NVFP4 decode batches), without the projection output passing through memory.  No counterpart in the reference (it names the fusion,
  * benchmarks/modeling_arc.py:112, and does not ship it).
  *   d_absmax  NULL, or fp32 [n_seg] ([1] for arcq_matmul_swiglu) zeroed by the caller: receives max |t| per
  *             expert (as the bits of a non-negative float, i.e. readable as fp32), the numerator of the
