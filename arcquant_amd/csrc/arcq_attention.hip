@@ -39,8 +39,9 @@ typedef v4s __attribute__((address_space(3))) lds_v4s;
 // rounding of every weight is then that of torch's kernel (one output in 3000 to 10000 differs, by a bf16 step), behind which a quantizer
 // makes the same codes.  (Raising the maximum only beyond 2^8 saves 4 %, but a row's largest weight is then no longer exactly 1:
 // error against 64 bits 2.1e-3 in norm, so 1.8e-3 as torch's, the bf16 output alone 1.66e-3.)  O is rescaled only when some query's
-// maximum moves.  us, torch's scaled_dot_product_attention before: 8 x 2048 tokens, 32 heads, 8 KV heads 744 -> 381
-// (723 TFLOP/s), 4 x 1024 165 -> 62, 3 x 777, 28 heads, 4 KV heads 109 -> 39, 1 x 100 25 -> 7.
+// maximum moves.  us, torch's scaled_dot_product_attention before, N(0, 1) operands: 8 x 2048 tokens, 32 heads, 8 KV heads 747 -> 361
+// (763 TFLOP/s; 339 in a layer), 4 x 1024 163 -> 58, 3 x 777, 28 heads, 4 KV heads 108 -> 39, 1 x 100 22 -> 11.  (Sequences of one token, 28
+// heads, 64 of them: 6.7 -> 16.9.)
 //
 // XCDs get contiguous runs of (sequence, KV head) groups, whose K and V their L2 then holds, the longest query tiles first.
 // ---------------------------------------------------------------------------------------------
