@@ -44,15 +44,22 @@ __global__ __launch_bounds__(256) void nvfp4_decode_f16_kernel(const uint32_t *c
 //
 // Eight waves, two per SIMD, in two groups of four: a wave owns 64 rows of the codes side (wave & 3) and 128 rows of
 // the fp16 side (wave >> 2).  A wave alternates between a memory phase (operand reads from LDS for the next 32 elements
-// of K, decoding of its codes, requests of later stages) and a compute phase (32 MFMAs, nothing else).  The second
-// group starts one phase late, so that at any time one wave of every SIMD multiplies while the other one reads and
-// decodes; the barrier between phases keeps them in step.
+// of K, requests of later stages) and a compute phase (32 MFMAs, and between them the decoding of its codes for the next
+// phase).  The second group starts one phase late, so that at any time one wave of every SIMD multiplies while the other one
+// reads; the barrier between phases keeps them in step.
+//
+// What bounds it is the longer of the two phases: 512 cycles of MFMAs, and in the other one what a lone wave can issue, an
+// instruction every 5 to 9 cycles.  Decoding in the memory phase (32 instructions) made that 63 to 84 instructions long, and the phase
+// of an odd step that also requests codes and scale bytes the longest of all; so the decoding goes between the MFMAs, which leave
+// room for one VALU instruction each, and the requests are spread (4 of 8 KB or less per phase at most).  us, decoding and the requests of
+// codes in the memory phases, and so: 2048 x 2048 x 14592 266 and 244
+// (its MFMAs and barriers alone: 216), 16384 x 28672 x 4352 2740 and 2630, where all CUs are busy and the clock gives way.  Neither more
+// stages on their way nor lines fetched into L2 ahead nor requests between the MFMAs, fewer barriers or raised wave
+// priority are faster.
 //
 // The matrix instruction is 16x16x32: the chip is power-limited under these kernels, and on decoded FP4 values a
 // register-only loop of it sustains 2.00 PFLOP/s against 1.83 for 32x32x16 (two waves per SIMD, all CUs), 2.08 when the fp16
 // tiles are walked back and forth, which keeps one operand of neighbours unchanged at the turns too (arcq_mfma_rate_probe).
-// 4096 x 28672 x 4352: 682 us with the decoding, 1.50 PFLOP/s (the matrix pipe is busy for 74 % of the cycles, the VALU for
-// 43 %); the kernel that decodes both operands in every workgroup: 832 us.
 //
 // LDS: three stages of the fp16 tile (64 elements of K: rows of 128 bytes), two of the codes (128 elements: rows of 64
 // bytes) and of the scale bytes (8 per row).  A stage is requested two steps ahead of its first read by LDS-direct
@@ -142,9 +149,9 @@ __device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, i
                             lds + kF + c_row * 64 + ((((g >> 1) + 2) ^ ((r >> 2) & 3)) << 4) + (g & 1) * 8};
   const uint8_t *s_rd = lds + kF + kC + c_row * 4 + g;
 
-  uint2 cq[2][4];           // codes of an even and of an odd step, eight bytes per 16 rows
-  uint32_t sq[2][4];        // their scale byte
-  v8h cf[4];                // decoded operands of a phase
+  uint2 cq[4];              // codes of a step, eight bytes per 16 rows
+  uint32_t sq[4];           // their scale byte
+  v8h cf[2][4];             // decoded operands of either phase
   v8h ff[TF];
   v4f acc[CODES_W ? 4 : TF][CODES_W ? TF : 4];
 #pragma unroll
@@ -154,8 +161,8 @@ __device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, i
 
   auto read_codes = [&](int j, auto odd_t, int i) {  // of step 2j or 2j + 1, 16-row tile i
     constexpr int o = decltype(odd_t)::value ? 1 : 0;
-    cq[o][i] = *reinterpret_cast<const uint2 *>(c_rd[o] + (j & 1) * (BC * 64) + i * 1024);
-    sq[o][i] = s_rd[(j & 1) * (BC * 8) + o * (BC * 4) + i * 64];
+    cq[i] = *reinterpret_cast<const uint2 *>(c_rd[o] + (j & 1) * (BC * 64) + i * 1024);
+    sq[i] = s_rd[(j & 1) * (BC * 8) + o * (BC * 4) + i * 64];
   };
   auto barrier = [&]() {
     asm volatile("" ::: "memory");
@@ -167,23 +174,30 @@ __device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, i
   auto read_f = [&](int st, int half, int t) {
     ff[t] = __builtin_bit_cast(v8h, *reinterpret_cast<const uint4 *>(f_rd[half] + st * (BF * 128) + t * 2048));
   };
-  auto decode = [&](int half, auto odd_t, int i) {
-    constexpr int o = decltype(odd_t)::value ? 1 : 0;
-    if (half == 0) sq[o][i] = (sq[o][i] << 7) + 0x1800u;  // scale byte -> fp16
-    cf[i] = decode8_nvfp4_f16<false>(half ? cq[o][i].y : cq[o][i].x, sq[o][i]);
-    asm volatile("" : "+v"(cf[i]));  // here, not behind the barrier
+  auto decode = [&](int half, int i) {
+    if (half == 0) sq[i] = (sq[i] << 7) + 0x1800u;  // scale byte -> fp16
+    cf[half][i] = decode8_nvfp4_f16<false>(half ? cq[i].y : cq[i].x, sq[i]);
   };
-  auto multiply = [&]() {
+  // the products of a phase, and between them the decoding of the next phase's codes (the last step's: of codes that nobody uses)
+  auto multiply = [&](auto half_t) {
+    constexpr int h = decltype(half_t)::value;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) decode(1 - h, i);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int s = 0; s < TF; ++s) {
         const int t = i & 1 ? TF - 1 - s : s;
         if constexpr (CODES_W)
-          acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cf[i], ff[t], acc[i][t], 0, 0, 0);
+          acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(cf[h][i], ff[t], acc[i][t], 0, 0, 0);
         else
-          acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ff[t], cf[i], acc[t][i], 0, 0, 0);
+          acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ff[t], cf[h][i], acc[t][i], 0, 0, 0);
       }
+#pragma unroll
+    for (int k = 0; k < 4 * TF; ++k) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, (8 + TF - 1) / TF, 0);
+    }
   };
 
 #pragma unroll
@@ -198,25 +212,27 @@ __device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, i
   barrier();
 #pragma unroll
   for (int i = 0; i < 4; ++i) read_codes(0, std::false_type{}, i);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < 4; ++i) decode(0, i);
   if (group) barrier();  // the second group runs one phase behind
 
   int st = 0, st2 = 2;   // stages of step u and u + 2
   auto step = [&](int u, auto odd_t) {
     constexpr bool ODD = decltype(odd_t)::value;
-    // A memory phase goes tile by tile: LDS reads, decoding and requests take turns, so that none of the three queues
-    // holds the other two up.
-    // first phase
+    // A memory phase goes tile by tile: LDS reads and requests take turns, so that neither queue holds the other up.
+    // first phase; the stage of the codes requested here was last read in step u - 1
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
       for (int t = i * TF / 4; t < (i + 1) * TF / 4; ++t) read_f(st, 0, t);
-      decode(0, odd_t, i);
       if (i < FI / 2) request_f(u + 2, st2, i);  // its stage was last read in step u - 1
+      if (ODD && (i == 2 || i == 3)) request_c((u + 3) >> 1, i - 2);
       __builtin_amdgcn_sched_barrier(0);
     }
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     barrier();
-    multiply();
+    multiply(std::integral_constant<int, 0>{});
     barrier();
     // second phase; the codes read are the next step's (behind the last one: not used)
 #pragma unroll
@@ -224,16 +240,15 @@ __device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, i
 #pragma unroll
       for (int t = i * TF / 4; t < (i + 1) * TF / 4; ++t) read_f(st, 1, t);
       read_codes((u + 1) >> 1, std::integral_constant<bool, !ODD>{}, i);
-      decode(1, odd_t, i);
       if (i < FI / 2) request_f(u + 2, st2, FI / 2 + i);
-      if (ODD && i > 0) request_c((u + 3) >> 1, i - 1);
+      if (ODD && i == 3) request_c((u + 3) >> 1, 2);
       __builtin_amdgcn_sched_barrier(0);
     }
     // the next step's fp16 stage (and everything older) has to be there behind this barrier; what this step has
     // requested may stay on its way
     asm volatile("s_waitcnt lgkmcnt(0) vmcnt(%0)" : : "n"(ODD ? FI + 3 : FI) : "memory");
     barrier();
-    multiply();
+    multiply(std::integral_constant<int, 1>{});
     barrier();
     st = st == 2 ? 0 : st + 1;
     st2 = st2 == 2 ? 0 : st2 + 1;
