@@ -1236,11 +1236,12 @@ int check_gemm_args(const void *a_codes, const void *a_scales, const void *b_cod
 }
 
 // Whether this problem goes to the kernel that multiplies one operand decoded to fp16 ahead (arcq_gemm_nv.hip).
-// Its tile is 256x256, one workgroup per CU, and a round of tiles takes the same time however few there are (K' = 4352:
-// 75-98 us).  The kernels without a workspace are faster as long as their 256x128 tiles fit one round (K' = 4352, without and
+// Its tile is 256 weight rows x 256, 192 or 128 activation rows (f16_plan), one workgroup per CU, and a round of tiles takes the same
+// time however few there are (K' = 4352, 256 rows: 75-98 us).  The kernels without a workspace are faster as long as their 256x128 tiles fit one round (K' = 4352, without and
 // with: 2048 x 4096 66 / 84 us, 1024 x 6144 55 / 82), and slower beyond (257 x 28672 100 / 98, 65 x 128256 241 / 239,
-// 1400 x 6144 115 / 85, 2331 x 4096 113 / 87, 4096 x 28672 832 / 725; K' = 14592, 4096 x 4096 360 / 346; K' = 1152,
-// 200 x 33024 44 / 34).
+// 1400 x 6144 115 / 68, 2331 x 4096 113 / 74, 4096 x 28672 832 / 682; K' = 14592, 4096 x 4096 360 / 328; K' = 1152,
+// 200 x 33024 44 / 34).  So are the plan's 256x256 tiles, for up to 128 rows on layers of more than 49000 columns (100 x 53248,
+// K' = 512, 1152: 20.5, 38.8 / 15.3, 24.2; 128 x 57344 x 4352 101 / 67).
 bool nvfp4_f16_wanted(int M, int N, int Kp, int fmt, int n_seg) {
   const int force = tuning().gemm_kernel;
   if (fmt != ARCQ_FMT_NVFP4 || Kp % 128 != 0 || Kp < 512 || (force >= 0 && force != 168)) return false;
@@ -1256,7 +1257,7 @@ bool nvfp4_f16_wanted(int M, int N, int Kp, int fmt, int n_seg) {
   if (n_seg > 0)
     return M / n_seg >= 768 && (N >= 6144 || (N > 2048 && ((M + 255) / 256 + n_seg / 2) * tiles_n >= 6 * 256));
   if (M <= 64) return false;  // a stream of the weights, however many tiles they make (16 x 70000 x 4352: 70 against 177 us)
-  return (long)((M + 127) / 128) * tiles_n > 256;
+  return (long)((M + 127) / 128) * tiles_n > 256 || (M <= 128 && tiles_n >= 192);
 }
 
 // The same, and whether its last round of tiles is cut along K, which some problems take that are otherwise left to the kernels
@@ -1265,7 +1266,7 @@ size_t nvfp4_split_scratch(int M, int N, int Kp, int fmt, int n_seg) {
   const int force = tuning().gemm_kernel;
   if (fmt != ARCQ_FMT_NVFP4 || force >= 0 || (size_t)M * Kp * 2 >= ((size_t)1 << 32) || (size_t)N * Kp / 2 >= ((size_t)1 << 32)) return 0;
   const size_t slots = nvfp4_split_bytes(M, N, Kp, n_seg);
-  return slots ? nvfp4_f16_bytes(M, N, Kp, n_seg > 0) + slots : 0;
+  return slots ? nvfp4_split_operand_bytes(M, N, Kp, n_seg > 0) + slots : 0;
 }
 
 // How a problem with this much workspace multiplies one operand decoded ahead: 0 not at all, 1 tile by tile, 2 with its last

@@ -40,19 +40,19 @@ __global__ __launch_bounds__(256) void nvfp4_decode_f16_kernel(const uint32_t *c
 }
 
 // ---------------------------------------------------------------------------------------------
-// 256 rows of codes x 256 rows of fp16 per workgroup, K in steps of 64.
+// 256 rows of codes x 32 TF rows of fp16 per workgroup (TF = 8, 6, 4 or 2), K in steps of 64.
 //
-// Eight waves, two per SIMD, in two groups of four: a wave owns 64 rows of the codes side (wave & 3) and 128 rows of
+// Eight waves, two per SIMD, in two groups of four: a wave owns 64 rows of the codes side (wave & 3) and 16 TF rows of
 // the fp16 side (wave >> 2).  A wave alternates between a memory phase (operand reads from LDS for the next 32 elements
-// of K, requests of later stages) and a compute phase (32 MFMAs, and between them the decoding of its codes for the next
+// of K, requests of later stages) and a compute phase (4 TF MFMAs, and between them the decoding of its codes for the next
 // phase).  The second group starts one phase late, so that at any time one wave of every SIMD multiplies while the other one
 // reads; the barrier between phases keeps them in step.
 //
-// What bounds it is the longer of the two phases: 512 cycles of MFMAs, and in the other one what a lone wave can issue, an
+// What bounds it is the longer of the two phases: 512 cycles of MFMAs (TF = 8), and in the other one what a lone wave can issue, an
 // instruction every 5 to 9 cycles.  Decoding in the memory phase (32 instructions) made that 63 to 84 instructions long, and the phase
 // of an odd step that also requests codes and scale bytes the longest of all; so the decoding goes between the MFMAs, which leave
 // room for one VALU instruction each, and the requests are spread (4 of 8 KB or less per phase at most).  us, decoding and the requests of
-// codes in the memory phases, and so: 2048 x 2048 x 14592 266 and 244
+// codes in the memory phases, and so: 2331 x 3584 x 19072 with TF = 6 316 and 262; 2048 x 2048 x 14592 with TF = 8 266 and 244
 // (its MFMAs and barriers alone: 216), 16384 x 28672 x 4352 2740 and 2630, where all CUs are busy and the clock gives way.  Neither more
 // stages on their way nor lines fetched into L2 ahead nor requests between the MFMAs, fewer barriers or raised wave
 // priority are faster.
@@ -72,12 +72,12 @@ __global__ __launch_bounds__(256) void nvfp4_decode_f16_kernel(const uint32_t *c
 // CODES_W: the weights are the codes side; they always take the MFMA's A slot (a lane then holds four consecutive output
 // columns).  Requires K' % 128 == 0, K' >= 256.
 // ---------------------------------------------------------------------------------------------
-template <bool CODES_W>
+template <bool CODES_W, int TF_ = 8>
 struct F16Shape {
-  static constexpr int TF = 8;  // 16-row tiles of the fp16 side per wave
+  static constexpr int TF = TF_;  // 16-row tiles of the fp16 side per wave
   static constexpr int BC = 256, BF = 32 * TF;
   static constexpr int BM = CODES_W ? BF : BC, BN = CODES_W ? BC : BF;
-  static constexpr int FI = BF / 64;                       // fp16 load instructions per wave and step
+  static constexpr int FI = BF / 64, FA = (FI + 1) / 2;    // fp16 load instructions per wave and step, and in its first phase
   static constexpr int kF = 3 * BF * 128, kC = 2 * BC * 64, kS = 2 * BC * 8;
   static constexpr int kRegion = 64 * 16 * TF * 2;         // bytes per wave of the epilogue's transpose
   static_assert(8 * kRegion <= kF + kC, "the epilogue's transpose");
@@ -88,28 +88,26 @@ struct F16Shape {
 // Rows of either side where tile lin begins.
 // An XCD's 32 workgroups run at the same time on consecutive tiles: 4 tiles of the fp16 side x 8 of the codes, so that
 // both operands are shared in its L2 (an fp16 tile is four times the bytes of a codes tile)
-template <bool CODES_W>
+template <bool CODES_W, int TF>
 __device__ __forceinline__ void f16_tile_at(const GemmParams &p, int lin, int &c_base, int &f_base) {
-  using S = F16Shape<CODES_W>;
+  using S = F16Shape<CODES_W, TF>;
   const int rows_c = CODES_W ? p.N : p.M, rows_f = CODES_W ? p.M : p.N;
   const int tc = (rows_c + S::BC - 1) / S::BC, tf = (rows_f + S::BF - 1) / S::BF;
   const int band = lin / (4 * tc), bw = min(4, tf - 4 * band), in_band = lin - band * 4 * tc;
   c_base = (in_band / bw) * S::BC, f_base = (4 * band + in_band % bw) * S::BF;
 }
 
-// Tile lin of p, nk steps of 64 elements from step u0 on (both even): the tile of C, or with `partial` the fp32 sums.
-template <bool CODES_W>
-__device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, int nk, float4 *partial, uint8_t *smem, int tid) {
-  using S = F16Shape<CODES_W>;
-  constexpr int TF = S::TF, BC = S::BC, BF = S::BF, FI = S::FI, kF = S::kF, kC = S::kC, kRegion = S::kRegion;
+// The tile at (c_base, f_base), nk steps of 64 elements from step u0 on (both even): the tile of C, or with `partial` the fp32 sums.
+template <bool CODES_W, int TF>
+__device__ __forceinline__ void f16_tile_of(const GemmParams &p, int c_base, int f_base, int u0, int nk, float4 *partial, uint8_t *smem, int tid) {
+  using S = F16Shape<CODES_W, TF>;
+  constexpr int BC = S::BC, BF = S::BF, FI = S::FI, FA = S::FA, kF = S::kF, kC = S::kC, kRegion = S::kRegion;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int cpos = wave & 3, group = wave >> 2;
   const int kbytes = p.Kp >> 1, ksc = p.Kp >> 4, fbytes = p.Kp << 1;
   const int rows_c = CODES_W ? p.N : p.M, rows_f = CODES_W ? p.M : p.N;
   const uint8_t *codes = (CODES_W ? p.b_codes : p.a_codes) + u0 * 32, *scales = (CODES_W ? p.b_scales : p.a_scales) + u0 * 4;
-  int c_base, f_base;
-  f16_tile_at<CODES_W>(p, lin, c_base, f_base);
 
   // ---- global -> LDS: a wave-uniform base plus a 32-bit byte offset per lane
   uint32_t fvo[FI], cvo[2], svo;
@@ -226,7 +224,7 @@ __device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, i
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
       for (int t = i * TF / 4; t < (i + 1) * TF / 4; ++t) read_f(st, 0, t);
-      if (i < FI / 2) request_f(u + 2, st2, i);  // its stage was last read in step u - 1
+      if (i < FA) request_f(u + 2, st2, i);  // its stage was last read in step u - 1
       if (ODD && (i == 2 || i == 3)) request_c((u + 3) >> 1, i - 2);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -240,7 +238,7 @@ __device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, i
 #pragma unroll
       for (int t = i * TF / 4; t < (i + 1) * TF / 4; ++t) read_f(st, 1, t);
       read_codes((u + 1) >> 1, std::integral_constant<bool, !ODD>{}, i);
-      if (i < FI / 2) request_f(u + 2, st2, FI / 2 + i);
+      if (i < FI - FA) request_f(u + 2, st2, FA + i);
       if (ODD && i == 3) request_c((u + 3) >> 1, 2);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -276,9 +274,25 @@ __device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, i
     store_wave_tile(p, Acc16<TF, 4>{acc}, region, c_base + 64 * cpos, f_base + 16 * TF * group, lane);
 }
 
-template <bool CODES_W>
+// The last rows of a problem or of an expert's: a tile of fewer fp16 rows, whose phases are shorter (the sums are the same).  Zipf-like
+// experts, 8192 rows over eight of 28672 x 4224 with the SwiGLU epilogue: 1616 us with whole tiles alone, 1595 so; 333 x 28672 x 4352:
+// 96 and 85.
+template <bool CODES_W, int TF>
+__device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, int nk, float4 *partial, uint8_t *smem, int tid) {
+  int c_base, f_base;
+  f16_tile_at<CODES_W, TF>(p, lin, c_base, f_base);
+  if constexpr (CODES_W) {
+    const int left = p.M - f_base;
+    if (TF > 2 && left <= 64) return f16_tile_of<CODES_W, 2>(p, c_base, f_base, u0, nk, partial, smem, tid);
+    if (TF > 4 && left <= 128) return f16_tile_of<CODES_W, 4>(p, c_base, f_base, u0, nk, partial, smem, tid);
+    if (TF > 6 && left <= 192) return f16_tile_of<CODES_W, 6>(p, c_base, f_base, u0, nk, partial, smem, tid);
+  }
+  f16_tile_of<CODES_W, TF>(p, c_base, f_base, u0, nk, partial, smem, tid);
+}
+
+template <bool CODES_W, int TF>
 __global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
-  using S = F16Shape<CODES_W>;
+  using S = F16Shape<CODES_W, TF>;
   __shared__ uint4 smem[(S::kF + S::kC + S::kS) / 16];
   int lin;
   if (p.seg) {
@@ -288,7 +302,7 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
     lin = (blockIdx.x & 7) * ((total + 7) >> 3) + (blockIdx.x >> 3);
     if (lin >= total) return;
   }
-  f16_tile<CODES_W>(p, lin, 0, p.Kp >> 6, nullptr, reinterpret_cast<uint8_t *>(smem), threadIdx.x);
+  f16_tile<CODES_W, TF>(p, lin, 0, p.Kp >> 6, nullptr, reinterpret_cast<uint8_t *>(smem), threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -361,23 +375,16 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_f16_split(GemmParams p) {
     wait_dma_and_sync();  // the LDS of the part before this one
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));  // what follows from it is formed per part: hoisted out of this loop it would be spilled
-    f16_tile<CODES_W>(q, lin, 2 * first, 2 * n, partial, reinterpret_cast<uint8_t *>(smem), tid);
+    f16_tile<CODES_W, 8>(q, lin, 2 * first, 2 * n, partial, reinterpret_cast<uint8_t *>(smem), tid);
     at += n;
   }
 }
 
 // a wave per eighth of a tile
-template <bool CODES_W>
-__global__ __launch_bounds__(64) void f16_split_add_kernel(GemmParams p) {
-  using S = F16Shape<CODES_W>;
-  __shared__ uint4 smem[S::kRegion / 16];
-  constexpr int TF = S::TF;
-  const int lane = threadIdx.x, wave = blockIdx.x & 7, tile = blockIdx.x >> 3, cpos = wave & 3, group = wave >> 2;
-  const LastRound r(f16_tiles<CODES_W>(p), p.Kp);
-  if (tile >= r.rest) return;
-  const int w0 = r.holder(tile * r.pairs), w1 = r.holder((tile + 1) * r.pairs - 1);
-  int lin = r.full + tile;
-  if (w0 == w1 || !f16_enter<CODES_W>(p, lin)) return;  // (one workgroup had the whole tile and stored it)
+template <bool CODES_W, int TF>
+__device__ __forceinline__ void f16_add_parts(const GemmParams &p, const LastRound &r, int w0, int w1, int c_base, int f_base, uint8_t *region) {
+  using S = F16Shape<CODES_W, TF>;
+  const int lane = threadIdx.x, wave = blockIdx.x & 7, cpos = wave & 3, group = wave >> 2;
   v4f acc[CODES_W ? 4 : TF][CODES_W ? TF : 4];
 #pragma unroll
   for (auto &a : acc)
@@ -385,7 +392,7 @@ __global__ __launch_bounds__(64) void f16_split_add_kernel(GemmParams p) {
     for (auto &b : a) b = v4f{0.f, 0.f, 0.f, 0.f};
   for (int w = w0; w <= w1; ++w) {
     if (r.begin(w) == r.begin(w + 1)) continue;
-    const float4 *src = p.split + (2 * w + (w == w1 ? 0 : 1)) * S::kSlot + (size_t)wave * S::kQuads * 64 + lane;
+    const float4 *src = p.split + (2 * w + (w == w1 ? 0 : 1)) * F16Shape<CODES_W>::kSlot + (size_t)wave * S::kQuads * 64 + lane;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -394,9 +401,6 @@ __global__ __launch_bounds__(64) void f16_split_add_kernel(GemmParams p) {
         (CODES_W ? acc[i][t] : acc[t][i]) += v4f{v.x, v.y, v.z, v.w};
       }
   }
-  int c_base, f_base;
-  f16_tile_at<CODES_W>(p, lin, c_base, f_base);
-  uint8_t *region = reinterpret_cast<uint8_t *>(smem);
   if constexpr (CODES_W)
     store_wave_tile(p, Acc16<4, TF>{acc}, region, f_base + 16 * TF * group, c_base + 64 * cpos, lane);
   else
@@ -404,14 +408,40 @@ __global__ __launch_bounds__(64) void f16_split_add_kernel(GemmParams p) {
 }
 
 template <bool CODES_W>
-int launch(const GemmParams &p, bool split, hipStream_t st) {
+__global__ __launch_bounds__(64) void f16_split_add_kernel(GemmParams p) {
+  using S = F16Shape<CODES_W>;
+  __shared__ uint4 smem[S::kRegion / 16];
+  const int tile = blockIdx.x >> 3;
+  const LastRound r(f16_tiles<CODES_W>(p), p.Kp);
+  if (tile >= r.rest) return;
+  const int w0 = r.holder(tile * r.pairs), w1 = r.holder((tile + 1) * r.pairs - 1);
+  int lin = r.full + tile;
+  if (w0 == w1 || !f16_enter<CODES_W>(p, lin)) return;  // (one workgroup had the whole tile and stored it)
+  int c_base, f_base;
+  f16_tile_at<CODES_W, 8>(p, lin, c_base, f_base);
+  uint8_t *region = reinterpret_cast<uint8_t *>(smem);
+  if constexpr (CODES_W) {  // as f16_tile
+    const int left = p.M - f_base;
+    if (left <= 64) return f16_add_parts<CODES_W, 2>(p, r, w0, w1, c_base, f_base, region);
+    if (left <= 128) return f16_add_parts<CODES_W, 4>(p, r, w0, w1, c_base, f_base, region);
+    if (left <= 192) return f16_add_parts<CODES_W, 6>(p, r, w0, w1, c_base, f_base, region);
+  }
+  f16_add_parts<CODES_W, 8>(p, r, w0, w1, c_base, f_base, region);
+}
+
+template <bool CODES_W, int TF>
+int launch_tiles(const GemmParams &p, hipStream_t st) {
+  using S = F16Shape<CODES_W, TF>;
+  const int total = ((p.M + S::BM - 1) / S::BM + (p.seg ? p.n_seg : 0)) * ((p.N + S::BN - 1) / S::BN);
+  hipLaunchKernelGGL((gemm_nvfp4_f16<CODES_W, TF>), dim3(((total + 7) / 8) * 8), dim3(512), 0, st, p);
+  ARCQ_HIP_TRY(hipGetLastError());
+  return ARCQ_OK;
+}
+
+template <bool CODES_W>
+int launch_split(const GemmParams &p, hipStream_t st) {
   const int total = ((p.M + 255) / 256 + (p.seg ? p.n_seg : 0)) * ((p.N + 255) / 256);
   const int grid = ((total + 7) / 8) * 8;
-  if (!split) {
-    hipLaunchKernelGGL((gemm_nvfp4_f16<CODES_W>), dim3(grid), dim3(512), 0, st, p);
-    ARCQ_HIP_TRY(hipGetLastError());
-    return ARCQ_OK;
-  }
   hipLaunchKernelGGL((gemm_nvfp4_f16_split<CODES_W>), dim3(grid + 256), dim3(512), 0, st, p);
   ARCQ_HIP_TRY(hipGetLastError());
   hipLaunchKernelGGL((f16_split_add_kernel<CODES_W>), dim3(8 * std::min(total, 255)), dim3(64), 0, st, p);
@@ -419,10 +449,30 @@ int launch(const GemmParams &p, bool split, hipStream_t st) {
   return ARCQ_OK;
 }
 
+// Which operand is decoded ahead, and the tile.  A round of 256 tiles takes its time however few there are: 0.78 of a 256-row round with
+// tiles of 192 rows of activations, 0.62 with 128, measured on 180 problems of 100 to 4096 rows, so the fewest rounds by those
+// weights.  us with 256, 192 and 128 rows: 2331 x 3584 x 3712 71, 62, 100; 2331 x 3584 x 19072 305, 268, 442; 1300 x 6144 x 4352 79, 68,
+// 112; 640 x 28672 x 4352 165, 143, 174; 300 x 37888 x 3712 132, 117, 103; 1024 x 28672 x 4352 187, 212, 234; 100 x 57344 x 4352 70, 70, 70.
+// The smaller tiles need the activations decoded; decoding a row takes 2.4e-5 of a round (about 5 TB/s, whatever K').
+struct F16Plan {
+  bool codes_w;
+  int tf;
+};
+F16Plan f16_plan(int M, int N, bool grouped) {
+  F16Plan plan{grouped || M <= N, 8};
+  if (grouped) return plan;
+  auto rounds = [&](long rows) { return (double)(((M + rows - 1) / rows * ((N + 255L) / 256) + 255) / 256); };
+  double least = rounds(256) - 2.4e-5 * std::max(0, M - N);
+  const struct { int tf; double weight; } smaller[] = {{6, 0.78}, {4, 0.62}};
+  for (const auto &s : smaller)
+    if (const double cost = rounds(32 * s.tf) * s.weight; cost < least) least = cost, plan = {true, s.tf};
+  return plan;
+}
+
 }  // namespace
 
 size_t nvfp4_f16_bytes(int M, int N, int Kp, bool grouped) {
-  return (size_t)(grouped || M <= N ? M : N) * Kp * 2;
+  return (size_t)(f16_plan(M, N, grouped).codes_w ? M : N) * Kp * 2;
 }
 
 // (Experts: the tiles are known on the device alone; from 512 rows per expert on, and where the most tiles that the rows can make are
@@ -442,17 +492,23 @@ size_t nvfp4_split_bytes(int M, int N, int Kp, int n_seg) {
   return 512 * F16Shape<true>::kSlot * sizeof(float4);
 }
 
+size_t nvfp4_split_operand_bytes(int M, int N, int Kp, bool grouped) { return (size_t)(grouped || M <= N ? M : N) * Kp * 2; }
+
 int run_nvfp4_f16(GemmParams p, void *workspace, hipStream_t st, bool split) {
-  const bool codes_w = p.seg || p.M <= p.N;
-  const int rows = codes_w ? p.M : p.N;
+  const F16Plan plan = split ? F16Plan{p.seg || p.M <= p.N, 8} : f16_plan(p.M, p.N, p.seg != nullptr);
+  const int rows = plan.codes_w ? p.M : p.N;
   const size_t dwords = (size_t)rows * (p.Kp >> 3);
   hipLaunchKernelGGL(nvfp4_decode_f16_kernel, dim3((unsigned)((dwords + 1023) / 1024)), dim3(256), 0, st,
-                     reinterpret_cast<const uint32_t *>(codes_w ? p.a_codes : p.b_codes), codes_w ? p.a_scales : p.b_scales,
+                     reinterpret_cast<const uint32_t *>(plan.codes_w ? p.a_codes : p.b_codes), plan.codes_w ? p.a_scales : p.b_scales,
                      static_cast<uint4 *>(workspace), dwords);
   ARCQ_HIP_TRY(hipGetLastError());
   p.f16 = static_cast<const uint16_t *>(workspace);
-  if (split) p.split = reinterpret_cast<float4 *>(static_cast<uint8_t *>(workspace) + nvfp4_f16_bytes(p.M, p.N, p.Kp, p.seg != nullptr));
-  return codes_w ? launch<true>(p, split, st) : launch<false>(p, split, st);
+  if (split) {
+    p.split = reinterpret_cast<float4 *>(static_cast<uint8_t *>(workspace) + nvfp4_split_operand_bytes(p.M, p.N, p.Kp, p.seg != nullptr));
+    return plan.codes_w ? launch_split<true>(p, st) : launch_split<false>(p, st);
+  }
+  if (!plan.codes_w) return launch_tiles<false, 8>(p, st);
+  return plan.tf == 8 ? launch_tiles<true, 8>(p, st) : plan.tf == 6 ? launch_tiles<true, 6>(p, st) : launch_tiles<true, 4>(p, st);
 }
 
 }  // namespace arcq

@@ -47,8 +47,7 @@ struct GemmParams {
   int swiglu = 0;
   uint32_t *absmax_bits = nullptr;
   int seg_index = 0;
-  // gemm_nvfp4_f16: one operand decoded to fp16 [rows, K'] ahead of the launch (the activations, or the weights
-  // where they have fewer rows)
+  // gemm_nvfp4_f16: one operand decoded to fp16 [rows, K'] ahead of the launch
   const uint16_t *f16 = nullptr;
   // gemm_nvfp4_f16 with its last round of tiles cut along K: the workgroups' fp32 sums of parts of tiles, two slots each
   float4 *split = nullptr;
@@ -62,8 +61,9 @@ struct GemmParams {
 // arcq_gemm_nv.hip: bytes of the decoded operand, and the GEMM on it
 size_t nvfp4_f16_bytes(int M, int N, int Kp, bool grouped);
 int run_nvfp4_f16(GemmParams p, void *workspace, hipStream_t st, bool split);
-// scratch of the same with its last round cut along K, 0 where that does not pay
+// scratch of the same with its last round cut along K behind the decoded operand, 0 where that does not pay
 size_t nvfp4_split_bytes(int M, int N, int Kp, int n_seg);
+size_t nvfp4_split_operand_bytes(int M, int N, int Kp, bool grouped);
 
 // arcq_gemm_nv_stream.hip: decode batches, plain (n_seg = 0, M <= 64) and grouped
 bool nvfp4_stream_able(int M, int Kp, int n_seg);

@@ -212,7 +212,7 @@ int arcq_matmul_add(const void *a_codes, const void *a_scales, const void *b_cod
  *                                the product: the same exact products in fp32 sums of another order, so that
  *                                results may differ by one bf16 rounding from this call's and are those of
  *                                arcq_matmul, arcq_matmul_noalloc and the other entry points, bit for bit.
- * NVFP4 problems of many rows use it: the operand with fewer rows is decoded to fp16 there once, instead of by every
+ * NVFP4 problems of many rows use it: one operand (the one with fewer rows as a rule) is decoded to fp16 there once, instead of by every
  * workgroup that multiplies it.  Fields that do not apply are 0 / NULL; n_seg > 0 makes it a grouped GEMM.
  */
 typedef struct arcq_gemm_args {

@@ -524,3 +524,66 @@ def test_nvfp4_captured_without_scratch(agemm, oracle, M, N, kp):
         torch.cuda.synchronize()
         assert rel_fro(y.float(), want) < 2.5e-3
         assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
+
+
+@pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
+@pytest.mark.parametrize("M,N,kp,decoded", [
+    (70, 49160, 512, 70), (128, 49152, 640, 128),                                   # tiles of 128 activation rows
+    (300, 22100, 512, 300), (385, 24576, 768, 385), (192, 33000, 640, 192),         # of 192, the last one of 108, 1 and 192
+    (3900, 4096, 512, 3900), (3960, 4090, 640, 3960), (4020, 4096, 512, 4020), (4090, 4096, 512, 4090),   # of 256: 60, 120, 180, 250
+    (3841, 4096, 512, 3841), (5331, 3584, 640, 5331), (4096, 3584, 512, 3584)])     # more rows than weights: either one decoded
+def test_nvfp4_decoded_ahead_tiles(agemm, oracle, M, N, kp, decoded):
+    """Every tile of the kernel on one operand decoded ahead, and every smaller one that the last rows take: against the kernels
+    without a workspace (exact products, sums in another order: one bf16 rounding at most), the residual exactly, and some rows
+    against the 64-bit product."""
+    import ctypes
+    from arcquant_amd import _lib
+    L = _lib.lib()
+    assert L.arcq_gemm_route(M, N, kp, 0, 0, 0) == 1 and L.arcq_gemm_workspace_bytes(M, N, kp, 0, 0) == 2 * decoded * kp
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    codes = lambda rows: (torch.randint(0, 256, (rows, kp // 2), generator=g, device="cuda", dtype=torch.uint8),
+                          torch.randint(60, 90, (rows * (kp // 16),), generator=g, device="cuda", dtype=torch.uint8))
+    (a, sfa), (b, sfb) = codes(M), codes(N)
+    res = torch.randn(M, N, generator=g, device="cuda").to(torch.bfloat16)
+    out = []
+    for residual, nbytes in ((None, 2 * decoded * kp), (None, 0), (res, 2 * decoded * kp)):
+        c = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+        work = torch.full((nbytes,), 0xff, dtype=torch.uint8, device="cuda") if nbytes else None
+        args = _lib.GemmArgs(a.data_ptr(), sfa.data_ptr(), b.data_ptr(), sfb.data_ptr(), M, N, kp, 0, 2.0 ** -9, 0, None, None,
+                             None if residual is None else residual.data_ptr(), c.data_ptr(), None, 0, None,
+                             None if work is None else work.data_ptr(), nbytes)
+        assert L.arcq_gemm(args, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        out.append(c)
+    assert rel_fro(out[0].float(), out[1].float()) < 1e-3
+    assert torch.allclose(out[0].float(), out[1].float(), rtol=2 ** -7, atol=1e-4 * float(out[1].float().abs().max()))
+    assert torch.equal(out[2], out[0] + res)
+    rows = torch.tensor([0, min(127, M - 1), M // 2, M - 1])
+    da = oracle_dq(oracle, a[rows.cuda()], sfa.view(M, -1)[rows.cuda()].reshape(-1), "NVFP4").double()
+    want = da @ oracle_dq(oracle, b, sfb, "NVFP4").double().T * 2.0 ** -9
+    assert rel_fro(out[0][rows.cuda()].float(), want) < 2.5e-3
+
+
+@pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
+@pytest.mark.parametrize("counts", [[830, 40, 2130], [1000, 950, 0, 1122], [2304, 1, 191, 1088]])
+def test_nvfp4_decoded_ahead_tiles_of_experts(agemm, counts):
+    """experts that end in a tile of 64, 128, 192 or 256 rows: each as a GEMM of its own (other tiles: one bf16 rounding at most),
+    and the fused SwiGLU epilogue's bits and maxima from the plain one's output"""
+    E, M, N, kp = len(counts), sum(counts), 6160, 512
+    g = torch.Generator(device="cuda").manual_seed(M)
+    codes = lambda rows: (torch.randint(0, 256, (rows, kp // 2), generator=g, device="cuda", dtype=torch.uint8),
+                          torch.randint(40, 60, (rows * (kp // 16),), generator=g, device="cuda", dtype=torch.uint8))
+    (a, sfa), (b, sfb) = codes(M), codes(E * N)
+    b, seg = b.view(E, N, -1), torch.tensor([0] + list(np.cumsum(counts)), dtype=torch.int32, device="cuda")
+    y = agemm.grouped_matmul(a, b, sfa, sfb, seg)
+    t, scales = agemm.grouped_matmul_swiglu(a, b, sfa, sfb, seg, tensor_scale=True)
+    assert torch.equal(t, torch.nn.functional.silu(y[:, 0::2]) * y[:, 1::2])
+    at = 0
+    for e, n in enumerate(counts):
+        if n == 0:
+            assert float(scales[e]) == 1.0
+            continue
+        rows = slice(at, at + n)
+        one = agemm.matmul(a[rows], b[e], sfa.view(M, -1)[rows].reshape(-1), sfb.view(E, -1)[e], 1.0)
+        assert rel_fro(y[rows].float(), one.float()) < 1e-3
+        assert float(scales[e]) == float(t[rows].abs().max().float().cpu() / torch.tensor(2688.0))
+        at += n
