@@ -995,11 +995,11 @@ struct GemmPlan {
 // the largest scratch the plan ever asks for (the stream workspaces are this big)
 constexpr size_t kSplitMaxBytes = kWorkspaceBytes[kWsSplitK];
 
-// The 256x256 MXFP4 tile: with a long K the ping-pong kernel (88, arcq_gemm_mx.hip), whose main loop is faster, else the one
-// that requests the next stage from one wave per SIMD (84), which gets in and out of a tile faster where that decides (grouped
-// launches; 2048 x 28672).  88's time against 84's, each forced for the whole of a process, whole and ragged problems of 2048 to
-// 16384 rows: K' = 19072 0.83-0.93, 14592 0.87-1.01, 11264 0.84-1.01, 9216 0.83-1.01, 8192 0.82-1.01, 2176 to 5248, ragged ones
-// (700 to 7300 rows), 0.93-1.10.
+// The 256x256 MXFP4 tile: the ping-pong kernel (88, arcq_gemm_mx.hip), whose main loop is faster, except where a short K or a
+// SwiGLU epilogue makes getting in and out of a tile decide: then the one that requests the next stage from one wave per SIMD (84).  88's
+// time against 84's, whole and ragged problems of 700 to 8192 rows: K' = 14592 0.92, 8064 0.83-0.96, 6272 0.85-0.98, 4352 0.88-0.99,
+// 3712 0.89-0.99, 2176 0.93-1.00, 1152 0.93-1.03, 640 0.91-1.07, 512 1.00-1.13.  (The plan names 88 from K' = 8192 on.)
+constexpr int kPingPongFrom = 2176;
 int large_mx_tile(int kernel, int Kp) { return kernel == 84 && Kp >= 8192 ? 88 : kernel; }
 
 // The eight-wave MXFP4 kernels address an operand's rows with 32-bit byte offsets from its base; beyond, the four-wave tile
@@ -1172,16 +1172,18 @@ int run_gemm(GemmParams p, const GemmPlan &plan, int fmt, float *scratch, hipStr
   if (plan.kernel == 1)
     return fmt == ARCQ_FMT_MXFP4 ? launch_skinny_for<ARCQ_FMT_MXFP4>(p, st) : launch_skinny_for<ARCQ_FMT_NVFP4>(p, st);
   if (fmt == ARCQ_FMT_MXFP4) {
-    // persistent workgroups: plain launches over whole tiles
-    // and more of them than one round of workgroups: with a single tile per CU there is nothing to overlap
-    // (gate_up at M = 4096, seven tiles per CU: 333 -> 325 us; qkv, one and a half: 77.5 -> 74.9; one round: 1-3 % slower)
+    // persistent workgroups (K' below kPingPongFrom): plain launches over whole tiles, and more of them than one round of workgroups:
+    // with a single tile per CU there is nothing to overlap (28672 x 4352, seven tiles per CU: 333 -> 325 us; 6144 x 4352, one and a
+    // half: 77.5 -> 74.9; one round: 1-3 % slower)
     const bool persist = !p.seg && !p.swiglu && tuning().gemm_persist != 0 && p.M % 256 == 0 && p.N % 256 == 0 &&
                          (long)(p.M / 256) * (p.N / 256) > 256;
     switch (addressable_tile(plan.kernel, p.M, p.N, p.Kp)) {
       case 88: return run_mxfp4_pingpong(p, st);
       case 44: return launch_mxfp4_tiled<4, 4>(p, st);
       // 256x256 tile, eight waves of 128x64, and 256x128 tile, eight waves of 128x32
-      case 84: return persist ? launch_mxfp4_persistent<4, 2>(p, st) : launch_mxfp4_tiled<4, 2, 2, 4>(p, st);
+      case 84:
+        if (!p.seg && !p.swiglu && p.Kp >= kPingPongFrom && tuning().gemm_kernel != 84) return run_mxfp4_pingpong(p, st);
+        return persist ? launch_mxfp4_persistent<4, 2>(p, st) : launch_mxfp4_tiled<4, 2, 2, 4>(p, st);
       case 82: return launch_mxfp4_tiled<4, 1, 2, 4>(p, st);
       case 42: return launch_mxfp4_tiled<4, 2>(p, st);
       case 224: return launch_mxfp4_tiled<2, 2, 4>(p, st);

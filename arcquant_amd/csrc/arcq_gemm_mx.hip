@@ -17,10 +17,16 @@ namespace {
 // compute phases (32 MFMAs, nothing else); the second group starts one phase late, so that one wave of every SIMD
 // multiplies while the other one reads, with a barrier between phases.
 //
+// What bounds it is the longer of the two phases: 512 cycles of MFMAs, and in the other one what a lone wave can issue, an
+// instruction every 5 to 9 cycles.  So a memory phase holds LDS reads and requests and next to nothing else: scale bytes are read a
+// stage ahead, two tiles per instruction, and taken apart between the MFMAs, addresses are formed there too, and stages come in
+// pairs so that their places in LDS are constants.  (With scale bytes read and taken apart where they are used, and addresses formed
+// where the requests are, 30 scalar and 12 vector instructions more: 2048 x 2048 x 14592, 64 workgroups, 84 us, so 69.5, the MFMAs and
+// barriers alone 57; 4096 x 4096 x 14592 111 / 102.5, 16384 x 28672 x 4352 1144 / 1066.)
+//
 // The matrix instruction is 16x16x128: a register-only loop of it sustains 7.0-7.2 PFLOP/s on random codes against 5.8-6.3 for
 // 32x32x64 (one and two waves per SIMD, arcq_mfma_rate_probe), the upper figure when the tiles are walked back and forth, so
-// that neighbouring instructions share an operand.  4096 x 4096 x 14592: 112-116 us, 4.2-4.4 PFLOP/s, one round of tiles (the
-// matrix pipe is busy for half of the cycles); against the kernel with 32x32x64: 116 / 120 us, 16384 rows 456 / 503.
+// that neighbouring instructions share an operand.  4096 x 4096 x 14592: 102-105 us, 4.6-4.8 PFLOP/s, one round of tiles.
 //
 // A stage has two phases: all activations with weight rows 0-63 of the wave, then with rows 64-127.  The activations and
 // the first half of the weights leave LDS in the first phase, so their buffers are requested again in the second one: two
@@ -29,7 +35,7 @@ namespace {
 //
 // LDS rows are 128 bytes of codes = 8 chunks, swizzled as the fp16 tile of the NVFP4 kernel (chunk ^ stage_swizzle(row)), and
 // windows of 16 scale bytes for two stages, the last of which ends with the row.  Lanes 16 g .. 16 g + 15 hold K blocks 2 g
-// and 2 g + 1 of the stage: their two scale bytes are one 16-bit read and picked by op_sel.
+// and 2 g + 1 of the stage: their two scale bytes are half of a dword and picked by op_sel.
 // Requires K' % 128 == 0, K' >= 512.
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
@@ -37,7 +43,7 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
   constexpr int kCodes = 2 * BT * 128, kScales = 2 * 2 * BT * 16;
   constexpr int kRegion = 128 * 64 * 2;
   static_assert(8 * kRegion <= 2 * kCodes, "the epilogue's transpose");
-  // weights, activations, scale bytes (512 rows per window; a lane without a block may read up to 4 bytes past its row)
+  // weights, activations, scale bytes (512 rows per window; those read behind the last stage may begin 12 bytes past their row)
   __shared__ uint4 smem[(2 * kCodes + kScales) / 16 + 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -57,7 +63,7 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
   const int n_base = (in_band / bw) * BT, m_base = (4 * band + in_band % bw) * BT;
 
   const int ns = (p.Kp + 255) >> 8;                 // stages
-  const bool short_last = (p.Kp & 255) != 0;        // the last one then has blocks 0..3 only
+  const bool short_last = (p.Kp & 255) != 0;        // the last one then has blocks 4..7 only
   const int nw = (ns + 1) >> 1, s_shift = 16 * nw - ksc;
 
   // ---- global -> LDS
@@ -73,18 +79,14 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
   const uint32_t svo = (uint32_t)(group ? min(m_base + 64 * pos + lane, p.M - 1) : min(n_base + 64 * pos + lane, p.N - 1)) * (uint32_t)ksc;
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(smem);
   // requests behind the last stage fetch it again into buffers that nobody reads any more: the number of loads on their
-  // way is the same in every stage.  A short last stage has chunks 0..3: those twice.
-  auto request_codes = [&](const uint8_t *codes, const uint32_t *vo, int area, int s, int i) {
-    const int sf = min(s, ns - 1);
-    const uint32_t back = short_last && sf == ns - 1 && ld_q >= 4 ? 64u : 0u;
-    lds_dma16_at(codes + (size_t)sf * 128, vo[i] - back, lds0 + area + (s & 1) * (BT * 128) + i * 8192 + wave * 1024);
-  };
-  auto request_x = [&](int s, int i) { request_codes(p.a_codes, xvo, kCodes, s, i); };
-  auto request_w = [&](int s, int i) { request_codes(p.b_codes, wvo, 0, s, i); };  // i even: first phase's rows, odd: second's
-  auto request_scales = [&](int w) {
-    const int wf = min(w, nw - 1);
-    lds_dma16_at(sbase + wf * 16 - (wf == nw - 1 ? s_shift : 0), svo, lds0 + 2 * kCodes + (w & 1) * (2 * BT * 16) + wave * 1024);
-  };
+  // way is the same in every stage.  A short last stage is the row's last 256 elements, the first half of which the stage before it has.
+  const int last_at = kbytes - 128;
+  auto stage_at = [&](int s) { return min(s * 128, last_at); };
+  auto request_x = [&](const uint8_t *x, int odd, int i) { lds_dma16_at(x, xvo[i], lds0 + wave * 1024, kCodes + odd * (BT * 128) + i * 8192); };
+  // i even: first phase's rows, odd: second's
+  auto request_w = [&](const uint8_t *w, int odd, int i) { lds_dma16_at(w, wvo[i], lds0 + wave * 1024, odd * (BT * 128) + i * 8192); };
+  auto window_at = [&](int w) { return min(w * 16, ksc - 16); };  // the last window ends with the row
+  auto request_scales = [&](const uint8_t *window, uint32_t at) { lds_dma16_at(window, svo, at, 2 * kCodes); };
 
   // ---- LDS -> operands
   const int r = lane & 15, g = lane >> 4;
@@ -96,12 +98,13 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
     w_rd[h] = lds + (128 * group + r) * 128 + c;
     x_rd[h] = lds + kCodes + (64 * pos + r) * 128 + c;
   }
-  const uint8_t *ws_rd = lds + 2 * kCodes + (128 * group + r) * 16 + 4 * (g >> 1);
-  const uint8_t *xs_rd = lds + 2 * kCodes + BT * 16 + (64 * pos + r) * 16 + 4 * (g >> 1);
+  const uint32_t ws_rd = 2 * kCodes + (128 * group + r) * 16 + 4 * (g >> 1);
+  const uint32_t xs_rd = 2 * kCodes + BT * 16 + (64 * pos + r) * 16 + 4 * (g >> 1);
   const int s_half = 16 * (g & 1);
 
   uint4 wq[4][2], xq[4][2];
-  int ws[4], xs[4];
+  int wr[8], xr[4];          // scale bytes of a stage as they are in LDS
+  int ws[2][4], xs[4];       // and this lane's two of each, by half of the weights
   v4f acc[8][4];
 #pragma unroll
   for (auto &a : acc)
@@ -115,12 +118,25 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("" ::: "memory");
   };
-  auto scale_offset = [&](int s) { return ((s >> 1) & 1) * (2 * BT * 16) + 8 * (s & 1) + ((s >> 1) == nw - 1 ? s_shift : 0); };
-  auto read_w = [&](int s, int so, int t, int i) {
-    wq[i][0] = *reinterpret_cast<const uint4 *>(w_rd[0] + (s & 1) * (BT * 128) + t * 2048);
-    wq[i][1] = *reinterpret_cast<const uint4 *>(w_rd[1] + (s & 1) * (BT * 128) + t * 2048);
-    ws[i] = *reinterpret_cast<const int *>(ws_rd + so + t * 256);
+  auto scale_offset = [&](int s) {
+    return ((s >> 1) & 1) * (2 * BT * 16) + 8 * (s & 1) + ((s >> 1) == nw - 1 ? s_shift : 0) - (short_last && s == ns - 1 ? 4 : 0);
   };
+  auto read_w = [&](int odd, int t, int i) {
+    wq[i][0] = *reinterpret_cast<const uint4 *>(w_rd[0] + odd * (BT * 128) + t * 2048);
+    wq[i][1] = *reinterpret_cast<const uint4 *>(w_rd[1] + odd * (BT * 128) + t * 2048);
+  };
+  auto read_scales = [&](uint32_t ws_at, uint32_t xs_at, int part) {  // of the activations and of the two halves of the weights: four tiles each
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (part == 0)
+        xr[i] = *reinterpret_cast<const int *>(lds + xs_at + i * 256);
+      else
+        wr[4 * part - 4 + i] = *reinterpret_cast<const int *>(lds + ws_at + (4 * part - 4 + i) * 256);
+    }
+  };
+  // lanes without blocks (g < 2 of a short last stage): both scales 2^-127, so that whatever codes they hold multiply to
+  // less than half the smallest number
+  auto present = [&](int s) { return short_last && s == ns - 1 && g < 2 ? 0 : 16; };
   auto multiply = [&](auto half_t) {
     constexpr int W0 = decltype(half_t)::value * 4;
 #pragma unroll
@@ -129,7 +145,7 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
       for (int t = 0; t < 4; ++t) {
         const int i = j & 1 ? 3 - t : t;
         acc[W0 + i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fp4_operand(wq[i][0]), fp4_operand(xq[j][0]), acc[W0 + i][j],
-                                                                         4, 4, 0, ws[i], 0, xs[j]);
+                                                                         4, 4, 0, ws[W0 >> 2][i], 0, xs[j]);
       }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
@@ -137,67 +153,100 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
       for (int t = 0; t < 4; ++t) {
         const int i = j & 1 ? 3 - t : t;
         acc[W0 + i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fp4_operand(wq[i][1]), fp4_operand(xq[j][1]), acc[W0 + i][j],
-                                                                         4, 4, 1, ws[i], 1, xs[j]);
+                                                                         4, 4, 1, ws[W0 >> 2][i], 1, xs[j]);
       }
   };
 
   // in the order of the steady state, so that the same wait counts apply
-  request_scales(0);
-  request_w(0, 1);
-  request_w(0, 3);
+  request_scales(sbase, lds0 + wave * 1024);
+  request_w(p.b_codes, 0, 1);
+  request_w(p.b_codes, 0, 3);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) request_x(0, i);
-  request_w(0, 0);
-  request_w(0, 2);
+  for (int i = 0; i < 4; ++i) request_x(p.a_codes, 0, i);
+  request_w(p.b_codes, 0, 0);
+  request_w(p.b_codes, 0, 2);
+  const uint8_t *x_next = p.a_codes + stage_at(1), *w_next = p.b_codes + stage_at(1);  // of the stage requested next
 #pragma unroll
-  for (int i = 0; i < 4; ++i) request_x(1, i);
-  request_w(1, 0);
-  request_w(1, 2);
+  for (int i = 0; i < 4; ++i) request_x(x_next, 1, i);
+  request_w(w_next, 1, 0);
+  request_w(w_next, 1, 2);
   asm volatile("s_waitcnt vmcnt(6)" ::: "memory");  // stage 0
   barrier();
+#pragma unroll
+  for (int i = 0; i < 3; ++i) read_scales(ws_rd + scale_offset(0), xs_rd + scale_offset(0), i);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    xs[i] = __builtin_amdgcn_ubfe(xr[i], s_half, 16);
+    ws[0][i] = __builtin_amdgcn_ubfe(wr[i], s_half, 16);
+  }
   if (group) barrier();  // the second group runs one phase behind
 
-  for (int s = 0; s < ns; ++s) {
-    const int so = scale_offset(s);
-    // lanes without blocks (g >= 2 of a short last stage): both scales 2^-127, so that whatever codes they hold multiply to
-    // less than half the smallest number
-    const int present = short_last && s == ns - 1 && g >= 2 ? 0 : 16;
+  const uint8_t *scales_next = sbase + window_at(1);   // of the window requested next, and its place
+  uint32_t scales_to = lds0 + wave * 1024 + 2 * BT * 16;
+  // What a memory phase needs of scalars is formed in the compute phase before it: there they are free.
+  auto stage = [&](int s, auto odd_t) {
+    constexpr int ODD = decltype(odd_t)::value;
     // first phase: activations and the first half of the weights
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      xq[i][0] = *reinterpret_cast<const uint4 *>(x_rd[0] + (s & 1) * (BT * 128) + i * 2048);
-      xq[i][1] = *reinterpret_cast<const uint4 *>(x_rd[1] + (s & 1) * (BT * 128) + i * 2048);
-      xs[i] = *reinterpret_cast<const int *>(xs_rd + so + i * 256);
-      read_w(s, so, i, i);
-      if (i == 0 && !(s & 1)) request_scales((s >> 1) + 1);
-      if (i == 1) request_w(s + 1, 1);
-      if (i == 2) request_w(s + 1, 3);
+      xq[i][0] = *reinterpret_cast<const uint4 *>(x_rd[0] + ODD * (BT * 128) + i * 2048);
+      xq[i][1] = *reinterpret_cast<const uint4 *>(x_rd[1] + ODD * (BT * 128) + i * 2048);
+      read_w(ODD, i, i);
+      if (i == 0 && !ODD) request_scales(scales_next, scales_to);
+      if (i == 1) request_w(w_next, 1 - ODD, 1);
+      if (i == 2) request_w(w_next, 1 - ODD, 3);
       __builtin_amdgcn_sched_barrier(0);
     }
     // the second half of this stage's weights has to be there behind this barrier (the counts leave out the scale load of an
     // even stage, which then may be waited for a little early)
     asm volatile("s_waitcnt lgkmcnt(0) vmcnt(8)" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < 4; ++i) xs[i] = __builtin_amdgcn_ubfe(xs[i], s_half, present), ws[i] = __builtin_amdgcn_ubfe(ws[i], s_half, present);
     barrier();
     multiply(std::integral_constant<int, 0>{});
+    const int here = present(s);
+    const uint32_t so = scale_offset(s + 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) ws[1][i] = __builtin_amdgcn_ubfe(wr[4 + i], s_half, here);  // the scales of the second half
+    x_next = p.a_codes + stage_at(s + 2), w_next = p.b_codes + stage_at(s + 2);
+    uint32_t ws_at = ws_rd + so, xs_at = xs_rd + so;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(ws[1][i]));
+    asm volatile("" : "+s"(x_next), "+s"(w_next), "+v"(ws_at), "+v"(xs_at));
     barrier();
-    // second phase: the second half of the weights
+    // second phase: the second half of the weights, and the next stage's scale bytes (behind the last stage: not used)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      read_w(s, so, 4 + i, i);
-      request_x(s + 2, i);
-      if (i & 1) request_w(s + 2, i - 1);
+      read_w(ODD, 4 + i, i);
+      if (i < 3) read_scales(ws_at, xs_at, i);
+      request_x(x_next, ODD, i);
+      if (i & 1) request_w(w_next, ODD, i - 1);
       __builtin_amdgcn_sched_barrier(0);
     }
     // the next stage's activations and first half of the weights
     asm volatile("s_waitcnt lgkmcnt(0) vmcnt(8)" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ws[i] = __builtin_amdgcn_ubfe(ws[i], s_half, present);
     barrier();
     multiply(std::integral_constant<int, 1>{});
+    const int next = present(s + 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      ws[0][i] = __builtin_amdgcn_ubfe(wr[i], s_half, next);
+      xs[i] = __builtin_amdgcn_ubfe(xr[i], s_half, next);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(ws[0][i]), "+v"(xs[i]));
+    if (ODD) {
+      scales_next = sbase + window_at((s + 3) >> 1);
+      scales_to = lds0 + wave * 1024 + ((s + 3) >> 1 & 1) * (2 * BT * 16);
+      asm volatile("" : "+s"(scales_next), "+s"(scales_to));
+    }
     barrier();
+  };
+  int s = 0;
+  for (; s + 1 < ns; s += 2) {
+    stage(s, std::integral_constant<int, 0>{});
+    stage(s + 1, std::integral_constant<int, 1>{});
   }
+  if (s < ns) stage(s, std::integral_constant<int, 0>{});
   if (!group) barrier();
   store_wave_tile(p, Acc16<8, 4>{acc}, reinterpret_cast<uint8_t *>(smem) + wave * kRegion, m_base + 64 * pos, n_base + 128 * group, lane);
 }

@@ -244,6 +244,14 @@ __device__ __forceinline__ void lds_dma16_at(const void *base, uint32_t lane_off
                : "memory");
 }
 
+// And with a constant part of the LDS address: one scalar instruction forms M0.
+__device__ __forceinline__ void lds_dma16_at(const void *base, uint32_t lane_offset, uint32_t lds_wave_base, int lds_offset) {
+  asm volatile("s_add_u32 m0, %0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+               :
+               : "s"(lds_wave_base), "v"(lane_offset), "s"(base), "i"(lds_offset)
+               : "memory", "scc");
+}
+
 __device__ __forceinline__ void lds_dma4_at(const void *base, uint32_t lane_offset, uint32_t lds_wave_base) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
                :
