@@ -15,6 +15,7 @@ HEADER_PATH = os.path.join(_HERE, "..", "include", "arcq.h")
 NVFP4 = 0
 MXFP4 = 1
 FORMATS = {"NVFP4": NVFP4, "MXFP4": MXFP4}
+SWIGLU_HALVES = 2                        # ARCQ_SWIGLU_HALVES
 
 _lib = None
 
@@ -105,6 +106,8 @@ def lib() -> ctypes.CDLL:
     L.arcq_gemm_workspace_bytes.restype = sz
     L.arcq_gemm_scratch_bytes.argtypes = [i, i, i, i, i]
     L.arcq_gemm_scratch_bytes.restype = sz
+    L.arcq_gemm_swiglu_halves.argtypes = [i, i, i, i]
+    L.arcq_gemm_swiglu_halves.restype = i
     L.arcq_gemm_kernel.argtypes = [i, i, i, i, i, i]
     L.arcq_gemm_kernel.restype = i
     L.arcq_gemm_route.argtypes = [i, i, i, i, i, i]

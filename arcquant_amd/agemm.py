@@ -239,6 +239,8 @@ def _gemm(A, SFA, B, SFB, M, N, Kp, f, c, *, alpha=1.0, da=None, db=None, residu
             break
         except torch.OutOfMemoryError:
             pass
+    if swiglu == _lib.SWIGLU_HALVES and f == _lib.NVFP4 and work is None:
+        return False
     args = _lib.GemmArgs(A.data_ptr(), SFA.data_ptr(), B.data_ptr(), SFB.data_ptr(), M, N, Kp, f, alpha, swiglu, da, db,
                          None if residual is None else residual.data_ptr(), c.data_ptr(),
                          None if seg is None else seg.data_ptr(), n_seg, None if absmax is None else absmax.data_ptr(),
@@ -248,6 +250,7 @@ def _gemm(A, SFA, B, SFB, M, N, Kp, f, c, *, alpha=1.0, da=None, db=None, residu
             _lib.check(L.arcq_gemm(args, _stream(A)), "arcq_gemm")
         else:
             _lib.check(L.arcq_gemm_parts(args, parts, _stream(A)), "arcq_gemm_parts")
+    return True
 
 
 def matmul(A, B, SFA, SFB, scale, *, fmt=None, residual=None):
@@ -308,11 +311,12 @@ def matmul(A, B, SFA, SFB, scale, *, fmt=None, residual=None):
     return C
 
 
-def matmul_parts(A, B, SFA, SFB, scale, part_rows, part_scales, *, fmt, bias=None):
+def matmul_parts(A, B, SFA, SFB, scale, part_rows, part_scales, *, fmt, bias=None, swiglu=False, tensor_scale=False):
     """Several linears over one quantized input in one launch: B u8 [N, K'/2] and SFB hold the parts' quantized weights one behind
     the other (q | k | v), part_rows[k] rows each, with the tensor scales part_scales[k] (0-dim fp32 CUDA tensors); scale: the
     input's (float or 0-dim fp32 CUDA tensor).  bf16 [M, N], what torch.cat of the parts' ``matmul(..., (scale, part_scales[k]))`` is
-    (sums in another order: one bf16 rounding at most), plus ``bias`` bf16 [N] where given, added in bf16."""
+    (sums in another order: one bf16 rounding at most), plus ``bias`` bf16 [N] where given, added in bf16.
+    swiglu=True (gate | up, no bias, where swiglu_halves_pay): matmul_swiglu(halves=True) of the two."""
     _require(A, "A", torch.uint8, 2)
     _require(B, "B", torch.uint8, 2)
     _require(SFA, "SFA", torch.uint8)
@@ -340,10 +344,28 @@ def matmul_parts(A, B, SFA, SFB, scale, part_rows, part_scales, *, fmt, bias=Non
             raise RuntimeError(f"bias must be bf16 [{N}] on the operands' device")
         parts.bias = bias.data_ptr()
     alpha, da, keep = _scalar(scale, A.device)
+    if swiglu:
+        return _swiglu_halves(A, SFA, B, SFB, M, N, Kp, f, tensor_scale, alpha=alpha, da=da, parts=parts)
     C = torch.empty((M, N), dtype=torch.bfloat16, device=A.device)
     _gemm(A, SFA, B, SFB, M, N, Kp, f, C, alpha=alpha, da=da, parts=parts)
     del keep
     return C
+
+
+@functools.lru_cache(maxsize=4096)
+def swiglu_halves_pay(M, N, Kp, fmt):
+    """whether matmul_swiglu(halves=True) takes a problem: those of many rows, where the pass over the projection's output that it saves is
+    more than its epilogue costs (us, GEMM and SwiGLU quantizer, and GEMM with the epilogue and plain quantizer: NVFP4 16384 x 28672 x
+    4352 3170 and 2870, 2331 x 37888 x 3712 600 and 535, MXFP4 4096 x 28672 x 4352 341 and 318)"""
+    return bool(_lib.lib().arcq_gemm_swiglu_halves(M, N, Kp, _fmt_id(fmt)))
+
+
+def _swiglu_halves(A, SFA, B, SFB, M, N, Kp, f, tensor_scale, **kw):
+    T = torch.empty((M, N // 2), dtype=torch.bfloat16, device=A.device)
+    amax = torch.zeros(1, dtype=torch.float32, device=A.device) if tensor_scale else None
+    if not _gemm(A, SFA, B, SFB, M, N, Kp, f, T, swiglu=_lib.SWIGLU_HALVES, absmax=amax, **kw):
+        return None
+    return (T, _absmax_to_scales(amax, 2688.0).reshape(())) if tensor_scale else T
 
 
 @functools.lru_cache(maxsize=4096)
@@ -523,12 +545,15 @@ def _absmax_to_scales(buf, divisor):
     return buf
 
 
-def matmul_swiglu(A, B, SFA, SFB, scale, *, fmt=None, tensor_scale=False):
+def matmul_swiglu(A, B, SFA, SFB, scale, *, fmt=None, tensor_scale=False, halves=False):
     """matmul for a fused gate/up projection whose weight rows alternate gate, up (interleave_gate_up), with
     act_fn(gate) * up formed in the epilogue: returns t bf16 [M, N/2], bit-identical to
     ``h = matmul(...); F.silu(h_gate) * h_up`` in bf16 (where matmul takes another kernel, NVFP4 decode batches, h's sums are in
     another order), without h going through memory.  tensor_scale=True
-    also returns the NVFP4 tensor scale max|t| / 2688 of t (0-dim fp32 device tensor, 1 for all zeros)."""
+    also returns the NVFP4 tensor scale max|t| / 2688 of t (0-dim fp32 device tensor, 1 for all zeros).
+    halves=True: the weights as they are, gate rows and then up rows, for the problems that swiglu_halves_pay says; None where there is
+    no memory for the scratch that such a GEMM takes.  (Where its last round of tiles is cut along K, other columns are in it than in
+    matmul's, whose sums are then in another order.)"""
     _require(A, "A", torch.uint8, 2)
     _require(B, "B", torch.uint8, 2)
     _require(SFA, "SFA", torch.uint8)
@@ -549,6 +574,8 @@ def matmul_swiglu(A, B, SFA, SFB, scale, *, fmt=None, tensor_scale=False):
     else:
         alpha, da, ka = _scalar(scale, A.device)
         db, kb = None, None
+    if halves:
+        return _swiglu_halves(A, SFA, B, SFB, M, N, Kp, f, tensor_scale, alpha=alpha, da=da, db=db)
     T = torch.empty((M, N // 2), dtype=torch.bfloat16, device=A.device)
     amax = torch.zeros(1, dtype=torch.float32, device=A.device) if tensor_scale else None
     _gemm(A, SFA, B, SFB, M, N, Kp, f, T, alpha=alpha, da=da, db=db, swiglu=1, absmax=amax)

@@ -1466,6 +1466,39 @@ extern "C" int arcq_grouped_matmul_swiglu(const void *a_codes, const void *a_sca
 
 namespace arcq {
 namespace {
+// Weights as they are ([gate; up] along N) with the SwiGLU epilogue: by the kernels for many rows, where the pass over the projection's
+// output that it saves (NVFP4: two, the tensor scale's too) is more than the epilogue costs.  us, plain and with it: NVFP4 16384 x 28672 x 4352
+// 2653 / 2722, the passes over its output 520 / 150; MXFP4 4096 x 28672 x 4352 271 / 290, 70 / 28.  (Grouped MXFP4 launches of
+// interleaved rows keep the kernel with 32x32 MFMAs: 768 / 797.)
+bool swiglu_halves_wanted(int M, int N, int Kp, int fmt) {
+  if (N % 32 != 0 || Kp % 128 != 0 || Kp < 512) return false;
+  if (fmt == ARCQ_FMT_NVFP4) return f16_way(M, N, Kp, fmt, 0, arcq_gemm_scratch_bytes(M, N, Kp, fmt, 0)) != 0;
+  if (tuning().gemm_kernel >= 0 && tuning().gemm_kernel != 88) return false;
+  const int kernel = addressable_tile(plan_gemm(M, N, Kp, fmt, true).kernel, M, N, Kp);
+  return kernel == 88 || (kernel == 84 && Kp >= kPingPongFrom);
+}
+
+int matmul_halves_impl(const arcq_gemm_args *a, const arcq_gemm_parts_args *parts, void *stream) {
+  GemmParams p;
+  const int rc = check_gemm_args(a->a_codes, a->a_scales, a->b_codes, a->b_scales, a->M, a->N, a->Kp, a->fmt, a->alpha, a->d_alpha_a,
+                                 a->d_alpha_b, nullptr, a->c, &p);
+  if (rc != ARCQ_OK || a->M == 0 || a->N == 0) return rc;
+  if (!swiglu_halves_wanted(a->M, a->N, a->Kp, a->fmt)) return ARCQ_ERR_SHAPE;
+  if (parts && (parts->n != 2 || parts->end[0] != a->N / 2 || parts->bias)) return ARCQ_ERR_SHAPE;
+  if (!aligned16(a->a_scales) || !aligned16(a->b_scales)) return ARCQ_ERR_ALIGN;
+  p.swiglu = kSwigluHalves;
+  p.absmax_bits = reinterpret_cast<uint32_t *>(a->d_absmax);
+  if (parts) {
+    p.parts = 2;
+    p.part_end[0] = parts->end[0];
+    p.part_alpha[0] = parts->d_alpha[0], p.part_alpha[1] = parts->d_alpha[1];
+  }
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (a->fmt == ARCQ_FMT_MXFP4) return run_mxfp4_pingpong(p, st);
+  const int way = a->workspace ? f16_way(a->M, a->N, a->Kp, a->fmt, 0, a->workspace_bytes) : 0;
+  return way ? run_nvfp4_f16(p, a->workspace, st, way == 2) : ARCQ_ERR_WORKSPACE;
+}
+
 int matmul_swiglu_impl(const void *a_codes, const void *a_scales, const void *b_codes, const void *b_scales, int M, int N,
                        int Kp, int fmt, float alpha, const float *d_alpha_a, const float *d_alpha_b, void *t, float *d_absmax,
                        void *workspace, size_t workspace_bytes, void *stream) {
@@ -1497,6 +1530,7 @@ extern "C" int arcq_gemm(const arcq_gemm_args *a, void *stream) {
   if (a->workspace && !arcq::aligned16(a->workspace)) return ARCQ_ERR_ALIGN;
   if (a->residual && !arcq::aligned16(a->residual)) return ARCQ_ERR_ALIGN;
   if (a->n_seg < 0 || (a->swiglu && a->residual)) return ARCQ_ERR_SHAPE;
+  if (a->swiglu == ARCQ_SWIGLU_HALVES) return a->n_seg > 0 ? ARCQ_ERR_SHAPE : arcq::matmul_halves_impl(a, nullptr, stream);
   if (a->n_seg > 0)
     return arcq::grouped_matmul_impl(a->a_codes, a->a_scales, a->b_codes, a->b_scales, a->seg_offsets, a->n_seg, a->M, a->N,
                                      a->Kp, a->fmt, a->alpha, a->d_alpha_a, a->d_alpha_b, a->residual, a->c, a->swiglu != 0,
@@ -1512,13 +1546,14 @@ extern "C" int arcq_gemm_parts(const arcq_gemm_args *a, const arcq_gemm_parts_ar
   if (!a || !parts) return ARCQ_ERR_NULL;
   if (a->workspace && !arcq::aligned16(a->workspace)) return ARCQ_ERR_ALIGN;
   if (parts->bias && !arcq::aligned16(parts->bias)) return ARCQ_ERR_ALIGN;
-  if (a->n_seg != 0 || a->swiglu || a->residual || a->d_alpha_b) return ARCQ_ERR_SHAPE;
+  if (a->n_seg != 0 || (a->swiglu && a->swiglu != ARCQ_SWIGLU_HALVES) || a->residual || a->d_alpha_b) return ARCQ_ERR_SHAPE;
   if (parts->n < 1 || parts->n > arcq::kMaxParts) return ARCQ_ERR_SHAPE;
   for (int k = 0; k < parts->n; ++k) {
     if (!parts->d_alpha[k]) return ARCQ_ERR_NULL;
     const int beg = k ? parts->end[k - 1] : 0;
     if (parts->end[k] <= beg || (k + 1 < parts->n ? parts->end[k] % 32 != 0 : parts->end[k] != a->N)) return ARCQ_ERR_SHAPE;
   }
+  if (a->swiglu) return arcq::matmul_halves_impl(a, parts, stream);
   return arcq::matmul_impl(a->a_codes, a->a_scales, a->b_codes, a->b_scales, a->M, a->N, a->Kp, a->fmt, a->alpha, a->d_alpha_a,
                            nullptr, nullptr, a->c, a->workspace, a->workspace_bytes, stream, parts);
 }
@@ -1531,6 +1566,11 @@ extern "C" size_t arcq_gemm_workspace_bytes(int M, int N, int Kp, int fmt, int n
 extern "C" size_t arcq_gemm_scratch_bytes(int M, int N, int Kp, int fmt, int n_seg) {
   if (M <= 0 || N <= 0 || Kp < 64 || n_seg < 0) return 0;
   return std::max(arcq::nvfp4_split_scratch(M, N, Kp, fmt, n_seg), arcq_gemm_workspace_bytes(M, N, Kp, fmt, n_seg));
+}
+
+extern "C" int arcq_gemm_swiglu_halves(int M, int N, int Kp, int fmt) {
+  if ((fmt != ARCQ_FMT_NVFP4 && fmt != ARCQ_FMT_MXFP4) || M <= 0 || N <= 0 || Kp < 64) return 0;
+  return arcq::swiglu_halves_wanted(M, N, Kp, fmt) ? 1 : 0;
 }
 
 extern "C" int arcq_gemm_kernel(int M, int N, int Kp, int fmt, int n_seg, int swiglu) {

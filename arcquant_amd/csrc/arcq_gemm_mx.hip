@@ -72,11 +72,11 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
   const uint32_t ld_q = (lane & 7) ^ stage_swizzle(ld_row);   // (the swizzle has a period of 16 rows)
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    wvo[i] = (uint32_t)min(n_base + 64 * i + ld_row, p.N - 1) * (uint32_t)kbytes + ld_q * 16;
+    wvo[i] = (uint32_t)weight_row<128>(p, n_base, 64 * i + ld_row) * (uint32_t)kbytes + ld_q * 16;
     xvo[i] = (uint32_t)min(m_base + 64 * i + ld_row, p.M - 1) * (uint32_t)kbytes + ld_q * 16;
   }
   const uint8_t *sbase = group ? p.a_scales : p.b_scales;
-  const uint32_t svo = (uint32_t)(group ? min(m_base + 64 * pos + lane, p.M - 1) : min(n_base + 64 * pos + lane, p.N - 1)) * (uint32_t)ksc;
+  const uint32_t svo = (uint32_t)(group ? min(m_base + 64 * pos + lane, p.M - 1) : weight_row<128>(p, n_base, 64 * pos + lane)) * (uint32_t)ksc;
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(smem);
   // requests behind the last stage fetch it again into buffers that nobody reads any more: the number of loads on their
   // way is the same in every stage.  A short last stage is the row's last 256 elements, the first half of which the stage before it has.

@@ -114,14 +114,14 @@ __device__ __forceinline__ void f16_tile_of(const GemmParams &p, int c_base, int
 #pragma unroll
   for (int i = 0; i < FI; ++i) {
     const int row = 64 * i + 8 * wave + (lane >> 3);
-    fvo[i] = (uint32_t)min(f_base + row, rows_f - 1) * (uint32_t)fbytes + (((lane & 7) ^ stage_swizzle(row)) << 4);
+    fvo[i] = (uint32_t)(CODES_W ? min(f_base + row, rows_f - 1) : weight_row<16 * TF>(p, f_base, row)) * (uint32_t)fbytes + (((lane & 7) ^ stage_swizzle(row)) << 4);
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int row = 128 * i + 16 * wave + (lane >> 2);
-    cvo[i] = (uint32_t)min(c_base + row, rows_c - 1) * (uint32_t)kbytes + (((lane & 3) ^ ((row >> 2) & 3)) << 4);
+    cvo[i] = (uint32_t)(CODES_W ? weight_row<64>(p, c_base, row) : min(c_base + row, rows_c - 1)) * (uint32_t)kbytes + (((lane & 3) ^ ((row >> 2) & 3)) << 4);
   }
-  svo = (uint32_t)min(c_base + 64 * cpos + lane, rows_c - 1) * (uint32_t)ksc + 4 * group;
+  svo = (uint32_t)(CODES_W ? weight_row<64>(p, c_base, 64 * cpos + lane) : min(c_base + 64 * cpos + lane, rows_c - 1)) * (uint32_t)ksc + 4 * group;
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(smem);
   const uint8_t *f16 = reinterpret_cast<const uint8_t *>(p.f16) + (size_t)u0 * 128;
   // (requests behind the last step fetch it again, into stages that nobody reads any more: the number of loads on their

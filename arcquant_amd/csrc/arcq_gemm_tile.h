@@ -18,6 +18,8 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 constexpr int kMaxParts = ARCQ_MAX_PARTS;
 
+constexpr int kSwigluPairs = 1, kSwigluHalves = 2;
+
 struct GemmParams {
   const uint8_t *a_codes, *a_scales;  // activations, M rows
   const uint8_t *b_codes, *b_scales;  // weights, N rows
@@ -44,6 +46,8 @@ struct GemmParams {
   // receives act_fn(gate) * up formed from the bf16-rounded GEMM outputs, exactly what the unfused sequence
   // (GEMM, then silu and multiply in bf16) gives.  absmax_bits: NULL, or one word per segment (one word when
   // not grouped) that collects max |output| as the bits of a non-negative float (zeroed by the caller).
+  // kSwigluHalves: the first N/2 weight rows are the gates, the others the ups; a tile takes half of its rows from either (weight_row), so
+  // that gate_j and up_j are kN / 2 apart in a wave's accumulators (gemm_nvfp4_f16 and gemm_mxfp4_pingpong, plain launches).
   int swiglu = 0;
   uint32_t *absmax_bits = nullptr;
   int seg_index = 0;
@@ -298,6 +302,65 @@ struct Acc16 {  // v_mfma_*_16x16x*: element e of a lane is n = 4 (lane / 16) + 
   __device__ __forceinline__ float4 quad(int q, int j) const { return make_float4(a[q][j][0], a[q][j][1], a[q][j][2], a[q][j][3]); }
 };
 
+// Row of the weights that local row `row` of the tile at n_base holds, kN of them to a wave.
+template <int kN>
+__device__ __forceinline__ int weight_row(const GemmParams &p, int n_base, int row) {
+  if (p.swiglu != kSwigluHalves) return min(n_base + row, p.N - 1);
+  const int o = row % kN, F = p.N >> 1;
+  return min((n_base >> 1) + row / kN * (kN / 2) + o % (kN / 2), F - 1) + (o >= kN / 2 ? F : 0);
+}
+
+// max |output| of a wave's lanes (bf16 bits without the sign) into its segment's word.  One atomic per wave, and only if its maximum is above
+// what the word, which never falls, is seen to hold: atomics on one word are served one after the other (16384 x 28672 x 4352, a
+// word for 57344 waves: 2852 us, so 2800; MXFP4 4096 rows 357 / 310).
+__device__ __forceinline__ void collect_absmax(const GemmParams &p, uint32_t amax, int lane) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint32_t v = (uint32_t)__shfl_xor((int)amax, o);
+    amax = v > amax ? v : amax;
+  }
+  uint32_t *word = p.absmax_bits + p.seg_index;
+  if (lane == 0 && (amax << 16) > *const_cast<volatile uint32_t *>(word)) atomicMax(word, amax << 16);  // bf16 bits -> fp32 bits
+}
+
+// kSwigluHalves: quads q and q + kQuads / 2 of a lane are the gates and the ups of the same four output columns.  m0: first row of C of the
+// wave's tile, n0: first output column.
+template <class Acc>
+__device__ __forceinline__ void store_wave_tile_halves(const GemmParams &p, const Acc &acc, uint8_t *region, int m0, int n0, int lane) {
+  constexpr int kNo = Acc::kN / 2, RB = 2 * kNo, LPR = RB / 16;  // output columns, bytes per row, lanes per row when reading 16 bytes each
+  static_assert((LPR & (LPR - 1)) == 0 && RB <= 256, "the swizzle needs a power of two");
+  const int F = p.N >> 1;
+  const Alpha by_column(p);
+  const float ag = by_column.at(p, 0), au = by_column.at(p, F);
+  // rows 256 bytes apart (all banks once) take turns
+  auto swizzle = [](int m) { return ((m / (256 / RB)) & (LPR - 1)) << 1; };
+  wait_dma_and_sync();  // every wave is done reading operands
+  const int rows = p.M - m0;
+  if (rows <= 0) return;
+  uint32_t amax = 0u;
+#pragma unroll
+  for (int q = 0; q < Acc::kQuads / 2; ++q)
+#pragma unroll
+    for (int j = 0; j < Acc::kTiles; ++j) {
+      const float4 g = acc.quad(q, j), u = acc.quad(q + Acc::kQuads / 2, j);
+      const uint2 t = swiglu_quad(make_uint2(pack_bf16_rne(g.x * ag, g.y * ag), pack_bf16_rne(g.z * ag, g.w * ag)),
+                                  make_uint2(pack_bf16_rne(u.x * au, u.y * au), pack_bf16_rne(u.z * au, u.w * au)));
+      const int m = Acc::m(j, lane), n = Acc::n(q, lane);
+      if (m < rows && n0 + n < F) amax = max(max(amax, max(t.x & 0x7fffu, (t.x >> 16) & 0x7fffu)), max(t.y & 0x7fffu, (t.y >> 16) & 0x7fffu));
+      *reinterpret_cast<uint2 *>(region + m * RB + (((n >> 2) ^ swizzle(m)) << 3)) = t;
+    }
+  const int rr = lane / LPR, tq = lane % LPR, col = n0 + 8 * tq;
+  uint16_t *cbase = p.c + (size_t)m0 * F + col;
+  const int lane_rows = col < F ? rows : 0;  // (F is a multiple of 8)
+#pragma unroll
+  for (int it = 0; it < (Acc::kM * LPR) / 64; ++it) {
+    const int m = it * (64 / LPR) + rr;
+    const uint4 v = *reinterpret_cast<const uint4 *>(region + m * RB + (((2 * tq) ^ swizzle(m)) << 3));
+    if (m < lane_rows) *reinterpret_cast<uint4 *>(cbase + (size_t)m * F) = v;
+  }
+  if (p.absmax_bits) collect_absmax(p, amax, lane);
+}
+
 // Fused SwiGLU epilogue of the tiled kernels (p.swiglu; N is a multiple of 16): a lane's four consecutive columns of one row are
 // (gate_j, up_j, gate_j+1, up_j+1); each is rounded to bf16 as the plain epilogue would store it, and the two
 // products act_fn(gate) * up leave through LDS, so that every store instruction writes 16 bytes per lane along output rows.
@@ -306,9 +369,10 @@ __device__ __forceinline__ void store_wave_tile_swiglu(const GemmParams &p, cons
   const float alpha = effective_alpha(p);
   const int No = p.N >> 1;  // output columns
   uint32_t amax = 0u;       // max |t| of this lane as bf16 bits without the sign
-  auto product = [&](int q, int j) {  // the hardware's RNE convert: the bits f32_to_bf16_bits gives
-    const float4 v = acc.quad(q, j);
-    return swiglu_pair(pack_bf16_rne(v.x * alpha, v.z * alpha), pack_bf16_rne(v.y * alpha, v.w * alpha));
+  auto products = [&](int q, int j) {  // of quads q and q + 1; the hardware's RNE convert: the bits f32_to_bf16_bits gives
+    const float4 v = acc.quad(q, j), w = acc.quad(q + 1, j);
+    return swiglu_quad(make_uint2(pack_bf16_rne(v.x * alpha, v.z * alpha), pack_bf16_rne(w.x * alpha, w.z * alpha)),
+                       make_uint2(pack_bf16_rne(v.y * alpha, v.w * alpha), pack_bf16_rne(w.y * alpha, w.w * alpha)));
   };
   wait_dma_and_sync();  // every wave is done reading operands
   const int rows = p.M - m0;  // of this wave's tile inside C
@@ -317,18 +381,22 @@ __device__ __forceinline__ void store_wave_tile_swiglu(const GemmParams &p, cons
   constexpr int LPR = Acc::kN / 16;  // lanes per row when reading 16 bytes each
   static_assert((LPR & (LPR - 1)) == 0, "the swizzle needs a power of two");
 #pragma unroll
-  for (int q = 0; q < Acc::kQuads; ++q)
+  for (int q2 = 0; q2 < Acc::kQuads; q2 += 2)
 #pragma unroll
     for (int j = 0; j < Acc::kTiles; ++j) {
-      const int m = Acc::m(j, lane), c = Acc::n(q, lane) >> 2;  // row and dword of the row
-      const int sw = m & (LPR - 1);                             // swizzle of the row's 16-byte groups
-      const uint32_t t = product(q, j);  // (every lane: the special-value test of the activation is a vote of the whole wave)
-      if (m < rows && n0 + Acc::n(q, lane) < p.N) {
-        const uint32_t lo = t & 0x7fffu, hi = (t >> 16) & 0x7fffu;
-        amax = lo > amax ? lo : amax;
-        amax = hi > amax ? hi : amax;
+      const uint2 two = products(q2, j);  // (every lane: the special-value test of the activation is a vote of the whole wave)
+#pragma unroll
+      for (int q = q2; q < q2 + 2; ++q) {
+        const int m = Acc::m(j, lane), c = Acc::n(q, lane) >> 2;  // row and dword of the row
+        const int sw = m & (LPR - 1);                             // swizzle of the row's 16-byte groups
+        const uint32_t t = q == q2 ? two.x : two.y;
+        if (m < rows && n0 + Acc::n(q, lane) < p.N) {
+          const uint32_t lo = t & 0x7fffu, hi = (t >> 16) & 0x7fffu;
+          amax = lo > amax ? lo : amax;
+          amax = hi > amax ? hi : amax;
+        }
+        *reinterpret_cast<uint32_t *>(region + m * RB + ((((c >> 2) ^ sw) << 2) | (c & 3)) * 4) = t;
       }
-      *reinterpret_cast<uint32_t *>(region + m * RB + ((((c >> 2) ^ sw) << 2) | (c & 3)) * 4) = t;
     }
   const int rr = lane / LPR, tq = lane % LPR, col = (n0 >> 1) + 8 * tq;
   uint16_t *cbase = p.c + (size_t)m0 * No + col;
@@ -340,14 +408,7 @@ __device__ __forceinline__ void store_wave_tile_swiglu(const GemmParams &p, cons
     const uint4 v = *reinterpret_cast<const uint4 *>(region + m * RB + ((tq ^ sw) << 4));
     if (m < lane_rows) *reinterpret_cast<uint4 *>(cbase + (size_t)m * No) = v;
   }
-  if (p.absmax_bits) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const uint32_t v = (uint32_t)__shfl_xor((int)amax, o);
-      amax = v > amax ? v : amax;
-    }
-    if (lane == 0 && amax) atomicMax(p.absmax_bits + p.seg_index, amax << 16);  // bf16 bits -> fp32 bits
-  }
+  if (p.absmax_bits) collect_absmax(p, amax, lane);
 }
 
 // Tile (i, j) of the wave's accumulators with bounds checks: the row is tested once per tile, the columns once per tile
@@ -398,6 +459,8 @@ __device__ __forceinline__ void store_tile(const GemmParams &p, const Acc &acc, 
 // reading operands.
 template <class Acc>
 __device__ __forceinline__ void store_wave_tile(const GemmParams &p, const Acc &acc, uint8_t *region, int m0, int n0, int lane) {
+  if constexpr (Acc::kSide == 16)
+    if (p.swiglu == kSwigluHalves) return store_wave_tile_halves(p, acc, region, m0, n0 >> 1, lane);
   if (p.swiglu) return store_wave_tile_swiglu(p, acc, region, m0, n0, lane);
   if (p.partial) {  // split-K: the unscaled fp32 tile of this K range
     float *part = p.partial + (size_t)blockIdx.y * p.M * p.N;

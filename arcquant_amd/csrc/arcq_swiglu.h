@@ -52,5 +52,28 @@ __device__ __forceinline__ uint32_t swiglu_pair(uint32_t gw, uint32_t uw) {
   return pack_bf16_rne(dot2_bf16(a, uw & 0xffffu), dot2_bf16(a, uw & 0xffff0000u));
 }
 
+// Four elements at once, for code that waits for its arithmetic: one vote for the special activations of all of them (halves of the
+// minimum below that are 0), among them every one that is infinite or NaN, so that the others need no vote of their own for the product.
+typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint2 swiglu_quad(uint2 g, uint2 u) {
+  auto halves = [](uint32_t x) { return __builtin_bit_cast(v2us, x); };
+  const v2us top = __builtin_elementwise_max(halves(g.x & 0x7fff7fffu), halves(g.y & 0x7fff7fffu));
+  const v2us equal = __builtin_elementwise_min(halves(g.x ^ 0x40be40beu), halves(g.y ^ 0x40be40beu));
+  const v2us below = __builtin_elementwise_sub_sat(halves(0x42ae42aeu), top);
+  const uint32_t least = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(equal, below));
+  const bool special = ((least - 0x00010001u) & ~least & 0x80008000u) != 0;
+  const float x0 = u2f(g.x << 16), x1 = u2f(g.x & 0xffff0000u), x2 = u2f(g.y << 16), x3 = u2f(g.y & 0xffff0000u);
+  if (__builtin_amdgcn_ballot_w64(special) != 0) {
+    const uint32_t a = pack_bf16_rne(x0 / (1.0f + expf(-x0)), x1 / (1.0f + expf(-x1)));
+    const uint32_t b = pack_bf16_rne(x2 / (1.0f + expf(-x2)), x3 / (1.0f + expf(-x3)));
+    return make_uint2(pack_bf16_rne(u2f(a << 16) * u2f(u.x << 16), u2f(a & 0xffff0000u) * u2f(u.x & 0xffff0000u)),
+                      pack_bf16_rne(u2f(b << 16) * u2f(u.y << 16), u2f(b & 0xffff0000u) * u2f(u.y & 0xffff0000u)));
+  }
+  auto silu = [](float x) { return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * -1.4426950408889634f)); };
+  const uint32_t a = pack_bf16_rne(silu(x0), silu(x1)), b = pack_bf16_rne(silu(x2), silu(x3));
+  return make_uint2(pack_bf16_rne(dot2_bf16(a, u.x & 0xffffu), dot2_bf16(a, u.x & 0xffff0000u)),
+                    pack_bf16_rne(dot2_bf16(b, u.y & 0xffffu), dot2_bf16(b, u.y & 0xffff0000u)));
+}
+
 }  // namespace arcq
 #endif  // ARCQ_SWIGLU_H_

@@ -246,13 +246,10 @@ def _linear(out_features, in_features, std, device, gen):
 class LlamaMLP(nn.Module):
     """SwiGLU MLP with gate and up projections fused into one [2*inter, hidden] linear
     (model/qLlamaLayer.py:380-443 with the fusion of benchmark configuration 4), followed by the fused
-    SwiGLU -> quantize pass.  interleave=True instead interleaves the fused weight's rows (gate_0, up_0,
-    gate_1, ...) and forms act_fn(gate) * up in the GEMM's epilogue, so that the [tokens, 2*inter] projection
-    output never goes through memory: the same bits, but not the default here, because on one large GEMM with
-    256x256 tiles (one workgroup per CU) the epilogue's activation arithmetic is exposed and costs more than
-    the pass it saves (16384 tokens, MXFP4: 2.01 against 1.73 ms for GEMM + quantizer; NVFP4 3.95 against
-    3.81).  The MoE block's grouped GEMMs run 128x128 tiles, two workgroups per CU, where one workgroup's
-    epilogue hides behind the other's main loop: there it is the default and a gain."""
+    SwiGLU -> quantize pass, or for many tokens (agemm.swiglu_halves_pay) by the quantizer alone, act_fn(gate) * up formed in the
+    GEMM's epilogue: the [tokens, 2*inter] projection output then never goes through memory; the same bits.  interleave=True
+    interleaves the fused weight's rows (gate_0, up_0, gate_1, ...), for which every GEMM has such an epilogue, as the MoE
+    block's grouped GEMMs need it."""
 
     def __init__(self, gate_up: nn.Linear, down: nn.Linear, select_num_in, select_num_down, in_index, down_index,
                  quant_type="NVFP4", interleave=False):
@@ -271,6 +268,20 @@ class LlamaMLP(nn.Module):
         self.register_buffer("down_reorder_index", down_index.to(torch.int16))
         self.quant_type = quant_type
 
+    def _activation(self, x):
+        """act_fn(gate) * up straight from the projection's epilogue, NVFP4 with its tensor scale; None where the projection is called
+        by itself: few tokens, hooks or another forward on it, a bias, no memory"""
+        qx, scale_x, scale, _, _ = x
+        p, nv = self.gate_up_proj, self.quant_type == "NVFP4"
+        if qx.dim() != 2 or not isinstance(scale, (float, int, torch.Tensor)) or \
+                not agemm.swiglu_halves_pay(qx.shape[0], 2 * self.inter, 2 * qx.shape[1], self.quant_type):
+            return None
+        if _unhooked(p, SplitQLinear):
+            return p._as_one(x, swiglu=True)
+        if not _unhooked(p, QLinearLayer) or p.bias is not None or p.out_features != 2 * self.inter or p.quant_type != self.quant_type:
+            return None
+        return agemm.matmul_swiglu(qx, p.W, scale_x, p.scale_w, (scale, p.scale), fmt=self.quant_type, tensor_scale=nv, halves=True)
+
     @_no_grad
     def forward(self, x, residual=None):
         """x: the tuple of the already quantized (normalised) hidden states; residual: added to the output"""
@@ -282,6 +293,14 @@ class LlamaMLP(nn.Module):
             qx, sfx = agemm.reorder_quantize_x(t, self.down_reorder_index, sel, fmt=self.quant_type,
                                                global_scale=scale if nv else None)
             return self.down_proj((qx, sfx, scale, x[3], x[4]), residual)
+        if self.inter <= 32736 and self.inter % 32 == 0:
+            t = self._activation(x)
+            if t is not None:
+                scale = t[1] if isinstance(t, tuple) else 1.0
+                t = t[0] if isinstance(t, tuple) else t
+                qx, sfx = agemm.reorder_quantize_x(t, self.down_reorder_index, sel, fmt=self.quant_type,
+                                                   global_scale=scale if self.quant_type == "NVFP4" else None)
+                return self.down_proj((qx, sfx, scale, x[3], x[4]), residual)
         gu = self.gate_up_proj(x)
         if self.inter <= 32736 and self.inter % 32 == 0:
             return self.down_proj(swiglu_quantize_tokens(gu, self.inter, self.down_reorder_index, sel, self.quant_type),
@@ -488,18 +507,21 @@ class SplitQLinear(nn.Module):
             rows += t.shape[0]
         return torch.as_strided(first, (rows, *first.shape[1:]), first.stride())
 
-    def _as_one(self, x):
-        """one GEMM over all parts, or None where they have to run one by one"""
+    def _as_one(self, x, swiglu=False):
+        """one GEMM over all parts, or None where they have to run one by one; swiglu: of a gate and an up projection, act_fn(gate) * up
+        instead of both (where agemm.swiglu_halves_pay), NVFP4 with its tensor scale"""
         qx, scale_x, scale, _, _ = x
         ps = list(self.parts)
         if not 2 <= len(ps) <= 4 or not all(_unhooked(p, QLinearLayer) and p.quant_type == ps[0].quant_type for p in ps) or \
                 any(p.out_features % 32 for p in ps) or not isinstance(scale, (float, int, torch.Tensor)):
             return None
         rows = tuple(p.out_features for p in ps)
-        if qx.dim() != 2 or not agemm.parts_pay(qx.shape[0], rows, 2 * qx.shape[1], ps[0].quant_type):
+        if qx.dim() != 2 or not (swiglu or agemm.parts_pay(qx.shape[0], rows, 2 * qx.shape[1], ps[0].quant_type)):
             return None
         bias = None
         if any(p.bias is not None for p in ps):
+            if swiglu:
+                return None
             bias = self._joint("bias")
             if bias is None or bias.dtype != torch.bfloat16:
                 return None
@@ -507,6 +529,11 @@ class SplitQLinear(nn.Module):
         scales = [p.scale for p in ps]
         if W is None or scale_w is None or any(s.dtype != torch.float32 or s.device != W.device for s in scales):
             return None
+        if swiglu:
+            if len(rows) != 2 or rows[0] != rows[1]:
+                return None
+            return agemm.matmul_parts(qx, W, scale_x, scale_w, scale, rows, scales, fmt=ps[0].quant_type, swiglu=True,
+                                      tensor_scale=ps[0].quant_type == "NVFP4")
         return agemm.matmul_parts(qx, W, scale_x, scale_w, scale, rows, scales, fmt=ps[0].quant_type, bias=bias)
 
     @_no_grad
@@ -517,6 +544,9 @@ class SplitQLinear(nn.Module):
         else:
             y = y.reshape(x[3], x[4], -1) if x[3] is not None else y.reshape(x[4], -1)
         return y if residual is None else y + residual
+
+
+_FORWARD[SplitQLinear] = SplitQLinear.forward
 
 
 class LlamaRMSNorm(nn.Module):

@@ -219,7 +219,7 @@ typedef struct arcq_gemm_args {
   const void *a_codes, *a_scales, *b_codes, *b_scales;
   int M, N, Kp, fmt;
   float alpha;
-  int swiglu;               /* 1: weight rows alternate gate, up; c is bf16 [M, N/2] (arcq_matmul_swiglu) */
+  int swiglu;               /* 1: weight rows alternate gate, up; c is bf16 [M, N/2] (arcq_matmul_swiglu); or ARCQ_SWIGLU_HALVES */
   const float *d_alpha_a, *d_alpha_b;
   const void *residual;     /* bf16 [M, N] or NULL (arcq_matmul_add) */
   void *c;
@@ -230,6 +230,11 @@ typedef struct arcq_gemm_args {
   size_t workspace_bytes;
 } arcq_gemm_args;
 int arcq_gemm(const arcq_gemm_args *args, void *stream);
+/* swiglu = ARCQ_SWIGLU_HALVES: the same output from weights as a fused gate_up projection has them, N/2 gate rows and then N/2 up rows (in
+ * arcq_gemm_parts one part each, without a bias), for the plain problems of many rows that arcq_gemm_swiglu_halves says 1 for; ARCQ_ERR_SHAPE
+ * for others, ARCQ_ERR_WORKSPACE without the workspace that arcq_gemm_workspace_bytes names. */
+#define ARCQ_SWIGLU_HALVES 2
+int arcq_gemm_swiglu_halves(int M, int N, int Kp, int fmt);
 size_t arcq_gemm_workspace_bytes(int M, int N, int Kp, int fmt, int n_seg);
 /* Bytes with which arcq_gemm may also cut the last round of its tiles along K (NVFP4 with a long K': fp32 sums of parts of tiles behind
  * the decoded operand, 128 MiB); arcq_gemm_workspace_bytes where it would not.  A workspace of either size is used for what it holds. */

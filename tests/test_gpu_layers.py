@@ -706,3 +706,35 @@ def test_prompts_of_one_token_and_more(layers, monkeypatch):
     assert ran == [2]
     one = layer(x[:, :1].contiguous())
     assert ran == [2] and torch.equal(one, two[:, :1])
+
+
+@pytest.mark.parametrize("fmt,tokens,split", [("NVFP4", 2100, False), ("NVFP4", 2100, True), ("MXFP4", 1100, False), ("MXFP4", 1100, True)])
+def test_mlp_of_many_tokens(layers, monkeypatch, fmt, tokens, split):
+    """Many tokens: act_fn(gate) * up comes from the projection's epilogue, with one scale or one each for gate and up; the bits of the
+    projection followed by the SwiGLU quantizer, which a hook on the projection brings back."""
+    H, I, S = 2048, 6400, 128
+    g = torch.Generator(device="cuda").manual_seed(3)
+
+    def linear(n, k, std):
+        lin = nn.Linear(k, n, bias=False, device="cuda", dtype=torch.bfloat16)
+        lin.weight.data.copy_(torch.randn(n, k, generator=g, device="cuda") * std)
+        return lin
+
+    index = lambda n: torch.randperm(n, generator=g, device="cuda").to(torch.int16)
+    idx, down_idx = index(H), index(I)
+    if split:
+        order = {f"layers.0.mlp.{n}.input": i for n, i in (("gate_proj", idx), ("up_proj", idx), ("down_proj", down_idx))}
+        mlp = layers.QLlamaMLP(linear(I, H, 0.1), linear(I, H, 0.02), linear(H, I, 0.02), {k: S for k in order}, order, 0, fmt)
+    else:
+        mlp = layers.LlamaMLP(linear(2 * I, H, 0.05), linear(H, I, 0.02), S, S, idx, down_idx, fmt)
+    assert layers.agemm.swiglu_halves_pay(tokens, 2 * I, H + S, fmt)
+    x = layers.quantize_tokens(torch.randn(1, tokens, H, generator=g, device="cuda").to(torch.bfloat16), idx, S, fmt)
+    res = torch.randn(1, tokens, H, generator=g, device="cuda").to(torch.bfloat16)
+    called, quantizer = [], layers.swiglu_quantize_tokens
+    monkeypatch.setattr(layers, "swiglu_quantize_tokens", lambda *a: called.append(1) or quantizer(*a))
+    fused = mlp(x, residual=res)
+    assert not called
+    handle = mlp.gate_up_proj.register_forward_hook(lambda *a: None)
+    assert torch.equal(mlp(x, residual=res), fused) and called
+    handle.remove()
+    assert torch.equal(mlp(x, residual=res), fused) and len(called) == 1

@@ -601,3 +601,64 @@ def test_mxfp4_rows_of_medium_length(agemm, oracle, M, N, K, S):
     assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
     res = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
     assert torch.equal(agemm.matmul(a, b, sfa, sfb, 0.5, fmt="MXFP4", residual=res), y + res)
+
+
+@pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
+@pytest.mark.parametrize("fmt,M,N,kp", [
+    ("NVFP4", 70, 49184, 512), ("NVFP4", 300, 22112, 640), ("NVFP4", 3900, 4096, 512), ("NVFP4", 3960, 4064, 512), ("NVFP4", 257, 43968, 512),
+    ("NVFP4", 8192, 3616, 512), ("NVFP4", 4100, 4096, 8192), ("NVFP4", 6144, 3008, 8320),          # the weights decoded; the last round cut
+    ("MXFP4", 2300, 4608, 2176), ("MXFP4", 2304, 4640, 2304), ("MXFP4", 4000, 3936, 8320)])
+def test_swiglu_of_weights_as_they_are(agemm, fmt, M, N, kp):
+    """gate rows and then up rows with the SwiGLU epilogue: the bits of the GEMM followed by silu and multiply in bf16, and the tensor scale
+    of the result; N / 2 a multiple of 16 that ends inside a tile, one scale for both and one each (parts), special activations
+    (5.9375 and beyond 87, where the epilogue leaves its estimate) among the gates.  Where the last round of tiles is cut along K, other
+    columns are in it: one bf16 rounding (2^-9, 1.7e-3 in norm) of a few gates and ups."""
+    from arcquant_amd import _lib
+    assert agemm.swiglu_halves_pay(M, N, kp, fmt)
+    cut = _lib.lib().arcq_gemm_route(M, N, kp, _lib.FORMATS[fmt], 0, 0) == 2
+    g, F, nv = torch.Generator(device="cuda").manual_seed(M + N), N // 2, fmt == "NVFP4"
+    lo, hi, G = (30, 60, 16) if nv else (118, 124, 32)
+    codes = lambda rows: (torch.randint(0, 256, (rows, kp // 2), generator=g, device="cuda", dtype=torch.uint8),
+                          torch.randint(lo, hi, (rows * (kp // G),), generator=g, device="cuda", dtype=torch.uint8))
+    (a, sfa), (b, sfb) = codes(M), codes(N)
+    y = agemm.matmul(a, b, sfa, sfb, 1.0, fmt=fmt)
+    big = 100.0 / float(y[:, :F].float().abs().max())      # gates of up to 100 in magnitude, most of them small
+    y = agemm.matmul(a, b, sfa, sfb, big, fmt=fmt)
+    want = torch.nn.functional.silu(y[:, :F]) * y[:, F:]
+    t, scale = agemm.matmul_swiglu(a, b, sfa, sfb, big, fmt=fmt, tensor_scale=True, halves=True)
+    assert rel_fro(t.float(), want.float()) < 1.7e-3 if cut else torch.equal(t, want)
+    assert float(scale) == float(t.abs().max().float().cpu() / torch.tensor(2688.0))
+    assert torch.equal(agemm.matmul_swiglu(a, b, sfa, sfb, big, fmt=fmt, halves=True), t)
+    scales = [torch.tensor(s, device="cuda") for s in (big, 0.5 * big)]
+    one = torch.tensor(1.0, device="cuda")
+    if F % 32 == 0:
+        y = agemm.matmul_parts(a, b, sfa, sfb, one, (F, F), scales, fmt=fmt)
+        want = torch.nn.functional.silu(y[:, :F]) * y[:, F:]
+        t, scale = agemm.matmul_parts(a, b, sfa, sfb, one, (F, F), scales, fmt=fmt, swiglu=True, tensor_scale=True)
+        assert rel_fro(t.float(), want.float()) < 1.7e-3 if cut else torch.equal(t, want)
+        assert float(scale) == float(t.abs().max().float().cpu() / torch.tensor(2688.0))
+
+
+def test_swiglu_of_weights_as_they_are_for_others(agemm, monkeypatch):
+    """problems that have no such epilogue are refused, and without memory for the scratch there is no result to be had"""
+    import ctypes
+    from arcquant_amd import _lib
+    L = _lib.lib()
+    for M, N, kp, f in ((64, 28672, 4352, 0), (16, 28672, 4352, 1), (4096, 28672, 1152, 1), (4096, 28688, 4352, 0), (4096, 28672, 448, 0)):
+        assert L.arcq_gemm_swiglu_halves(M, N, kp, f) == 0
+        ok = 0x1000
+        args = _lib.GemmArgs(ok, ok, ok, ok, M, N, kp, f, 1.0, _lib.SWIGLU_HALVES, None, None, None, ok, None, 0, None, None, 0)
+        assert L.arcq_gemm(args, None) == 2
+    if "ARCQ_GEMM_KERNEL" in os.environ:
+        pytest.skip("another kernel is forced")
+    M, N, K = 2100, 6400, 512
+    (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, K, 128, "NVFP4", seed=31)
+    empty = torch.empty
+
+    def full(*size, **kw):
+        if kw.get("dtype") is torch.uint8:
+            raise torch.OutOfMemoryError("no memory for the workspace")
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(torch, "empty", full)
+    assert agemm.matmul_swiglu(a, b, sfa, sfb, gx * gw, tensor_scale=True, halves=True) is None
