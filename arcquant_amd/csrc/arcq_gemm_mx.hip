@@ -52,7 +52,7 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
 
   int lin;
   if (p.seg) {
-    if (!enter_segment<BT, BT, 32>(p, lin)) return;
+    if (!enter_segment_in_turn<BT, BT, 32, 32>(p, lin)) return;
   } else {
     const int total = ((p.M + BT - 1) / BT) * ((p.N + BT - 1) / BT);
     lin = (blockIdx.x & 7) * ((total + 7) >> 3) + (blockIdx.x >> 3);
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
 
 int run_mxfp4_pingpong(const GemmParams &p, hipStream_t st) {
   const int total = ((p.M + 255) / 256 + (p.seg ? p.n_seg : 0)) * ((p.N + 255) / 256);
-  hipLaunchKernelGGL(gemm_mxfp4_pingpong, dim3(((total + 7) / 8) * 8), dim3(512), 0, st, p);
+  hipLaunchKernelGGL(gemm_mxfp4_pingpong, dim3(p.seg ? grid_in_turn<32>(total) : grid_in_turn<1>(total)), dim3(512), 0, st, p);
   ARCQ_HIP_TRY(hipGetLastError());
   return ARCQ_OK;
 }

@@ -296,7 +296,7 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
   __shared__ uint4 smem[(S::kF + S::kC + S::kS) / 16];
   int lin;
   if (p.seg) {
-    if (!enter_segment<S::BM, S::BN, 16>(p, lin)) return;
+    if (!enter_segment_in_turn<S::BM, S::BN, 16, 32>(p, lin)) return;
   } else {
     const int total = ((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN);
     lin = (blockIdx.x & 7) * ((total + 7) >> 3) + (blockIdx.x >> 3);
@@ -433,7 +433,7 @@ template <bool CODES_W, int TF>
 int launch_tiles(const GemmParams &p, hipStream_t st) {
   using S = F16Shape<CODES_W, TF>;
   const int total = ((p.M + S::BM - 1) / S::BM + (p.seg ? p.n_seg : 0)) * ((p.N + S::BN - 1) / S::BN);
-  hipLaunchKernelGGL((gemm_nvfp4_f16<CODES_W, TF>), dim3(((total + 7) / 8) * 8), dim3(512), 0, st, p);
+  hipLaunchKernelGGL((gemm_nvfp4_f16<CODES_W, TF>), dim3(p.seg ? grid_in_turn<32>(total) : grid_in_turn<1>(total)), dim3(512), 0, st, p);
   ARCQ_HIP_TRY(hipGetLastError());
   return ARCQ_OK;
 }

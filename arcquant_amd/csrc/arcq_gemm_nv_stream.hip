@@ -278,7 +278,7 @@ __global__ __launch_bounds__(64 * WN * WK) void gemm_nvfp4_stream(GemmParams p) 
   uint8_t *lds = reinterpret_cast<uint8_t *>(smem);
   int lin;
   if constexpr (GROUPED) {
-    if (!enter_segment<S::BM, S::BN, 16>(p, lin)) return;
+    if (!enter_segment_in_turn<S::BM, S::BN, 16, 2>(p, lin)) return;
   } else {
     const int total = ((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN);
     lin = (blockIdx.x & 7) * ((total + 7) >> 3) + (blockIdx.x >> 3);
@@ -299,7 +299,7 @@ template <int MT, int NT, int WN, int WK, int NS, bool GROUPED = false>
 int launch(const GemmParams &p, hipStream_t st) {
   using S = StreamShape<MT, NT, WN, WK, NS>;
   const int total = ((p.M + S::BM - 1) / S::BM + (GROUPED ? p.n_seg : 0)) * ((p.N + S::BN - 1) / S::BN);
-  hipLaunchKernelGGL((gemm_nvfp4_stream<MT, NT, WN, WK, NS, GROUPED>), dim3(((total + 7) / 8) * 8), dim3(64 * S::NW), 0, st, p);
+  hipLaunchKernelGGL((gemm_nvfp4_stream<MT, NT, WN, WK, NS, GROUPED>), dim3(grid_in_turn<GROUPED ? 2 : 1>(total)), dim3(64 * S::NW), 0, st, p);
   ARCQ_HIP_TRY(hipGetLastError());
   return ARCQ_OK;
 }

@@ -181,6 +181,23 @@ __device__ __forceinline__ bool enter_segment(GemmParams &p, int &lin) {
   return segments.enter(p, lin);
 }
 
+// The same with runs of RUN tiles that go to the XCDs in turn, for kernels whose tiles take less time for fewer rows: with one run per XCD,
+// the XCD that has the experts of most rows, or none of those that end in a small tile, is the last one.  The grid is a multiple of
+// 8 RUN (grid_in_turn).  us, one run per XCD and so, Zipf-like and even sizes: gemm_nvfp4_f16, RUN = 32, 8192 rows over eight of 28672 x
+// 4224 1497, 1378 / 1472, 1373, 50000 over 64 of 4096 x 2176 824 / 791; gemm_mxfp4_pingpong, 8192 over eight of 4096 x 14464 342, 243 / 330, 247.
+// gemm_nvfp4_stream, RUN = 2 (the tiles of an expert's first and second rows, which share their weights): 128 rows over eight of 28672 x 4224
+// 134, 125 / 128, 124, 64 rows 132 / 122, 200 rows 151 / 139; of 4096 x 14464 84, 55 / 83, 56; 1024 over 64 of 2048 x 1536 44.1 / 36.6.
+template <int RUN>
+inline int grid_in_turn(int tiles) { return (tiles + 8 * RUN - 1) / (8 * RUN) * (8 * RUN); }
+
+template <int BM, int BN, int G, int RUN>
+__device__ __forceinline__ bool enter_segment_in_turn(GemmParams &p, int &lin) {
+  Segments<BM, BN, G> segments(p);
+  const int of_xcd = blockIdx.x >> 3;
+  lin = (of_xcd / RUN * 8 + (blockIdx.x & 7)) * RUN + of_xcd % RUN;
+  return segments.enter(p, lin);
+}
+
 // two bf16 pairs + two bf16 pairs, each sum rounded to bf16
 __device__ __forceinline__ uint32_t add_bf16_pair(uint32_t a, uint32_t b) {
   return pack_bf16_rne(u2f(a << 16) + u2f(b << 16), u2f(a & 0xffff0000u) + u2f(b & 0xffff0000u));
