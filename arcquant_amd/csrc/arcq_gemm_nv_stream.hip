@@ -38,7 +38,7 @@ __device__ __forceinline__ void wait_vmcnt(int n) {
 // What bounds such a problem is the stream of the weights, and in front of it everything that keeps a CU from asking for
 // more of them: waves that wait for one another, load instructions that touch a cache line for a few bytes, and the decoding,
 // which costs 8 VALU instructions (a wave's takes 2 ns on its SIMD once two or more waves offer them, 4 ns alone) per 512
-// codes and operand.  So:
+// codes and operand.  So (EK = 64 elements of a step per wave, or 128 where workgroups have a CU to themselves):
 //  - NT is as large as the grid allows: the activations are decoded once per workgroup (WN = 1), whatever its rows.
 //  - Codes travel by LDS-direct loads in whole rows of 128 to 512 bytes, scale bytes in 64-byte windows (1024 elements): with
 //    16-byte windows, or straight to registers, the cache lines fetched for scale bytes outweigh the codes.
@@ -49,11 +49,11 @@ __device__ __forceinline__ void wait_vmcnt(int n) {
 // 14336 x 4352 17.8 / 26 / 26.4, now 10.9 / 14 / 16.9; 6144 x 4352 10.0 / 14.6 / 17.1, now 7.8 / 8.8 / 11.5; 4096 x 4352 6.6 / 9.0 /
 // 12.5, now 6.0 / 6.9 / 9.4; 4096 x 14592 16.9 / 20.8 / 22.2, now 12.1 / 15.3 / 21.3.
 // ---------------------------------------------------------------------------------------------
-template <int MT, int NT, int WN, int WK, int NS>
+template <int MT, int NT, int WN, int WK, int NS, int EK = 64>
 struct StreamShape {
   static constexpr int NW = WN * WK, BN = 16 * NT * WN, BM = 16 * MT;
-  static constexpr int RB = 32 * WK;             // code bytes of a row in one step (64 elements per wave)
-  static constexpr int SB = WK >= 16 ? 1 : 16 / WK;  // steps per scale window of 64 bytes
+  static constexpr int RB = EK / 2 * WK;         // code bytes of a row in one step (EK elements per wave)
+  static constexpr int SB = RB >= 512 ? 1 : 512 / RB;  // steps per scale window of 64 bytes
   static constexpr int NB = (NS + SB - 2) / SB + 1;  // windows on their way or in use
   static constexpr int kCodes = NS * (BN + BM) * RB, kScales = NB * (BN + BM) * 64;
   static constexpr int kLds = kCodes + kScales;
@@ -62,9 +62,9 @@ struct StreamShape {
   static_assert(NW * kBatch * 1024 <= kLds, "a batch of sums fits");
 };
 
-template <int MT, int NT, int WN, int WK, int NS, bool GROUPED>
+template <int MT, int NT, int WN, int WK, int NS, bool GROUPED, int EK = 64>
 __device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, int m_base, uint8_t *smem) {
-  using S = StreamShape<MT, NT, WN, WK, NS>;
+  using S = StreamShape<MT, NT, WN, WK, NS, EK>;
   constexpr int NW = S::NW, BN = S::BN, BM = S::BM, RB = S::RB, SB = S::SB, NB = S::NB;
   constexpr int CPR = RB / 16, RPI = 64 / CPR;      // 16-byte chunks per row, rows per load instruction
   constexpr int WI = BN / RPI, NI = (BN + BM) / RPI;  // load instructions of the weights and of both operands per step
@@ -131,9 +131,9 @@ __device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, 
 #pragma unroll
     for (auto &b : a) b = v4f{0.f, 0.f, 0.f, 0.f};
   const int w_row = 16 * NT * wn + r, x_row = BN + r;
-  const int chunk = 2 * wk + (g >> 1);
-  const int w_rd = w_row * RB + ((chunk ^ swizzle(w_row)) << 4) + (g & 1) * 8;
-  const int x_rd = x_row * RB + ((chunk ^ swizzle(r)) << 4) + (g & 1) * 8;
+  const int chunk = EK == 64 ? 2 * wk + (g >> 1) : 4 * wk + g, in_chunk = EK == 64 ? (g & 1) * 8 : 0;
+  const int w_rd = w_row * RB + ((chunk ^ swizzle(w_row)) << 4) + in_chunk;
+  const int x_rd = x_row * RB + ((chunk ^ swizzle(r)) << 4) + in_chunk;
   const int swz_s = (r >> 2) & 3;
 
   auto compute = [&](int kt, int st, int win) {
@@ -171,6 +171,60 @@ __device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, 
       }
     }
   };
+  // The same with 128 elements of a step per wave (EK = 128): a lane's 32 codes are one 16-byte read, their two scale bytes another one, and
+  // the products of one quarter run with the decoding of the next between them.
+  struct Operands {
+    v8h w[NT], x[MT];
+  };
+  Operands quarter[EK == 128 ? 2 : 1];
+  if constexpr (EK == 128) {
+#pragma unroll
+    for (auto &v : quarter[1].w) v = v8h{};
+#pragma unroll
+    for (auto &v : quarter[1].x) v = v8h{};
+  }
+  auto multiply = [&](const Operands &o) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(o.w[i], o.x[j], acc[i][j], 0, 0, 0);
+  };
+  auto compute128 = [&](int kt, int st, int win) {
+    const int c = kt * WK + wk;  // this wave's 128 elements
+    const int piece = c >> 1;
+    const int sb = (((piece & 3) ^ swz_s) << 4) + 8 * (c & 1) + 2 * g + ((ksc & 15) && piece == (ksc >> 4) ? 8 : 0);
+    const uint8_t *cs = smem + st * ((BN + BM) * RB), *ss = smem + S::kCodes + win * ((BN + BM) * 64) + sb;
+    uint4 wq[NT], xq[MT];
+    uint32_t wsc[NT], xsc[MT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      wq[i] = *reinterpret_cast<const uint4 *>(cs + w_rd + i * (16 * RB));
+      wsc[i] = *reinterpret_cast<const uint16_t *>(ss + (w_row + 16 * i) * 64);
+    }
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+      xq[j] = *reinterpret_cast<const uint4 *>(cs + x_rd + j * (16 * RB));
+      xsc[j] = *reinterpret_cast<const uint16_t *>(ss + (x_row + 16 * j) * 64);
+    }
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      multiply(quarter[(h & 1) ^ 1]);  // (the step before's last quarter first)
+      Operands &next = quarter[h & 1];
+      auto scale = [&](uint32_t &two) { return ((h < 2 ? two & 0xffu : two >> 8) << 7) + 0x1800u; };
+      auto dword = [&](const uint4 &q) { return h == 0 ? q.x : h == 1 ? q.y : h == 2 ? q.z : q.w; };
+#pragma unroll
+      for (int j = 0; j < MT; ++j) next.x[j] = decode8_nvfp4_f16<false>(dword(xq[j]), scale(xsc[j]));
+#pragma unroll
+      for (int i = 0; i < NT; ++i) next.w[i] = decode8_nvfp4_f16<false>(dword(wq[i]), scale(wsc[i]));
+      constexpr int kEach = (10 * (NT + MT) + NT * MT - 1) / (NT * MT);
+#pragma unroll
+      for (int k = 0; k < NT * MT; ++k) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, kEach, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
   auto barrier = [&]() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
@@ -189,12 +243,17 @@ __device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, 
     wait_vmcnt(younger);
     barrier();  // step kt is there, and everyone is done with the stage of step kt - 1
     if (kt + NS - 1 < nk) request(kt + NS - 1, st_req, win_req);
-    compute(kt, st, win);
+    if constexpr (EK == 64)
+      compute(kt, st, win);
+    else if ((kt * WK + wk) * 64 < kbytes)
+      compute128(kt, st, win);
     st = st == NS - 1 ? 0 : st + 1;
     st_req = st_req == NS - 1 ? 0 : st_req + 1;
     if ((kt + 1) % SB == 0) win = win == NB - 1 ? 0 : win + 1;
     if ((kt + NS) % SB == 0) win_req = win_req == NB - 1 ? 0 : win_req + 1;
   }
+
+  if constexpr (EK == 128) multiply(quarter[1]);
 
   // the sums of the waves that share a tile meet in LDS, added in the order of K
   float4 *red = reinterpret_cast<float4 *>(smem);
@@ -271,9 +330,9 @@ __device__ __forceinline__ void nv_stream_tile(const GemmParams &p, int n_base, 
   }
 }
 
-template <int MT, int NT, int WN, int WK, int NS, bool GROUPED>
+template <int MT, int NT, int WN, int WK, int NS, bool GROUPED, int EK = 64>
 __global__ __launch_bounds__(64 * WN * WK) void gemm_nvfp4_stream(GemmParams p) {
-  using S = StreamShape<MT, NT, WN, WK, NS>;
+  using S = StreamShape<MT, NT, WN, WK, NS, EK>;
   __shared__ uint4 smem[S::kLds / 16];
   uint8_t *lds = reinterpret_cast<uint8_t *>(smem);
   int lin;
@@ -292,20 +351,21 @@ __global__ __launch_bounds__(64 * WN * WK) void gemm_nvfp4_stream(GemmParams p) 
     if (MT > 2 && rows <= 32) return nv_stream_tile<2, NT, WN, WK, NS, GROUPED>(p, n_base, m_base, lds);
     if (MT > 3 && rows <= 48) return nv_stream_tile<3, NT, WN, WK, NS, GROUPED>(p, n_base, m_base, lds);
   }
-  nv_stream_tile<MT, NT, WN, WK, NS, GROUPED>(p, n_base, m_base, lds);
+  nv_stream_tile<MT, NT, WN, WK, NS, GROUPED, EK>(p, n_base, m_base, lds);
 }
 
-template <int MT, int NT, int WN, int WK, int NS, bool GROUPED = false>
+template <int MT, int NT, int WN, int WK, int NS, bool GROUPED = false, int EK = 64>
 int launch(const GemmParams &p, hipStream_t st) {
-  using S = StreamShape<MT, NT, WN, WK, NS>;
+  using S = StreamShape<MT, NT, WN, WK, NS, EK>;
   const int total = ((p.M + S::BM - 1) / S::BM + (GROUPED ? p.n_seg : 0)) * ((p.N + S::BN - 1) / S::BN);
-  hipLaunchKernelGGL((gemm_nvfp4_stream<MT, NT, WN, WK, NS, GROUPED>), dim3(grid_in_turn<GROUPED ? 2 : 1>(total)), dim3(64 * S::NW), 0, st, p);
+  hipLaunchKernelGGL((gemm_nvfp4_stream<MT, NT, WN, WK, NS, GROUPED, EK>), dim3(grid_in_turn<GROUPED ? 2 : 1>(total)), dim3(64 * S::NW), 0, st, p);
   ARCQ_HIP_TRY(hipGetLastError());
   return ARCQ_OK;
 }
 
 // Rows per workgroup.  Up to 12288 rows of weights make at most one workgroup per CU of 16, 32 or 48 rows, which then has
-// sixteen waves (us at 16 rows: 6144 x 4352 7.8, eight waves 8.9; 10240 x 8320 15.0 and 17.6).  Beyond, eight waves, and the
+// sixteen waves, or eight that take 128 elements of a step each (us at 16 rows: 6144 x 4352 7.8, eight waves of 64 elements 8.9; 10240 x
+// 8320 15.0 and 17.6; at 16, 32, 64 rows of 6144 x 4352 sixteen waves 6.8, 8.0, 11.0, eight of 128 elements 6.5, 7.7, 10.7).  Beyond, eight waves, and the
 // rows per workgroup by how many rounds of 256 workgroups they make: the rows and activation rows of a CU's workgroups
 // together, a quarter more where up to 32 rows, or a K' of one or two steps, have a single workgroup per CU to themselves (nothing else
 // asks for weights while it starts, waits and ends): 28672 rows take 64 per workgroup up to 32 rows and 112 above (64 rows, K' = 4352:
@@ -313,7 +373,7 @@ int launch(const GemmParams &p, hipStream_t st) {
 template <int MT>
 int launch_plain(const GemmParams &p, hipStream_t st) {
   if (p.N <= 4096) return launch<MT, 1, 1, 16, (MT == 1 ? 3 : 2)>(p, st);
-  if (p.N <= 8192) return launch<MT, 2, 1, 16, 2>(p, st);
+  if (p.N <= 8192) return launch<MT, 2, 1, 8, 2, false, 128>(p, st);
   if (p.N <= 12288) return launch<MT, 3, 1, 16, 2>(p, st);
   int best = 0;
   double least = 0;
@@ -388,15 +448,19 @@ bool nvfp4_stream_wanted(int M, int N, int Kp, int n_seg, bool swiglu) {
 // do not.  A workgroup's time per K' = 4352 and its wait to start and end (6 us; less for the smallest shapes, as long as they make one
 // round), measured, by shape; where workgroups have a CU to themselves, each of several rounds takes an eighth more (us; workgroups of 1
 // to 14 per CU; 1900 problems of 65 to 1024 rows, 256 to 28672 weight rows and K' = 512 to 14592 to within 10 % in one round):
+// The larger shapes, whose workgroups have a CU to themselves in one round anyway, then take 128 elements of a step per wave (`one`): half as
+// many LDS reads, barriers and waits, twice the bytes on their way.  us, 64 elements and 128: 333 x 6144 x 4352 27.9 / 25.4, 400 x 4096 x
+// 4352 25.1 / 22.4, 512 x 4096 x 4352 25.5 / 23.1, 300 x 4608 x 3712 26.4 / 23.8.  (In several rounds two of the workgroups of 64 share a CU.)
 struct MidShape {
   int mt, nt, wn, wk;
   double us, rounds;
   double short_start, short_us;
+  double one;
 };
 constexpr double kMidStart = 6;
-constexpr MidShape kMid[] = {{4, 3, 1, 8, 8.2, 1.0, 4.0, 10.0}, {4, 4, 1, 8, 9.8, 1.0, 4.7, 11.8},   {5, 3, 1, 8, 9.2, 1.0, 4.7, 11.3},
-                             {6, 4, 1, 8, 14.8, 1.12, 6, 14.8}, {7, 3, 1, 8, 13.8, 1.12, 6, 13.8},   {5, 3, 2, 4, 16.6, 1.0, 6, 16.6},
-                             {4, 4, 2, 4, 18.0, 1.0, 6, 18.0},  {6, 3, 2, 4, 22.5, 1.0, 6, 22.5},    {5, 4, 2, 4, 25.0, 1.0, 6, 25.0}};
+constexpr MidShape kMid[] = {{4, 3, 1, 8, 8.2, 1.0, 4.0, 10.0, 8.2},    {4, 4, 1, 8, 9.8, 1.0, 4.7, 11.8, 9.8},    {5, 3, 1, 8, 9.2, 1.0, 4.7, 11.3, 9.2},
+                             {6, 4, 1, 8, 14.8, 1.12, 6, 14.8, 14.8}, {7, 3, 1, 8, 13.8, 1.12, 6, 13.8, 13.8}, {5, 3, 2, 4, 16.6, 1.0, 6, 16.8, 16.8},
+                             {4, 4, 2, 4, 18.0, 1.0, 6, 17.6, 17.6},  {6, 3, 2, 4, 22.5, 1.0, 6, 19.8, 19.8},  {5, 4, 2, 4, 25.0, 1.0, 6, 21.5, 21.5}};
 
 // The shape for a problem that the plan would give to 128x64 (21, K in `slices`), 128x128 (22) or 256x128 tiles (42), -1 where those
 // are faster by their own measured times (`always`: the best one whatever theirs are).  Over 1888 measured problems 0.81 of the tiles'
@@ -423,13 +487,22 @@ int nvfp4_mid_shape(int M, int N, int Kp, int kernel, int slices, bool always) {
   for (int i = 0; i < (int)(sizeof(kMid) / sizeof(kMid[0])); ++i) {
     const MidShape &s = kMid[i];
     const double r = rounds(tiles(16 * s.mt, 16 * s.nt * s.wn));
-    const double us = r > 1 ? kMidStart + s.us * k * r * s.rounds : std::min(kMidStart + s.us * k, s.short_start + s.short_us * k);
+    const double us = r > 1 ? kMidStart + s.us * k * r * s.rounds : std::min(kMidStart + s.one * k, s.short_start + s.short_us * k);
     if (us < least) best = i, least = us;
   }
   return best;
 }
 
 int run_nvfp4_mid(const GemmParams &p, int shape, hipStream_t st) {
+  if (shape < 0 || shape >= (int)(sizeof(kMid) / sizeof(kMid[0]))) return ARCQ_ERR_SHAPE;
+  const int bm = 16 * kMid[shape].mt, bn = 16 * kMid[shape].nt * kMid[shape].wn;
+  if ((long)((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn) <= 256) switch (shape) {
+      case 5: return launch<5, 3, 2, 4, 2, false, 128>(p, st);
+      case 6: return launch<4, 4, 2, 4, 2, false, 128>(p, st);
+      case 7: return launch<6, 3, 2, 4, 2, false, 128>(p, st);
+      case 8: return launch<5, 4, 2, 4, 2, false, 128>(p, st);
+      default: break;
+    }
   switch (shape) {
     case 0: return launch<4, 3, 1, 8, 2>(p, st);
     case 1: return launch<4, 4, 1, 8, 2>(p, st);

@@ -662,3 +662,23 @@ def test_swiglu_of_weights_as_they_are_for_others(agemm, monkeypatch):
 
     monkeypatch.setattr(torch, "empty", full)
     assert agemm.matmul_swiglu(a, b, sfa, sfb, gx * gw, tensor_scale=True, halves=True) is None
+
+
+@pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
+@pytest.mark.parametrize("M,N,kp,route", [
+    (8, 8192, 4224, 3), (5, 5121, 4096, 3), (17, 6145, 2176, 3), (33, 6144, 1152, 3), (48, 5121, 1152, 3), (64, 8190, 4224, 3), (64, 4112, 8320, 3),
+    (523, 3001, 1792, 21), (349, 4099, 2048, 21), (375, 5122, 2432, 22), (297, 6145, 1664, 22), (644, 3001, 1536, 23), (326, 6144, 1792, 23),
+    (333, 6144, 1152, 23), (556, 4099, 2048, 24), (80, 28672, 640, 24)])
+def test_nvfp4_steps_of_128_elements_per_wave(agemm, oracle, M, N, kp, route):
+    """the streams whose waves take 128 elements of a step: K' ending after any number of waves' shares of the last step and inside a
+    16-byte piece of scale bytes, rows and columns ending inside a tile; exact products and fp32 sums as for the other shapes"""
+    from arcquant_amd import _lib
+    assert _lib.lib().arcq_gemm_route(M, N, kp, 0, 0, 0) == route
+    (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, kp - 64, 64, "NVFP4", seed=91)
+    want = oracle_dq(oracle, a, sfa, "NVFP4") @ oracle_dq(oracle, b, sfb, "NVFP4").T * (gx * gw)
+    scale = (torch.tensor(gx, device="cuda"), torch.tensor(gw, device="cuda"))
+    y = agemm.matmul(a, b, sfa, sfb, scale)
+    assert rel_fro(y.float(), want) < 2.5e-3
+    assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
+    res = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
+    assert torch.equal(agemm.matmul(a, b, sfa, sfb, scale, residual=res), y + res)
