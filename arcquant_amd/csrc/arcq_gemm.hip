@@ -726,7 +726,7 @@ __global__ __launch_bounds__(128 * NWM) void gemm_nvfp4_tiled(GemmParams p) {
 // ---------------------------------------------------------------------------------------------
 // Skinny kernels for M <= 64 (decode batches; NVFP4: few rows, narrow layers and a short K', see kStreamFrom): the GEMM is a stream of the weight matrix, read
 // exactly once, so nothing is staged through LDS.  A workgroup owns 16 weight rows; its NW waves
-// take the K steps of 128 round-robin in pairs (split-K: with four waves wave w does steps 2w, 2w+1, 2w+8, 2w+9, ...:
+// take the K steps of 128 round-robin in pairs (split-K; MXFP4 in runs of four: with four waves wave w does steps 2w, 2w+1, 2w+8, 2w+9, ...:
 // a pair of steps is one whole 128-byte line of every row, and the four waves walk neighbouring lines) and their partial sums meet in LDS.  A lane loads
 // the 16 bytes (32 codes) the 16x16 MFMA wants from it straight from global memory: row lane%16,
 // K group lane/16, i.e. 64 contiguous bytes per row and step.  The activations (<= 64 rows) come
@@ -778,7 +778,7 @@ template <int MT, int AT, int NW>
 __global__ __launch_bounds__(64 * NW) void gemm_mxfp4_skinny(GemmParams p) {
   __shared__ float red[NW - 1][MT * AT][64][4];
   constexpr int D = (MT * AT >= 4) ? 4 : 8;  // K steps whose loads are in flight together
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int T = p.Kp >> 7;
   const size_t rowb = (size_t)(p.Kp >> 1), rows = (size_t)(p.Kp >> 5);
@@ -799,35 +799,51 @@ __global__ __launch_bounds__(64 * NW) void gemm_mxfp4_skinny(GemmParams p) {
 #pragma unroll
   for (int j = 0; j < AT * MT; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
   const uint32_t sh = 8u * (uint32_t)g;
-  for (int t0 = 2 * wave; t0 < T; t0 += NW * D) {
-    uint4 a[AT][D], b[MT][D];
-    uint32_t sa[AT][D], sb[MT][D];
+  // A wave takes runs of four steps (two lines of codes per row, 16 scale bytes) NW runs apart: the scale bytes of a run are one load.  us,
+  // a load per step and pairs of steps by wave, and so: 8 x 4096 x 14592 11.8 / 10.7, 16 rows 14.4 / 12.9, 20 rows 16.5 / 14.9; 8 x 3584 x
+  // 19072 14.2 / 11.6; 3 x 28672 x 4352 17.6 / 15.3; 16 x 6144 x 4352 7.2 / 6.7.
+  auto scales_of = [&](const uint8_t *row, int t) {
+    const uint8_t *at = row + 4 * t;
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (t + 4 <= T) {  // (4-byte aligned)
+      __builtin_memcpy(&v, at, 16);
+      return v;
+    }
+    if (t < T) __builtin_memcpy(&v.x, at, 4);
+    if (t + 1 < T) __builtin_memcpy(&v.y, at + 4, 4);
+    if (t + 2 < T) __builtin_memcpy(&v.z, at + 8, 4);
+    return v;
+  };
+  auto dword = [](const uint4 &v, int d) { return d == 0 ? v.x : d == 1 ? v.y : d == 2 ? v.z : v.w; };
+  for (int t0 = 4 * wave; t0 < T; t0 += NW * D) {
+    uint4 a[AT][D], b[MT][D], sa[AT][D / 4], sb[MT][D / 4];
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int t = t0 + 2 * NW * (d >> 1) + (d & 1);
-      if (t < T) {  // uniform over the wave
+    for (int k = 0; k < D / 4; ++k) {
+      const int t1 = t0 + 4 * NW * k;
+      if (t1 >= T) continue;  // (uniform over the wave, as all of these)
 #pragma unroll
-        for (int i = 0; i < AT; ++i) {
-          a[i][d] = *reinterpret_cast<const uint4 *>(wc[i] + 64 * t);
-          sa[i][d] = *reinterpret_cast<const uint32_t *>(ws[i] + 4 * t);
+      for (int i = 0; i < AT; ++i) sa[i][k] = scales_of(ws[i], t1);
+#pragma unroll
+      for (int j = 0; j < MT; ++j) sb[j][k] = scales_of(xs[j], t1);
+#pragma unroll
+      for (int d = 0; d < 4; ++d)
+        if (t1 + d < T) {
+#pragma unroll
+          for (int i = 0; i < AT; ++i) a[i][4 * k + d] = *reinterpret_cast<const uint4 *>(wc[i] + 64 * (t1 + d));
+#pragma unroll
+          for (int j = 0; j < MT; ++j) b[j][4 * k + d] = *reinterpret_cast<const uint4 *>(xc[j] + 64 * (t1 + d));
         }
-#pragma unroll
-        for (int j = 0; j < MT; ++j) {
-          b[j][d] = *reinterpret_cast<const uint4 *>(xc[j] + 64 * t);
-          sb[j][d] = *reinterpret_cast<const uint32_t *>(xs[j] + 4 * t);
-        }
-      }
     }
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      if (t0 + 2 * NW * (d >> 1) + (d & 1) < T) {
+      if (t0 + 4 * NW * (d / 4) + d % 4 < T) {
 #pragma unroll
         for (int i = 0; i < AT; ++i)
 #pragma unroll
           for (int j = 0; j < MT; ++j)
             acc[i * MT + j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                fp4_operand(a[i][d]), fp4_operand(b[j][d]), acc[i * MT + j], 4, 4, 0, (int)(sa[i][d] >> sh), 0,
-                (int)(sb[j][d] >> sh));
+                fp4_operand(a[i][d]), fp4_operand(b[j][d]), acc[i * MT + j], 4, 4, 0, (int)(dword(sa[i][d / 4], d % 4) >> sh), 0,
+                (int)(dword(sb[j][d / 4], d % 4) >> sh));
       }
     }
   }
@@ -902,7 +918,9 @@ int launch_skinny(const GemmParams &p, hipStream_t st) {
   const int grid = (p.N + 16 * AT - 1) / (16 * AT);
   const bool eight = grid <= 512 && AT == 1;
   if (FMT == ARCQ_FMT_MXFP4) {
-    if (eight)
+    if (MT == 1 && grid <= 256 && p.Kp >= 8192)  // a workgroup per CU: all of a long row on its way at once (8 x 4096 x 14592: 10.7 / 10.2 us)
+      hipLaunchKernelGGL((gemm_mxfp4_skinny<1, 1, 16>), dim3(grid), dim3(1024), 0, st, p);
+    else if (eight)
       hipLaunchKernelGGL((gemm_mxfp4_skinny<MT, 1, 8>), dim3(grid), dim3(512), 0, st, p);
     else
       hipLaunchKernelGGL((gemm_mxfp4_skinny<MT, AT, 4>), dim3(grid), dim3(256), 0, st, p);

@@ -698,17 +698,28 @@ __global__ __launch_bounds__(64 * kDecodeWaves) void kv_decode_i4_mfma_kernel(ui
   }
 }
 
-// one workgroup of 128 threads per (sequence, query head): softmax-weighted sum of the ranges' partials
+// one workgroup of 128 threads per (sequence, query head): softmax-weighted sum of the ranges' partials.  What bounds it is latency: all
+// ranges' values are asked for before the first one is used.
+constexpr int kMaxSplits = 16;
 template <bool BF16>
 __global__ __launch_bounds__(128) void kv_decode_merge_kernel(uint16_t *o, const float *partial, int splits) {
   const float *src = partial + (size_t)blockIdx.x * splits * kPartialStride;
+  float m[kMaxSplits], l[kMaxSplits], v[kMaxSplits];
+#pragma unroll
+  for (int z = 0; z < kMaxSplits; ++z) {
+    const float *at = src + min(z, splits - 1) * kPartialStride;  // (ranges behind the last one: its values, without weight)
+    m[z] = at[0], l[z] = at[1], v[z] = at[2 + threadIdx.x];
+  }
   float M = -1e30f;
-  for (int z = 0; z < splits; ++z) M = fmaxf(M, src[z * kPartialStride]);
+#pragma unroll
+  for (int z = 0; z < kMaxSplits; ++z) M = fmaxf(M, m[z]);
   float num = 0.0f, den = 0.0f;
-  for (int z = 0; z < splits; ++z) {
-    const float wgt = __builtin_amdgcn_exp2f(src[z * kPartialStride] - M);
-    num = __builtin_fmaf(wgt, src[z * kPartialStride + 2 + threadIdx.x], num);
-    den = __builtin_fmaf(wgt, src[z * kPartialStride + 1], den);
+#pragma unroll
+  for (int z = 0; z < kMaxSplits; ++z) {
+    if (z >= splits) break;
+    const float wgt = __builtin_amdgcn_exp2f(m[z] - M);
+    num = __builtin_fmaf(wgt, v[z], num);
+    den = __builtin_fmaf(wgt, l[z], den);
   }
   const float out = den > 0.0f ? num / den : 0.0f;
   o[(size_t)blockIdx.x * kHeadDim + threadIdx.x] = (uint16_t)to_bits<BF16>(out);
@@ -877,7 +888,7 @@ int arcq_kv_decode_i4(void *o, const void *q, int dtype, int batch, int num_qo_h
     const long pairs = (long)batch * num_kv_heads;
     const int split_env = tuning().kv_decode_splits;
     splits = split_env > 0 ? split_env : (pairs >= 256 ? 1 : (int)((512 + pairs - 1) / pairs));
-    if (splits > 16) splits = 16;
+    if (splits > kMaxSplits) splits = kMaxSplits;
     if (splits > 1 &&
         (size_t)batch * num_qo_heads * splits * kPartialStride * sizeof(float) > kWorkspaceBytes[kWsDecode])
       splits = 1;

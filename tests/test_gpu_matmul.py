@@ -682,3 +682,17 @@ def test_nvfp4_steps_of_128_elements_per_wave(agemm, oracle, M, N, kp, route):
     assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
     res = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
     assert torch.equal(agemm.matmul(a, b, sfa, sfb, scale, residual=res), y + res)
+
+
+@pytest.mark.parametrize("M,N,kp", [(1, 24, 128), (3, 100, 256), (8, 4096, 384), (16, 513, 640), (5, 4096, 8320), (16, 4090, 8448), (8, 2048, 8576), (1, 4096, 8192),
+                                    (17, 1000, 896), (40, 4096, 1408), (64, 333, 4352), (4, 8200, 1152), (33, 4096, 8320), (8, 6144, 8576)])
+def test_mxfp4_decode_batches(agemm, oracle, M, N, kp):
+    """MXFP4 decode batches straight from global memory: K' ending after one to four steps of a wave's run, fewer runs than waves and many
+    more, sixteen waves for long rows; the bf16 rounding and the order of the fp32 sum remain"""
+    (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, kp - 64, 64, "MXFP4", seed=93)
+    want = oracle_dq(oracle, a, sfa, "MXFP4") @ oracle_dq(oracle, b, sfb, "MXFP4").T * 0.5
+    y = agemm.matmul(a, b, sfa, sfb, 0.5, fmt="MXFP4")
+    assert rel_fro(y.float(), want) < 2.5e-3
+    assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
+    res = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
+    assert torch.equal(agemm.matmul(a, b, sfa, sfb, 0.5, fmt="MXFP4", residual=res), y + res)
