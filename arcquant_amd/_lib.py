@@ -102,6 +102,8 @@ def lib() -> ctypes.CDLL:
     L.arcq_rmsnorm.restype = i
     L.arcq_attention_prefill.argtypes = [vp, i, vp, i, vp, i, i, i, i, i, i, f, vp, i, vp]
     L.arcq_attention_prefill.restype = i
+    L.arcq_attention_prefill_rope.argtypes = [vp, i, vp, vp, i, vp, i, vp, i, i, i, i, i, i, f, vp, i, vp]
+    L.arcq_attention_prefill_rope.restype = i
     L.arcq_gemm_workspace_bytes.argtypes = [i, i, i, i, i]
     L.arcq_gemm_workspace_bytes.restype = sz
     L.arcq_gemm_scratch_bytes.argtypes = [i, i, i, i, i]

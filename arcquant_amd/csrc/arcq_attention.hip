@@ -16,6 +16,8 @@ struct AttentionParams {
   int ldq, ldk, ldv, ldo;     // elements from token to token
   int batch, seq, heads, kv_heads;
   float scale;                // of q k^T, times log2 e
+  const uint16_t *cos, *sin;  // [positions, 64], of queries that are not rotated yet
+  int positions;
 };
 
 typedef short v4s __attribute__((ext_vector_type(4)));
@@ -43,10 +45,24 @@ typedef v4s __attribute__((address_space(3))) lds_v4s;
 // (763 TFLOP/s; 339 in a layer), 4 x 1024 163 -> 58, 3 x 777, 28 heads, 4 KV heads 108 -> 39, 1 x 100 22 -> 11.  (Sequences of one token, 28
 // heads, 64 of them: 6.7 -> 16.9.)
 //
+// ROTATE: the queries come as the projection left them and take their rotary embedding in registers.  Channels c and c + 64 of a query
+// are the same lane's, every (query, head) is some workgroup's once, and the products are rounded as rope_rows_kernel rounds them: the
+// same bits, without q written and read again.  Rotary pass + attention, us, q in the pass / here: 8 x 2048 tokens, 32 heads, 8 KV heads
+// 71 + 354 / 19 + 367, 4096 tokens 23 + 67 / 8 + 71; a layer of 8 x 2048 tokens 5672 / 5624, of 4096 (MXFP4) 650 / 638.
+//
 // XCDs get contiguous runs of (sequence, KV head) groups, whose K and V their L2 then holds, the longest query tiles first.
 // ---------------------------------------------------------------------------------------------
 constexpr int kQ = 128, kKeys = 64, kStage = kKeys * 256;
 
+// two channels of a query and the two 64 further on, each a pair of bf16: x cos - y sin and y cos + x sin, every product and sum rounded
+__device__ __forceinline__ void rotate(uint32_t &x, uint32_t &y, uint32_t cs, uint32_t sn) {
+  const float x0 = u2f(x << 16), x1 = u2f(x & 0xffff0000u), y0 = u2f(y << 16), y1 = u2f(y & 0xffff0000u);
+  const float c0 = u2f(cs << 16), c1 = u2f(cs & 0xffff0000u), s0 = u2f(sn << 16), s1 = u2f(sn & 0xffff0000u);
+  x = add_bf16_pair(pack_bf16_rne(x0 * c0, x1 * c1), pack_bf16_rne(-y0 * s0, -y1 * s1));
+  y = add_bf16_pair(pack_bf16_rne(y0 * c0, y1 * c1), pack_bf16_rne(x0 * s0, x1 * s1));
+}
+
+template <bool ROTATE>
 __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(AttentionParams p) {
   __shared__ uint4 smem[4 * kStage / 16];  // K and V, two stages each
   const int tid = threadIdx.x, lane = tid & 63;
@@ -69,6 +85,19 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(AttentionPara
     const uint16_t *src = p.q + (row0 + min(qw + r, p.seq - 1)) * p.ldq + head * 128 + 8 * h;
 #pragma unroll
     for (int c = 0; c < 8; ++c) qf[c] = __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4 *>(src + 16 * c));
+    if constexpr (ROTATE) {
+      const int at = min(min(qw + r, p.seq - 1), p.positions - 1) * 64 + 8 * h;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint4 cs = *reinterpret_cast<const uint4 *>(p.cos + at + 16 * c), sn = *reinterpret_cast<const uint4 *>(p.sin + at + 16 * c);
+        uint4 x = __builtin_bit_cast(uint4, qf[c]), y = __builtin_bit_cast(uint4, qf[c + 4]);
+        rotate(x.x, y.x, cs.x, sn.x);
+        rotate(x.y, y.y, cs.y, sn.y);
+        rotate(x.z, y.z, cs.z, sn.z);
+        rotate(x.w, y.w, cs.w, sn.w);
+        qf[c] = __builtin_bit_cast(v8bf, x), qf[c + 4] = __builtin_bit_cast(v8bf, y);
+      }
+    }
   }
 
   // ---- global -> LDS: four instructions per wave, tile and operand, four keys each
@@ -204,29 +233,45 @@ __global__ __launch_bounds__(256, 2) void attention_prefill_kernel(AttentionPara
   }
 }
 
-}  // namespace
-}  // namespace arcq
-
-extern "C" int arcq_attention_prefill(const void *q, int ldq, const void *k, int ldk, const void *v, int ldv, int batch, int seq,
-                                      int num_qo_heads, int num_kv_heads, int head_dim, float sm_scale, void *o, int ldo, void *stream) {
-  using namespace arcq;
+// cos_t, sin_t: null for rotated queries
+int attention_entry(const void *q, int ldq, bool rotate, const void *cos_t, const void *sin_t, int positions, const void *k, int ldk,
+                    const void *v, int ldv, int batch, int seq, int num_qo_heads, int num_kv_heads, int head_dim, float sm_scale, void *o,
+                    int ldo, void *stream) {
   const float scale = sm_scale * 1.44269504088896341f;
   if (!(scale > 0.0f) || std::isinf(scale)) return ARCQ_ERR_SHAPE;  // the maximum is taken, and masked, ahead of the scale
   if (batch < 0 || seq < 0 || head_dim != 128 || num_kv_heads < 1 || num_qo_heads < num_kv_heads || num_qo_heads % num_kv_heads != 0)
     return ARCQ_ERR_SHAPE;
   const int need_q = num_qo_heads * 128, need_kv = num_kv_heads * 128;
+  if (rotate && (positions < 1 || positions > (1 << 24))) return ARCQ_ERR_SHAPE;
   if (ldq < need_q || ldo < need_q || ldk < need_kv || ldv < need_kv || (ldq | ldk | ldv | ldo) % 8 != 0) return ARCQ_ERR_SHAPE;
   // 32-bit byte offsets of a sequence's keys
   if ((size_t)seq * (size_t)std::max(ldk, ldv) * 2 >= ((size_t)1 << 32)) return ARCQ_ERR_SHAPE;
   if (batch == 0 || seq == 0) return ARCQ_OK;
-  if (!q || !k || !v || !o) return ARCQ_ERR_NULL;
-  if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o)) return ARCQ_ERR_ALIGN;
+  if (!q || !k || !v || !o || (rotate && (!cos_t || !sin_t))) return ARCQ_ERR_NULL;
+  if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o) || !aligned16(cos_t) || !aligned16(sin_t)) return ARCQ_ERR_ALIGN;
   const long total = (long)batch * num_qo_heads * ((seq + kQ - 1) / kQ);
   if (total > (1l << 30)) return ARCQ_ERR_SHAPE;
   AttentionParams p{static_cast<const uint16_t *>(q), static_cast<const uint16_t *>(k), static_cast<const uint16_t *>(v),
                     static_cast<uint16_t *>(o), ldq, ldk, ldv, ldo, batch, seq, num_qo_heads, num_kv_heads,
-                    scale};
-  hipLaunchKernelGGL(attention_prefill_kernel, dim3((unsigned)(((total + 7) / 8) * 8)), dim3(256), 0, static_cast<hipStream_t>(stream), p);
+                    scale,  static_cast<const uint16_t *>(cos_t),  static_cast<const uint16_t *>(sin_t),  positions};
+  const auto kernel = rotate ? attention_prefill_kernel<true> : attention_prefill_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(((total + 7) / 8) * 8)), dim3(256), 0, static_cast<hipStream_t>(stream), p);
   ARCQ_HIP_TRY(hipGetLastError());
   return ARCQ_OK;
+}
+
+}  // namespace
+}  // namespace arcq
+
+extern "C" int arcq_attention_prefill(const void *q, int ldq, const void *k, int ldk, const void *v, int ldv, int batch, int seq,
+                                      int num_qo_heads, int num_kv_heads, int head_dim, float sm_scale, void *o, int ldo, void *stream) {
+  return arcq::attention_entry(q, ldq, false, nullptr, nullptr, 0, k, ldk, v, ldv, batch, seq, num_qo_heads, num_kv_heads, head_dim,
+                               sm_scale, o, ldo, stream);
+}
+
+extern "C" int arcq_attention_prefill_rope(const void *q, int ldq, const void *cos_table, const void *sin_table, int max_positions,
+                                           const void *k, int ldk, const void *v, int ldv, int batch, int seq, int num_qo_heads,
+                                           int num_kv_heads, int head_dim, float sm_scale, void *o, int ldo, void *stream) {
+  return arcq::attention_entry(q, ldq, true, cos_table, sin_table, max_positions, k, ldk, v, ldv, batch, seq, num_qo_heads, num_kv_heads,
+                               head_dim, sm_scale, o, ldo, stream);
 }

@@ -115,7 +115,11 @@ def rope(qkv, q_len, pos0, num_qo_heads, num_kv_heads, cos_table, sin_table):
 def attention_prefill(q, k, v, q_len):
     """Causal attention of whole prompts over their own keys (model/qLlamaLayer.py:340-370): q [tokens, heads, 128], k [tokens,
     kv heads, 128] bf16 contiguous, v [tokens, kv heads * 128] bf16 with rows possibly strided (a slice of the fused projection's
-    output), q_len tokens per sequence.  Returns [tokens, heads * 128]; None for operands that arcq_attention_prefill does not take."""
+    output), q_len tokens per sequence.  Returns [tokens, heads * 128]; None for operands that arcq_attention_prefill does not take.
+    q (rows, cos, sin): the queries [tokens, heads * 128] as the projection left them (rows possibly strided) and the tables of
+    rope(): rotated on the way, token t of a sequence at position t, to the bits of rope()'s."""
+    if isinstance(q, tuple):
+        return _attention_prefill_rope(*q, k, v, q_len)
     tokens, heads, d = q.shape
     kv_heads = k.shape[1]
     ld = v.stride(0) if tokens > 1 else v.shape[1]
@@ -129,6 +133,28 @@ def attention_prefill(q, k, v, q_len):
         rc = _lib.lib().arcq_attention_prefill(_ptr(q), heads * d, _ptr(k), kv_heads * d, _ptr(v), int(ld), tokens // q_len,
                                                int(q_len), heads, kv_heads, d, 1.0 / math.sqrt(d), _ptr(o), heads * d, _stream(q))
     _lib.check(rc, "arcq_attention_prefill")
+    return o
+
+
+def _attention_prefill_rope(q, cos, sin, k, v, q_len):
+    tokens, kv_heads, d = k.shape
+    if q.dim() != 2 or v.dim() != 2 or d != 128 or any(t.dtype != torch.bfloat16 or not t.is_cuda or t.device != k.device or t.data_ptr() % 16
+                                                       for t in (q, k, v, cos, sin)):
+        return None
+    heads = q.shape[1] // d
+    ldq, ldv = ((t.stride(0) if tokens > 1 else t.shape[1]) for t in (q, v))
+    if tuple(q.shape) != (tokens, heads * d) or tuple(v.shape) != (tokens, kv_heads * d) or kv_heads < 1 or heads < 1 or heads % kv_heads or \
+            q.stride(1) != 1 or v.stride(1) != 1 or ldq % 8 or ldv % 8 or ldq < heads * d or ldv < kv_heads * d or not k.is_contiguous() or \
+            any(t.dim() != 2 or t.shape[1] != 64 or t.shape[0] != cos.shape[0] or not 1 <= t.shape[0] <= 1 << 24 or not t.is_contiguous()
+                for t in (cos, sin)) or \
+            q_len < 1 or tokens % q_len or 2 * q_len * max(ldv, kv_heads * d) >= 1 << 32 or tokens * heads >= 1 << 30:
+        return None
+    o = torch.empty(tokens, heads * d, dtype=q.dtype, device=q.device)
+    with _lib.on_device_of(q):
+        rc = _lib.lib().arcq_attention_prefill_rope(_ptr(q), int(ldq), _ptr(cos), _ptr(sin), int(cos.shape[0]), _ptr(k), kv_heads * d,
+                                                    _ptr(v), int(ldv), tokens // q_len, int(q_len), heads, kv_heads, d,
+                                                    1.0 / math.sqrt(d), _ptr(o), heads * d, _stream(q))
+    _lib.check(rc, "arcq_attention_prefill_rope")
     return o
 
 

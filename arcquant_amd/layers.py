@@ -324,6 +324,10 @@ class LlamaAttention(nn.Module):
         self.quant_type = quant_type
         self._rope = None                    # cos / sin tables of the fused rotary embedding, built on first use
 
+    def _rotated(self, rows, q_len):
+        q, tables = rows[0], rows[1:]
+        return _kvc.rope(q, q_len, 0, self.num_heads, 0, *tables)[0].view(-1, q_len, self.num_heads, self.head_dim).transpose(1, 2)
+
     @_no_grad
     def forward(self, x, kv_cache=None, past_len=0, layer_idx=0, residual=None):
         """x: quantized hidden states (tuple); residual: added to the output.  kv_cache: None, or (k, v) bf16 [bsz, kv_heads, L, d]
@@ -347,9 +351,15 @@ class LlamaAttention(nn.Module):
             need = past_len + q_len
             if self._rope is None or self._rope[0].shape[0] < need:
                 self._rope = _kvc.rope_tables(max(need, 4096), d, qkv.dtype, qkv.device)
-            q, k = _kvc.rope(qkv.view(bsz * q_len, -1), q_len, past_len, nh, nkv, *self._rope)
-            rows = (q, k, qkv.view(bsz * q_len, -1)[:, (nh + nkv) * d:(nh + 2 * nkv) * d])
-            q = q.view(bsz, q_len, nh, d).transpose(1, 2)
+            flat = qkv.view(bsz * q_len, -1)
+            # a prompt's own keys, read where they are (one token sees itself alone: torch's kernel for it, 64 sequences of 28 heads 6.7
+            # us, has not 128 queries' work, 16.9); the queries are then rotated by the attention, and only the keys here
+            if past_len == 0 and q_len > 1 and not isinstance(kv_cache, tuple) and _plain(flat, *self._rope):
+                k = _kvc.rope(flat[:, nh * d:(nh + nkv) * d], q_len, 0, nkv, 0, *self._rope)[0]
+                rows = ((flat[:, :nh * d], *self._rope), k, flat[:, (nh + nkv) * d:(nh + 2 * nkv) * d])
+            else:
+                q, k = _kvc.rope(flat, q_len, past_len, nh, nkv, *self._rope)
+                q = q.view(bsz, q_len, nh, d).transpose(1, 2)
             k = k.view(bsz, q_len, nkv, d).transpose(1, 2)
         else:
             q = qkv[..., :nh * d].view(bsz, q_len, nh, d).transpose(1, 2)
@@ -358,6 +368,8 @@ class LlamaAttention(nn.Module):
         if kv_cache is not None and not isinstance(kv_cache, tuple):
             r = kv_cache.update(k.transpose(1, 2), v.transpose(1, 2), layer_idx)
             if callable(r):                                   # decode: attention over the INT4 pages
+                if rows is not None:
+                    q = self._rotated(rows[0], q_len)
                 out = r(q.transpose(1, 2)).reshape(bsz, q_len, nh * d)
                 return self.o_proj(quantize_tokens(out, self.o_reorder_index, self.o_proj.select_num,
                                                    self.quant_type), residual)
@@ -367,13 +379,12 @@ class LlamaAttention(nn.Module):
             kc[:, :, past_len:past_len + q_len] = k
             vc[:, :, past_len:past_len + q_len] = v
             k, v = kc[:, :, :past_len + q_len], vc[:, :, :past_len + q_len]
-        # a prompt's own keys, read where they are (one token sees itself alone: torch's kernel for it, 64 sequences of 28 heads 6.7
-        # us, has not 128 queries' work, 16.9)
-        if rows is not None and kv_cache is None and past_len == 0 and q_len > 1 and _plain(*rows):
+        if rows is not None:
             out = _kvc.attention_prefill(*rows, q_len)
             if out is not None:
                 return self.o_proj(quantize_tokens(out.view(bsz, q_len, nh * d), self.o_reorder_index, self.o_proj.select_num,
                                                    self.quant_type), residual)
+            q = self._rotated(rows[0], q_len)
         if q_len == 1:
             mask, causal = None, False
         elif isinstance(past_len, int) and past_len == 0:

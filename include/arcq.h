@@ -367,6 +367,11 @@ int arcq_scales_from_absmax(float *d_values, int n, float divisor, void *stream)
  */
 int arcq_attention_prefill(const void *q, int ldq, const void *k, int ldk, const void *v, int ldv, int batch, int seq,
                            int num_qo_heads, int num_kv_heads, int head_dim, float sm_scale, void *o, int ldo, void *stream);
+/* the same with the rotary embedding of the queries ahead of it, token t of a sequence at position t: q as the projection left it, the bits
+ * of arcq_rope's queries; tables as there (bf16, at most 2^24 positions, 16-byte aligned).  k is rotated already. */
+int arcq_attention_prefill_rope(const void *q, int ldq, const void *cos_table, const void *sin_table, int max_positions, const void *k,
+                                int ldk, const void *v, int ldv, int batch, int seq, int num_qo_heads, int num_kv_heads, int head_dim,
+                                float sm_scale, void *o, int ldo, void *stream);
 
 /*
  * Routing of a mixture-of-experts block (model/qMixtralLayer.py:441-452: softmax over the experts in fp32,

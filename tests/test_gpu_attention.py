@@ -91,3 +91,27 @@ def test_attention_prefill_refuses():
     for c in (0.0, -0.1, float("inf"), float("-inf"), float("nan"), 3e38):             # 3e38 log2 e is not finite
         assert call(c=c) == 2
     assert call(b=1, q=None) == 1 and call(b=1, v=0x1008) == 4 and call(b=1, s=1 << 23, ldk=512) == 2
+
+
+@pytest.mark.parametrize("batch,seq,heads,kv_heads,positions", [(1, 1, 1, 1, 1), (3, 2, 4, 4, 8), (2, 33, 4, 2, 33), (1, 127, 8, 8, 100), (2, 128, 6, 2, 128),
+                                                                (3, 129, 8, 1, 4096), (1, 257, 28, 4, 300)])
+def test_attention_prefill_rotates_queries(batch, seq, heads, kv_heads, positions):
+    """Queries rotated by the attention itself, read from the projection's rows: the bits of the rotary pass followed by the attention,
+    also behind the table's last position (which stands for every later one)"""
+    from arcquant_amd import _lib, kv_cache
+    _, _, qkv = operands(batch, seq, heads, kv_heads)
+    qkv = torch.cat([qkv, qkv[:, :8]], 1).cuda()                    # rows that end behind the heads
+    qkv[0, :2] = torch.tensor([float("nan"), 0.0])                  # what is not finite stays where it was
+    tables = kv_cache.rope_tables(positions, 128, torch.bfloat16, "cuda")
+    q, k = kv_cache.rope(qkv, seq, 0, heads, kv_heads, *tables)
+    rows, v = qkv[:, :heads * 128], qkv[:, (heads + kv_heads) * 128:(heads + 2 * kv_heads) * 128]
+    want = kv_cache.attention_prefill(q, k, v, seq)
+    got = kv_cache.attention_prefill((rows, *tables), k, v, seq)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+    assert kv_cache.attention_prefill((rows.half(), *tables), k, v, seq) is None
+    assert kv_cache.attention_prefill((rows, tables[0][:, :32], tables[1]), k, v, seq) is None
+    assert kv_cache.attention_prefill((rows[:, :64], *tables), k, v, seq) is None
+    ok, f = 0x1000, _lib.lib().arcq_attention_prefill_rope
+    args = lambda cos, n: (ok, 128, cos, ok, n, ok, 128, ok, 128, 1, 1, 1, 1, 128, 1.0, ok, 128, None)
+    null, shape, align = (f(*args(*a)) for a in ((None, 1), (ok, 0), (ok + 2, 1)))
+    assert len({null, shape, align}) == 3 and 0 not in (null, shape, align)      # refused ahead of any launch
