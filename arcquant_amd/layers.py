@@ -294,7 +294,7 @@ class LlamaMLP(nn.Module):
                                                global_scale=scale if nv else None)
             return self.down_proj((qx, sfx, scale, x[3], x[4]), residual)
         if self.inter <= 32736 and self.inter % 32 == 0:
-            t = self._activation(x)
+            t = self._activation(x) if x[0].shape[0] > 64 else None
             if t is not None:
                 scale = t[1] if isinstance(t, tuple) else 1.0
                 t = t[0] if isinstance(t, tuple) else t
