@@ -371,9 +371,10 @@ def _swiglu_halves(A, SFA, B, SFB, M, N, Kp, f, tensor_scale, **kw):
 @functools.lru_cache(maxsize=4096)
 def parts_pay(M, part_rows, Kp, fmt):
     """Whether matmul_parts over part_rows (a tuple) is faster than a GEMM per part and a concatenation: nearly always, 0.6 of the time on
-    average.  Not where the parts by themselves fit smaller NVFP4 tiles and all of them together make 256x256 ones, whose last round
-    is nearly empty (two parts of 18944 x 4352, 300 rows, 296 tiles: 171 against 133 us; 11008, 600 rows, 258 tiles: 174 / 141) or whose rows
-    are (28672 x 4352, 80 rows: 101 / 71, 128 rows 103 / 90)."""
+    average.  Not where the parts by themselves fit smaller NVFP4 tiles and all of them together make tiles of 256 weight rows whose last
+    round is nearly empty or whose rows are (two parts of 28672 x 4352, 80 rows, 66 against 60 us without the concatenation, of 38016 x
+    4352, 66 rows, 119 / 79; since those tiles come with fewer activation rows there is little in it elsewhere: two of 18944 x 4352, 300
+    rows, 111 / 117, of 11008 x 4352, 600 rows, 118 / 115, three of 4096 x 4352, 1500 rows, 141 / 160)."""
     f = _fmt_id(fmt)
     if f != _lib.NVFP4 or M <= 64:
         return True
