@@ -232,7 +232,7 @@ typedef struct arcq_gemm_args {
 int arcq_gemm(const arcq_gemm_args *args, void *stream);
 /* swiglu = ARCQ_SWIGLU_HALVES: the same output from weights as a fused gate_up projection has them, N/2 gate rows and then N/2 up rows (in
  * arcq_gemm_parts one part each, without a bias), for the plain problems of many rows that arcq_gemm_swiglu_halves says 1 for; ARCQ_ERR_SHAPE
- * for others, ARCQ_ERR_WORKSPACE without the workspace that arcq_gemm_workspace_bytes names. */
+ * for others.  NVFP4: with a workspace of arcq_gemm_scratch_bytes, or of arcq_gemm_workspace_bytes where that is not 0, else ARCQ_ERR_WORKSPACE. */
 #define ARCQ_SWIGLU_HALVES 2
 int arcq_gemm_swiglu_halves(int M, int N, int Kp, int fmt);
 size_t arcq_gemm_workspace_bytes(int M, int N, int Kp, int fmt, int n_seg);
