@@ -270,14 +270,15 @@ class LlamaMLP(nn.Module):
 
     def _activation(self, x):
         """act_fn(gate) * up straight from the projection's epilogue, NVFP4 with its tensor scale; None where the projection is called
-        by itself: few tokens, hooks or another forward on it, a bias, no memory"""
+        by itself: few tokens, hooks or another forward on it, another format or other sizes than the MLP's, a bias, no memory"""
         qx, scale_x, scale, _, _ = x
         p, nv = self.gate_up_proj, self.quant_type == "NVFP4"
         if qx.dim() != 2 or not isinstance(scale, (float, int, torch.Tensor)) or \
                 not agemm.swiglu_halves_pay(qx.shape[0], 2 * self.inter, 2 * qx.shape[1], self.quant_type):
             return None
         if _unhooked(p, SplitQLinear):
-            return p._as_one(x, swiglu=True)
+            ours = all(getattr(q, "quant_type", None) == self.quant_type and q.out_features == self.inter for q in p.parts)
+            return p._as_one(x, swiglu=True) if ours else None
         if not _unhooked(p, QLinearLayer) or p.bias is not None or p.out_features != 2 * self.inter or p.quant_type != self.quant_type:
             return None
         return agemm.matmul_swiglu(qx, p.W, scale_x, p.scale_w, (scale, p.scale), fmt=self.quant_type, tensor_scale=nv, halves=True)

@@ -217,6 +217,52 @@ def test_split_linear_runs_part_by_part_where_that_is_faster(monkeypatch):
     assert ran == ["one", "part", "part"]
 
 
+def _mlp(projection, down, quant_type):
+    """a LlamaMLP over given linears"""
+    mlp = layers.LlamaMLP.__new__(layers.LlamaMLP)
+    nn.Module.__init__(mlp)
+    mlp.gate_up_proj, mlp.down_proj, mlp.quant_type = projection, down, quant_type
+    mlp.inter, mlp.interleaved = 64, False
+    mlp.register_buffer("down_reorder_index", torch.arange(64, dtype=torch.int16))
+    return mlp
+
+
+@pytest.mark.parametrize("split", [False, True])
+def test_mlp_projection_of_another_format(monkeypatch, split):
+    """gate and up in another format than the MLP's own (projections or quant_type assigned after construction), or of other sizes: the
+    projection is called by itself and its output quantized in the MLP's format, never the epilogue's output with the other's scale"""
+    ran = []
+    epilogue = lambda *a, tensor_scale=False, **kw: ran.append("epilogue") or (("t", "scale") if tensor_scale else "t")
+    monkeypatch.setattr(layers.agemm, "swiglu_halves_pay", lambda *a: True)
+    monkeypatch.setattr(layers.agemm, "matmul_swiglu", epilogue)
+    monkeypatch.setattr(layers.agemm, "matmul_parts", lambda A, B, *a, swiglu=False, **kw: epilogue(**kw) if swiglu else
+                        ran.append("projection") or torch.zeros(A.shape[0], B.shape[0], dtype=torch.bfloat16))
+    monkeypatch.setattr(layers.agemm, "matmul", lambda A, B, *a, **kw: ran.append("projection") or
+                        torch.zeros(A.shape[0], B.shape[0], dtype=torch.bfloat16))
+    monkeypatch.setattr(layers.agemm, "reorder_quantize_x", lambda t, *a, fmt, global_scale=None: ran.append((t, fmt, global_scale)) or ("q", "s"))
+    monkeypatch.setattr(layers, "swiglu_quantize_tokens", lambda gu, inter, index, select, fmt: ran.append(("gate_up", fmt)) or
+                        ("q", "s", 0.5, None, 100))
+
+    class Down(nn.Module):
+        select_num, out_features = 0, 32
+
+        def forward(self, x, residual=None):
+            return x
+
+    def run(fmt, own, sizes=(64, 64)):
+        parts = [_quantized_linear(n, 32) for n in (sizes if split else [sum(sizes)])]
+        for p in parts:
+            p.quant_type = fmt
+        mlp = _mlp(layers.SplitQLinear(parts) if split else parts[0], Down(), own)
+        ran.clear()
+        return mlp((torch.zeros(100, 32, dtype=torch.uint8), torch.zeros(400, dtype=torch.uint8), 1.0, None, 100))
+
+    assert run("NVFP4", "NVFP4")[2] == "scale" and ran == ["epilogue", ("t", "NVFP4", "scale")]
+    assert run("MXFP4", "MXFP4")[2] == 1.0 and ran == ["epilogue", ("t", "MXFP4", None)]
+    for fmt, own, sizes in (("NVFP4", "MXFP4", (64, 64)), ("MXFP4", "NVFP4", (64, 64)), ("NVFP4", "NVFP4", (96, 96))):
+        assert run(fmt, own, sizes)[2] == 0.5 and ran == ["projection", ("gate_up", own)], (fmt, own, sizes)
+
+
 def test_norm_ahead_of_a_quantizer_is_the_module(monkeypatch):
     """the norm's launch that also forms the tensor scale stands in for LlamaRMSNorm's own forward alone"""
     layer = layers.QLlamaDecoderLayer.__new__(layers.QLlamaDecoderLayer)
