@@ -361,6 +361,8 @@ def swiglu_halves_pay(M, N, Kp, fmt):
 
 
 def _swiglu_halves(A, SFA, B, SFB, M, N, Kp, f, tensor_scale, **kw):
+    if (SFA.data_ptr() | SFB.data_ptr()) % 16:      # (a GEMM with one of the plain kernels takes them)
+        return None
     T = torch.empty((M, N // 2), dtype=torch.bfloat16, device=A.device)
     amax = torch.zeros(1, dtype=torch.float32, device=A.device) if tensor_scale else None
     if not _gemm(A, SFA, B, SFB, M, N, Kp, f, T, swiglu=_lib.SWIGLU_HALVES, absmax=amax, **kw):
@@ -553,7 +555,8 @@ def matmul_swiglu(A, B, SFA, SFB, scale, *, fmt=None, tensor_scale=False, halves
     another order), without h going through memory.  tensor_scale=True
     also returns the NVFP4 tensor scale max|t| / 2688 of t (0-dim fp32 device tensor, 1 for all zeros).
     halves=True: the weights as they are, gate rows and then up rows, for the problems that swiglu_halves_pay says; None where there is
-    no memory for the scratch that such a GEMM takes.  (Where its last round of tiles is cut along K, other columns are in it than in
+    no memory for the scratch that such a GEMM takes, and for scale bytes that do not begin at a multiple of 16 (a slice of quantized
+    rows).  (Where its last round of tiles is cut along K, other columns are in it than in
     matmul's, whose sums are then in another order.)"""
     _require(A, "A", torch.uint8, 2)
     _require(B, "B", torch.uint8, 2)

@@ -270,7 +270,8 @@ class LlamaMLP(nn.Module):
 
     def _activation(self, x):
         """act_fn(gate) * up straight from the projection's epilogue, NVFP4 with its tensor scale; None where the projection is called
-        by itself: few tokens, hooks or another forward on it, another format or other sizes than the MLP's, a bias, no memory"""
+        by itself: few tokens, hooks or another forward on it, another format or other sizes than the MLP's, a bias, no memory,
+        unaligned scale bytes"""
         qx, scale_x, scale, _, _ = x
         p, nv = self.gate_up_proj, self.quant_type == "NVFP4"
         if qx.dim() != 2 or not isinstance(scale, (float, int, torch.Tensor)) or \
