@@ -449,10 +449,12 @@ int launch_split(const GemmParams &p, hipStream_t st) {
   return ARCQ_OK;
 }
 
-// Which operand is decoded ahead, and the tile.  A round of 256 tiles takes its time however few there are: 0.78 of a 256-row round with
-// tiles of 192 rows of activations, 0.62 with 128, measured on 180 problems of 100 to 4096 rows, so the fewest rounds by those
-// weights.  us with 256, 192 and 128 rows: 2331 x 3584 x 3712 71, 62, 100; 2331 x 3584 x 19072 305, 268, 442; 1300 x 6144 x 4352 79, 68,
-// 112; 640 x 28672 x 4352 165, 143, 174; 300 x 37888 x 3712 132, 117, 103; 1024 x 28672 x 4352 187, 212, 234; 100 x 57344 x 4352 70, 70, 70.
+// Which operand is decoded ahead, and the tile: the fewest rounds of 256 tiles, a round with 192 rows of activations counting 0.82 of one
+// with 256 rows, and with 128 rows 0.70 (a round takes more than its share of rows: codes and their decoding are the same; partly
+// empty ones less).  On 400 problems of 65 to 16384 rows, 2048 to 57344 columns and K' = 512 to 8064 that is 0.1 % above the fastest tile
+// on average, 6 % at most, and nowhere more than 3 % above 256 rows (with 0.78 and 0.62: 0.4, 11 and 11 %).  us with 256, 192 and 128 rows: 2331
+// x 3584 x 3712 71, 62, 99; 1300 x 6144 x 4352 79, 68, 112; 640 x 28672 x 4352 164, 134, 170; 300 x 37888 x 3712 133, 117, 101; 1024 x 28672
+// x 4352 184, 213, 229; 4096 x 6144 x 4352 175, 215, 185; 600 x 37888 x 3712 147, 174, 159; 6144 x 28672 x 1152 326, 363, 393.
 // The smaller tiles need the activations decoded; decoding a row takes 2.4e-5 of a round (about 5 TB/s, whatever K').
 struct F16Plan {
   bool codes_w;
@@ -463,7 +465,7 @@ F16Plan f16_plan(int M, int N, bool grouped) {
   if (grouped) return plan;
   auto rounds = [&](long rows) { return (double)(((M + rows - 1) / rows * ((N + 255L) / 256) + 255) / 256); };
   double least = rounds(256) - 2.4e-5 * std::max(0, M - N);
-  const struct { int tf; double weight; } smaller[] = {{6, 0.78}, {4, 0.62}};
+  const struct { int tf; double weight; } smaller[] = {{6, 0.82}, {4, 0.70}};
   for (const auto &s : smaller)
     if (const double cost = rounds(32 * s.tf) * s.weight; cost < least) least = cost, plan = {true, s.tf};
   return plan;

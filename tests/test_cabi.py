@@ -176,6 +176,18 @@ def test_gemm_workspace(M, N, kp, decoded_rows):
     assert ask(M, N, kp, 1, 0) == 0
 
 
+@pytest.mark.parametrize("M,N,decoded_rows", [
+    (8100, 3072, 3072),      # two rounds of 256 rows (less the decoding of fewer rows), and not three of 128: 1.88 to 2.1
+    (8300, 6144, 6144),      # four of 256 rows, and not five of 192: 3.95 to 4.1
+    (6216, 3584, 6216),      # two of 192 rows, and not two of 256: 1.64 to 1.94
+])
+def test_gemm_workspace_by_rounds_of_tiles(M, N, decoded_rows):
+    """more rows of activations than of weights: the weights are decoded for tiles of 256 rows of activations, the activations for
+    smaller ones, whichever make the fewest rounds, counted by what a round of each was measured to take"""
+    for kp in (512, 1152, 4352):
+        assert _lib.lib().arcq_gemm_workspace_bytes(M, N, kp, 0, 0) == 2 * decoded_rows * kp
+
+
 def test_gemm_rejects_bad_arguments():
     """arcq_gemm checks the forms against each other, alignment, shapes and pointers before any launch"""
     L, ok, odd = _lib.lib(), 0x1000, 0x1004

@@ -529,7 +529,8 @@ def test_nvfp4_captured_without_scratch(agemm, oracle, M, N, kp):
 @pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
 @pytest.mark.parametrize("M,N,kp,decoded", [
     (70, 49160, 512, 70), (128, 49152, 640, 128),                                   # tiles of 128 activation rows
-    (300, 22100, 512, 300), (385, 24576, 768, 385), (192, 33000, 640, 192),         # of 192, the last one of 108, 1 and 192
+    (300, 22100, 512, 300), (385, 20480, 768, 385), (192, 33000, 640, 192),         # of 192, the last one of 108, 1 and 192
+    (385, 24576, 768, 385),                                                          # of 256, the last one of 129
     (3900, 4096, 512, 3900), (3960, 4090, 640, 3960), (4020, 4096, 512, 4020), (4090, 4096, 512, 4090),   # of 256: 60, 120, 180, 250
     (3841, 4096, 512, 3841), (5331, 3584, 640, 5331), (4096, 3584, 512, 3584)])     # more rows than weights: either one decoded
 def test_nvfp4_decoded_ahead_tiles(agemm, oracle, M, N, kp, decoded):
