@@ -726,8 +726,8 @@ __global__ __launch_bounds__(128 * NWM) void gemm_nvfp4_tiled(GemmParams p) {
 // ---------------------------------------------------------------------------------------------
 // Skinny kernels for M <= 64 (decode batches; NVFP4: few rows, narrow layers and a short K', see kStreamFrom): the GEMM is a stream of the weight matrix, read
 // exactly once, so nothing is staged through LDS.  A workgroup owns 16 weight rows; its NW waves
-// take the K steps of 128 round-robin in pairs (split-K; MXFP4 in runs of four: with four waves wave w does steps 2w, 2w+1, 2w+8, 2w+9, ...:
-// a pair of steps is one whole 128-byte line of every row, and the four waves walk neighbouring lines) and their partial sums meet in LDS.  A lane loads
+// take the K steps of 128 round-robin in pairs (split-K; with four waves wave w does steps 2w, 2w+1, 2w+8, 2w+9, ...: a pair of steps is one
+// whole 128-byte line of every row, and the four waves walk neighbouring lines; MXFP4 mostly in runs of four) and their partial sums meet in LDS.  A lane loads
 // the 16 bytes (32 codes) the 16x16 MFMA wants from it straight from global memory: row lane%16,
 // K group lane/16, i.e. 64 contiguous bytes per row and step.  The activations (<= 64 rows) come
 // from L2 the same way, one 16-column tile at a time, each reusing the weight registers.
@@ -774,7 +774,7 @@ __device__ __forceinline__ void skinny_reduce_store(const GemmParams &p, v4f (&a
   }
 }
 
-template <int MT, int AT, int NW>
+template <int MT, int AT, int NW, int R = 4>
 __global__ __launch_bounds__(64 * NW) void gemm_mxfp4_skinny(GemmParams p) {
   __shared__ float red[NW - 1][MT * AT][64][4];
   constexpr int D = (MT * AT >= 4) ? 4 : 8;  // K steps whose loads are in flight together
@@ -799,51 +799,54 @@ __global__ __launch_bounds__(64 * NW) void gemm_mxfp4_skinny(GemmParams p) {
 #pragma unroll
   for (int j = 0; j < AT * MT; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
   const uint32_t sh = 8u * (uint32_t)g;
-  // A wave takes runs of four steps (two lines of codes per row, 16 scale bytes) NW runs apart: the scale bytes of a run are one load.  us,
-  // a load per step and pairs of steps by wave, and so: 8 x 4096 x 14592 11.8 / 10.7, 16 rows 14.4 / 12.9, 20 rows 16.5 / 14.9; 8 x 3584 x
-  // 19072 14.2 / 11.6; 3 x 28672 x 4352 17.6 / 15.3; 16 x 6144 x 4352 7.2 / 6.7.
+  // A wave takes runs of R steps NW runs apart: four (two lines of codes per row, 16 scale bytes), two where the row is short (launch_skinny).
+  // The scale bytes of a run are one load; where the row ends inside it, one for each step, clamped to the row, of which nothing is waited
+  // for ahead of the others (with the bytes behind the row's end set to 0: 1 x 4096 x 4352 4.34 us, so 4.05, 1 x 18944 x 2176 6.04 / 5.67).
+  // us, a load per step and pairs of steps by wave, and runs of four: 8 x 4096 x 14592 11.8 / 10.7, 16 rows 14.4 / 12.9, 20 rows 16.5 /
+  // 14.9; 8 x 3584 x 19072 14.2 / 11.6; 3 x 28672 x 4352 17.6 / 15.3; 16 x 6144 x 4352 7.2 / 6.7.
   auto scales_of = [&](const uint8_t *row, int t) {
-    const uint8_t *at = row + 4 * t;
-    uint4 v = make_uint4(0, 0, 0, 0);
-    if (t + 4 <= T) {  // (4-byte aligned)
-      __builtin_memcpy(&v, at, 16);
-      return v;
+    uint4 v;  // (dwords of steps behind the run's or the row's last one: not read)
+    if (t + R <= T) {  // (4-byte aligned)
+      __builtin_memcpy(&v, row + 4 * t, 4 * R);
+    } else {
+      __builtin_memcpy(&v.x, row + 4 * t, 4);
+      if (R > 2) {
+        __builtin_memcpy(&v.y, row + 4 * min(t + 1, T - 1), 4);
+        __builtin_memcpy(&v.z, row + 4 * min(t + 2, T - 1), 4);
+      }
     }
-    if (t < T) __builtin_memcpy(&v.x, at, 4);
-    if (t + 1 < T) __builtin_memcpy(&v.y, at + 4, 4);
-    if (t + 2 < T) __builtin_memcpy(&v.z, at + 8, 4);
     return v;
   };
   auto dword = [](const uint4 &v, int d) { return d == 0 ? v.x : d == 1 ? v.y : d == 2 ? v.z : v.w; };
-  for (int t0 = 4 * wave; t0 < T; t0 += NW * D) {
-    uint4 a[AT][D], b[MT][D], sa[AT][D / 4], sb[MT][D / 4];
+  for (int t0 = R * wave; t0 < T; t0 += NW * D) {
+    uint4 a[AT][D], b[MT][D], sa[AT][D / R], sb[MT][D / R];
 #pragma unroll
-    for (int k = 0; k < D / 4; ++k) {
-      const int t1 = t0 + 4 * NW * k;
+    for (int k = 0; k < D / R; ++k) {
+      const int t1 = t0 + R * NW * k;
       if (t1 >= T) continue;  // (uniform over the wave, as all of these)
 #pragma unroll
       for (int i = 0; i < AT; ++i) sa[i][k] = scales_of(ws[i], t1);
 #pragma unroll
       for (int j = 0; j < MT; ++j) sb[j][k] = scales_of(xs[j], t1);
 #pragma unroll
-      for (int d = 0; d < 4; ++d)
+      for (int d = 0; d < R; ++d)
         if (t1 + d < T) {
 #pragma unroll
-          for (int i = 0; i < AT; ++i) a[i][4 * k + d] = *reinterpret_cast<const uint4 *>(wc[i] + 64 * (t1 + d));
+          for (int i = 0; i < AT; ++i) a[i][R * k + d] = *reinterpret_cast<const uint4 *>(wc[i] + 64 * (t1 + d));
 #pragma unroll
-          for (int j = 0; j < MT; ++j) b[j][4 * k + d] = *reinterpret_cast<const uint4 *>(xc[j] + 64 * (t1 + d));
+          for (int j = 0; j < MT; ++j) b[j][R * k + d] = *reinterpret_cast<const uint4 *>(xc[j] + 64 * (t1 + d));
         }
     }
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      if (t0 + 4 * NW * (d / 4) + d % 4 < T) {
+      if (t0 + R * NW * (d / R) + d % R < T) {
 #pragma unroll
         for (int i = 0; i < AT; ++i)
 #pragma unroll
           for (int j = 0; j < MT; ++j)
             acc[i * MT + j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
-                fp4_operand(a[i][d]), fp4_operand(b[j][d]), acc[i * MT + j], 4, 4, 0, (int)(dword(sa[i][d / 4], d % 4) >> sh), 0,
-                (int)(dword(sb[j][d / 4], d % 4) >> sh));
+                fp4_operand(a[i][d]), fp4_operand(b[j][d]), acc[i * MT + j], 4, 4, 0, (int)(dword(sa[i][d / R], d % R) >> sh), 0,
+                (int)(dword(sb[j][d / R], d % R) >> sh));
       }
     }
   }
@@ -913,17 +916,21 @@ __global__ __launch_bounds__(64 * NW) void gemm_nvfp4_skinny(GemmParams p) {
 
 // NW waves per workgroup split K among them: eight where the layer is narrow (few workgroups, one wave
 // per SIMD otherwise), four where the grid alone fills the machine
-template <int FMT, int MT, int AT>
+template <int FMT, int MT>
 int launch_skinny(const GemmParams &p, hipStream_t st) {
-  const int grid = (p.N + 16 * AT - 1) / (16 * AT);
-  const bool eight = grid <= 512 && AT == 1;
+  const int grid = (p.N + 15) / 16;
+  const bool eight = grid <= 512;
   if (FMT == ARCQ_FMT_MXFP4) {
-    if (MT == 1 && grid <= 256 && p.Kp >= 8192)  // a workgroup per CU: all of a long row on its way at once (8 x 4096 x 14592: 10.7 / 10.2 us)
+    // Short rows in runs of two steps, which keep all four waves busy (us in runs of four and in twos: 1 x 28672 x 1152 5.4, 5.2, 1 x 28672
+    // x 1408 5.9, 5.75, 48 x 2048 x 256 3.15, 2.95)
+    if ((!eight && p.Kp <= 2304) || p.Kp < 512)
+      hipLaunchKernelGGL((gemm_mxfp4_skinny<MT, 1, 4, 2>), dim3(grid), dim3(256), 0, st, p);
+    else if (MT == 1 && grid <= 256 && p.Kp >= 8192)  // a workgroup per CU: all of a long row on its way at once (8 x 4096 x 14592: 10.7 / 10.2 us)
       hipLaunchKernelGGL((gemm_mxfp4_skinny<1, 1, 16>), dim3(grid), dim3(1024), 0, st, p);
     else if (eight)
       hipLaunchKernelGGL((gemm_mxfp4_skinny<MT, 1, 8>), dim3(grid), dim3(512), 0, st, p);
     else
-      hipLaunchKernelGGL((gemm_mxfp4_skinny<MT, AT, 4>), dim3(grid), dim3(256), 0, st, p);
+      hipLaunchKernelGGL((gemm_mxfp4_skinny<MT, 1, 4>), dim3(grid), dim3(256), 0, st, p);
   } else {
     if (eight)
       hipLaunchKernelGGL((gemm_nvfp4_skinny<MT, 8>), dim3(grid), dim3(512), 0, st, p);
@@ -936,9 +943,9 @@ int launch_skinny(const GemmParams &p, hipStream_t st) {
 
 template <int FMT>
 int launch_skinny_for(const GemmParams &p, hipStream_t st) {
-  if (p.M <= 16) return launch_skinny<FMT, 1, 1>(p, st);
-  if (p.M <= 32) return launch_skinny<FMT, 2, 1>(p, st);
-  return launch_skinny<FMT, 4, 1>(p, st);
+  if (p.M <= 16) return launch_skinny<FMT, 1>(p, st);
+  if (p.M <= 32) return launch_skinny<FMT, 2>(p, st);
+  return launch_skinny<FMT, 4>(p, st);
 }
 
 template <int WN, int WM, int NWM = 2>

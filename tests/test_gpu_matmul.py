@@ -686,10 +686,12 @@ def test_nvfp4_steps_of_128_elements_per_wave(agemm, oracle, M, N, kp, route):
 
 
 @pytest.mark.parametrize("M,N,kp", [(1, 24, 128), (3, 100, 256), (8, 4096, 384), (16, 513, 640), (5, 4096, 8320), (16, 4090, 8448), (8, 2048, 8576), (1, 4096, 8192),
-                                    (17, 1000, 896), (40, 4096, 1408), (64, 333, 4352), (4, 8200, 1152), (33, 4096, 8320), (8, 6144, 8576)])
+                                    (17, 1000, 896), (40, 4096, 1408), (64, 333, 4352), (4, 8200, 1152), (33, 4096, 8320), (8, 6144, 8576),
+                                    (1, 8208, 1280), (2, 8200, 2304), (3, 9000, 2176), (4, 8193, 2432), (20, 300, 384), (48, 2048, 256), (33, 100, 128)])
 def test_mxfp4_decode_batches(agemm, oracle, M, N, kp):
     """MXFP4 decode batches straight from global memory: K' ending after one to four steps of a wave's run, fewer runs than waves and many
-    more, sixteen waves for long rows; the bf16 rounding and the order of the fp32 sum remain"""
+    more, sixteen waves for long rows, runs of two steps for short rows of wide layers and for those of less than four steps; the bf16
+    rounding and the order of the fp32 sum remain"""
     (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, kp - 64, 64, "MXFP4", seed=93)
     want = oracle_dq(oracle, a, sfa, "MXFP4") @ oracle_dq(oracle, b, sfb, "MXFP4").T * 0.5
     y = agemm.matmul(a, b, sfa, sfb, 0.5, fmt="MXFP4")
