@@ -365,7 +365,9 @@ int launch(const GemmParams &p, hipStream_t st) {
 
 // Rows per workgroup.  Up to 12288 rows of weights make at most one workgroup per CU of 16, 32 or 48 rows, which then has
 // sixteen waves, or eight that take 128 elements of a step each (us at 16 rows: 6144 x 4352 7.8, eight waves of 64 elements 8.9; 10240 x
-// 8320 15.0 and 17.6; at 16, 32, 64 rows of 6144 x 4352 sixteen waves 6.8, 8.0, 11.0, eight of 128 elements 6.5, 7.7, 10.7).  Beyond, eight waves, and the
+// 8320 15.0 and 17.6; at 16, 32, 64 rows of 6144 x 4352 sixteen waves 6.8, 8.0, 11.0, eight of 128 elements 6.5, 7.7, 10.7; but 64 rows of a
+// longer K' are decoded faster by sixteen: 8192 x 6272 14.4 / 14.8, 8192 x 8448 18.2 / 19.1, 6144 x 14592 27.1 / 29.3, 48 rows 16.0 /
+// 15.7 and 23.7 / 23.3).  Beyond, eight waves, and the
 // rows per workgroup by how many rounds of 256 workgroups they make: the rows and activation rows of a CU's workgroups
 // together, a quarter more where up to 32 rows, or a K' of one or two steps, have a single workgroup per CU to themselves (nothing else
 // asks for weights while it starts, waits and ends): 28672 rows take 64 per workgroup up to 32 rows and 112 above (64 rows, K' = 4352:
@@ -373,6 +375,7 @@ int launch(const GemmParams &p, hipStream_t st) {
 template <int MT>
 int launch_plain(const GemmParams &p, hipStream_t st) {
   if (p.N <= 4096) return launch<MT, 1, 1, 16, (MT == 1 ? 3 : 2)>(p, st);
+  if (MT == 4 && p.N <= 8192 && p.Kp >= 6144) return launch<MT, 2, 1, 16, 2>(p, st);
   if (p.N <= 8192) return launch<MT, 2, 1, 8, 2, false, 128>(p, st);
   if (p.N <= 12288) return launch<MT, 3, 1, 16, 2>(p, st);
   int best = 0;

@@ -668,6 +668,7 @@ def test_swiglu_of_weights_as_they_are_for_others(agemm, monkeypatch):
 @pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
 @pytest.mark.parametrize("M,N,kp,route", [
     (8, 8192, 4224, 3), (5, 5121, 4096, 3), (17, 6145, 2176, 3), (33, 6144, 1152, 3), (48, 5121, 1152, 3), (64, 8190, 4224, 3), (64, 4112, 8320, 3),
+    (64, 8190, 6016, 3), (49, 4112, 6144, 3), (48, 8177, 6144, 3),                   # (more than 48 rows from K' = 6144 on: 64 elements)
     (523, 3001, 1792, 21), (349, 4099, 2048, 21), (375, 5122, 2432, 22), (297, 6145, 1664, 22), (644, 3001, 1536, 23), (326, 6144, 1792, 23),
     (333, 6144, 1152, 23), (556, 4099, 2048, 24), (80, 28672, 640, 24)])
 def test_nvfp4_steps_of_128_elements_per_wave(agemm, oracle, M, N, kp, route):
