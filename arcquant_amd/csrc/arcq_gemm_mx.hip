@@ -52,7 +52,7 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
 
   int lin;
   if (p.seg) {
-    if (!enter_segment_in_turn<BT, BT, 32, 32>(p, lin)) return;
+    if (!enter_segment_in_runs<BT, BT, 32>(p, lin)) return;
   } else {
     const int total = ((p.M + BT - 1) / BT) * ((p.N + BT - 1) / BT);
     lin = (blockIdx.x & 7) * ((total + 7) >> 3) + (blockIdx.x >> 3);

@@ -296,7 +296,7 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
   __shared__ uint4 smem[(S::kF + S::kC + S::kS) / 16];
   int lin;
   if (p.seg) {
-    if (!enter_segment_in_turn<S::BM, S::BN, 16, 32>(p, lin)) return;
+    if (!enter_segment_in_runs<S::BM, S::BN, 16>(p, lin)) return;
   } else {
     const int total = ((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN);
     lin = (blockIdx.x & 7) * ((total + 7) >> 3) + (blockIdx.x >> 3);

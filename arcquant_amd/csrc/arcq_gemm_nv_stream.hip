@@ -337,7 +337,7 @@ __global__ __launch_bounds__(64 * WN * WK) void gemm_nvfp4_stream(GemmParams p) 
   uint8_t *lds = reinterpret_cast<uint8_t *>(smem);
   int lin;
   if constexpr (GROUPED) {
-    if (!enter_segment_in_turn<S::BM, S::BN, 16, 2>(p, lin)) return;
+    if (!enter_segment_in_twos<S::BM, S::BN, 16>(p, lin)) return;
   } else {
     const int total = ((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN);
     lin = (blockIdx.x & 7) * ((total + 7) >> 3) + (blockIdx.x >> 3);

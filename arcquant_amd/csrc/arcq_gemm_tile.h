@@ -181,20 +181,46 @@ __device__ __forceinline__ bool enter_segment(GemmParams &p, int &lin) {
   return segments.enter(p, lin);
 }
 
-// The same with runs of RUN tiles that go to the XCDs in turn, for kernels whose tiles take less time for fewer rows: with one run per XCD,
+// The same in shorter runs that go to the XCDs in turn, for kernels whose tiles take less time for fewer rows: with one run per XCD,
 // the XCD that has the experts of most rows, or none of those that end in a small tile, is the last one.  The grid is a multiple of
-// 8 RUN (grid_in_turn).  us, one run per XCD and so, Zipf-like and even sizes: gemm_nvfp4_f16, RUN = 32, 8192 rows over eight of 28672 x
-// 4224 1497, 1378 / 1472, 1373, 50000 over 64 of 4096 x 2176 824 / 791; gemm_mxfp4_pingpong, 8192 over eight of 4096 x 14464 342, 243 / 330, 247.
-// gemm_nvfp4_stream, RUN = 2 (the tiles of an expert's first and second rows, which share their weights): 128 rows over eight of 28672 x 4224
-// 134, 125 / 128, 124, 64 rows 132 / 122, 200 rows 151 / 139; of 4096 x 14464 84, 55 / 83, 56; 1024 over 64 of 2048 x 1536 44.1 / 36.6.
+// 8 RUN (grid_in_turn).
 template <int RUN>
 inline int grid_in_turn(int tiles) { return (tiles + 8 * RUN - 1) / (8 * RUN) * (8 * RUN); }
 
-template <int BM, int BN, int G, int RUN>
-__device__ __forceinline__ bool enter_segment_in_turn(GemmParams &p, int &lin) {
+// Large tiles: runs of at most 32 tiles, as many for every XCD and all of one length (whole runs of 32 for some XCDs and none for
+// others: 2048 rows over eight of 4096 x 14464, 128 tiles, 129 us with one run per XCD, 135, so 129).  More than 32 experts keep one run
+// per XCD: a run then ends inside an expert, whose operands another XCD's L2 has to fetch again, as often as it evens anything out.  us, one run
+// per XCD, runs of 32 wherever they end, and so, even and Zipf-like sizes: gemm_nvfp4_f16, 8192 rows over eight of 14336 x 4224 672, 717 / 668,
+// 708 / 670, 706, 20800 over 16 of 6144 x 4224 864, 843 / 870, 845 / 858, 821, 83200 over 64 of 2816 x 2176 969, 904 / 998, 926 / 969, 904;
+// gemm_mxfp4_pingpong, 2048 over eight of 4096 x 14464 130, 130 / 135, 133 / 129, 130, 8192 241, 341 / 246, 331 / 245, 325, 24576 over 16 of
+// 2048 x 14464 382, 456 / 374, 437 / 375, 426.
+template <int BM, int BN, int G>
+__device__ __forceinline__ bool enter_segment_in_runs(GemmParams &p, int &lin) {
+  constexpr int kMost = 32;
   Segments<BM, BN, G> segments(p);
-  const int of_xcd = blockIdx.x >> 3;
-  lin = (of_xcd / RUN * 8 + (blockIdx.x & 7)) * RUN + of_xcd % RUN;
+  if (segments.total == 0) return false;
+  const int runs = p.n_seg > 32 ? 1 : (segments.total + 8 * kMost - 1) / (8 * kMost);  // of an XCD
+  const int run = (segments.total + 8 * runs - 1) / (8 * runs), of_xcd = blockIdx.x >> 3;
+  lin = (of_xcd / run * 8 + (blockIdx.x & 7)) * run + of_xcd % run;  // (of_xcd >= run * runs: behind the last tile)
+  return segments.enter(p, lin);
+}
+
+// Small tiles: in twos (those of an expert's first and second rows, which share their weights).  A few narrow experts with a long K' keep one
+// run per XCD: there are one or two tiles per slot, and which of them come last decides more than the XCDs' shares.  us, one run per XCD and in
+// twos, even sizes, Zipf-like ones and those in reverse: 128 rows over eight of 28672 x 4224 118, 130, 128 / 117, 124, 126, 200 rows 126, 146, 146 /
+// 123, 133, 135; 1024 over 64 of 2048 x 1536 31.6, 44, 44 / 31.4, 36.6, 37; of 4096 x 14464, eight experts, 128 rows 55.2, 83.6, 84.2 / 55.6, 82.3, 91.5,
+// 200 rows 58.2, 86.8, 90.3 / 59.3, 83.4, 91.5.
+template <int BM, int BN, int G>
+__device__ __forceinline__ bool enter_segment_in_twos(GemmParams &p, int &lin) {
+  Segments<BM, BN, G> segments(p);
+  const int of_xcd = blockIdx.x >> 3, xcd = blockIdx.x & 7;
+  if (p.Kp >= 8192 && p.N <= 4096) {
+    const int per_xcd = (segments.total + 7) >> 3;
+    if (of_xcd >= per_xcd) return false;
+    lin = xcd * per_xcd + of_xcd;
+  } else {
+    lin = (of_xcd / 2 * 8 + xcd) * 2 + of_xcd % 2;
+  }
   return segments.enter(p, lin);
 }
 
