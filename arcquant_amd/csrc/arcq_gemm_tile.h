@@ -188,12 +188,12 @@ template <int RUN>
 inline int grid_in_turn(int tiles) { return (tiles + 8 * RUN - 1) / (8 * RUN) * (8 * RUN); }
 
 // Large tiles: runs of at most 32 tiles, as many for every XCD and all of one length (whole runs of 32 for some XCDs and none for
-// others: 2048 rows over eight of 4096 x 14464, 128 tiles, 129 us with one run per XCD, 135, so 129).  More than 32 experts keep one run
-// per XCD: a run then ends inside an expert, whose operands another XCD's L2 has to fetch again, as often as it evens anything out.  us, one run
-// per XCD, runs of 32 wherever they end, and so, even and Zipf-like sizes: gemm_nvfp4_f16, 8192 rows over eight of 14336 x 4224 672, 717 / 668,
-// 708 / 670, 706, 20800 over 16 of 6144 x 4224 864, 843 / 870, 845 / 858, 821, 83200 over 64 of 2816 x 2176 969, 904 / 998, 926 / 969, 904;
-// gemm_mxfp4_pingpong, 2048 over eight of 4096 x 14464 130, 130 / 135, 133 / 129, 130, 8192 241, 341 / 246, 331 / 245, 325, 24576 over 16 of
-// 2048 x 14464 382, 456 / 374, 437 / 375, 426.
+// others: 2048 even rows over eight of 4096 x 14464, 128 tiles, 135 us, so 129).  More than 32 experts keep one run per XCD: a shorter run
+// ends inside an expert, whose operands another XCD's L2 then fetches again, as often as it evens anything out.  us, one run per XCD, runs of 32
+// wherever they end, and runs of one length, each for even sizes, Zipf-like ones and those in reverse: gemm_nvfp4_f16, 8192 rows over eight of
+// 14336 x 4224 672, 733, 735 / 668, 723, 736 / 670, 712, 724, 20800 over 16 of 6144 x 4224 864, 840, 838 / 870, 833, 824 / 858, 803, 820, 83200 over 64
+// of 2816 x 2176 969, 881, 909 / 998, 916, 933 / 1001, 893, 884; gemm_mxfp4_pingpong, 2048 over eight of 4096 x 14464 130, 130, 128 / 135, 129, 134 /
+// 129, 130, 128, 8192 241, 343, 336 / 247, 328, 322 / 245, 331, 298, 24576 over 16 of 2048 x 14464 382, 458, 451 / 374, 455, 430 / 375, 435, 418.
 template <int BM, int BN, int G>
 __device__ __forceinline__ bool enter_segment_in_runs(GemmParams &p, int &lin) {
   constexpr int kMost = 32;
@@ -207,9 +207,9 @@ __device__ __forceinline__ bool enter_segment_in_runs(GemmParams &p, int &lin) {
 
 // Small tiles: in twos (those of an expert's first and second rows, which share their weights).  A few narrow experts with a long K' keep one
 // run per XCD: there are one or two tiles per slot, and which of them come last decides more than the XCDs' shares.  us, one run per XCD and in
-// twos, even sizes, Zipf-like ones and those in reverse: 128 rows over eight of 28672 x 4224 118, 130, 128 / 117, 124, 126, 200 rows 126, 146, 146 /
-// 123, 133, 135; 1024 over 64 of 2048 x 1536 31.6, 44, 44 / 31.4, 36.6, 37; of 4096 x 14464, eight experts, 128 rows 55.2, 83.6, 84.2 / 55.6, 82.3, 91.5,
-// 200 rows 58.2, 86.8, 90.3 / 59.3, 83.4, 91.5.
+// twos, even sizes, Zipf-like ones and those in reverse: 128 rows over eight of 28672 x 4224 118, 129, 128 / 117, 124, 127, 200 rows 126, 144, 145 /
+// 124, 133, 136; 1024 over 64 of 2048 x 1536 31.7, 44.2, 44.1 / 30.9, 35.9, 37.9; over eight of 4096 x 14464 128 rows 55.4, 85, 84.8 / 56.1, 82.6, 91.5, 320
+// rows 70.5, 91.7, 98.7 / 70.1, 84.5, 101.3.
 template <int BM, int BN, int G>
 __device__ __forceinline__ bool enter_segment_in_twos(GemmParams &p, int &lin) {
   Segments<BM, BN, G> segments(p);
