@@ -1021,10 +1021,8 @@ struct GemmPlan {
 constexpr size_t kSplitMaxBytes = kWorkspaceBytes[kWsSplitK];
 
 // The 256x256 MXFP4 tile: the ping-pong kernel (88, arcq_gemm_mx.hip), whose main loop is faster, except where a short K or a
-// SwiGLU epilogue makes getting in and out of a tile decide: then the one that requests the next stage from one wave per SIMD (84).  88's
-// time against 84's, whole and ragged problems of 700 to 8192 rows: K' = 14592 0.92, 8064 0.83-0.96, 6272 0.85-0.98, 4352 0.88-0.99,
-// 3712 0.89-0.99, 2176 0.93-1.00, 1152 0.93-1.03, 640 0.91-1.07, 512 1.00-1.13.  (The plan names 88 from K' = 8192 on.)
-constexpr int kPingPongFrom = 2176;
+// SwiGLU epilogue makes getting in and out of a tile decide: then the one that requests the next stage from one wave per SIMD (84).  The plan
+// names 88 from K' = 8192 on, whatever the epilogue; plain problems take it from plain_tile's K' on.
 int large_mx_tile(int kernel, int Kp) { return kernel == 84 && Kp >= 8192 ? 88 : kernel; }
 
 // The eight-wave MXFP4 kernels address an operand's rows with 32-bit byte offsets from its base; beyond, the four-wave tile
@@ -1032,6 +1030,25 @@ int large_mx_tile(int kernel, int Kp) { return kernel == 84 && Kp >= 8192 ? 88 :
 int addressable_tile(int kernel, int M, int N, int Kp) {
   if ((size_t)std::max(M, N) * (size_t)(Kp >> 1) < ((size_t)1 << 32)) return kernel;
   return kernel == 84 || kernel == 88 ? 44 : (kernel == 82 ? 42 : kernel);
+}
+
+// 84's workgroups as persistent ones: plain launches over whole tiles, and more of them than one round of workgroups.  us without and so:
+// 4096 x 28672, K' = 512 74.5 / 64.8, 1152 125 / 120, 2048 157 / 150, 8192 x 4096 x 768 27.0 / 25.8; in between K' that are no multiple of 256 lose as
+// much as they gain (4096 x 6144 x 1152 29.6 / 29.4, 16384 x 6144 x 1152 104 / 108), one round 1-3 %.
+bool persistent_84(int M, int N) {
+  return tuning().gemm_persist != 0 && M % 256 == 0 && N % 256 == 0 && (long)(M / 256) * (N / 256) > 256;
+}
+
+// What a plain problem's plan of 84 is launched as.  88's time against the faster of 84's two forms, averages over whole and ragged problems of 512
+// to 16384 rows: K' = 512 1.15, 640 1.04, 1152 1.00, 1664 0.97, 2176 0.96, 2688 0.95, 3712 0.94; multiples of 256, which 84 takes as fast as the K' 128
+// below, 768 1.08, 1280 1.04, 2048 1.02, 2304 1.01, 2560 1.00, 3072 0.98, 3840 0.96, 4352 0.95.  There persistent workgroups are faster on many columns
+// up to 3584 (us, 88 and so: 4096 x 28672 x 2560 181, 173, 2048 x 28672 x 3072 110, 108, 4096 x 37888 x 3584 319, 308; but 8192 x 16384 x 2560 203, 210).
+constexpr int kPingPongFrom = 2176;
+int plain_tile(int kernel, int M, int N, int Kp) {
+  kernel = addressable_tile(kernel, M, N, Kp);
+  if (kernel != 84 || tuning().gemm_kernel == 84) return kernel;
+  const int from = Kp % 256 != 0 ? kPingPongFrom : persistent_84(M, N) && M <= 4096 && N >= 16384 ? 3840 : 2560;
+  return Kp >= from ? 88 : 84;
 }
 
 // The tiled kernels a format has: a kernel forced through the environment that is not among them is ignored.
@@ -1197,18 +1214,12 @@ int run_gemm(GemmParams p, const GemmPlan &plan, int fmt, float *scratch, hipStr
   if (plan.kernel == 1)
     return fmt == ARCQ_FMT_MXFP4 ? launch_skinny_for<ARCQ_FMT_MXFP4>(p, st) : launch_skinny_for<ARCQ_FMT_NVFP4>(p, st);
   if (fmt == ARCQ_FMT_MXFP4) {
-    // persistent workgroups (K' below kPingPongFrom): plain launches over whole tiles, and more of them than one round of workgroups:
-    // with a single tile per CU there is nothing to overlap (28672 x 4352, seven tiles per CU: 333 -> 325 us; 6144 x 4352, one and a
-    // half: 77.5 -> 74.9; one round: 1-3 % slower)
-    const bool persist = !p.seg && !p.swiglu && tuning().gemm_persist != 0 && p.M % 256 == 0 && p.N % 256 == 0 &&
-                         (long)(p.M / 256) * (p.N / 256) > 256;
-    switch (addressable_tile(plan.kernel, p.M, p.N, p.Kp)) {
+    const bool plain = !p.seg && !p.swiglu;
+    switch (plain ? plain_tile(plan.kernel, p.M, p.N, p.Kp) : addressable_tile(plan.kernel, p.M, p.N, p.Kp)) {
       case 88: return run_mxfp4_pingpong(p, st);
       case 44: return launch_mxfp4_tiled<4, 4>(p, st);
       // 256x256 tile, eight waves of 128x64, and 256x128 tile, eight waves of 128x32
-      case 84:
-        if (!p.seg && !p.swiglu && p.Kp >= kPingPongFrom && tuning().gemm_kernel != 84) return run_mxfp4_pingpong(p, st);
-        return persist ? launch_mxfp4_persistent<4, 2>(p, st) : launch_mxfp4_tiled<4, 2, 2, 4>(p, st);
+      case 84: return plain && persistent_84(p.M, p.N) ? launch_mxfp4_persistent<4, 2>(p, st) : launch_mxfp4_tiled<4, 2, 2, 4>(p, st);
       case 82: return launch_mxfp4_tiled<4, 1, 2, 4>(p, st);
       case 42: return launch_mxfp4_tiled<4, 2>(p, st);
       case 224: return launch_mxfp4_tiled<2, 2, 4>(p, st);

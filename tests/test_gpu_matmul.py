@@ -590,7 +590,22 @@ def test_nvfp4_decoded_ahead_tiles_of_experts(agemm, counts):
         at += n
 
 
-@pytest.mark.parametrize("M,N,K,S", [(2300, 4600, 2048, 128), (2304, 4608, 2048, 256), (2049, 4601, 2304, 128), (2300, 4610, 2304, 256)])
+@pytest.mark.parametrize("M,N,K,S", [(4096, 4352, 512, 0), (4096, 4352, 512, 128), (4352, 4096, 2048, 0), (2048, 16384, 3328, 256), (4096, 4352, 2048, 256)])
+def test_mxfp4_persistent_workgroups(agemm, oracle, M, N, K, S):
+    """MXFP4 on whole 256x256 tiles, more than one for every CU, with a short K': one workgroup per CU walks its tiles; the bf16 rounding and
+    the fp32 sum's order remain."""
+    assert_kernel(M, N, K + S, "MXFP4", 84)
+    (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, K, S, "MXFP4", seed=37)
+    want = oracle_dq(oracle, a, sfa, "MXFP4") @ oracle_dq(oracle, b, sfb, "MXFP4").T * 0.5
+    y = agemm.matmul(a, b, sfa, sfb, 0.5, fmt="MXFP4")
+    assert rel_fro(y.float(), want) < 2.5e-3
+    assert torch.allclose(y.float(), want, rtol=2 ** -7, atol=1e-4 * float(want.abs().max()))
+    res = torch.randn(M, N, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
+    assert torch.equal(agemm.matmul(a, b, sfa, sfb, 0.5, fmt="MXFP4", residual=res), y + res)
+
+
+@pytest.mark.parametrize("M,N,K,S", [(2300, 4600, 2048, 128), (2304, 4608, 2048, 256), (2049, 4601, 2304, 128), (2300, 4610, 2304, 256),
+                                     (2304, 4608, 2048, 128), (4096, 4352, 2304, 256)])
 def test_mxfp4_rows_of_medium_length(agemm, oracle, M, N, K, S):
     """MXFP4 on 256x256 tiles from K' = 2176 on: the ping-pong kernel with an odd and an even number of stages, the last one whole and
     half; the bf16 rounding (1.7e-3 in norm) and the fp32 sum's order remain."""
