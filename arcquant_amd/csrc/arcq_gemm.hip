@@ -1626,6 +1626,8 @@ extern "C" int arcq_gemm_route(int M, int N, int Kp, int fmt, int n_seg, int swi
     return ahead == 2 ? ARCQ_ROUTE_AHEAD_CUT : ARCQ_ROUTE_AHEAD;
   const GemmPlan plan = n_seg > 0 ? plan_grouped(M, Kp, fmt, n_seg)
                         : swiglu ? plan_swiglu(M, N, Kp, fmt) : plan_gemm(M, N, Kp, fmt, true);
+  if (fmt == ARCQ_FMT_MXFP4 && n_seg == 0 && !swiglu && addressable_tile(plan.kernel, M, N, Kp) == 84 && plain_tile(plan.kernel, M, N, Kp) == 88)
+    return ARCQ_ROUTE_PINGPONG;
   const int way = stream_way(plan, M, N, Kp, fmt, n_seg, swiglu != 0);
   return way == kByPlan ? ARCQ_ROUTE_PLAN : way == kAsStream ? ARCQ_ROUTE_STREAM : ARCQ_ROUTE_STREAM_SHAPE + way - kMidRows;
 }

@@ -258,12 +258,14 @@ int arcq_gemm_parts(const arcq_gemm_args *args, const arcq_gemm_parts_args *part
 /* The plan that arcq_gemm has for a problem when it has the workspace and aligned operands, by the numbers that the ARCQ_GEMM_KERNEL
  * environment variable forces (168 = one operand decoded ahead, 88 = MXFP4 ping-pong, ..., 1 = skinny, 0 = direct; 11 = NVFP4, up to 32
  * rows on a wide layer, which no kernel of its own serves any more); -1 for arguments arcq_gemm refuses.  Unforced, NVFP4 problems may
- * take another route than their plan, which arcq_gemm_route tells.  Host only, both: for tests of the dispatch and for tuning. */
+ * take another route than their plan, and plain MXFP4 problems with a plan of 84 the ping-pong kernel, which arcq_gemm_route tells.  Host
+ * only, both: for tests of the dispatch and for tuning. */
 int arcq_gemm_kernel(int M, int N, int Kp, int fmt, int n_seg, int swiglu);
 #define ARCQ_ROUTE_PLAN 0          /* the kernel of the plan */
 #define ARCQ_ROUTE_AHEAD 1         /* one operand decoded to fp16 ahead */
 #define ARCQ_ROUTE_AHEAD_CUT 2     /* the same, the last round of tiles cut along K (grouped: if the device counts more than a round) */
 #define ARCQ_ROUTE_STREAM 3        /* one pass over the weights, nothing cut: decode batches, experts of few rows */
+#define ARCQ_ROUTE_PINGPONG 4      /* MXFP4, plan 84: the ping-pong kernel, with the same tiles */
 #define ARCQ_ROUTE_STREAM_SHAPE 16 /* the same for 65 to 1024 rows, + the workgroup's shape */
 /* What arcq_gemm launches for a problem, given arcq_gemm_scratch_bytes of workspace and aligned operands; -1 as above. */
 int arcq_gemm_route(int M, int N, int Kp, int fmt, int n_seg, int swiglu);

@@ -271,6 +271,20 @@ def test_route_of_other_nvfp4_problems():
     assert route(0, 4096, 4352, 0, 0, 0) == route(64, 256, 448, 0, 2, 0) == route(64, 256, 512, 2, 0, 0) == -1
 
 
+@pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
+def test_route_of_mxfp4_problems_on_large_tiles():
+    """what a plan of 84 is launched as: the ping-pong kernel from K' = 2176 on, of multiples of 256 from 2560, 3840 where persistent workgroups
+    walk many columns; not with the interleaved SwiGLU epilogue or over experts, and not where rows lie beyond 32-bit offsets"""
+    L, PINGPONG = _lib.lib(), 4
+    for M, N, first, before in ((2300, 4600, 2176, 2048), (2304, 4608, 2560, 2304), (2300, 4610, 2560, 2304), (2300, 4610, 2432, 2048), (4096, 28672, 3840, 3584),
+                                (4096, 28672, 2176, 2048), (4090, 28672, 2560, 2304), (8192, 28672, 2560, 2304), (4096, 14336, 2560, 2304)):
+        assert L.arcq_gemm_kernel(M, N, first, 1, 0, 0) == L.arcq_gemm_kernel(M, N, before, 1, 0, 0) == 84
+        assert L.arcq_gemm_route(M, N, first, 1, 0, 0) == PINGPONG and L.arcq_gemm_route(M, N, before, 1, 0, 0) == PLAN, (M, N)
+        assert L.arcq_gemm_route(M, N, first, 1, 0, 1) == L.arcq_gemm_route(8 * 800, N, first, 1, 8, 0) == PLAN
+    assert L.arcq_gemm_kernel(4096, 4096, 14592, 1, 0, 0) == 88 and L.arcq_gemm_route(4096, 4096, 14592, 1, 0, 0) == PLAN
+    assert L.arcq_gemm_route(2_000_000, 4096, 8064, 1, 0, 0) == L.arcq_gemm_route(16, 4096, 4352, 1, 0, 0) == PLAN
+
+
 def test_release_stream_without_buffers_needs_no_gpu_work():
     assert hasattr(_lib.lib(), "arcq_release_stream")
 

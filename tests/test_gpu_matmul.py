@@ -41,6 +41,12 @@ def assert_kernel(M, N, Kp, fmt, kernel, n_seg=0, swiglu=0):
         assert _lib.lib().arcq_gemm_kernel(M, N, Kp, _lib.FORMATS[fmt], n_seg, swiglu) == kernel
 
 
+def assert_route(M, N, Kp, fmt, route):
+    from arcquant_amd import _lib
+    if "ARCQ_GEMM_KERNEL" not in os.environ:
+        assert _lib.lib().arcq_gemm_route(M, N, Kp, _lib.FORMATS[fmt], 0, 0) == route
+
+
 def quantized_pair(agemm, M, N, K, S, fmt, seed):
     x = recipes.activations(M, K, seed=seed)
     w = recipes.weights(N, K, seed=seed + 1)
@@ -595,6 +601,7 @@ def test_mxfp4_persistent_workgroups(agemm, oracle, M, N, K, S):
     """MXFP4 on whole 256x256 tiles, more than one for every CU, with a short K': one workgroup per CU walks its tiles; the bf16 rounding and
     the fp32 sum's order remain."""
     assert_kernel(M, N, K + S, "MXFP4", 84)
+    assert_route(M, N, K + S, "MXFP4", 0)
     (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, K, S, "MXFP4", seed=37)
     want = oracle_dq(oracle, a, sfa, "MXFP4") @ oracle_dq(oracle, b, sfb, "MXFP4").T * 0.5
     y = agemm.matmul(a, b, sfa, sfb, 0.5, fmt="MXFP4")
@@ -607,9 +614,10 @@ def test_mxfp4_persistent_workgroups(agemm, oracle, M, N, K, S):
 @pytest.mark.parametrize("M,N,K,S", [(2300, 4600, 2048, 128), (2304, 4608, 2048, 256), (2049, 4601, 2304, 128), (2300, 4610, 2304, 256),
                                      (2304, 4608, 2048, 128), (4096, 4352, 2304, 256)])
 def test_mxfp4_rows_of_medium_length(agemm, oracle, M, N, K, S):
-    """MXFP4 on 256x256 tiles from K' = 2176 on: the ping-pong kernel with an odd and an even number of stages, the last one whole and
-    half; the bf16 rounding (1.7e-3 in norm) and the fp32 sum's order remain."""
+    """MXFP4 on 256x256 tiles from K' = 2176 on: the ping-pong kernel (2304 excepted) with an odd and an even number of stages, the last one
+    whole and half; the bf16 rounding (1.7e-3 in norm) and the fp32 sum's order remain."""
     assert_kernel(M, N, K + S, "MXFP4", 84)
+    assert_route(M, N, K + S, "MXFP4", 0 if K + S == 2304 else 4)
     (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, K, S, "MXFP4", seed=29)
     want = oracle_dq(oracle, a, sfa, "MXFP4") @ oracle_dq(oracle, b, sfb, "MXFP4").T * 0.5
     y = agemm.matmul(a, b, sfa, sfb, 0.5, fmt="MXFP4")
