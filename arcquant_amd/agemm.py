@@ -372,21 +372,18 @@ def _swiglu_halves(A, SFA, B, SFB, M, N, Kp, f, tensor_scale, **kw):
 
 @functools.lru_cache(maxsize=4096)
 def parts_pay(M, part_rows, Kp, fmt):
-    """Whether matmul_parts over part_rows (a tuple) is faster than a GEMM per part and a concatenation: nearly always, 0.6 of the time on
-    average.  Not where the parts by themselves fit smaller NVFP4 tiles and all of them together make tiles of 256 weight rows whose last
-    round is nearly empty or whose rows are (two parts of 28672 x 4352, 80 rows, 66 against 60 us without the concatenation, of 38016 x
-    4352, 66 rows, 119 / 79; since those tiles come with fewer activation rows there is little in it elsewhere: two of 18944 x 4352, 300
-    rows, 111 / 117, of 11008 x 4352, 600 rows, 118 / 115, three of 4096 x 4352, 1500 rows, 141 / 160)."""
+    """Whether matmul_parts over part_rows (a tuple) is faster than a GEMM per part and a concatenation: nearly always, 0.57 to 0.98 of the
+    time.  Not where up to 80 rows of activations make one tile of each part's weight stream, and all parts together the tiles of 256 weight
+    rows for many rows (us, joint and by part: two parts of 28672 x 8448, 65 rows 118, 110, 80 rows 117, 112, of 38016 x 4352, 80 rows 124, 93;
+    but two of 28672 x 8448, 100 rows 117, 158, of 28672 x 4352, 82 rows 71, 94, of 38016 x 4352, 100 rows 125, 122, of 18944 x 4352, 300 rows
+    116, 138, of 11008 x 4352, 600 rows 122, 140, three of 4096 x 4352, 1500 rows 148, 199)."""
     f = _fmt_id(fmt)
-    if f != _lib.NVFP4 or M <= 64:
+    if f != _lib.NVFP4 or not 64 < M <= 80:
         return True
-    L, N = _lib.lib(), sum(part_rows)
+    L = _lib.lib()
     large = lambda n: L.arcq_gemm_route(M, n, Kp, f, 0, 0) in (1, 2) or \
         (L.arcq_gemm_route(M, n, Kp, f, 0, 0) == 0 and L.arcq_gemm_kernel(M, n, Kp, f, 0, 0) == 44)
-    if not large(N) or any(large(n) for n in part_rows):
-        return True
-    tiles = -(-M // 256) * -(-N // 256)
-    return M > 128 and not (tiles > 256 and 0 < tiles % 256 <= 64)
+    return not large(sum(part_rows)) or any(large(n) for n in part_rows)
 
 
 def rmsnorm(X, W, eps, *, tensor_scale=False):

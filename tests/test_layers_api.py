@@ -199,11 +199,13 @@ def test_split_linear_runs_part_by_part_where_a_part_is_not_itself(monkeypatch):
 
 @pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
 def test_split_linear_runs_part_by_part_where_that_is_faster(monkeypatch):
-    """one GEMM over all parts, but for the sizes at which its 256x256 tiles leave most of a round, or most of their rows, empty"""
-    for M, rows, kp, one in ((300, (18944, 18944), 4352, False), (384, (18944, 18944), 4352, False), (600, (11008, 11008), 4352, False),
-                             (80, (28672, 28672), 8320, False), (128, (28672, 28672), 8320, False), (129, (28672, 28672), 8320, True),
-                             (64, (28672, 28672), 8320, True), (200, (18944, 18944), 4352, True), (300, (14336, 14336), 4352, True),
-                             (2331, (3584, 512, 512), 3712, True), (2331, (18944, 18944), 3712, True)):
+    """one GEMM over all parts, but for up to 80 rows where each part by itself is a stream of one tile of them and all parts together are not
+    (the measured times stand at parts_pay)"""
+    for M, rows, kp, one in ((300, (18944, 18944), 4352, True), (384, (18944, 18944), 4352, True), (600, (11008, 11008), 4352, True),
+                             (1500, (4096, 4096, 4096), 4352, True), (65, (28672, 28672), 8320, False), (80, (28672, 28672), 8320, False),
+                             (81, (28672, 28672), 8320, True), (128, (28672, 28672), 8320, True), (80, (38016, 38016), 4352, False),
+                             (64, (28672, 28672), 8320, True), (80, (18944, 18944), 4352, True), (200, (18944, 18944), 4352, True),
+                             (300, (14336, 14336), 4352, True), (2331, (3584, 512, 512), 3712, True), (2331, (18944, 18944), 3712, True)):
         assert layers.agemm.parts_pay(M, rows, kp, "NVFP4") == one, (M, rows)
         assert layers.agemm.parts_pay(M, rows, kp, "MXFP4")
     ran = []
