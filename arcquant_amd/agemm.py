@@ -316,7 +316,7 @@ def matmul_parts(A, B, SFA, SFB, scale, part_rows, part_scales, *, fmt, bias=Non
     the other (q | k | v), part_rows[k] rows each, with the tensor scales part_scales[k] (0-dim fp32 CUDA tensors); scale: the
     input's (float or 0-dim fp32 CUDA tensor).  bf16 [M, N], what torch.cat of the parts' ``matmul(..., (scale, part_scales[k]))`` is
     (sums in another order: one bf16 rounding at most), plus ``bias`` bf16 [N] where given, added in bf16.
-    swiglu=True (gate | up, no bias, where swiglu_halves_pay): matmul_swiglu(halves=True) of the two."""
+    swiglu=True (gate | up, no bias, where swiglu_halves_pay; others are refused): matmul_swiglu(halves=True) of the two."""
     _require(A, "A", torch.uint8, 2)
     _require(B, "B", torch.uint8, 2)
     _require(SFA, "SFA", torch.uint8)
@@ -361,6 +361,8 @@ def swiglu_halves_pay(M, N, Kp, fmt):
 
 
 def _swiglu_halves(A, SFA, B, SFB, M, N, Kp, f, tensor_scale, **kw):
+    if not swiglu_halves_pay(M, N, Kp, f):
+        raise RuntimeError(f"Value error in matmul_swiglu: no such epilogue for {M} x {N} x {Kp}")
     if (SFA.data_ptr() | SFB.data_ptr()) % 16:      # (a GEMM with one of the plain kernels takes them)
         return None
     T = torch.empty((M, N // 2), dtype=torch.bfloat16, device=A.device)
@@ -553,8 +555,9 @@ def matmul_swiglu(A, B, SFA, SFB, scale, *, fmt=None, tensor_scale=False, halves
     also returns the NVFP4 tensor scale max|t| / 2688 of t (0-dim fp32 device tensor, 1 for all zeros).
     halves=True: the weights as they are, gate rows and then up rows, for the problems that swiglu_halves_pay says; None where there is
     no memory for the scratch that such a GEMM takes, and for scale bytes that do not begin at a multiple of 16 (a slice of quantized
-    rows).  (Where its last round of tiles is cut along K, other columns are in it than in
-    matmul's, whose sums are then in another order.)"""
+    rows).  (The sums are matmul's, but NVFP4's are in another order where its last round
+    of tiles is cut along K, from K' = 8192 on, as other columns are in it, and MXFP4's with K' a multiple of 256 below 3840, which matmul may
+    have another kernel for.)"""
     _require(A, "A", torch.uint8, 2)
     _require(B, "B", torch.uint8, 2)
     _require(SFA, "SFA", torch.uint8)

@@ -247,7 +247,9 @@ class LlamaMLP(nn.Module):
     """SwiGLU MLP with gate and up projections fused into one [2*inter, hidden] linear
     (model/qLlamaLayer.py:380-443 with the fusion of benchmark configuration 4), followed by the fused
     SwiGLU -> quantize pass, or for many tokens (agemm.swiglu_halves_pay) by the quantizer alone, act_fn(gate) * up formed in the
-    GEMM's epilogue: the [tokens, 2*inter] projection output then never goes through memory; the same bits.  interleave=True
+    GEMM's epilogue: the [tokens, 2*inter] projection output then never goes through memory.  The same bits, but where the GEMM's fp32 sums are
+    in another order: NVFP4 with its last tiles cut along K (from K' = 8192 on), MXFP4 with K' a multiple of 256 below 3840, which other
+    kernels have without the epilogue, and gate and up that would run as two GEMMs (agemm.parts_pay).  interleave=True
     interleaves the fused weight's rows (gate_0, up_0, gate_1, ...), for which every GEMM has such an epilogue, as the MoE
     block's grouped GEMMs need it."""
 

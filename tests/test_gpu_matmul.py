@@ -677,6 +677,11 @@ def test_swiglu_of_weights_as_they_are_for_others(agemm, monkeypatch):
         pytest.skip("another kernel is forced")
     M, N, K = 2100, 6400, 512
     (x, w, idx, gx, gw), (a, sfa, b, sfb) = quantized_pair(agemm, M, N, K, 128, "NVFP4", seed=31)
+    few, scale, one = 64, torch.tensor(1.0, device="cuda"), torch.tensor(1.0, device="cuda")
+    with pytest.raises(RuntimeError):
+        agemm.matmul_swiglu(a[:few], b, sfa.view(M, -1)[:few].reshape(-1), sfb, 1.0, tensor_scale=True, halves=True)
+    with pytest.raises(RuntimeError):
+        agemm.matmul_parts(a[:few], b, sfa.view(M, -1)[:few].reshape(-1), sfb, one, (N // 2, N // 2), (scale, scale), fmt="NVFP4", swiglu=True)
     empty = torch.empty
 
     def full(*size, **kw):
