@@ -38,6 +38,7 @@ namespace {
 // and 2 g + 1 of the stage: their two scale bytes are half of a dword and picked by op_sel.
 // Requires K' % 128 == 0, K' >= 512.
 // ---------------------------------------------------------------------------------------------
+template <bool HALVES>
 __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
   constexpr int BT = 256;
   constexpr int kCodes = 2 * BT * 128, kScales = 2 * 2 * BT * 16;
@@ -72,11 +73,11 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
   const uint32_t ld_q = (lane & 7) ^ stage_swizzle(ld_row);   // (the swizzle has a period of 16 rows)
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    wvo[i] = (uint32_t)weight_row<128>(p, n_base, 64 * i + ld_row) * (uint32_t)kbytes + ld_q * 16;
+    wvo[i] = (uint32_t)weight_row<128, HALVES>(p, n_base, 64 * i + ld_row) * (uint32_t)kbytes + ld_q * 16;
     xvo[i] = (uint32_t)min(m_base + 64 * i + ld_row, p.M - 1) * (uint32_t)kbytes + ld_q * 16;
   }
   const uint8_t *sbase = group ? p.a_scales : p.b_scales;
-  const uint32_t svo = (uint32_t)(group ? min(m_base + 64 * pos + lane, p.M - 1) : weight_row<128>(p, n_base, 64 * pos + lane)) * (uint32_t)ksc;
+  const uint32_t svo = (uint32_t)(group ? min(m_base + 64 * pos + lane, p.M - 1) : weight_row<128, HALVES>(p, n_base, 64 * pos + lane)) * (uint32_t)ksc;
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(smem);
   // requests behind the last stage fetch it again into buffers that nobody reads any more: the number of loads on their
   // way is the same in every stage.  A short last stage is the row's last 256 elements, the first half of which the stage before it has.
@@ -248,14 +249,15 @@ __global__ __launch_bounds__(512) void gemm_mxfp4_pingpong(GemmParams p) {
   }
   if (s < ns) stage(s, std::integral_constant<int, 0>{});
   if (!group) barrier();
-  store_wave_tile(p, Acc16<8, 4>{acc}, reinterpret_cast<uint8_t *>(smem) + wave * kRegion, m_base + 64 * pos, n_base + 128 * group, lane);
+  store_wave_tile<HALVES>(p, Acc16<8, 4>{acc}, reinterpret_cast<uint8_t *>(smem) + wave * kRegion, m_base + 64 * pos, n_base + 128 * group, lane);
 }
 
 }  // namespace
 
 int run_mxfp4_pingpong(const GemmParams &p, hipStream_t st) {
   const int total = ((p.M + 255) / 256 + (p.seg ? p.n_seg : 0)) * ((p.N + 255) / 256);
-  hipLaunchKernelGGL(gemm_mxfp4_pingpong, dim3(p.seg ? grid_in_turn<32>(total) : grid_in_turn<1>(total)), dim3(512), 0, st, p);
+  const auto kernel = p.swiglu == kSwigluHalves ? gemm_mxfp4_pingpong<true> : gemm_mxfp4_pingpong<false>;
+  hipLaunchKernelGGL(kernel, dim3(p.seg ? grid_in_turn<32>(total) : grid_in_turn<1>(total)), dim3(512), 0, st, p);
   ARCQ_HIP_TRY(hipGetLastError());
   return ARCQ_OK;
 }

@@ -98,7 +98,7 @@ __device__ __forceinline__ void f16_tile_at(const GemmParams &p, int lin, int &c
 }
 
 // The tile at (c_base, f_base), nk steps of 64 elements from step u0 on (both even): the tile of C, or with `partial` the fp32 sums.
-template <bool CODES_W, int TF>
+template <bool CODES_W, int TF, bool HALVES>
 __device__ __forceinline__ void f16_tile_of(const GemmParams &p, int c_base, int f_base, int u0, int nk, float4 *partial, uint8_t *smem, int tid) {
   using S = F16Shape<CODES_W, TF>;
   constexpr int BC = S::BC, BF = S::BF, FI = S::FI, FA = S::FA, kF = S::kF, kC = S::kC, kRegion = S::kRegion;
@@ -114,14 +114,14 @@ __device__ __forceinline__ void f16_tile_of(const GemmParams &p, int c_base, int
 #pragma unroll
   for (int i = 0; i < FI; ++i) {
     const int row = 64 * i + 8 * wave + (lane >> 3);
-    fvo[i] = (uint32_t)(CODES_W ? min(f_base + row, rows_f - 1) : weight_row<16 * TF>(p, f_base, row)) * (uint32_t)fbytes + (((lane & 7) ^ stage_swizzle(row)) << 4);
+    fvo[i] = (uint32_t)(CODES_W ? min(f_base + row, rows_f - 1) : weight_row<16 * TF, HALVES>(p, f_base, row)) * (uint32_t)fbytes + (((lane & 7) ^ stage_swizzle(row)) << 4);
   }
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int row = 128 * i + 16 * wave + (lane >> 2);
-    cvo[i] = (uint32_t)(CODES_W ? weight_row<64>(p, c_base, row) : min(c_base + row, rows_c - 1)) * (uint32_t)kbytes + (((lane & 3) ^ ((row >> 2) & 3)) << 4);
+    cvo[i] = (uint32_t)(CODES_W ? weight_row<64, HALVES>(p, c_base, row) : min(c_base + row, rows_c - 1)) * (uint32_t)kbytes + (((lane & 3) ^ ((row >> 2) & 3)) << 4);
   }
-  svo = (uint32_t)(CODES_W ? weight_row<64>(p, c_base, 64 * cpos + lane) : min(c_base + 64 * cpos + lane, rows_c - 1)) * (uint32_t)ksc + 4 * group;
+  svo = (uint32_t)(CODES_W ? weight_row<64, HALVES>(p, c_base, 64 * cpos + lane) : min(c_base + 64 * cpos + lane, rows_c - 1)) * (uint32_t)ksc + 4 * group;
   const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>(smem);
   const uint8_t *f16 = reinterpret_cast<const uint8_t *>(p.f16) + (size_t)u0 * 128;
   // (requests behind the last step fetch it again, into stages that nobody reads any more: the number of loads on their
@@ -269,28 +269,31 @@ __device__ __forceinline__ void f16_tile_of(const GemmParams &p, int c_base, int
   }
   uint8_t *region = smem + wave * kRegion;
   if constexpr (CODES_W)
-    store_wave_tile(p, Acc16<4, TF>{acc}, region, f_base + 16 * TF * group, c_base + 64 * cpos, lane);
+    store_wave_tile<HALVES>(p, Acc16<4, TF>{acc}, region, f_base + 16 * TF * group, c_base + 64 * cpos, lane);
   else
-    store_wave_tile(p, Acc16<TF, 4>{acc}, region, c_base + 64 * cpos, f_base + 16 * TF * group, lane);
+    store_wave_tile<HALVES>(p, Acc16<TF, 4>{acc}, region, c_base + 64 * cpos, f_base + 16 * TF * group, lane);
 }
 
 // The last rows of a problem or of an expert's: a tile of fewer fp16 rows, whose phases are shorter (the sums are the same).  Zipf-like
 // experts, 8192 rows over eight of 28672 x 4224 with the SwiGLU epilogue: 1616 us with whole tiles alone, 1595 so; 333 x 28672 x 4352:
 // 96 and 85.
-template <bool CODES_W, int TF>
+template <bool CODES_W, int TF, bool HALVES, bool SMALL>
 __device__ __forceinline__ void f16_tile(const GemmParams &p, int lin, int u0, int nk, float4 *partial, uint8_t *smem, int tid) {
   int c_base, f_base;
   f16_tile_at<CODES_W, TF>(p, lin, c_base, f_base);
-  if constexpr (CODES_W) {
+  if constexpr (CODES_W && SMALL) {
     const int left = p.M - f_base;
-    if (TF > 2 && left <= 64) return f16_tile_of<CODES_W, 2>(p, c_base, f_base, u0, nk, partial, smem, tid);
-    if (TF > 4 && left <= 128) return f16_tile_of<CODES_W, 4>(p, c_base, f_base, u0, nk, partial, smem, tid);
-    if (TF > 6 && left <= 192) return f16_tile_of<CODES_W, 6>(p, c_base, f_base, u0, nk, partial, smem, tid);
+    if (TF > 2 && left <= 64) return f16_tile_of<CODES_W, 2, HALVES>(p, c_base, f_base, u0, nk, partial, smem, tid);
+    if (TF > 4 && left <= 128) return f16_tile_of<CODES_W, 4, HALVES>(p, c_base, f_base, u0, nk, partial, smem, tid);
+    if (TF > 6 && left <= 192) return f16_tile_of<CODES_W, 6, HALVES>(p, c_base, f_base, u0, nk, partial, smem, tid);
   }
-  f16_tile_of<CODES_W, TF>(p, c_base, f_base, u0, nk, partial, smem, tid);
+  f16_tile_of<CODES_W, TF, HALVES>(p, c_base, f_base, u0, nk, partial, smem, tid);
 }
 
-template <bool CODES_W, int TF>
+// HALVES, and SMALL (a problem with rows for a smaller last tile, or experts, which may have some): what a launch does not need is not in its
+// kernel, 39 KB of code for 256 rows with neither, against 177 KB with every epilogue and height in one.  us, that one and so: 2048 x 16384 x 512 44.1,
+// 43.0, 4096 x 16384 x 640 90.8, 88.7, 640 x 28672 x 1152 48.2, 47.7.
+template <bool CODES_W, int TF, bool HALVES, bool SMALL>
 __global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
   using S = F16Shape<CODES_W, TF>;
   __shared__ uint4 smem[(S::kF + S::kC + S::kS) / 16];
@@ -302,7 +305,7 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_f16(GemmParams p) {
     lin = (blockIdx.x & 7) * ((total + 7) >> 3) + (blockIdx.x >> 3);
     if (lin >= total) return;
   }
-  f16_tile<CODES_W, TF>(p, lin, 0, p.Kp >> 6, nullptr, reinterpret_cast<uint8_t *>(smem), threadIdx.x);
+  f16_tile<CODES_W, TF, HALVES, SMALL>(p, lin, 0, p.Kp >> 6, nullptr, reinterpret_cast<uint8_t *>(smem), threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -346,7 +349,7 @@ __device__ __forceinline__ bool f16_enter(GemmParams &p, int &lin) {
   return segments.enter(p, lin);
 }
 
-template <bool CODES_W>
+template <bool CODES_W, bool HALVES>
 __global__ __launch_bounds__(512) void gemm_nvfp4_f16_split(GemmParams p) {
   using S = F16Shape<CODES_W>;
   __shared__ uint4 smem[(S::kF + S::kC + S::kS) / 16];
@@ -375,13 +378,13 @@ __global__ __launch_bounds__(512) void gemm_nvfp4_f16_split(GemmParams p) {
     wait_dma_and_sync();  // the LDS of the part before this one
     int tid = threadIdx.x;
     asm volatile("" : "+v"(tid));  // what follows from it is formed per part: hoisted out of this loop it would be spilled
-    f16_tile<CODES_W, 8>(q, lin, 2 * first, 2 * n, partial, reinterpret_cast<uint8_t *>(smem), tid);
+    f16_tile<CODES_W, 8, HALVES, true>(q, lin, 2 * first, 2 * n, partial, reinterpret_cast<uint8_t *>(smem), tid);
     at += n;
   }
 }
 
 // a wave per eighth of a tile
-template <bool CODES_W, int TF>
+template <bool CODES_W, int TF, bool HALVES>
 __device__ __forceinline__ void f16_add_parts(const GemmParams &p, const LastRound &r, int w0, int w1, int c_base, int f_base, uint8_t *region) {
   using S = F16Shape<CODES_W, TF>;
   const int lane = threadIdx.x, wave = blockIdx.x & 7, cpos = wave & 3, group = wave >> 2;
@@ -402,12 +405,12 @@ __device__ __forceinline__ void f16_add_parts(const GemmParams &p, const LastRou
       }
   }
   if constexpr (CODES_W)
-    store_wave_tile(p, Acc16<4, TF>{acc}, region, f_base + 16 * TF * group, c_base + 64 * cpos, lane);
+    store_wave_tile<HALVES>(p, Acc16<4, TF>{acc}, region, f_base + 16 * TF * group, c_base + 64 * cpos, lane);
   else
-    store_wave_tile(p, Acc16<TF, 4>{acc}, region, c_base + 64 * cpos, f_base + 16 * TF * group, lane);
+    store_wave_tile<HALVES>(p, Acc16<TF, 4>{acc}, region, c_base + 64 * cpos, f_base + 16 * TF * group, lane);
 }
 
-template <bool CODES_W>
+template <bool CODES_W, bool HALVES>
 __global__ __launch_bounds__(64) void f16_split_add_kernel(GemmParams p) {
   using S = F16Shape<CODES_W>;
   __shared__ uint4 smem[S::kRegion / 16];
@@ -422,29 +425,31 @@ __global__ __launch_bounds__(64) void f16_split_add_kernel(GemmParams p) {
   uint8_t *region = reinterpret_cast<uint8_t *>(smem);
   if constexpr (CODES_W) {  // as f16_tile
     const int left = p.M - f_base;
-    if (left <= 64) return f16_add_parts<CODES_W, 2>(p, r, w0, w1, c_base, f_base, region);
-    if (left <= 128) return f16_add_parts<CODES_W, 4>(p, r, w0, w1, c_base, f_base, region);
-    if (left <= 192) return f16_add_parts<CODES_W, 6>(p, r, w0, w1, c_base, f_base, region);
+    if (left <= 64) return f16_add_parts<CODES_W, 2, HALVES>(p, r, w0, w1, c_base, f_base, region);
+    if (left <= 128) return f16_add_parts<CODES_W, 4, HALVES>(p, r, w0, w1, c_base, f_base, region);
+    if (left <= 192) return f16_add_parts<CODES_W, 6, HALVES>(p, r, w0, w1, c_base, f_base, region);
   }
-  f16_add_parts<CODES_W, 8>(p, r, w0, w1, c_base, f_base, region);
+  f16_add_parts<CODES_W, 8, HALVES>(p, r, w0, w1, c_base, f_base, region);
 }
 
-template <bool CODES_W, int TF>
+template <bool CODES_W, int TF, bool HALVES>
 int launch_tiles(const GemmParams &p, hipStream_t st) {
   using S = F16Shape<CODES_W, TF>;
-  const int total = ((p.M + S::BM - 1) / S::BM + (p.seg ? p.n_seg : 0)) * ((p.N + S::BN - 1) / S::BN);
-  hipLaunchKernelGGL((gemm_nvfp4_f16<CODES_W, TF>), dim3(p.seg ? grid_in_turn<32>(total) : grid_in_turn<1>(total)), dim3(512), 0, st, p);
+  const int total = ((p.M + S::BM - 1) / S::BM + (p.seg ? p.n_seg : 0)) * ((p.N + S::BN - 1) / S::BN), left = p.M % S::BM;
+  const bool small = CODES_W && (p.seg || (left > 0 && left <= S::BM - 64));
+  const auto kernel = small ? gemm_nvfp4_f16<CODES_W, TF, HALVES, CODES_W> : gemm_nvfp4_f16<CODES_W, TF, HALVES, false>;
+  hipLaunchKernelGGL(kernel, dim3(p.seg ? grid_in_turn<32>(total) : grid_in_turn<1>(total)), dim3(512), 0, st, p);
   ARCQ_HIP_TRY(hipGetLastError());
   return ARCQ_OK;
 }
 
-template <bool CODES_W>
+template <bool CODES_W, bool HALVES>
 int launch_split(const GemmParams &p, hipStream_t st) {
   const int total = ((p.M + 255) / 256 + (p.seg ? p.n_seg : 0)) * ((p.N + 255) / 256);
   const int grid = ((total + 7) / 8) * 8;
-  hipLaunchKernelGGL((gemm_nvfp4_f16_split<CODES_W>), dim3(grid + 256), dim3(512), 0, st, p);
+  hipLaunchKernelGGL((gemm_nvfp4_f16_split<CODES_W, HALVES>), dim3(grid + 256), dim3(512), 0, st, p);
   ARCQ_HIP_TRY(hipGetLastError());
-  hipLaunchKernelGGL((f16_split_add_kernel<CODES_W>), dim3(8 * std::min(total, 255)), dim3(64), 0, st, p);
+  hipLaunchKernelGGL((f16_split_add_kernel<CODES_W, HALVES>), dim3(8 * std::min(total, 255)), dim3(64), 0, st, p);
   ARCQ_HIP_TRY(hipGetLastError());
   return ARCQ_OK;
 }
@@ -505,12 +510,14 @@ int run_nvfp4_f16(GemmParams p, void *workspace, hipStream_t st, bool split) {
                      static_cast<uint4 *>(workspace), dwords);
   ARCQ_HIP_TRY(hipGetLastError());
   p.f16 = static_cast<const uint16_t *>(workspace);
-  if (split) {
-    p.split = reinterpret_cast<float4 *>(static_cast<uint8_t *>(workspace) + nvfp4_split_operand_bytes(p.M, p.N, p.Kp, p.seg != nullptr));
-    return plan.codes_w ? launch_split<true>(p, st) : launch_split<false>(p, st);
-  }
-  if (!plan.codes_w) return launch_tiles<false, 8>(p, st);
-  return plan.tf == 8 ? launch_tiles<true, 8>(p, st) : plan.tf == 6 ? launch_tiles<true, 6>(p, st) : launch_tiles<true, 4>(p, st);
+  if (split) p.split = reinterpret_cast<float4 *>(static_cast<uint8_t *>(workspace) + nvfp4_split_operand_bytes(p.M, p.N, p.Kp, p.seg != nullptr));
+  auto launch = [&](auto halves) {
+    constexpr bool HALVES = decltype(halves)::value;
+    if (split) return plan.codes_w ? launch_split<true, HALVES>(p, st) : launch_split<false, HALVES>(p, st);
+    if (!plan.codes_w) return launch_tiles<false, 8, HALVES>(p, st);
+    return plan.tf == 8 ? launch_tiles<true, 8, HALVES>(p, st) : plan.tf == 6 ? launch_tiles<true, 6, HALVES>(p, st) : launch_tiles<true, 4, HALVES>(p, st);
+  };
+  return p.swiglu == kSwigluHalves ? launch(std::true_type{}) : launch(std::false_type{});
 }
 
 }  // namespace arcq

@@ -346,9 +346,9 @@ struct Acc16 {  // v_mfma_*_16x16x*: element e of a lane is n = 4 (lane / 16) + 
 };
 
 // Row of the weights that local row `row` of the tile at n_base holds, kN of them to a wave.
-template <int kN>
+template <int kN, bool HALVES>
 __device__ __forceinline__ int weight_row(const GemmParams &p, int n_base, int row) {
-  if (p.swiglu != kSwigluHalves) return min(n_base + row, p.N - 1);
+  if (!HALVES) return min(n_base + row, p.N - 1);
   const int o = row % kN, F = p.N >> 1;
   return min((n_base >> 1) + row / kN * (kN / 2) + o % (kN / 2), F - 1) + (o >= kN / 2 ? F : 0);
 }
@@ -500,12 +500,11 @@ __device__ __forceinline__ void store_tile(const GemmParams &p, const Acc &acc, 
 // Epilogue shared by the tiled kernels, called by every wave of the workgroup (there is a barrier in it).  m0 / n0: first row /
 // column of C of this wave's tile.  region: 2 * kM * kN bytes of LDS of this wave's own, free for reuse once every wave is done
 // reading operands.
-template <class Acc>
+template <bool HALVES = false, class Acc>
 __device__ __forceinline__ void store_wave_tile(const GemmParams &p, const Acc &acc, uint8_t *region, int m0, int n0, int lane) {
-  if constexpr (Acc::kSide == 16)
-    if (p.swiglu == kSwigluHalves) return store_wave_tile_halves(p, acc, region, m0, n0 >> 1, lane);
+  if constexpr (HALVES) return store_wave_tile_halves(p, acc, region, m0, n0 >> 1, lane);
   if (p.swiglu) return store_wave_tile_swiglu(p, acc, region, m0, n0, lane);
-  if (p.partial) {  // split-K: the unscaled fp32 tile of this K range
+  if (Acc::kSide == 32 && p.partial) {  // split-K: the unscaled fp32 tile of this K range
     float *part = p.partial + (size_t)blockIdx.y * p.M * p.N;
     const bool quads = (p.N & 3) == 0, inside = quads && n0 + Acc::kN <= p.N;
 #pragma unroll
