@@ -328,8 +328,11 @@ class LlamaAttention(nn.Module):
         self.quant_type = quant_type
         self._rope = None                    # cos / sin tables of the fused rotary embedding, built on first use
 
-    def _rotated(self, rows, q_len):
-        q, tables = rows[0], rows[1:]
+    def _rotated(self, q, q_len):
+        """the queries handed to the attention as [batch, heads, tokens, head_dim]: rotated already, or (rows, cos, sin)"""
+        if not isinstance(q, tuple):
+            return q.view(-1, q_len, self.num_heads, self.head_dim).transpose(1, 2)
+        q, *tables = q
         return _kvc.rope(q, q_len, 0, self.num_heads, 0, *tables)[0].view(-1, q_len, self.num_heads, self.head_dim).transpose(1, 2)
 
     @_no_grad
@@ -357,12 +360,18 @@ class LlamaAttention(nn.Module):
                 self._rope = _kvc.rope_tables(max(need, 4096), d, qkv.dtype, qkv.device)
             flat = qkv.view(bsz * q_len, -1)
             # a prompt's own keys, read where they are (one token sees itself alone: torch's kernel for it, 64 sequences of 28 heads 6.7
-            # us, has not 128 queries' work, 16.9); the queries are then rotated by the attention, and only the keys here
-            if past_len == 0 and q_len > 1 and not isinstance(kv_cache, tuple) and _plain(flat, *self._rope):
+            # us, has not 128 queries' work, 16.9)
+            prompt = past_len == 0 and q_len > 1 and not isinstance(kv_cache, tuple) and _plain(flat, *self._rope)
+            if prompt and q_len >= 32 and bsz * q_len * nh >= 8192:
+                # The attention rotates the queries, and only the keys are rotated here: in tiles of 128 queries of a head, however few of them
+                # there are, ahead of a tile's products (us, both rotated in one pass and so, 32 heads: 1 x 100 tokens 10.6, 11.6, 64 x 8 26.6,
+                # 30.2; 4 x 64 10.4, 10.2, 1 x 300 16.2, 15.2, 8 x 100 17.0, 14.3, 8 x 2048 413, 367; 8 heads, 1 x 300 14.3, 14.5)
                 k = _kvc.rope(flat[:, nh * d:(nh + nkv) * d], q_len, 0, nkv, 0, *self._rope)[0]
                 rows = ((flat[:, :nh * d], *self._rope), k, flat[:, (nh + nkv) * d:(nh + 2 * nkv) * d])
             else:
                 q, k = _kvc.rope(flat, q_len, past_len, nh, nkv, *self._rope)
+                if prompt:
+                    rows = (q, k, flat[:, (nh + nkv) * d:(nh + 2 * nkv) * d])
                 q = q.view(bsz, q_len, nh, d).transpose(1, 2)
             k = k.view(bsz, q_len, nkv, d).transpose(1, 2)
         else:

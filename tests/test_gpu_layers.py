@@ -769,3 +769,38 @@ def test_mlp_of_a_slice_of_quantized_tokens(layers, monkeypatch, fmt, split):
     assert torch.equal(mlp(sliced), y)
     aligned = (sliced[0], sliced[1].clone(), scale, None, tokens)
     assert rel_fro(mlp(aligned), y) < 2e-2                  # other kernels' sums: a few codes of t move
+
+
+@pytest.mark.parametrize("batch,tokens,heads,rotates", [(3, 31, 4, False), (2, 127, 32, False), (2, 128, 32, True), (512, 16, 4, False), (64, 32, 4, True)])
+@pytest.mark.parametrize("paged", [False, True])
+def test_prompt_queries_are_rotated_where_that_is_faster(layers, monkeypatch, batch, tokens, heads, rotates, paged):
+    """short prompts rotate queries and keys in one pass, others leave the queries to the attention: the same bits, and those of the rotary pass
+    with torch's attention up to its bf16 probabilities"""
+    from arcquant_amd.kv_cache import MultiLayerPagedKVCache4Bit
+    kv_heads, hidden = 2, heads * 128
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    attn = layers.LlamaAttention.__new__(layers.LlamaAttention)
+    nn.Module.__init__(attn)
+    attn.num_heads, attn.num_kv_heads, attn.head_dim, attn._rope, attn.quant_type = heads, kv_heads, 128, None, "MXFP4"
+    qkv = torch.randn(batch, tokens, (heads + 2 * kv_heads) * 128, generator=g, device="cuda").to(torch.bfloat16)
+    attn.qkv_proj = lambda x: qkv
+    out = lambda t, residual: t
+    out.select_num = 0
+    object.__setattr__(attn, "o_proj", out)
+    attn.o_reorder_index = None
+    monkeypatch.setattr(layers, "quantize_tokens", lambda t, *a: t)
+    seen, own = [], layers._kvc.attention_prefill
+    monkeypatch.setattr(layers._kvc, "attention_prefill", lambda q, k, v, n: seen.append(isinstance(q, tuple)) or own(q, k, v, n))
+
+    def run():
+        cache = MultiLayerPagedKVCache4Bit(batch, 16, tokens + 16, "cuda", 1, kv_heads, 128, dtype=torch.bfloat16) if paged else None
+        return attn((None, None, None, batch, tokens), cache).view(batch * tokens, hidden)
+
+    y = run()
+    assert seen == [rotates]
+    flat = qkv.view(batch * tokens, -1)
+    tables = attn._rope
+    q, k = layers._kvc.rope(flat, tokens, 0, heads, kv_heads, *tables)
+    assert torch.equal(y, own(q, k, flat[:, (heads + kv_heads) * 128:], tokens))
+    monkeypatch.setattr(layers, "_plain", lambda *a: False)             # torch's attention
+    assert rel_fro(run(), y) < 1e-2 and len(seen) == 1
