@@ -136,6 +136,12 @@ struct Segments {
     }
   }
 
+  // (up to 64 segments) much the same rows in each: one 16-row tile of an MFMA at most, or no more than one and a half times the average
+  __device__ __forceinline__ bool even(int n_seg) const {
+    const int most = __builtin_amdgcn_readlane(wave_prefix<true>(end - beg), 63);
+    return most <= 16 || 2l * most * n_seg <= 3l * (__builtin_amdgcn_readlane(end, 63) - first);
+  }
+
   // Turns p into the problem of the segment that tile lin belongs to, lin into the tile's number inside it; false past the end.
   // (Up to 64 segments the constructor's one read still holds; beyond, p is read anew, so it has to be the launch's own.)
   __device__ __forceinline__ bool enter(GemmParams &p, int &lin) {
@@ -205,16 +211,17 @@ __device__ __forceinline__ bool enter_segment_in_runs(GemmParams &p, int &lin) {
   return segments.enter(p, lin);
 }
 
-// Small tiles: in twos (those of an expert's first and second rows, which share their weights).  A few narrow experts with a long K' keep one
-// run per XCD: there are one or two tiles per slot, and which of them come last decides more than the XCDs' shares.  us, one run per XCD and in
-// twos, even sizes, Zipf-like ones and those in reverse: 128 rows over eight of 28672 x 4224 118, 129, 128 / 117, 124, 127, 200 rows 126, 144, 145 /
-// 124, 133, 136; 1024 over 64 of 2048 x 1536 31.7, 44.2, 44.1 / 30.9, 35.9, 37.9; over eight of 4096 x 14464 128 rows 55.4, 85, 84.8 / 56.1, 82.6, 91.5, 320
-// rows 70.5, 91.7, 98.7 / 70.1, 84.5, 101.3.
+// Small tiles: in twos (those of an expert's first and second rows, which share their weights).  A few narrow experts with a long K' and much
+// the same rows keep one run per XCD, which then has an expert or two and their activations to itself.  us, one run per XCD, in twos, and so, even
+// sizes, Zipf-like ones, those in reverse and top-2 of skewed scores: 128 rows over eight of 28672 x 4224 118, 129, 129, 139 / 117, 123, 126, 120, of 4096 x
+// 14464 55.2, 84.1, 84.3, 68.7 / 55.8, 82.2, 92.2, 57.3 / 55.3, 82.3, 92.1, 57.5, of 8192 x 14464 99.6, 132, 132, 134 / 109, 127, 145, 113 / 99.9, 127, 146, 114.
+// (Sizes that grow from expert to expert are the ones that lose: their longest tiles come last.  With the experts sorted, 7 to 10 % are lost on
+// 16 even ones, whose XCDs then share all of them.)
 template <int BM, int BN, int G>
 __device__ __forceinline__ bool enter_segment_in_twos(GemmParams &p, int &lin) {
   Segments<BM, BN, G> segments(p);
   const int of_xcd = blockIdx.x >> 3, xcd = blockIdx.x & 7;
-  if (p.Kp >= 8192 && p.N <= 4096) {
+  if (p.Kp >= 8192 && p.N <= 8192 && p.n_seg <= 16 && segments.even(p.n_seg)) {
     const int per_xcd = (segments.total + 7) >> 3;
     if (of_xcd >= per_xcd) return false;
     lin = xcd * per_xcd + of_xcd;
