@@ -272,12 +272,11 @@ class LlamaMLP(nn.Module):
 
     def _activation(self, x):
         """act_fn(gate) * up straight from the projection's epilogue, NVFP4 with its tensor scale; None where the projection is called
-        by itself: few tokens, hooks or another forward on it, another format or other sizes than the MLP's, a bias, no memory,
+        by itself: hooks or another forward on it, another format or other sizes than the MLP's, a bias, no memory,
         unaligned scale bytes"""
         qx, scale_x, scale, _, _ = x
         p, nv = self.gate_up_proj, self.quant_type == "NVFP4"
-        if qx.dim() != 2 or not isinstance(scale, (float, int, torch.Tensor)) or \
-                not agemm.swiglu_halves_pay(qx.shape[0], 2 * self.inter, 2 * qx.shape[1], self.quant_type):
+        if not isinstance(scale, (float, int, torch.Tensor)):
             return None
         if _unhooked(p, SplitQLinear):
             ours = all(getattr(q, "quant_type", None) == self.quant_type and q.out_features == self.inter for q in p.parts)
@@ -298,7 +297,9 @@ class LlamaMLP(nn.Module):
                                                global_scale=scale if nv else None)
             return self.down_proj((qx, sfx, scale, x[3], x[4]), residual)
         if self.inter <= 32736 and self.inter % 32 == 0:
-            t = self._activation(x) if x[0].shape[0] > 64 else None
+            rows = x[0].shape
+            t = self._activation(x) if rows[0] > 64 and len(rows) == 2 and \
+                agemm.swiglu_halves_pay(rows[0], 2 * self.inter, 2 * rows[1], self.quant_type) else None
             if t is not None:
                 scale = t[1] if isinstance(t, tuple) else 1.0
                 t = t[0] if isinstance(t, tuple) else t
