@@ -363,10 +363,11 @@ class LlamaAttention(nn.Module):
             # a prompt's own keys, read where they are (one token sees itself alone: torch's kernel for it, 64 sequences of 28 heads 6.7
             # us, has not 128 queries' work, 16.9)
             prompt = past_len == 0 and q_len > 1 and not isinstance(kv_cache, tuple) and _plain(flat, *self._rope)
-            if prompt and q_len >= 32 and bsz * q_len * nh >= 8192:
+            if prompt and q_len >= 32 and bsz * q_len * nh >= 32768:
                 # The attention rotates the queries, and only the keys are rotated here: in tiles of 128 queries of a head, however few of them
-                # there are, ahead of a tile's products (us, both rotated in one pass and so, 32 heads: 1 x 100 tokens 10.6, 11.6, 64 x 8 26.6,
-                # 30.2; 4 x 64 10.4, 10.2, 1 x 300 16.2, 15.2, 8 x 100 17.0, 14.3, 8 x 2048 413, 367; 8 heads, 1 x 300 14.3, 14.5)
+                # there are, ahead of a tile's products, and for 5 us more of the host's time, which a layer of fewer tokens waits for (us, both
+                # rotated in one pass and so, 32 heads: 64 x 8 tokens 26.6, 30.2, 1 x 300 16.2, 15.2, 4 x 256 23.1, 17.7, 1 x 1000 41.8, 34.5, 8 x
+                # 2048 413, 367; the host's: 22.5, 28)
                 k = _kvc.rope(flat[:, nh * d:(nh + nkv) * d], q_len, 0, nkv, 0, *self._rope)[0]
                 rows = ((flat[:, :nh * d], *self._rope), k, flat[:, (nh + nkv) * d:(nh + 2 * nkv) * d])
             else:

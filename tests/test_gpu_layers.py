@@ -771,7 +771,7 @@ def test_mlp_of_a_slice_of_quantized_tokens(layers, monkeypatch, fmt, split):
     assert rel_fro(mlp(aligned), y) < 2e-2                  # other kernels' sums: a few codes of t move
 
 
-@pytest.mark.parametrize("batch,tokens,heads,rotates", [(3, 31, 4, False), (2, 127, 32, False), (2, 128, 32, True), (512, 16, 4, False), (64, 32, 4, True)])
+@pytest.mark.parametrize("batch,tokens,heads,rotates", [(3, 33, 4, False), (1, 1023, 32, False), (1, 1024, 32, True), (512, 16, 4, False), (256, 32, 4, True)])
 @pytest.mark.parametrize("paged", [False, True])
 def test_prompt_queries_are_rotated_where_that_is_faster(layers, monkeypatch, batch, tokens, heads, rotates, paged):
     """short prompts rotate queries and keys in one pass, others leave the queries to the attention: the same bits, and those of the rotary pass
