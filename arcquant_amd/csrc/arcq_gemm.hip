@@ -1277,7 +1277,7 @@ int check_gemm_args(const void *a_codes, const void *a_scales, const void *b_cod
 // Its tile is 256 weight rows x 256, 192 or 128 activation rows (f16_plan), one workgroup per CU, and a round of tiles takes the same
 // time however few there are (K' = 4352, 256 rows: 75-98 us).  The kernels without a workspace are faster as long as their 256x128 tiles fit one round (K' = 4352, without and
 // with: 2048 x 4096 66 / 84 us, 1024 x 6144 55 / 82), and slower beyond (257 x 28672 100 / 98, 65 x 128256 241 / 239,
-// 1400 x 6144 115 / 68, 2331 x 4096 113 / 74, 4096 x 28672 832 / 682; K' = 14592, 4096 x 4096 360 / 328; K' = 1152,
+// 1400 x 6144 115 / 68, 2331 x 4096 113 / 74, 4096 x 28672 832 / 675; K' = 14592, 4096 x 4096 360 / 328; K' = 1152,
 // 200 x 33024 44 / 34).  So are the plan's 256x256 tiles, for up to 128 rows on layers of more than 49000 columns (100 x 53248,
 // K' = 512, 1152: 20.5, 38.8 / 15.3, 24.2; 128 x 57344 x 4352 101 / 67).
 bool nvfp4_f16_wanted(int M, int N, int Kp, int fmt, int n_seg) {

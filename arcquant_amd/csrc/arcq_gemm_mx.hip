@@ -26,7 +26,8 @@ namespace {
 //
 // The matrix instruction is 16x16x128: a register-only loop of it sustains 7.0-7.2 PFLOP/s on random codes against 5.8-6.3 for
 // 32x32x64 (one and two waves per SIMD, arcq_mfma_rate_probe), the upper figure when the tiles are walked back and forth, so
-// that neighbouring instructions share an operand.  4096 x 4096 x 14592: 102-105 us, 4.6-4.8 PFLOP/s, one round of tiles.
+// that neighbouring instructions share an operand.  4096 x 4096 x 14592, one round of tiles: 102-107 us, 4.6-4.8 PFLOP/s, once the
+// clock is up; 110-120 us in the first milliseconds after a pause.
 //
 // A stage has two phases: all activations with weight rows 0-63 of the wave, then with rows 64-127.  The activations and
 // the first half of the weights leave LDS in the first phase, so their buffers are requested again in the second one: two

@@ -53,7 +53,7 @@ __global__ __launch_bounds__(256) void nvfp4_decode_f16_kernel(const uint32_t *c
 // of an odd step that also requests codes and scale bytes the longest of all; so the decoding goes between the MFMAs, which leave
 // room for one VALU instruction each, and the requests are spread (4 of 8 KB or less per phase at most).  us, decoding and the requests of
 // codes in the memory phases, and so: 2331 x 3584 x 19072 with TF = 6 316 and 262; 2048 x 2048 x 14592 with TF = 8 266 and 244
-// (its MFMAs and barriers alone: 216), 16384 x 28672 x 4352 2740 and 2630, where all CUs are busy and the clock gives way.  Neither more
+// (its MFMAs and barriers alone: 216), 16384 x 28672 x 4352 2715 and 2645, where all CUs are busy and the clock gives way.  Neither more
 // stages on their way nor lines fetched into L2 ahead nor requests between the MFMAs, fewer barriers or raised wave
 // priority are faster.
 //

@@ -2,6 +2,8 @@
 restated with the torch oracle on the CPU: same quantizers (bit-exact, see test_gpu_quantize.py),
 so what remains is GEMM accumulation order and bf16 roundings between ops.  Tolerances are
 relative Frobenius errors, written at each comparison."""
+import os
+
 import pytest
 import torch
 import torch.nn as nn
@@ -740,6 +742,7 @@ def test_mlp_of_many_tokens(layers, monkeypatch, fmt, tokens, split):
     assert torch.equal(mlp(x, residual=res), fused) and len(called) == 1
 
 
+@pytest.mark.skipif("ARCQ_GEMM_KERNEL" in os.environ, reason="another kernel is forced")
 @pytest.mark.parametrize("fmt", FMTS)
 @pytest.mark.parametrize("split", [False, True])
 def test_mlp_of_a_slice_of_quantized_tokens(layers, monkeypatch, fmt, split):
